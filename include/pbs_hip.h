@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 4
+#define PBS_ABI_VERSION 5
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -73,7 +73,8 @@ int pbs_build_indices(const uint8_t* mask, const int64_t* block_ptr, int X, int 
  * changed and pass it to every pbs_blocksparse_matmul call of that direction.  It is what the
  * reference's kernel derives again in every thread block from ptr/indices
  * (cutlass/gemm/block_loader_crosswise_prune_dense.h:254-264, :398-444), hoisted out of the hot
- * path: per group of 8 result block columns, the merged list of k-blocks they touch.
+ * path: per result block column the list of its blocks, longest column first, and, for the bf16 kernels
+ * with shared operand panels, the merged lists of groups of 16 columns.
  *
  *   transpose = 1 (forward):        ptr = row_start_ends_a, indices = cols_a, n = out, k = in
  *   transpose = 0 (input gradient): ptr = col_start_ends_b, indices = rows_b, n = in,  k = out
@@ -82,6 +83,19 @@ int pbs_build_indices(const uint8_t* mask, const int64_t* block_ptr, int X, int 
 size_t pbs_blocksparse_matmul_plan_bytes(int n, int k);
 int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz,
                                 void* plan, size_t plan_bytes, void* stream);
+
+/*
+ * The plan in parts, for callers whose pattern changes often: a product reads one part only, and the first
+ * (PBS_PLAN_LIST, one launch) is all that fp32 and small bf16 products need.  `part` is a sum of PBS_PLAN_*;
+ * pbs_blocksparse_matmul_part() tells which part a product of these sizes reads, given whether the call has a
+ * workspace.  PBS_PLAN_LIST has to be there in any case.  pbs_blocksparse_matmul_plan builds everything.
+ */
+#define PBS_PLAN_LIST 1
+#define PBS_PLAN_WIDE 2
+#define PBS_PLAN_COLUMN 4
+int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, int part,
+                                     void* plan, size_t plan_bytes, void* stream);
+int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace);
 
 /*
  * dense x block-sparse -> dense.  Replaces blocksparse_matmul_cutlass
@@ -223,7 +237,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
  * the device.  The Python layer checks it after every product when PBS_DEBUG is set and raises.
  *
  * pbs_blocksparse_matmul_kernel_name / ..._back_kernel_name: which kernel(s) a call with these sizes runs
- * ("dds_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_seg_kernel", "sdd_kernel", "sdd_bf16_kernel", with
+ * ("stream_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_seg_kernel", "sdd_kernel", "sdd_bf16_kernel", with
  * " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
  */

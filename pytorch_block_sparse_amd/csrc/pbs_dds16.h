@@ -37,10 +37,9 @@
 // LDS: [A ring: RS steps x 16 KB][block ring: RB x 2 KB][epilogue staging: 8 x 2304 B][progress words][plan records].
 // Panel rows are 128 bytes (8 chunks of 16 bytes); chunk c of row r sits at position c ^ ((r >> 1) & 7),
 // which makes the 16-byte fragment reads of 16 consecutive rows conflict-free.  Packed blocks are laid
-// out as in the narrow kernel (pbs_dds.h).
+// out with chunk c of row r at c ^ ((r >> 2) & 3) for the input gradient, as stored ([k][n]) for the forward.
 #pragma once
 #include "pbs_common.h"
-#include "pbs_dds.h"
 
 namespace pbs {
 
@@ -241,7 +240,7 @@ __global__ __launch_bounds__((8 + NP) * 64) void dds16_kernel(D16Args g) {
         for (int q = 0; q < 2; ++q) {
             if constexpr (TRANS) {
                 const int row = q * 16 + (lane >> 2);
-                b_voff[q] = row * 64 + (((lane & 3) ^ swz<4>(row)) * 16);
+                b_voff[q] = row * 64 + (((lane & 3) ^ ((row >> 2) & 3)) * 16);
             } else {
                 b_voff[q] = q * 1024 + lane * 16;
             }
@@ -370,7 +369,7 @@ __global__ __launch_bounds__((8 + NP) * 64) void dds16_kernel(D16Args g) {
     const int a_lane_off = ((ms * TM) * 32 + lrow) * C::ROWB + (((h * 2) ^ ((lrow >> 1) & 7)) * 16);
     int b_lane_off;
     if constexpr (TRANS) {
-        b_lane_off = lrow * 64 + (((h * 2) ^ swz<4>(lrow)) * 16);   // register q: ^ (q * 16)
+        b_lane_off = lrow * 64 + (((h * 2) ^ ((lrow >> 2) & 3)) * 16);   // register q: ^ (q * 16)
     } else {
         // transposing 8-byte reads: within 16 lanes, lane s addresses 4 consecutive columns of row s/4
         // and receives, for its own column, the 4 rows as 4 consecutive k

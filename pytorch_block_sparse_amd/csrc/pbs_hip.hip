@@ -9,9 +9,9 @@
 #include <mutex>
 
 #include "pbs_common.h"
-#include "pbs_dds.h"
 #include "pbs_dds16.h"
 #include "pbs_ddsc.h"
+#include "pbs_stream.h"
 #include "pbs_index.h"
 #include "pbs_sdd.h"
 #include "pbs_sdd_bf16.h"
@@ -41,65 +41,46 @@ static int raise_lds_limit(K kernel, int bytes, std::atomic<uint64_t>& done) {
     return 0;
 }
 
-template <typename T, int TRANS, int TM, int SK, int RS, int RB, int NP, int NBW = DDS_NBW, int NSL = 4>
-static int launch_dds(DdsArgs g, hipStream_t stream) {
-    using C = DdsCfg<T, TRANS, TM, SK, RS, RB, NP, NBW, NSL>;
-    static std::atomic<uint64_t> done{0};
-    auto kernel = dds_kernel<T, TRANS, TM, SK, RS, RB, NP, NBW, NSL>;
-    constexpr int LDS_MAX = 160 * 1024;
-    // rings (or the epilogue staging) plus this group's plan records
-    const size_t lds = (size_t)C::WORK_BYTES + (size_t)g.group_ints * sizeof(int);
-    if (lds > (size_t)LDS_MAX) return PBS_ERR_TOO_LARGE;
-    if (int rc = raise_lds_limit(kernel, LDS_MAX, done)) return rc;
-    g.m_tiles = (g.M + C::BM - 1) / C::BM;
-    const long long tiles = (long long)g.m_tiles * g.n_groups * C::NSUB;
-    if (tiles > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)tiles)), dim3(C::NT), lds, stream, g);
-    return (int)hipGetLastError();
-}
+struct DdsArgs {
+    const void* a;         // [M, K] row-major
+    const void* data;      // [nnz*32, 32]
+    const int* plan;       // built by pbs_blocksparse_matmul_plan for this pattern and direction
+    const void* bias;      // nullptr or [N]
+    void* out;             // [M, N] row-major
+    int M, N, K, nnz;
+};
 
-// ---- wide-tile persistent bf16 kernel ----
-// The plan buffer holds the narrow plan first, then (when k is a multiple of 64) the wide one.
-// The narrow plan exists in four versions that differ in how many block columns of the result a
-// group of 8 places holds (8, 7, 6 or 5; the other places stay empty): one workgroup runs per CU, so a
-// launch whose tiles number 192 leaves a quarter of the chip idle, while the same columns in groups
-// of 6 make 256 tiles of three quarters the work each.  Which version a launch uses depends on the
-// token count, which is not known when the plan is built.
-constexpr int DDS_NWIDTHS = 4;
-constexpr int DDS_WIDTHS[DDS_NWIDTHS] = {8, 7, 6, 5};
-static_assert(DDS_WIDTHS[DDS_NWIDTHS - 1] == DDS_MIN_WIDTH, "dds_slots_kernel sizes its table for the narrowest group");
-static inline size_t narrow_groups(int n, int wi) { return ((size_t)(n / 32) + DDS_WIDTHS[wi] - 1) / DDS_WIDTHS[wi]; }
-static inline size_t narrow_plan_bytes_w(int n, int k, int wi) {
-    return narrow_groups(n, wi) * dds_plan_group_ints(k / 32) * sizeof(int);
-}
-static inline size_t slot_table_bytes_w(int n, int wi) {   // the block column in every place of every group
-    return ((narrow_groups(n, wi) * DDS_NB * sizeof(int)) + 63) / 64 * 64;
-}
-// Plan buffer: [narrow plan, 8 columns per group][wide plan][slot table, 8][narrow 7][slots 7][narrow 6][slots 6]
-// [narrow 5][slots 5].
-static inline size_t narrow_plan_bytes(int n, int k) { return narrow_plan_bytes_w(n, k, 0); }
-static inline size_t slot_table_bytes(int n) { return slot_table_bytes_w(n, 0); }
+// ---- plan buffer ----
+// [work list, pbs_stream.h][wide plan, pbs_dds16.h][block column tables][column plan, pbs_ddsc.h].  Its size and the
+// places of its parts are those callers of the C ABI have sized and read it by since plans held records for groups of
+// 8, 7, 6 and 5 block columns: per width an area of 64-byte records and a table of the block column in each of a group's
+// 8 places.  The work list fills the area of the first width exactly; the tables are still written (they tell
+// which columns exist), the other widths' records are not.
+constexpr int PLAN_NWIDTHS = 4;
+constexpr int PLAN_WIDTHS[PLAN_NWIDTHS] = {8, 7, 6, 5};
+constexpr int PLAN_PLACES = 8;
+static inline size_t width_groups(int n, int wi) { return ((size_t)(n / 32) + PLAN_WIDTHS[wi] - 1) / PLAN_WIDTHS[wi]; }
+static inline size_t width_bytes(int n, int k, int wi) { return width_groups(n, wi) * ((size_t)k / 32 + 2) * 64; }
+static inline size_t slot_table_bytes_w(int n, int wi) { return (width_groups(n, wi) * PLAN_PLACES * sizeof(int) + 63) / 64 * 64; }
+static inline size_t list_area_bytes(int n, int k) { return width_bytes(n, k, 0); }   // >= list_plan_bytes(n, k)
 static inline size_t wide_plan_bytes(int n, int k) {
     if (k % 64) return 0;
     const size_t groups = ((size_t)(n / 32) + D16_NB - 1) / D16_NB;
     return (groups * dds16_plan_group_ints(k / 32) + D16_SEQ_INTS) * sizeof(int);
 }
 
-static inline size_t narrow_plan_offset(int n, int k, int wi) {
+static inline size_t width_offset(int n, int k, int wi) {
     if (wi == 0) return 0;
-    size_t off = narrow_plan_bytes(n, k) + wide_plan_bytes(n, k) + slot_table_bytes(n);
-    for (int i = 1; i < wi; ++i) off += narrow_plan_bytes_w(n, k, i) + slot_table_bytes_w(n, i);
+    size_t off = list_area_bytes(n, k) + wide_plan_bytes(n, k) + slot_table_bytes_w(n, 0);
+    for (int i = 1; i < wi; ++i) off += width_bytes(n, k, i) + slot_table_bytes_w(n, i);
     return off;
 }
 static inline size_t slot_table_offset(int n, int k, int wi) {
-    if (wi == 0) return narrow_plan_bytes(n, k) + wide_plan_bytes(n, k);
-    return narrow_plan_offset(n, k, wi) + narrow_plan_bytes_w(n, k, wi);
+    if (wi == 0) return list_area_bytes(n, k) + wide_plan_bytes(n, k);
+    return width_offset(n, k, wi) + width_bytes(n, k, wi);
 }
-// ... and behind all of those the plan of the kernel with one block column per wave (pbs_ddsc.h), where it can
-// apply: [column table][per-group lists][the table 0, 1, 2, ...].
 static inline size_t column_plan_offset(int n, int k) {
-    return narrow_plan_offset(n, k, DDS_NWIDTHS - 1) + narrow_plan_bytes_w(n, k, DDS_NWIDTHS - 1) +
-           slot_table_bytes_w(n, DDS_NWIDTHS - 1);
+    return width_offset(n, k, PLAN_NWIDTHS - 1) + width_bytes(n, k, PLAN_NWIDTHS - 1) + slot_table_bytes_w(n, PLAN_NWIDTHS - 1);
 }
 static inline int column_groups(int n) { return (n / 32 + DC_NB - 1) / DC_NB; }
 static inline size_t column_table_bytes(int n) { return ((size_t)column_groups(n) * DC_NB * sizeof(int) + 63) / 64 * 64; }
@@ -109,6 +90,22 @@ static inline size_t column_plan_bytes(int n, int k) {
     return column_table_bytes(n) + ((size_t)column_groups(n) * ddsc_plan_group_ints(k / 32) + DC_SEQ_INTS) * sizeof(int);
 }
 static inline size_t all_plan_bytes(int n, int k) { return column_plan_offset(n, k) + column_plan_bytes(n, k); }
+
+// the block column in each of the 8 places of each group, one table per width: every column once, -1 elsewhere
+struct SlotTables {
+    int* table[PLAN_NWIDTHS];
+    int groups[PLAN_NWIDTHS];
+};
+__global__ __launch_bounds__(256) void slot_tables_kernel(SlotTables t, int nblk_n) {
+#pragma unroll
+    for (int wi = 0; wi < PLAN_NWIDTHS; ++wi) {
+        const int width = PLAN_WIDTHS[wi];
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < t.groups[wi] * PLAN_PLACES; i += gridDim.x * 256) {
+            const int j = i % PLAN_PLACES, c = i / PLAN_PLACES * width + j;
+            t.table[wi][i] = j < width && c < nblk_n ? c : -1;
+        }
+    }
+}
 
 constexpr int D16_TM = 2, D16_RS = 3, D16_RB = 32, D16_NP = 4;
 constexpr double DDSC_MIN_BLOCKS_PER_COLUMN = 32.0;
@@ -133,7 +130,7 @@ static int launch_dds16(const DdsArgs& g, hipStream_t stream) {
     D16Args a;
     a.a = g.a;
     a.data = g.data;
-    a.plan = reinterpret_cast<const int*>(reinterpret_cast<const unsigned char*>(g.plan) + narrow_plan_bytes(g.N, g.K));
+    a.plan = reinterpret_cast<const int*>(reinterpret_cast<const unsigned char*>(g.plan) + list_area_bytes(g.N, g.K));
     a.bias = g.bias;
     a.out = g.out;
     a.M = g.M;
@@ -188,9 +185,8 @@ static inline ColumnLaunch column_launch(long long M, int n) {
 // faster one for sparse patterns (4096 x 4096: 6 to 30 % at 1 to 24 blocks per column; 2048 x 2048: level at 2 to 4
 // blocks per column, 5 to 13 % from 8), while results of 512 to 1024 columns stay 10 to 30 % faster in the other
 // kernels until their columns hold 32 blocks.
-static bool column_kernel_fits(long long M, int n, int k, int nnz, const void* bias) {
+static bool column_kernel_fits(long long M, int n, int k, int nnz) {
     if (!column_plan_bytes(n, k) || nnz < 1 || nnz > DC_MAX_BLOCKS || M < 1) return false;
-    if (reinterpret_cast<uintptr_t>(bias) & 3u) return false;
     const ColumnLaunch c = column_launch(M, n);
     const long long tiles_per_wg = (c.m_tiles + c.wg_per_group - 1) / c.wg_per_group;
     if (tiles_per_wg * (k / 64) >= DC_SEQ_INTS) return false;   // a workgroup's steps are numbered through the table
@@ -235,96 +231,161 @@ static int launch_ddsc(const DdsArgs& g, const void* data_nk, hipStream_t stream
     return (int)hipGetLastError();
 }
 
-// Tile shapes: 256 tokens x 8 block columns, 128 x 8, or 128 x 4 (twice as many, half as wide tiles).
-// One workgroup runs per CU, so a launch takes ceil(tiles / 256) rounds of one tile time each; the shape
-// with the smallest rounds x tile area wins (smaller tiles move more operand bytes per product, hence the
-// small handicaps), e.g. 384 tiles of 128 x 8 take two rounds, of which the second is half empty, while
-// the same problem in 768 tiles of 128 x 4 takes three full rounds of half the length.  A shape whose
-// rings and plan records do not fit in LDS (very long contractions) is skipped.
-// bf16 steps cover two k-blocks (the matrix cores go through a k-block 16x faster than in fp32).
+// ---- one block column per workgroup ----
+struct StreamShape {
+    int tt, ks;   // token tile 16 * tt, waves per workgroup
+};
+// The shapes that are built, of the 15 with tt in {1, 2, 4, 8} and ks in {1, 2, 4, 8} that were timed on 140 problems (1 to
+// 16384 tokens, 256 to 4096 features, densities 0.05 to 0.75, even and Zipf columns).  In fp32 the number of waves
+// follows from the pattern alone, so that a token's result does not depend, to the last bit, on how many tokens share the call: four from 14
+// blocks per column (then within 1 to 4 % of the best on average), two below (within 5 %; four are 6 to 14 % slower there,
+// the sum of the waves' parts weighs more).
+constexpr StreamShape STREAM_F32[] = {{1, 2}, {2, 2}, {4, 2}, {1, 4}, {2, 4}, {4, 4}};
+constexpr StreamShape STREAM_BF16[] = {{1, 4}, {1, 8}, {2, 2}, {2, 4}, {4, 1}, {4, 2}, {4, 4}, {8, 2}};
+static int stream_waves_f32(int n, int nnz) { return (double)nnz / (n / 32) >= 14.0 ? 4 : 2; }
+
+// Estimated time of a shape in us: workgroups per CU x (what a block costs a CU that is kept busy, and what a workgroup
+// costs apart from its blocks), plus one workgroup's own chain (launch, list, first operands; then its blocks one after
+// the other).  The constants were fitted to the timings above, which they meet within 9 % (bf16) and 11 % (fp32); the
+// choice they make is 1.5 % (fp32) and 6 % (bf16) slower than the best built shape on average.  0.0589 us per 16 tokens
+// and block is close to the matrix instructions' own rate in fp32.  bf16 tiles of 128 tokens leave a CU one tile at most
+// times, so short columns, whose start and end weigh more, do not take them (from 12 blocks per column they are 10 to 20 % faster).
+static double stream_us(int esz, long long M, int n, int nnz, StreamShape s) {
+    const double cols = n / 32, c = nnz / cols, tt = s.tt, ks = s.ks;
+    const double per_cu = (double)((M + 16 * s.tt - 1) / (16 * s.tt)) * cols / 256.0;
+    if (esz == 4)
+        return std::ceil(per_cu) * (c * (0.0589 * tt + 0.0058) + 0.0976 * tt + 0.0819 * ks) + 3.6 + std::ceil(std::ceil(c) / ks) * 0.235 * tt;
+    const double rounds = 0.7 * per_cu + 0.3 * std::ceil(per_cu);
+    const double t = rounds * (c * (0.0177 * tt + 0.0067) + 0.0344 * tt + 0.0638 * ks) + 3.8 + std::ceil(std::ceil(c) / ks) * (0.12 + 0.0196 * tt);
+    return s.tt == 8 && c < 12.0 ? 2.0 * t : t;
+}
+struct StreamChoice {
+    StreamShape shape;
+    double us;
+};
+static StreamChoice choose_stream(int esz, long long M, int n, int k, int nnz) {
+    StreamChoice best{{0, 0}, -1.0};
+    auto consider = [&](StreamShape s) {
+        // a lane's offset into its token tile is a 32-bit number
+        if (16ll * s.tt * k * esz > 0xffffffffll) return;
+        const double us = stream_us(esz, M, n, nnz, s);
+        if (best.us < 0 || us < best.us) best = StreamChoice{s, us};
+    };
+    if (esz == 4)
+        for (const StreamShape& s : STREAM_F32) {
+            if (s.ks == stream_waves_f32(n, nnz)) consider(s);
+        }
+    else
+        for (const StreamShape& s : STREAM_BF16) consider(s);
+    return best;
+}
+
+template <typename T, int TRANS, int TT, int KS>
+static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
+    constexpr int WPE = TT == 8 ? 2 : (TT == 4 ? 3 : 4);   // waves per SIMD that the registers have to allow
+    StreamArgs a;
+    a.a = g.a;
+    a.data = g.data;
+    a.plan = g.plan;
+    a.bias = g.bias;
+    a.out = g.out;
+    a.M = g.M;
+    a.N = g.N;
+    a.K = g.K;
+    a.m_tiles = (g.M + 16 * TT - 1) / (16 * TT);
+    // The 8 XCDs as xcd_t ranges of token tiles x 8 / xcd_t sets of columns (every 8 / xcd_t-th of the ranking, so the sets
+    // are equally heavy): the split that gives the fullest XCD the fewest workgroups, and of those within 3 % of it the one
+    // with the least to read per XCD.
+    const int cols = g.N / 32;
+    const double tile_bytes = 16.0 * TT * g.K * sizeof(T), col_bytes = 1024.0 * sizeof(T) * g.nnz / cols;
+    long long fewest = 1ll << 62;
+    double least = 0.0;
+    a.xcd_t = 1;
+    for (int pass = 0; pass < 2; ++pass) {
+        for (int t = 1; t <= NUM_XCD; t *= 2) {
+            const long long tiles = (a.m_tiles + t - 1) / t, sets = (cols + NUM_XCD / t - 1) / (NUM_XCD / t);
+            if (pass == 0) {
+                if (tiles * sets < fewest) fewest = tiles * sets;
+            } else if (tiles * sets <= fewest + fewest / 32) {
+                const double bytes = tiles * tile_bytes + sets * col_bytes;
+                if (least == 0.0 || bytes < least) {
+                    least = bytes;
+                    a.xcd_t = t;
+                }
+            }
+        }
+    }
+    // as many token tiles to a pass over the columns as an XCD's L2 (4 MB) holds, at least one
+    const double fit = 4e6 / tile_bytes;
+    a.group = fit < 1.0 ? 1 : (fit > a.m_tiles ? a.m_tiles : (int)fit);
+    const long long grid = NUM_XCD * (((long long)a.m_tiles + a.xcd_t - 1) / a.xcd_t) * ((cols + NUM_XCD / a.xcd_t - 1) / (NUM_XCD / a.xcd_t));
+    if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    hipLaunchKernelGGL((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)grid), dim3(KS * 64), 0, stream, a);
+    return (int)hipGetLastError();
+}
+
+template <typename T, int TRANS>
+static int launch_stream(const DdsArgs& g, hipStream_t stream) {
+    const StreamShape s = choose_stream(sizeof(T), g.M, g.N, g.K, g.nnz).shape;
+#define PBS_STREAM(TT, KS) \
+    if (s.tt == TT && s.ks == KS) return launch_stream_shape<T, TRANS, TT, KS>(g, stream);
+    PBS_STREAM(1, 4) PBS_STREAM(2, 2) PBS_STREAM(2, 4) PBS_STREAM(4, 2) PBS_STREAM(4, 4)
+    if constexpr (sizeof(T) == 4) {
+        PBS_STREAM(1, 2)
+    } else {
+        PBS_STREAM(1, 8) PBS_STREAM(4, 1) PBS_STREAM(8, 2)
+    }
+#undef PBS_STREAM
+    return PBS_ERR_TOO_LARGE;
+}
+
+// ---- which kernel runs a product ----
+enum MatmulPart { PART_LIST = PBS_PLAN_LIST, PART_WIDE = PBS_PLAN_WIDE, PART_COLUMN = PBS_PLAN_COLUMN };   // and so which part of the plan it reads
+
+// Estimated times of the two bf16 kernels with shared panels, in us, from the same kind of fit (140 shapes of 768 to 4096
+// features, 1024 to 16384 tokens, within 9 % / 8 %): both walk R token tiles per workgroup, of S k-pairs each.
+static double wide_us(long long M, int n, int k, int nnz) {
+    const long long m_tiles = (M + D16_BM - 1) / D16_BM, groups = (n / 32 + D16_NB - 1) / D16_NB;
+    long long P = 256 / groups;
+    P = P < 1 ? 1 : (P > m_tiles ? m_tiles : P);
+    return 3.7 + (double)((m_tiles + P - 1) / P) * (0.258 * (k / 64) + 1.394 * nnz / (n / 32) + 5.4);
+}
+static double column_us(long long M, int n, int k, int nnz, bool copy) {
+    const ColumnLaunch c = column_launch(M, n);
+    return (double)((c.m_tiles + c.wg_per_group - 1) / c.wg_per_group) * (0.262 * (k / 64) + 0.429 * nnz / (n / 32) + 12.2) + (copy ? 0.0031 * nnz : 0.0);
+}
+// The column kernel where column_kernel_fits: from 8192 tokens without further question (it is the faster one in nearly
+// all of that range and within a few us in the rest), below that where its estimate is the smallest.
+static int choose_part(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
+    if (esz == 4) return PART_LIST;
+    const int wish = column_kernel_wish();
+    const bool wide = wide_kernel_fits(M, n, k);
+    const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz);
+    if (wish == 1 && column) return PART_COLUMN;
+    if (wish == 0 && wide) return PART_WIDE;
+    if (column && M >= 8192) return PART_COLUMN;
+    const double ts = choose_stream(esz, M, n, k, nnz).us;
+    const double tw = wide ? wide_us(M, n, k, nnz) : 1e300, tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
+    if (tc < ts && tc < tw) return PART_COLUMN;
+    return tw < ts ? PART_WIDE : PART_LIST;
+}
+
 template <typename T, int TRANS>
 static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
-        if (column_kernel_fits(g.M, g.N, g.K, g.nnz, g.bias)) {
+        const bool copy = workspace && workspace_bytes >= (size_t)g.nnz * 2048 && aligned16(workspace);
+        const int part = choose_part(2, g.M, g.N, g.K, g.nnz, !TRANS, copy);
+        if (part == PART_COLUMN && (reinterpret_cast<uintptr_t>(g.bias) & 3u) == 0) {   // (it reads the bias in words)
             // the kernel wants every block with k along its rows: as stored for TRANS, a transposed copy otherwise
             if constexpr (TRANS) return launch_ddsc<false>(g, g.data, stream);
-            const size_t need = (size_t)g.nnz * 2048;
-            if (workspace && workspace_bytes >= need && aligned16(workspace)) {
-                hipLaunchKernelGGL(transpose_blocks_kernel, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream,
-                                   static_cast<const uint16_t*>(g.data), static_cast<uint16_t*>(workspace), g.nnz);
-                if (int rc = (int)hipGetLastError()) return rc;
-                return launch_ddsc<true>(g, workspace, stream);
-            }
+            hipLaunchKernelGGL(transpose_blocks_kernel, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream,
+                               static_cast<const uint16_t*>(g.data), static_cast<uint16_t*>(workspace), g.nnz);
+            if (int rc = (int)hipGetLastError()) return rc;
+            return launch_ddsc<true>(g, workspace, stream);
         }
-        if (wide_kernel_fits(g.M, g.N, g.K)) return launch_dds16<TRANS>(g, stream);
+        if (part == PART_WIDE) return launch_dds16<TRANS>(g, stream);
     }
-    // shapes: 0 = 256 x 8 (4 token slices x 2 column halves), 1 = 128 x 8, 2 = 128 x 4,
-    //         3 = 256 x 8 with 8 token slices (every wave has all 8 columns; fp32 only: 8 accumulators of fp32
-    //             fragments fit the registers, and balanced waves are worth more than the larger fragments cost)
-    //         fp32 shapes 1 to 3 have four copy waves beside the eight compute waves (their registers allow three
-    //         waves per SIMD): a compute wave that also issues the DMA spends 900 to 1400 cycles of every step on
-    //         it, at the start of the step when no wave of its SIMD has products in flight (4096 x 4096 forward
-    //         1.37 -> 1.27 ms).  Shape 0 needs 200 registers per lane and keeps copying with its compute waves.
-    //         4 = 128 x 4 with one k-block per step (fp32 only).  The fp32 shapes of 128 tokens take two k-blocks
-    //             per step in two ring stages: their steps are short (a k-block is one or two block products per
-    //             wave), so a barrier per k-block costs them a fifth of their time (768 -> 3072 input gradient at
-    //             4096 tokens 0.142 -> 0.116 ms); shape 4 needs half the LDS and is what very long contractions
-    //             fall through to.
-    // widths: 8, 7, 6 or 5 of a tile's 8 (4) places hold a block column.  A tile's time falls with the columns it
-    //         holds, though not in proportion (its panel traffic and per-step overhead stay); bf16 tiles are
-    //         bound by their operand stream rather than by the matrix cores and gain less.
-    constexpr int NSHAPES = sizeof(T) == 4 ? 5 : 3;
-    constexpr int NCAND = NSHAPES * DDS_NWIDTHS;
-    const double area[5] = {2048.0, 1024.0 * 1.04, 512.0 * 1.10, 2048.0 * 0.8, 512.0 * 1.35};
-    const double fixed = sizeof(T) == 4 ? 0.15 : 0.35;   // share of a tile's time that does not depend on its columns
-    double cost[NCAND];
-    int order[NCAND];
-    for (int wi = 0; wi < DDS_NWIDTHS; ++wi) {
-        const long long groups = (long long)narrow_groups(g.N, wi);
-        // of the widths that give the same number of groups only the narrowest (most even) is tried
-        const bool useful = wi == 0 || (groups > (long long)narrow_groups(g.N, 0) &&
-                                        (wi == DDS_NWIDTHS - 1 || groups != (long long)narrow_groups(g.N, wi + 1)));
-        const long long tiles[5] = {
-            (long long)((g.M + 255) / 256) * groups,
-            (long long)((g.M + 127) / 128) * groups,
-            (long long)((g.M + 127) / 128) * groups * 2,
-            (long long)((g.M + 255) / 256) * groups,
-            (long long)((g.M + 127) / 128) * groups * 2,
-        };
-        for (int c = 0; c < NSHAPES; ++c) {
-            const int i = wi * NSHAPES + c;
-            order[i] = i;
-            cost[i] = useful ? (double)((tiles[c] + 255) / 256) * area[c] * (fixed + (1.0 - fixed) * DDS_WIDTHS[wi] / 8.0) * (1.0 + 0.01 * wi)
-                             : 1e300;
-        }
-    }
-    for (int i = 0; i < NCAND; ++i)
-        for (int j = i + 1; j < NCAND; ++j)
-            if (cost[order[j]] < cost[order[i]]) {
-                const int t = order[i];
-                order[i] = order[j];
-                order[j] = t;
-            }
-    int rc = PBS_ERR_TOO_LARGE;
-    for (int i = 0; i < NCAND && rc == PBS_ERR_TOO_LARGE; ++i) {
-        if (cost[order[i]] >= 1e300) break;
-        const int wi = order[i] / NSHAPES, c = order[i] % NSHAPES;
-        DdsArgs gw = g;
-        gw.plan = reinterpret_cast<const int*>(reinterpret_cast<const unsigned char*>(g.plan) + narrow_plan_offset(g.N, g.K, wi));
-        gw.n_groups = (int)narrow_groups(g.N, wi);
-        if constexpr (sizeof(T) == 4) {
-            rc = c == 0 ? launch_dds<T, TRANS, 2, 1, 3, 8, 0>(gw, stream)
-                 : c == 1 ? launch_dds<T, TRANS, 1, 2, 2, 16, 4>(gw, stream)
-                 : c == 2 ? launch_dds<T, TRANS, 1, 2, 2, 16, 4, 2>(gw, stream)
-                 : c == 3 ? launch_dds<T, TRANS, 1, 1, 3, 8, 4, 8, 8>(gw, stream)
-                          : launch_dds<T, TRANS, 1, 1, 3, 8, 0, 2>(gw, stream);
-        } else {
-            rc = c == 0 ? launch_dds<T, TRANS, 2, 2, 3, 16, 4>(gw, stream)
-                 : c == 1 ? launch_dds<T, TRANS, 1, 2, 3, 16, 4>(gw, stream)
-                          : launch_dds<T, TRANS, 1, 2, 3, 16, 4, 2>(gw, stream);
-        }
-    }
-    return rc;
+    return launch_stream<T, TRANS>(g, stream);
 }
 
 // ---- sparse-output product ----
@@ -579,51 +640,73 @@ size_t pbs_blocksparse_matmul_plan_bytes(int n, int k) {
     return all_plan_bytes(n, k);
 }
 
-int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, void* plan,
-                                size_t plan_bytes, void* stream) {
+static int plan_checks(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, const void* plan, size_t plan_bytes) {
     if (n <= 0 || k <= 0 || nnz < 0 || (n % 32) || (k % 32)) return PBS_ERR_BAD_SHAPE;
     if ((long long)nnz > (long long)(n / 32) * (k / 32) || k > (1 << 24)) return PBS_ERR_TOO_LARGE;
     if (!ptr || !plan || (nnz > 0 && !indices)) return PBS_ERR_NULL_POINTER;
-    if (!aligned16(plan) || plan_bytes < pbs_blocksparse_matmul_plan_bytes(n, k)) return PBS_ERR_WORKSPACE;
-    for (int wi = 0; wi < DDS_NWIDTHS; ++wi) {
-        const int groups = (int)narrow_groups(n, wi);
-        int* slots = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + slot_table_offset(n, k, wi));
-        int* narrow = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + narrow_plan_offset(n, k, wi));
-        hipLaunchKernelGGL(dds_slots_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream), ptr, n / 32, groups,
-                           DDS_WIDTHS[wi], slots);
-        if (int rc = (int)hipGetLastError()) return rc;
-        hipLaunchKernelGGL(dds_plan_kernel, dim3(groups), dim3(256), 0, static_cast<hipStream_t>(stream), ptr, indices,
-                           slots, n / 32, k / 32, nnz, narrow, (int)dds_plan_group_ints(k / 32));
+    if (!aligned16(plan) || plan_bytes < all_plan_bytes(n, k)) return PBS_ERR_WORKSPACE;
+    return PBS_OK;
+}
+
+int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, int part, void* plan,
+                                     size_t plan_bytes, void* stream) {
+    if (int rc = plan_checks(ptr, indices, n, k, nnz, plan, plan_bytes)) return rc;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    unsigned char* base = static_cast<unsigned char*>(plan);
+    if (part & PART_LIST) {
+        const long long work = (long long)nnz > 64ll * (n / 32) ? nnz : 64ll * (n / 32);
+        const unsigned grid = (unsigned)(work < 256 ? 1 : (work > 256ll * 1024 ? 1024 : (work + 255) / 256));
+        hipLaunchKernelGGL(list_plan_kernel, dim3(grid), dim3(256), 0, s, ptr, indices, n / 32, k / 32, nnz, reinterpret_cast<int*>(base));
         if (int rc = (int)hipGetLastError()) return rc;
     }
-    if (wide_plan_bytes(n, k)) {
+    if ((part & PART_WIDE) && wide_plan_bytes(n, k)) {
         const int groups16 = (n / 32 + D16_NB - 1) / D16_NB;
-        int* wide = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + narrow_plan_bytes(n, k));
-        hipLaunchKernelGGL(dds16_plan_kernel, dim3(groups16), dim3(256), 0, static_cast<hipStream_t>(stream), ptr, indices,
-                           n / 32, k / 32, nnz, wide, (int)dds16_plan_group_ints(k / 32),
-                           wide + (size_t)groups16 * dds16_plan_group_ints(k / 32));
+        int* wide = reinterpret_cast<int*>(base + list_area_bytes(n, k));
+        hipLaunchKernelGGL(dds16_plan_kernel, dim3(groups16), dim3(256), 0, s, ptr, indices, n / 32, k / 32, nnz, wide,
+                           (int)dds16_plan_group_ints(k / 32), wide + (size_t)groups16 * dds16_plan_group_ints(k / 32));
         if (int rc = (int)hipGetLastError()) return rc;
     }
-    if (column_plan_bytes(n, k)) {
+    if ((part & PART_COLUMN) && column_plan_bytes(n, k)) {
         const int groups = column_groups(n);
         const int group_ints = (int)ddsc_plan_group_ints(k / 32);
-        int* cols = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + column_plan_offset(n, k));
-        int* lists = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + column_plan_offset(n, k) + column_table_bytes(n));
-        hipStream_t s = static_cast<hipStream_t>(stream);
+        int* cols = reinterpret_cast<int*>(base + column_plan_offset(n, k));
+        int* lists = reinterpret_cast<int*>(base + column_plan_offset(n, k) + column_table_bytes(n));
         hipLaunchKernelGGL(ddsc_cols_kernel, dim3(1), dim3(256), 0, s, ptr, n / 32, groups, nnz, cols);
         if (int rc = (int)hipGetLastError()) return rc;
         hipLaunchKernelGGL(ddsc_plan_kernel, dim3(groups), dim3(256), 0, s, ptr, indices, cols, n / 32, k / 32, nnz, lists,
                            group_ints, lists + (size_t)groups * group_ints);
         if (int rc = (int)hipGetLastError()) return rc;
         hipLaunchKernelGGL(ddsc_plan_ahead_kernel, dim3(groups), dim3(64), 0, s, k / 32, lists, group_ints);
+        if (int rc = (int)hipGetLastError()) return rc;
     }
+    return PBS_OK;
+}
+
+int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, void* plan,
+                                size_t plan_bytes, void* stream) {
+    if (int rc = pbs_blocksparse_matmul_plan_part(ptr, indices, n, k, nnz, PART_LIST | PART_WIDE | PART_COLUMN, plan, plan_bytes, stream))
+        return rc;
+    SlotTables t;
+    for (int wi = 0; wi < PLAN_NWIDTHS; ++wi) {
+        t.table[wi] = reinterpret_cast<int*>(static_cast<unsigned char*>(plan) + slot_table_offset(n, k, wi));
+        t.groups[wi] = (int)width_groups(n, wi);
+    }
+    const int places = t.groups[PLAN_NWIDTHS - 1] * PLAN_PLACES;
+    hipLaunchKernelGGL(slot_tables_kernel, dim3((unsigned)(places < 16384 ? (places + 255) / 256 : 64)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), t, n / 32);
     return (int)hipGetLastError();
+}
+
+int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace) {
+    if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || nnz < 0 || (n % 32) || (k % 32))
+        return PART_LIST;
+    return choose_part(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
 }
 
 size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype) {
     if (dtype != PBS_DTYPE_BF16 || !transpose || tokens <= 0 || n <= 0 || k <= 0 || nnz <= 0 || (n % 32) || (k % 32)) return 0;
     if ((long long)nnz > (long long)(n / 32) * (k / 32)) return 0;
-    return column_kernel_fits(tokens, n, k, nnz, nullptr) ? (size_t)nnz * 2048 : 0;
+    return choose_part(2, tokens, n, k, nnz, 1, true) == PART_COLUMN ? (size_t)nnz * 2048 : 0;
 }
 
 int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* plan, const void* bias, void* dense_out,
@@ -652,9 +735,6 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
     g.N = n;
     g.K = k;
     g.nnz = nnz;
-    g.m_tiles = 0;
-    g.n_groups = (n / 32 + DDS_NB - 1) / DDS_NB;
-    g.group_ints = (int)dds_plan_group_ints(k / 32);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == PBS_DTYPE_F32) {
         return transpose ? dispatch_dds<float, 0>(g, nullptr, 0, s) : dispatch_dds<float, 1>(g, nullptr, 0, s);
@@ -823,11 +903,8 @@ int pbs_protocol_failures(unsigned* count) {
 const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int nnz, int transpose, int dtype,
                                                int with_workspace) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || (n % 32) || (k % 32)) return "";
-    if (dtype == PBS_DTYPE_BF16) {
-        if ((!transpose || with_workspace) && column_kernel_fits(tokens, n, k, nnz, nullptr)) return "ddsc_kernel";
-        if (wide_kernel_fits(tokens, n, k)) return "dds16_kernel";
-    }
-    return "dds_kernel";
+    const int part = pbs_blocksparse_matmul_part(tokens, n, k, nnz, transpose, dtype, with_workspace);
+    return part == PART_COLUMN ? "ddsc_kernel" : (part == PART_WIDE ? "dds16_kernel" : "stream_kernel");
 }
 
 const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
