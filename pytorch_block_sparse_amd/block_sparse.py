@@ -86,7 +86,7 @@ class BlockSparseMatrixBase(torch.nn.Module):
         self.register_buffer("rows_b", rows_b)
         self.register_buffer("col_start_ends_b", col_start_ends_b)
         self.register_buffer("blocks", blocks)
-        self._plans = {}
+        self._schedule = None
         self.validate_indices()
         self.check_ = False
         if callback:
@@ -377,7 +377,7 @@ class BlockSparseMatrixBase(torch.nn.Module):
         before = {n: getattr(self, n).clone() for n in names}
         super()._load_from_state_dict(state_dict, prefix, *args, **kwargs)
         error_msgs = args[4] if len(args) > 4 else kwargs.get("error_msgs")
-        self._plans = {}
+        self._schedule = None
         try:
             self.validate_indices()
         except Exception as e:  # reported the way torch reports the other problems of a state dict
@@ -462,27 +462,19 @@ class BlockSparseMatrixBase(torch.nn.Module):
         k, n = (cols, rows) if transpose else (rows, cols)
         if dense_a.shape[1] != k:
             raise Exception("Invalid matrices sizes (%d, %d) x (%d, %d)" % (dense_a.shape[0], dense_a.shape[1], k, n))
-        dense_a = self.tensor_prepare(dense_a)
-        data = self.data.detach()
-        if not data.is_contiguous():
-            raise Exception("block data must be contiguous")
-        plan = self._matmul_plan(bool(transpose), n, k)
-        return native.blocksparse_matmul(dense_a, data, plan, n, k, self.cols_a.shape[0], transpose, bias=bias)
+        return native.torch_path().matmul(dense_a, self.data, bias, bool(transpose), self._buffers, self.schedule())
 
-    def _matmul_plan(self, transpose, n, k):
-        """Kernel schedule of this pattern for one direction, built on first use and kept until the
-        index buffers change (rebuild, load_state_dict, move to another device)."""
-        if transpose:
-            ptr, indices = self.row_start_ends_a, self.cols_a
-        else:
-            ptr, indices = self.col_start_ends_b, self.rows_b
-        plans = self.__dict__.setdefault("_plans", {})
-        key = (transpose, ptr.data_ptr(), indices.data_ptr(), ptr._version, indices._version)
-        hit = plans.get(transpose)
-        if hit is None or hit[0] != key:
-            hit = (key, native.blocksparse_matmul_plan(ptr, indices, n, k))
-            plans[transpose] = hit
-        return hit[1]
+    def schedule(self):
+        """Where the native path keeps what it derives from the index buffers (the kernels' plans), for as long as the
+        buffers stay as they are."""
+        s = self.__dict__.get("_schedule")
+        if s is None:
+            s = self._schedule = native.torch_path().Schedule()
+        return s
+
+    def __getstate__(self):
+        # copies and pickles of the matrix derive their own
+        return {**self.__dict__, "_schedule": None}
 
     def reverse_matmul(self, dense_a, transpose, bias=None):
         """Any leading dims.  reference: block_sparse.py:597-604."""
@@ -497,9 +489,7 @@ class BlockSparseMatrixBase(torch.nn.Module):
                 % (tuple(dense_a.shape), tuple(dense_b.shape), tuple(self.shape))
             )
         out = self.data.detach() if overwrite_data else torch.empty_like(self.data, requires_grad=False)
-        native.blocksparse_matmul_back(
-            self.tensor_prepare(dense_a), self.tensor_prepare(dense_b), self.row_start_ends_a, self.cols_a, out
-        )
+        native.torch_path().matmul_back(dense_a, dense_b, out, self._buffers, self.schedule())
         return self.data if overwrite_data else out
 
     def matmul_with_output_sparse_support(self, dense_a, dense_b, overwrite_data=False):

@@ -13,6 +13,7 @@ import torch
 import torch.autograd
 import torch.nn as nn
 
+from . import native
 from .block_sparse import BlockSparseMatrix, BlockSparseMatrixBase, BlockSparseMatrixEmulator
 
 
@@ -109,6 +110,9 @@ class BlockSparseLinear(nn.Module):
             self.register_parameter("bias", None)
 
     def forward(self, x):
+        weight = self.weight
+        if isinstance(weight, BlockSparseMatrix):
+            return native.torch_path().linear(x, weight.data, self.bias, weight._buffers, weight.schedule())
         return self.fn(x, self.weight.get_differentiable_data(), self.weight, self.bias)
 
     def extra_repr(self):

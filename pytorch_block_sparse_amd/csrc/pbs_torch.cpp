@@ -1,0 +1,375 @@
+// The host path of the three products between torch and the C ABI of pbs_hip.h: a CPython module (no pybind11) whose
+// functions take torch tensors, allocate results and workspaces, build and keep the plans, launch on the current stream
+// and record the autograd node.
+//
+// Why native: a product of a small layer runs 4 us on the GPU.  Issued from Python (autograd.Function, ctypes, the
+// checks and the plan cache in Python) a call took 21 us of host time and a training step of one layer 160 us, so every
+// case below some thousand tokens was bound by it; the same calls take 7.7 us and 70 us here (most of the latter in torch's
+// autograd engine).
+#include <Python.h>
+
+#include <cstdlib>
+#include <memory>
+#include <mutex>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+
+#include "../../include/pbs_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+void check(int code, const char* what) {
+    TORCH_CHECK(code == PBS_OK, what, " failed with code ", code, ": ", pbs_error_string(code));
+}
+
+// With PBS_DEBUG set (read at every call: tests switch it): raise if a bounded wait of a barrier-free kernel has run out
+// since the last check.  The kernel marks the affected results NaN and counts the event; without this the call reports success.
+void check_protocol(const char* what, int device) {
+    const char* e = std::getenv("PBS_DEBUG");
+    if (!e || !*e) return;
+    static std::mutex lock;
+    static unsigned seen[64];
+    unsigned count = 0;
+    check(pbs_protocol_failures(&count), "pbs_protocol_failures");
+    std::lock_guard<std::mutex> hold(lock);
+    const unsigned before = seen[device & 63];
+    seen[device & 63] = count;
+    TORCH_CHECK(count == before, what, ": ", count - before,
+                " wait(s) of the kernel's progress protocol ran into their bound; the results of the affected tiles are NaN");
+}
+
+int dtype_code(const Tensor& t) {
+    switch (t.scalar_type()) {
+        case at::kFloat: return PBS_DTYPE_F32;
+        case at::kBFloat16: return PBS_DTYPE_BF16;
+        default: TORCH_CHECK(false, "unsupported dtype ", t.dtype(), "; supported: float32, bfloat16");
+    }
+}
+
+void check_gpu(const Tensor& t) {
+    TORCH_CHECK(!t.defined() || t.is_cuda(),
+                "pytorch_block_sparse_amd: the block-sparse matmuls run only on a GPU through libpbs_hip.so; got a tensor on ", t.device());
+}
+
+void* current_stream(const Tensor& t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
+
+// An index tensor as it was when the plans were made.
+struct Seen {
+    Tensor t;
+    const void* data = nullptr;
+    uint32_t version = 0;
+
+    static uint32_t version_of(const Tensor& t) {   // (tensors made in inference mode do not count)
+        const auto& v = t.unsafeGetTensorImpl()->version_counter();
+        return v.enabled() ? v.current_version() : 0;
+    }
+    void take(const Tensor& now) {
+        t = now;
+        data = now.const_data_ptr();
+        version = version_of(now);
+    }
+    bool still(const Tensor& now) const {
+        return now.unsafeGetTensorImpl() == t.unsafeGetTensorImpl() && now.const_data_ptr() == data && version_of(now) == version;
+    }
+};
+
+// One pattern: its index arrays and the plans of both directions.  Never changed once made, except that parts of
+// the plans are added when a product first needs them; a matrix whose index arrays change gets a new one, and autograd
+// nodes keep the one of their forward product.
+struct Pattern {
+    Seen row_ptr, cols, col_ptr, rows;
+    int out_features = 0, in_features = 0, nnz = 0;
+    std::mutex lock;
+    Tensor plan[2];      // [transpose]
+    int parts[2] = {0, 0};
+
+    bool still(const Tensor& rp, const Tensor& c, const Tensor& cp, const Tensor& r) const {
+        return row_ptr.still(rp) && cols.still(c) && col_ptr.still(cp) && rows.still(r);
+    }
+
+    const void* plan_for(bool transpose, int n, int k, int part, void* stream) {
+        std::lock_guard<std::mutex> hold(lock);
+        part |= PBS_PLAN_LIST;
+        if ((parts[transpose] & part) != part) {
+            const Tensor& ptr = transpose ? row_ptr.t : col_ptr.t;
+            const Tensor& idx = transpose ? cols.t : rows.t;
+            TORCH_CHECK(ptr.is_cuda() && idx.is_cuda(), "the index buffers are not on the GPU");
+            const size_t bytes = pbs_blocksparse_matmul_plan_bytes(n, k);
+            if (!plan[transpose].defined()) plan[transpose] = at::empty({(int64_t)bytes}, ptr.options().dtype(at::kByte));
+            check(pbs_blocksparse_matmul_plan_part(ptr.const_data_ptr<int>(), idx.const_data_ptr<int>(), n, k, nnz, part & ~parts[transpose],
+                                                   plan[transpose].mutable_data_ptr(), bytes, stream),
+                  "pbs_blocksparse_matmul_plan_part");
+            parts[transpose] |= part;
+        }
+        return plan[transpose].const_data_ptr();
+    }
+};
+using PatternPtr = std::shared_ptr<Pattern>;
+
+const void* data_or_null(const Tensor& t) { return t.defined() && t.numel() ? t.const_data_ptr() : nullptr; }
+
+// a [..., k] -> [..., n]
+Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose) {
+    check_gpu(a_any);
+    check_gpu(data);
+    check_gpu(bias);
+    const int code = dtype_code(a_any);
+    TORCH_CHECK(data.scalar_type() == a_any.scalar_type(), "dense operand is ", a_any.dtype(), " but the block data is ", data.dtype());
+    TORCH_CHECK(!bias.defined() || bias.scalar_type() == a_any.scalar_type(), "bias is ", bias.dtype(), ", expected ", a_any.dtype());
+    TORCH_CHECK(data.is_contiguous(), "block data must be contiguous");
+    TORCH_CHECK(data.device() == a_any.device() && (!bias.defined() || bias.device() == a_any.device()),
+                "the operands are on different devices");
+    const int n = transpose ? p.out_features : p.in_features, k = transpose ? p.in_features : p.out_features;
+    TORCH_CHECK(a_any.dim() >= 2, "Invalid dimensions for dense_a ", a_any.sizes(), " : dense_a should have at least 2 dimensions.");
+    TORCH_CHECK(a_any.size(-1) == k, "Invalid matrices sizes ", a_any.sizes(), " x (", k, ", ", n, ")");
+    TORCH_CHECK(data.numel() == (int64_t)p.nnz * 1024, "the block data does not match the index buffers");
+    TORCH_CHECK(!bias.defined() || (bias.numel() == n && bias.is_contiguous()), "bias should be contiguous and hold ", n, " values");
+    const Tensor a = a_any.is_contiguous() ? a_any : a_any.contiguous();
+    const int64_t tokens = a.numel() / k;
+    c10::DeviceGuard guard(a.device());
+    void* stream = current_stream(a);
+    c10::SmallVector<int64_t, 6> sizes(a.sizes().begin(), a.sizes().end());
+    sizes.back() = n;
+    Tensor out = at::empty(sizes, a.options());
+    if (tokens == 0) return out;
+    const int part = pbs_blocksparse_matmul_part(tokens, n, k, p.nnz, transpose, code, 1);
+    const void* plan = p.plan_for(transpose, n, k, part, stream);
+    // the transposed copy of the blocks that the bf16 column kernel's forward product works from
+    const size_t ws_bytes = transpose && part == PBS_PLAN_COLUMN ? pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, p.nnz, 1, code) : 0;
+    Tensor ws;
+    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+    check(pbs_blocksparse_matmul_ws(a.const_data_ptr(), data_or_null(data), plan, data_or_null(bias), out.mutable_data_ptr(), tokens, n, k,
+                                    p.nnz, transpose, code, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
+          "pbs_blocksparse_matmul_ws");
+    check_protocol("pbs_blocksparse_matmul_ws", a.device().index());
+    return out;
+}
+
+// packed blocks of a^T b on the pattern, into `out`
+void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out) {
+    check_gpu(a_any);
+    check_gpu(b_any);
+    check_gpu(out);
+    const int code = dtype_code(a_any);
+    TORCH_CHECK(b_any.scalar_type() == a_any.scalar_type() && out.scalar_type() == a_any.scalar_type(), "operands and result must share one dtype");
+    TORCH_CHECK(b_any.device() == a_any.device() && out.device() == a_any.device() && p.cols.t.device() == a_any.device(),
+                "the operands are on different devices");
+    TORCH_CHECK(a_any.size(-1) == p.out_features && b_any.size(-1) == p.in_features && out.numel() == (int64_t)p.nnz * 1024 && out.is_contiguous(),
+                "Invalid matrices sizes ", a_any.sizes(), "^T x ", b_any.sizes());
+    const Tensor a = a_any.is_contiguous() ? a_any : a_any.contiguous();
+    const Tensor b = b_any.is_contiguous() ? b_any : b_any.contiguous();
+    const int64_t tokens = a.numel() / p.out_features;
+    TORCH_CHECK(b.numel() / p.in_features == tokens, "Invalid matrices sizes ", a.sizes(), "^T x ", b.sizes());
+    c10::DeviceGuard guard(a.device());
+    const size_t ws_bytes = pbs_blocksparse_matmul_back_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
+    Tensor ws;
+    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
+    check(pbs_blocksparse_matmul_back(data_or_null(a), data_or_null(b), p.row_ptr.t.const_data_ptr<int>(),
+                                      static_cast<const int*>(data_or_null(p.cols.t)), out.numel() ? out.mutable_data_ptr() : nullptr, tokens,
+                                      p.out_features, p.in_features, p.nnz, code, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes,
+                                      current_stream(a)),
+          "pbs_blocksparse_matmul_back");
+}
+
+// y = x W^T + bias.  Backward: dx = dy W, dW on the pattern's blocks, dbias = sum of dy over the tokens.
+struct BlockSparseLinearBackward : public torch::autograd::Node {
+    PatternPtr pattern;
+    torch::autograd::SavedVariable x, data;
+    bool has_bias = false;
+
+    std::string name() const override { return "BlockSparseLinearBackward"; }
+    void release_variables() override {
+        x.reset_data();
+        data.reset_data();
+    }
+    torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+        torch::autograd::variable_list out(3);
+        const Tensor& g = grads[0];
+        if (!g.defined()) return out;
+        at::NoGradGuard no_grad;
+        const Tensor dy = g.is_contiguous() ? g : g.contiguous();
+        if (task_should_compute_output(0)) out[0] = matmul(*pattern, dy, data.unpack(shared_from_this()), Tensor(), false);
+        if (task_should_compute_output(1)) {
+            const Tensor xs = x.unpack(shared_from_this());
+            out[1] = at::empty({(int64_t)pattern->nnz * 32, 32}, xs.options());
+            matmul_back(*pattern, dy, xs, out[1]);
+        }
+        if (has_bias && task_should_compute_output(2)) out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
+        return out;
+    }
+};
+
+Tensor linear(const PatternPtr& p, const Tensor& x, const Tensor& data, const Tensor& bias) {
+    Tensor y;
+    {
+        at::NoGradGuard no_grad;
+        y = matmul(*p, x, data, bias, true);
+    }
+    if (torch::autograd::compute_requires_grad(x, data, bias)) {
+        auto node = std::shared_ptr<BlockSparseLinearBackward>(new BlockSparseLinearBackward(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(x, data, bias));
+        node->pattern = p;
+        node->has_bias = bias.defined();
+        if (data.requires_grad()) node->x = torch::autograd::SavedVariable(x, false);
+        if (x.requires_grad()) node->data = torch::autograd::SavedVariable(data, false);
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// Python side
+// ---------------------------------------------------------------------------------------------------------------
+
+// Where a matrix keeps its Pattern.
+struct Schedule {
+    PyObject_HEAD
+    PatternPtr* pattern;
+    std::mutex* lock;
+};
+
+PyObject* schedule_new(PyTypeObject* type, PyObject*, PyObject*) {
+    Schedule* self = reinterpret_cast<Schedule*>(type->tp_alloc(type, 0));
+    if (self) {
+        self->pattern = new PatternPtr();
+        self->lock = new std::mutex();
+    }
+    return reinterpret_cast<PyObject*>(self);
+}
+void schedule_dealloc(PyObject* o) {
+    Schedule* self = reinterpret_cast<Schedule*>(o);
+    delete self->pattern;
+    delete self->lock;
+    Py_TYPE(o)->tp_free(o);
+}
+PyTypeObject ScheduleType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyObject *s_row_ptr, *s_cols, *s_col_ptr, *s_rows;   // buffer names, interned
+
+Tensor tensor_arg(PyObject* o, const char* what) {
+    TORCH_CHECK_TYPE(THPVariable_Check(o), what, " should be a tensor, not ", Py_TYPE(o)->tp_name);
+    return THPVariable_Unpack(o);
+}
+Tensor optional_tensor(PyObject* o, const char* what) { return o == Py_None ? Tensor() : tensor_arg(o, what); }
+
+const Tensor& buffer(PyObject* buffers, PyObject* name) {
+    PyObject* o = PyDict_GetItem(buffers, name);   // borrowed
+    TORCH_CHECK(o && THPVariable_Check(o), "the matrix has no index buffer ", PyUnicode_AsUTF8(name));
+    return THPVariable_Unpack(o);
+}
+
+// The pattern of a matrix, from its `_buffers` and its Schedule; a new one if the buffers are not those it was made from.
+PatternPtr pattern_arg(PyObject* buffers, PyObject* schedule) {
+    TORCH_CHECK_TYPE(PyDict_Check(buffers) && Py_TYPE(schedule) == &ScheduleType, "expected a matrix's buffers and Schedule");
+    Schedule* s = reinterpret_cast<Schedule*>(schedule);
+    const Tensor &rp = buffer(buffers, s_row_ptr), &c = buffer(buffers, s_cols), &cp = buffer(buffers, s_col_ptr), &r = buffer(buffers, s_rows);
+    std::lock_guard<std::mutex> hold(*s->lock);
+    PatternPtr& p = *s->pattern;
+    if (!p || !p->still(rp, c, cp, r)) {
+        for (const Tensor* t : {&rp, &c, &cp, &r})
+            TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous(), "index buffers should be contiguous int32 tensors");
+        auto q = std::make_shared<Pattern>();
+        q->row_ptr.take(rp);
+        q->cols.take(c);
+        q->col_ptr.take(cp);
+        q->rows.take(r);
+        q->out_features = (int)(rp.numel() - 1) * 32;
+        q->in_features = (int)(cp.numel() - 1) * 32;
+        q->nnz = (int)(c.numel() / 2);
+        TORCH_CHECK(r.numel() == c.numel(), "cols_a and rows_b differ in length");
+        p = std::move(q);
+    }
+    return p;
+}
+
+void need(Py_ssize_t got, Py_ssize_t want, const char* what) { TORCH_CHECK_TYPE(got == want, what, " takes ", want, " arguments, got ", got); }
+
+struct NoGil {
+    PyThreadState* s = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(s); }
+};
+
+// linear(x, data, bias or None, buffers, schedule) -> y, recorded for autograd
+PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 5, "linear");
+    const Tensor x = tensor_arg(args[0], "x"), data = tensor_arg(args[1], "data"), bias = optional_tensor(args[2], "bias");
+    const PatternPtr p = pattern_arg(args[3], args[4]);
+    Tensor y;
+    {
+        NoGil no_gil;
+        y = linear(p, x, data, bias);
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// matmul(a, data, bias or None, transpose, buffers, schedule) -> a W^T or a W, outside autograd
+PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 6, "matmul");
+    const Tensor a = tensor_arg(args[0], "dense_a"), data = tensor_arg(args[1], "data"), bias = optional_tensor(args[2], "bias");
+    const bool transpose = PyObject_IsTrue(args[3]) == 1;
+    const PatternPtr p = pattern_arg(args[4], args[5]);
+    Tensor y;
+    {
+        NoGil no_gil;
+        at::NoGradGuard no_grad;
+        y = matmul(*p, a, data, bias, transpose);
+    }
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// matmul_back(a, b, out, buffers, schedule): packed blocks of a^T b into out
+PyObject* py_matmul_back(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 5, "matmul_back");
+    const Tensor a = tensor_arg(args[0], "dense_a"), b = tensor_arg(args[1], "dense_b"), out = tensor_arg(args[2], "out");
+    const PatternPtr p = pattern_arg(args[3], args[4]);
+    {
+        NoGil no_gil;
+        at::NoGradGuard no_grad;
+        matmul_back(*p, a, b, out);
+    }
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {{"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_linear)), METH_FASTCALL, nullptr},
+                         {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_matmul)), METH_FASTCALL, nullptr},
+                         {"matmul_back", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_matmul_back)), METH_FASTCALL, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pbs_torch", nullptr, -1, methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__pbs_torch() {
+    ScheduleType.tp_name = "pytorch_block_sparse_amd.csrc._pbs_torch.Schedule";
+    ScheduleType.tp_basicsize = sizeof(Schedule);
+    ScheduleType.tp_flags = Py_TPFLAGS_DEFAULT;
+    ScheduleType.tp_new = schedule_new;
+    ScheduleType.tp_dealloc = schedule_dealloc;
+    if (PyType_Ready(&ScheduleType) < 0) return nullptr;
+    s_row_ptr = PyUnicode_InternFromString("row_start_ends_a");
+    s_cols = PyUnicode_InternFromString("cols_a");
+    s_col_ptr = PyUnicode_InternFromString("col_start_ends_b");
+    s_rows = PyUnicode_InternFromString("rows_b");
+    PyObject* m = PyModule_Create(&module);
+    if (!m) return nullptr;
+    Py_INCREF(&ScheduleType);
+    if (PyModule_AddObject(m, "Schedule", reinterpret_cast<PyObject*>(&ScheduleType)) < 0) return nullptr;
+    return m;
+}

@@ -83,6 +83,25 @@ def load():
     return lib
 
 
+_torch_path = None
+
+
+def torch_path():
+    """The extension module csrc/_pbs_torch.so: the products on torch tensors (result and workspace allocation, plans,
+    autograd node) on top of the C ABI.  Loaded on first use; like the library it has no stand-in."""
+    global _torch_path
+    if _torch_path is None:
+        load()
+        try:
+            from .csrc import _pbs_torch
+        except ImportError as e:
+            raise NativeLibraryMissing(
+                f"{_HERE}/csrc/_pbs_torch.so cannot be loaded ({e}). Run `python -m pytorch_block_sparse_amd.csrc.build`."
+            ) from e
+        _torch_path = _pbs_torch
+    return _torch_path
+
+
 def error_string(code):
     return load().pbs_error_string(int(code)).decode()
 
@@ -90,26 +109,6 @@ def error_string(code):
 def _check(code, what):
     if code != 0:
         raise RuntimeError(f"{what} failed with code {code}: {error_string(code)}")
-
-
-_failures_seen = {}
-
-
-def check_protocol(what):
-    """With PBS_DEBUG set: raise if a bounded wait of a barrier-free kernel has run out since the last check
-    (the kernel marks the affected results NaN and counts the event; without this the call reports success)."""
-    if not os.environ.get("PBS_DEBUG"):
-        return
-    count = ctypes.c_uint(0)
-    _check(load().pbs_protocol_failures(ctypes.byref(count)), "pbs_protocol_failures")
-    dev = torch.cuda.current_device()
-    before = _failures_seen.get(dev, 0)
-    _failures_seen[dev] = count.value
-    if count.value != before:
-        raise RuntimeError(
-            f"{what}: {count.value - before} wait(s) of the kernel's progress protocol ran into their bound; "
-            "the results of the affected tiles are NaN"
-        )
 
 
 def matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace=True):
@@ -128,25 +127,6 @@ def _stream(index=None):
         index = torch.cuda.current_device()
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # the handle without a Stream object around it
     return ctypes.c_void_p(raw(index) if raw is not None else torch.cuda.current_stream(index).cuda_stream)
-
-
-class _on_device:
-    """`with torch.cuda.device(d)` only when d is not the current device already (the context manager costs
-    several microseconds, which is most of a small product's host time)."""
-
-    def __init__(self, device):
-        self.index = device.index if device.index is not None else torch.cuda.current_device()
-        self.ctx = None if self.index == torch.cuda.current_device() else torch.cuda.device(self.index)
-
-    def __enter__(self):
-        if self.ctx is not None:
-            self.ctx.__enter__()
-        return self.index
-
-    def __exit__(self, *exc):
-        if self.ctx is not None:
-            self.ctx.__exit__(*exc)
-        return False
 
 
 def _ptr(t):
@@ -208,60 +188,3 @@ def blocksparse_matmul_plan(ptr, indices, n, k):
         )
     _check(code, "pbs_blocksparse_matmul_plan")
     return plan
-
-
-def blocksparse_matmul(dense_a, data, plan, n, k, nnz, transpose, bias=None, out=None):
-    """out[tokens, n] = dense_a[tokens, k] . W^T (transpose) or . W (not transpose)."""
-    lib = _lib or load()
-    dtype = dense_a.dtype
-    if not (dense_a.is_cuda and data.is_cuda and plan.is_cuda and (bias is None or bias.is_cuda)):
-        _require_cuda(dense_a, data, plan, bias)
-    code_dtype = DTYPE_CODES.get(dtype)
-    if code_dtype is None:
-        raise RuntimeError(f"unsupported dtype {dtype}; supported: {SUPPORTED_DTYPES}")
-    if data.dtype != dtype:
-        raise RuntimeError(f"dense operand is {dtype} but the block data is {data.dtype}")
-    if bias is not None and bias.dtype != dtype:
-        raise RuntimeError(f"bias is {bias.dtype}, expected {dtype}")
-    tokens = dense_a.shape[0]
-    if out is None:
-        out = torch.empty((tokens, n), dtype=dtype, device=dense_a.device)
-    tr = 1 if transpose else 0
-    # the transposed copy of the blocks that the forward bf16 kernel for dense patterns works from (made by the library)
-    ws, ws_bytes = None, 0
-    if tr and code_dtype == 1:
-        ws_bytes = lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, code_dtype)
-        if ws_bytes:
-            ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dense_a.device)
-    with _on_device(dense_a.device) as index:
-        code = lib.pbs_blocksparse_matmul_ws(
-            _ptr(dense_a), _ptr(data), _ptr(plan), _ptr(bias), _ptr(out), tokens, n, k, nnz, tr, code_dtype,
-            _ptr(ws), ws_bytes, _stream(index),
-        )
-    if code != 0:
-        _check(code, "pbs_blocksparse_matmul_ws")
-    check_protocol("pbs_blocksparse_matmul_ws")
-    return out
-
-
-def blocksparse_matmul_back(dense_a, dense_b, row_start_ends_a, cols_a, out):
-    """out (packed [nnz*32, 32]) = blocks of dense_a^T . dense_b on the pattern's support."""
-    lib = load()
-    _require_cuda(dense_a, dense_b, row_start_ends_a, cols_a, out)
-    if dense_a.dtype not in DTYPE_CODES:
-        raise RuntimeError(f"unsupported dtype {dense_a.dtype}; supported: {SUPPORTED_DTYPES}")
-    if dense_b.dtype != dense_a.dtype or out.dtype != dense_a.dtype:
-        raise RuntimeError("operands and result must share one dtype")
-    tokens, out_features = dense_a.shape
-    in_features = dense_b.shape[1]
-    nnz = cols_a.shape[0]
-    code_dtype = DTYPE_CODES[dense_a.dtype]
-    ws_bytes = lib.pbs_blocksparse_matmul_back_workspace_bytes(tokens, out_features, in_features, nnz, code_dtype)
-    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dense_a.device) if ws_bytes else None
-    with _on_device(dense_a.device) as index:
-        code = lib.pbs_blocksparse_matmul_back(
-            _ptr(dense_a), _ptr(dense_b), _ptr(row_start_ends_a), _ptr(cols_a), _ptr(out), tokens, out_features,
-            in_features, nnz, code_dtype, _ptr(ws), ws_bytes, _stream(index),
-        )
-    _check(code, "pbs_blocksparse_matmul_back")
-    return out
