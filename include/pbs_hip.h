@@ -68,6 +68,40 @@ int pbs_build_indices(const uint8_t* mask, const int64_t* block_ptr, int X, int 
                       int32_t* blocks, int32_t* status, void* stream);
 
 /*
+ * Move data blocks to other positions and write all five index arrays again, in one launch
+ * (BlockSparseMatrixBase.block_replace, block_sparse.py:167-219).
+ *
+ *   old_blocks [2*nnz]  the present `blocks` array
+ *   moves   [n_moves,3] int64: (block row, block column, data block)
+ *   status     one int32 word the GPU can write (device or pinned host memory): 0, or a sum of 1 (a data block outside
+ *              [0, nnz)), 2 (a position outside the grid), 4 (two blocks at one position); nothing else is written then
+ *   workspace  pbs_replace_blocks_workspace_bytes(X, Y, nnz) bytes of device memory
+ */
+size_t pbs_replace_blocks_workspace_bytes(int X, int Y, int nnz);
+int pbs_replace_blocks(const int32_t* old_blocks, const int64_t* moves, int n_moves, int X, int Y, int nnz,
+                       int32_t* cols_a, int32_t* row_start_ends_a, int32_t* rows_b, int32_t* col_start_ends_b,
+                       int32_t* blocks, int32_t* status, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * Consistency of the five index arrays (sanity_check, block_sparse.py:431-463, and what the kernels rely on beyond it).
+ * `status` as above: a sum of the bits below; the conditions of rows_b / col_start_ends_b have those of cols_a /
+ * row_start_ends_a times 16.
+ */
+#define PBS_BAD_ROW_STARTS 1       /* does not start at 0, or decreases */
+#define PBS_BAD_ROW_END 2          /* the last one is not nnz */
+#define PBS_BAD_COLS 4             /* a coordinate outside the grid */
+#define PBS_BAD_COLS_IDS 8         /* the data blocks are not a permutation */
+#define PBS_BAD_BLOCKS 256         /* a position of `blocks` outside the grid */
+#define PBS_BAD_COLS_ORDER 512     /* the coordinates of a list do not increase: cols_a */
+#define PBS_BAD_ROWS_ORDER 1024    /* ... rows_b */
+#define PBS_BAD_LISTS_DIFFER 2048  /* cols_a and rows_b hold different blocks */
+#define PBS_BAD_BLOCKS_DIFFER 4096 /* `blocks` and cols_a hold different blocks */
+size_t pbs_validate_indices_workspace_bytes(int nnz);
+int pbs_validate_indices(const int32_t* cols_a, const int32_t* row_start_ends_a, const int32_t* rows_b,
+                         const int32_t* col_start_ends_b, const int32_t* blocks, int X, int Y, int nnz,
+                         int32_t* status, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Schedule ("plan") of the dense x block-sparse product for one pattern and one direction.
  * It depends only on the index arrays, not on the data: build it when the pattern is created or
  * changed and pass it to every pbs_blocksparse_matmul call of that direction.  It is what the

@@ -153,9 +153,12 @@ class BlockSparseMatrixBase(torch.nn.Module):
 
         reference: block_sparse.py:167-219.
         """
+        X, Y = self.blocks_count()
+        if self.blocks.is_cuda and not self.check_:
+            self._block_replace_on_gpu(block_replacements, X, Y)
+            return
         pos = self.build_coo_block_index().long()
         rep = block_replacements.to(dtype=torch.long, device=pos.device).reshape(-1, 3)
-        X, Y = self.blocks_count()
         if self.check_:
             refs = torch.zeros(X * Y, dtype=torch.long, device=pos.device)
             refs[pos[0] * Y + pos[1]] = 1
@@ -167,6 +170,21 @@ class BlockSparseMatrixBase(torch.nn.Module):
         mask = self.block_mask_build(pos)
         block_ptr = torch.argsort(pos[0] * Y + pos[1])
         self.rebuild(mask, block_ptr)
+
+    def _block_replace_on_gpu(self, block_replacements, X, Y):
+        """The same in one kernel, which writes arrays that are consistent by construction or reports why it cannot."""
+        rep = block_replacements.to(dtype=torch.long, device=self.blocks.device).reshape(-1, 3)
+        status, arrays = native.torch_path().replace_blocks(self.blocks, rep, X, Y)
+        if status & 1:
+            raise Exception("block_replacements names a data block outside [0, %d)" % (self.data.shape[0] // self.block_shape[0]))
+        if status & 2:
+            raise Exception("block_replacements holds a position outside the %d x %d grid of blocks" % (X, Y))
+        if status & 4:
+            raise RuntimeError("block_replacements leaves two blocks at one position")
+        for name, array in zip(("blocks", "cols_a", "row_start_ends_a", "rows_b", "col_start_ends_b"), arrays):
+            self._buffers[name] = array
+        self._schedule = None
+        self.updated_data()
 
     # ------------------------------------------------------------------ constructors
     @classmethod
@@ -327,49 +345,66 @@ class BlockSparseMatrixBase(torch.nn.Module):
         blocks = self.blocks
         if blocks.dim() != 1 or blocks.shape[0] != 2 * nnz or blocks.dtype != it:
             raise Exception("blocks should be %s of shape (%d,), not %s %s" % (it, 2 * nnz, blocks.dtype, tuple(blocks.shape)))
+        if blocks.is_cuda:
+            bad = native.torch_path().validate(self.cols_a, self.row_start_ends_a, self.rows_b, self.col_start_ends_b, blocks)
+            if bad:
+                raise Exception(self._index_problems(nnz, X, Y)[(bad & -bad).bit_length() - 1])
+            return
+        messages = self._index_problems(nnz, X, Y)
         problems = []   # (message, 0-d bool tensor: True = broken)
-        for name, ids, ends_name, ends, _, limit in lists:
+        for i, (name, ids, ends_name, ends, _, limit) in enumerate(lists):
             e = ends.long()
-            problems.append(("%s should start at 0 and never decrease" % ends_name, (e[0] != 0) | (e[1:] < e[:-1]).any()))
-            problems.append(("%s last element should be equal to the block count (%d)" % (ends_name, nnz), e[-1] != nnz))
+            problems.append((messages[4 * i], (e[0] != 0) | (e[1:] < e[:-1]).any()))
+            problems.append((messages[4 * i + 1], e[-1] != nnz))
             if nnz:
                 c, b = ids[:, 0].long(), ids[:, 1].long()
-                problems.append(("%s holds a block coordinate outside [0, %d)" % (name, limit), (c.min() < 0) | (c.max() >= limit)))
+                problems.append((messages[4 * i + 2], (c.min() < 0) | (c.max() >= limit)))
                 b_ok = (b >= 0) & (b < nnz)
                 seen = torch.zeros(nnz, dtype=torch.long, device=ids.device)
                 seen.index_add_(0, b.clamp(0, nnz - 1), b_ok.long())
-                problems.append(
-                    ("the data block ids of %s should be a permutation of 0..%d" % (name, nnz - 1), (seen != 1).any())
-                )
+                problems.append((messages[4 * i + 3], (seen != 1).any()))
         if nnz:
             b2 = blocks.view(-1, 2).long()
-            problems.append((
-                "blocks holds a block position outside the %d x %d grid" % (X, Y),
-                (b2.min() < 0) | (b2[:, 0].max() >= Y) | (b2[:, 1].max() >= X),
-            ))
+            problems.append((messages[8], (b2.min() < 0) | (b2[:, 0].max() >= Y) | (b2[:, 1].max() >= X)))
             # Within one list the coordinates must increase strictly (sorted, no duplicates): the weight-gradient
             # kernels binary-search a row's entries and size their tables for at most one entry per position.
             # And the two compressed lists and `blocks` must describe the same (row, column) for every data block.
             where = {}
             pos = torch.arange(nnz, device=blocks.device)
-            for name, ids, ends_name, ends, n_lists, _ in lists:
+            for i, (name, ids, ends_name, ends, n_lists, _) in enumerate(lists):
                 e = ends.long().to(blocks.device).clamp(0, nnz)
                 owner = torch.searchsorted(e[1:].contiguous(), pos, right=True)   # the list each entry belongs to
                 c, b = ids[:, 0].long().to(blocks.device), ids[:, 1].long().to(blocks.device)
                 same = owner[1:] == owner[:-1]
-                problems.append(("the coordinates of %s should increase strictly within each of its lists" % name,
-                                 (same & (c[1:] <= c[:-1])).any()))
+                problems.append((messages[9 + i], (same & (c[1:] <= c[:-1])).any()))
                 at = torch.full((nnz, 2), -1, dtype=torch.long, device=blocks.device)
                 at[b.clamp(0, nnz - 1)] = torch.stack((owner, c), 1)
                 where[name] = at
             rc_a = where["cols_a"]                 # (row, column) of every data block according to the row lists
             rc_b = where["rows_b"].flip(1)         # the column lists hold (column, row)
-            problems.append(("cols_a and rows_b should hold the same blocks", (rc_a != rc_b).any()))
-            problems.append(("blocks should hold the (column, row) of every data block of cols_a", (b2 != rc_a.flip(1)).any()))
+            problems.append((messages[11], (rc_a != rc_b).any()))
+            problems.append((messages[12], (b2 != rc_a.flip(1)).any()))
         flags = torch.stack([p[1].to(self.blocks.device) for p in problems]).tolist()
         for (message, _), broken in zip(problems, flags):
             if broken:
                 raise Exception(message)
+
+    @staticmethod
+    def _index_problems(nnz, X, Y):
+        """What is wrong with the index buffers, in the order of the bits of pbs_validate_indices."""
+        out = []
+        for name, ends_name, limit in (("cols_a", "row_start_ends_a", Y), ("rows_b", "col_start_ends_b", X)):
+            out += [
+                "%s should start at 0 and never decrease" % ends_name,
+                "%s last element should be equal to the block count (%d)" % (ends_name, nnz),
+                "%s holds a block coordinate outside [0, %d)" % (name, limit),
+                "the data block ids of %s should be a permutation of 0..%d" % (name, nnz - 1),
+            ]
+        out.append("blocks holds a block position outside the %d x %d grid" % (X, Y))
+        out += ["the coordinates of %s should increase strictly within each of its lists" % n for n in ("cols_a", "rows_b")]
+        out.append("cols_a and rows_b should hold the same blocks")
+        out.append("blocks should hold the (column, row) of every data block of cols_a")
+        return out
 
     def _load_from_state_dict(self, state_dict, prefix, *args, **kwargs):
         """Index buffers copied in from a checkpoint are validated before any kernel reads them."""

@@ -635,6 +635,39 @@ int pbs_build_indices(const uint8_t* mask, const int64_t* block_ptr, int X, int 
     return (int)hipGetLastError();
 }
 
+size_t pbs_replace_blocks_workspace_bytes(int X, int Y, int nnz) {
+    return X < 1 || Y < 1 || nnz < 0 ? 0 : replace_ws_bytes(X, Y, nnz);
+}
+
+int pbs_replace_blocks(const int32_t* old_blocks, const int64_t* moves, int n_moves, int X, int Y, int nnz, int32_t* cols_a,
+                       int32_t* row_start_ends_a, int32_t* rows_b, int32_t* col_start_ends_b, int32_t* blocks, int32_t* status,
+                       void* workspace, size_t workspace_bytes, void* stream) {
+    if (X < 1 || Y < 1 || nnz < 0 || n_moves < 0 || (long long)nnz > (long long)X * Y) return PBS_ERR_BAD_SHAPE;
+    if ((long long)X * Y > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    if (!row_start_ends_a || !col_start_ends_b || !status || (n_moves > 0 && !moves)) return PBS_ERR_NULL_POINTER;
+    if (nnz > 0 && (!old_blocks || !cols_a || !rows_b || !blocks)) return PBS_ERR_NULL_POINTER;
+    const size_t need = replace_ws_bytes(X, Y, nnz);
+    if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
+    hipLaunchKernelGGL(replace_blocks_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), old_blocks, moves, n_moves, X,
+                       Y, nnz, cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks, status, static_cast<int*>(workspace));
+    return (int)hipGetLastError();
+}
+
+size_t pbs_validate_indices_workspace_bytes(int nnz) { return nnz < 0 ? 0 : validate_ws_bytes(nnz); }
+
+int pbs_validate_indices(const int32_t* cols_a, const int32_t* row_start_ends_a, const int32_t* rows_b,
+                         const int32_t* col_start_ends_b, const int32_t* blocks, int X, int Y, int nnz, int32_t* status,
+                         void* workspace, size_t workspace_bytes, void* stream) {
+    if (X < 1 || Y < 1 || nnz < 0) return PBS_ERR_BAD_SHAPE;
+    if ((long long)X * Y > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    if (!row_start_ends_a || !col_start_ends_b || !status || (nnz > 0 && (!cols_a || !rows_b || !blocks))) return PBS_ERR_NULL_POINTER;
+    const size_t need = validate_ws_bytes(nnz);
+    if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
+    hipLaunchKernelGGL(validate_indices_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), cols_a, row_start_ends_a,
+                       rows_b, col_start_ends_b, blocks, X, Y, nnz, status, static_cast<int*>(workspace));
+    return (int)hipGetLastError();
+}
+
 size_t pbs_blocksparse_matmul_plan_bytes(int n, int k) {
     if (n <= 0 || k <= 0 || (n % 32) || (k % 32)) return 0;
     return all_plan_bytes(n, k);

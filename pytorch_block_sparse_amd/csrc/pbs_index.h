@@ -156,6 +156,161 @@ __global__ __launch_bounds__(INDEX_THREADS) void csr_from_owner_kernel(const int
     if (tid == 0) row_ptr[X] = counted;
 }
 
+// ---- move data blocks (block_replace): all five arrays from the old `blocks` list and a list of moves ----
+// One workgroup, five short phases over the data blocks instead of scans over the grid: every block sets its bit in a bitmap
+// of its row and in one of its column; a row's (column's) start is the sum of the popcounts before it, and a block's place within it
+// the popcount of the bits below its own.  No sort, no search; the bitmaps sit in LDS while they fit (16 K positions take
+// 4 KB, 24 x 96 positions and 1152 blocks 6 us in all, where building a mask, sorting the positions and the two scans of
+// build_indices_kernel took 150 us in a dozen launches).
+constexpr int REPLACE_LDS_WORDS = 12 * 1024;
+enum ReplaceError { REPLACE_BAD_ID = 1, REPLACE_BAD_POSITION = 2, REPLACE_TAKEN = 4 };
+static inline size_t replace_bitmap_words(int X, int Y) { return (size_t)X * ((Y + 31) / 32) + (size_t)Y * ((X + 31) / 32); }
+static inline size_t replace_ws_bytes(int X, int Y, int nnz) {
+    const size_t words = replace_bitmap_words(X, Y);
+    return ((size_t)nnz + (words > REPLACE_LDS_WORDS ? words : 0)) * sizeof(int);
+}
+__global__ __launch_bounds__(INDEX_THREADS) void replace_blocks_kernel(
+    const int32_t* __restrict__ old_blocks, const int64_t* __restrict__ moves, int n_moves, int X, int Y, int nnz, int32_t* cols_a,
+    int32_t* row_ptr, int32_t* rows_b, int32_t* col_ptr, int32_t* blocks, int32_t* status, int* ws) {
+    __shared__ unsigned s_bits[REPLACE_LDS_WORDS];
+    __shared__ int s_wave[17];
+    __shared__ int s_err;
+    const int tid = threadIdx.x;
+    const int wr = (Y + 31) / 32, wc = (X + 31) / 32;   // words per row, per column
+    const int words = X * wr + Y * wc;
+    int* pos = ws;                                      // [nnz] row-major position of every data block
+    unsigned* bits = words > REPLACE_LDS_WORDS ? reinterpret_cast<unsigned*>(ws + nnz) : s_bits;
+    unsigned* row_bits = bits;
+    unsigned* col_bits = bits + (size_t)X * wr;
+    if (tid == 0) s_err = 0;
+    for (int i = tid; i < words; i += INDEX_THREADS) bits[i] = 0u;
+    for (int b = tid; b < nnz; b += INDEX_THREADS) {
+        const int c = old_blocks[2 * b], r = old_blocks[2 * b + 1];
+        pos[b] = c >= 0 && c < Y && r >= 0 && r < X ? r * Y + c : -1;
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int i = tid; i < n_moves; i += INDEX_THREADS) {
+        const int64_t r = moves[3 * (size_t)i], c = moves[3 * (size_t)i + 1], b = moves[3 * (size_t)i + 2];
+        if (b < 0 || b >= nnz) atomicOr(&s_err, REPLACE_BAD_ID);
+        else pos[b] = r >= 0 && r < X && c >= 0 && c < Y ? (int)(r * Y + c) : -1;
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int b = tid; b < nnz; b += INDEX_THREADS) {
+        const int p = pos[b];
+        if (p < 0) {
+            atomicOr(&s_err, REPLACE_BAD_POSITION);
+            continue;
+        }
+        const int r = p / Y, c = p - r * Y;
+        const unsigned was = atomicOr(&row_bits[(size_t)r * wr + (c >> 5)], 1u << (c & 31));
+        if ((was >> (c & 31)) & 1u) atomicOr(&s_err, REPLACE_TAKEN);
+        atomicOr(&col_bits[(size_t)c * wc + (r >> 5)], 1u << (r & 31));
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (s_err) {   // the same for every thread
+        if (tid == 0) *status = s_err;
+        return;
+    }
+    auto starts = [&](const unsigned* line, int n, int w, int32_t* ptr) {
+        int carry = 0;
+        for (int base = 0; base < n; base += INDEX_THREADS) {
+            const int i = base + tid;
+            int cnt = 0;
+            if (i < n)
+                for (int k = 0; k < w; ++k) cnt += __popc(line[(size_t)i * w + k]);
+            int total;
+            const int before = block_exclusive_scan(cnt, s_wave, &total);
+            if (i < n) ptr[i] = carry + before;
+            carry += total;
+        }
+        if (tid == 0) ptr[n] = carry;
+    };
+    starts(row_bits, X, wr, row_ptr);
+    starts(col_bits, Y, wc, col_ptr);
+    __threadfence_block();
+    __syncthreads();
+    auto below = [](const unsigned* line, int at) {
+        int n = __popc(line[at >> 5] & ((1u << (at & 31)) - 1u));
+        for (int k = 0; k < at >> 5; ++k) n += __popc(line[k]);
+        return n;
+    };
+    for (int b = tid; b < nnz; b += INDEX_THREADS) {
+        const int p = pos[b], r = p / Y, c = p - r * Y;
+        const int i = row_ptr[r] + below(row_bits + (size_t)r * wr, c), j = col_ptr[c] + below(col_bits + (size_t)c * wc, r);
+        reinterpret_cast<int2*>(cols_a)[i] = make_int2(c, b);
+        reinterpret_cast<int2*>(rows_b)[j] = make_int2(r, b);
+        reinterpret_cast<int2*>(blocks)[b] = make_int2(c, r);
+    }
+    if (tid == 0) *status = 0;
+}
+
+// ---- consistency of the five arrays, one bit of *status per broken condition (PBS_BAD_* in pbs_hip.h) ----
+// One workgroup; every index is checked before it is used, so any contents are safe to look at.  (The same checks as some
+// seventy tensor operations took 0.5 ms of launches.)
+static inline size_t validate_ws_bytes(int nnz) { return (size_t)nnz * 6 * sizeof(int); }
+__global__ __launch_bounds__(INDEX_THREADS) void validate_indices_kernel(
+    const int32_t* __restrict__ cols_a, const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ rows_b,
+    const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ blocks, int X, int Y, int nnz, int32_t* status, int* ws) {
+    __shared__ int s_bad;
+    const int tid = threadIdx.x;
+    int* seen[2] = {ws, ws + nnz};                                   // times a data block is listed
+    int2* at[2] = {reinterpret_cast<int2*>(ws + 2 * (size_t)nnz), reinterpret_cast<int2*>(ws + 4 * (size_t)nnz)};   // (list, coordinate) of it
+    if (tid == 0) s_bad = 0;
+    for (int b = tid; b < nnz; b += INDEX_THREADS) {
+        seen[0][b] = seen[1][b] = 0;
+        at[0][b] = at[1][b] = make_int2(-1, -1);
+    }
+    __threadfence_block();
+    __syncthreads();
+    int bad = 0;
+    auto list = [&](int which, const int32_t* ids, const int32_t* ends, int lists, int limit) {
+        const int base = 4 * which;
+        for (int i = tid; i <= lists; i += INDEX_THREADS) {
+            const int e = ends[i];
+            if (i == 0 ? e != 0 : e < ends[i - 1]) bad |= PBS_BAD_ROW_STARTS << base;
+            if (i == lists && e != nnz) bad |= PBS_BAD_ROW_END << base;
+        }
+        auto owner = [&](int e) {   // the list that entry e belongs to: the last one that starts at or before it
+            int lo = 0, hi = lists;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (ends[mid + 1] <= e) lo = mid + 1; else hi = mid;
+            }
+            return lo;
+        };
+        for (int e = tid; e < nnz; e += INDEX_THREADS) {
+            const int c = ids[2 * (size_t)e], b = ids[2 * (size_t)e + 1], o = owner(e);
+            if (c < 0 || c >= limit) bad |= PBS_BAD_COLS << base;
+            if (e > 0 && o == owner(e - 1) && c <= ids[2 * (size_t)e - 2]) bad |= which ? PBS_BAD_ROWS_ORDER : PBS_BAD_COLS_ORDER;
+            if (b < 0 || b >= nnz) {
+                bad |= PBS_BAD_COLS_IDS << base;
+            } else {
+                atomicAdd(&seen[which][b], 1);
+                at[which][b] = make_int2(o, c);
+            }
+        }
+    };
+    list(0, cols_a, row_ptr, X, Y);
+    list(1, rows_b, col_ptr, Y, X);
+    __threadfence_block();
+    __syncthreads();
+    for (int b = tid; b < nnz; b += INDEX_THREADS) {
+        if (seen[0][b] != 1) bad |= PBS_BAD_COLS_IDS;
+        if (seen[1][b] != 1) bad |= PBS_BAD_COLS_IDS << 4;
+        const int2 a = at[0][b], t = at[1][b];   // (row, column), (column, row)
+        if (a.x != t.y || a.y != t.x) bad |= PBS_BAD_LISTS_DIFFER;
+        const int c = blocks[2 * (size_t)b], r = blocks[2 * (size_t)b + 1];
+        if (c < 0 || c >= Y || r < 0 || r >= X) bad |= PBS_BAD_BLOCKS;
+        if (c != a.y || r != a.x) bad |= PBS_BAD_BLOCKS_DIFFER;
+    }
+    if (bad) atomicOr(&s_bad, bad);
+    __syncthreads();
+    if (tid == 0) *status = s_bad;
+}
+
 // out[c][r] = in[r][c] for a rows x cols matrix of 2- or 4-byte elements (tiles of 32 x 32 through LDS)
 template <typename U>
 __global__ __launch_bounds__(256) void transpose_dense_kernel(const U* __restrict__ in, U* __restrict__ out, long long rows,

@@ -15,7 +15,6 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
-#include <ATen/ops/empty_like.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
 #include <torch/csrc/Exceptions.h>
@@ -348,7 +347,85 @@ PyObject* py_matmul_back(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {{"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_linear)), METH_FASTCALL, nullptr},
+// one status word that the GPU writes and the host reads after waiting for the stream
+int read_status(const Tensor& status, void* stream) {
+    const hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    TORCH_CHECK(e == hipSuccess, "hipStreamSynchronize: ", hipGetErrorString(e));
+    return *static_cast<const volatile int*>(status.const_data_ptr());
+}
+Tensor status_word() { return at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true)); }
+Tensor workspace(size_t bytes, const Tensor& like) { return at::empty({(int64_t)(bytes ? bytes : 16)}, like.options().dtype(at::kByte)); }
+const int* ints(const Tensor& t) { return static_cast<const int*>(data_or_null(t)); }
+int* ints_out(Tensor& t) { return t.numel() ? t.mutable_data_ptr<int>() : nullptr; }
+
+// replace_blocks(blocks, moves [n, 3] int64, X, Y) -> (status, (blocks, cols_a, row_start_ends_a, rows_b, col_start_ends_b))
+PyObject* py_replace_blocks(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 4, "replace_blocks");
+    const Tensor old = tensor_arg(args[0], "blocks"), moves_any = tensor_arg(args[1], "moves");
+    const int X = (int)PyLong_AsLong(args[2]), Y = (int)PyLong_AsLong(args[3]);
+    check_gpu(old);
+    TORCH_CHECK(old.scalar_type() == at::kInt && old.is_contiguous() && moves_any.scalar_type() == at::kLong && moves_any.device() == old.device() &&
+                    moves_any.dim() == 2 && moves_any.size(1) == 3,
+                "moves should be a [n, 3] int64 tensor on the device of the matrix");
+    const int nnz = (int)(old.numel() / 2);
+    Tensor made[5];
+    int status = 0;
+    {
+        NoGil no_gil;
+        at::NoGradGuard no_grad;
+        const Tensor moves = moves_any.contiguous();
+        c10::DeviceGuard guard(old.device());
+        void* stream = current_stream(old);
+        const int64_t sizes[5][2] = {{2 * (int64_t)nnz, 0}, {nnz, 2}, {X + 1, 0}, {nnz, 2}, {Y + 1, 0}};
+        for (int i = 0; i < 5; ++i) made[i] = at::empty(at::IntArrayRef(sizes[i], sizes[i][1] ? 2 : 1), old.options());
+        const size_t bytes = pbs_replace_blocks_workspace_bytes(X, Y, nnz);
+        Tensor ws = workspace(bytes, old), word = status_word();
+        check(pbs_replace_blocks(ints(old), moves.numel() ? moves.const_data_ptr<int64_t>() : nullptr, (int)moves.size(0), X, Y, nnz,
+                                 ints_out(made[1]), ints_out(made[2]), ints_out(made[3]), ints_out(made[4]), ints_out(made[0]),
+                                 word.mutable_data_ptr<int>(), ws.mutable_data_ptr(), bytes, stream),
+              "pbs_replace_blocks");
+        status = read_status(word, stream);
+    }
+    PyObject* arrays = PyTuple_New(5);
+    for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(arrays, i, THPVariable_Wrap(std::move(made[i])));
+    return Py_BuildValue("(iN)", status, arrays);
+    END_HANDLE_TH_ERRORS
+}
+
+// validate(cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks) -> status
+PyObject* py_validate(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 5, "validate");
+    Tensor t[5];
+    for (int i = 0; i < 5; ++i) {
+        t[i] = tensor_arg(args[i], "index buffer");
+        check_gpu(t[i]);
+        TORCH_CHECK(t[i].scalar_type() == at::kInt && t[i].device() == t[0].device(), "index buffers should be int32 and on one device");
+    }
+    TORCH_CHECK(t[0].numel() == t[2].numel() && t[0].numel() == t[4].numel() && t[1].numel() >= 2 && t[3].numel() >= 2, "index buffers differ in length");
+    int status = 0;
+    {
+        NoGil no_gil;
+        at::NoGradGuard no_grad;
+        for (Tensor& x : t) x = x.contiguous();
+        c10::DeviceGuard guard(t[0].device());
+        void* stream = current_stream(t[0]);
+        const int nnz = (int)(t[0].numel() / 2);
+        const size_t bytes = pbs_validate_indices_workspace_bytes(nnz);
+        Tensor ws = workspace(bytes, t[0]), word = status_word();
+        check(pbs_validate_indices(ints(t[0]), ints(t[1]), ints(t[2]), ints(t[3]), ints(t[4]), (int)t[1].numel() - 1, (int)t[3].numel() - 1, nnz,
+                                   word.mutable_data_ptr<int>(), ws.mutable_data_ptr(), bytes, stream),
+              "pbs_validate_indices");
+        status = read_status(word, stream);
+    }
+    return PyLong_FromLong(status);
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {{"replace_blocks", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_replace_blocks)), METH_FASTCALL, nullptr},
+                         {"validate", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_validate)), METH_FASTCALL, nullptr},
+                         {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_linear)), METH_FASTCALL, nullptr},
                          {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_matmul)), METH_FASTCALL, nullptr},
                          {"matmul_back", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_matmul_back)), METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

@@ -29,6 +29,10 @@ _PROTOTYPES = {
     "pbs_abi_version": (ctypes.c_int, []),
     "pbs_error_string": (ctypes.c_char_p, [_i32]),
     "pbs_build_indices": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "pbs_replace_blocks_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32]),
+    "pbs_replace_blocks": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]),
+    "pbs_validate_indices_workspace_bytes": (ctypes.c_size_t, [_i32]),
+    "pbs_validate_indices": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "pbs_blocksparse_matmul_plan_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "pbs_blocksparse_matmul_plan": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "pbs_blocksparse_matmul_plan_part": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),

@@ -1,0 +1,65 @@
+"""block_replace and validate_indices of a matrix on the GPU (one kernel each) against the host versions, bit for bit and
+message for message: grids whose bitmaps fit LDS and one whose do not, line lengths around multiples of 32."""
+import numpy as np
+import pytest
+import torch
+
+from pytorch_block_sparse_amd import BlockSparseMatrix
+
+pytestmark = pytest.mark.gpu
+NAMES = ("blocks", "cols_a", "row_start_ends_a", "rows_b", "col_start_ends_b")
+
+
+def _pair(X, Y, nnz, cuda):
+    np.random.seed(X + Y + nnz)
+    host = BlockSparseMatrix.zeros((32 * X, 32 * Y), nnz, device="cpu")
+    gpu = BlockSparseMatrix.zeros((32 * X, 32 * Y), nnz, device="cpu").to(cuda)
+    gpu.load_state_dict(host.state_dict())
+    return host, gpu
+
+
+@pytest.mark.parametrize("X, Y, nnz, moved", [(1, 2, 1, 1), (31, 33, 200, 20), (64, 32, 1500, 548), (96, 24, 1152, 0), (640, 640, 5000, 1234)])
+def test_moves_match_the_host(cuda, X, Y, nnz, moved):
+    print(X, Y, nnz, moved, flush=True)
+    host, gpu = _pair(X, Y, nnz, cuda)
+    for turn in range(2):   # the second turn starts from recycled data blocks
+        free = (~host.block_mask_build(None)).nonzero()
+        to = free[torch.randperm(free.shape[0])[:moved]]
+        rep = torch.cat([to, torch.randperm(nnz)[:moved, None]], 1)
+        host.block_replace(rep)
+        gpu.block_replace(rep.to(cuda))
+        for name in NAMES:
+            assert torch.equal(getattr(host, name), getattr(gpu, name).cpu()), name
+        gpu.validate_indices()
+
+
+def test_bad_moves_raise_and_change_nothing(cuda):
+    _, gpu = _pair(8, 6, 20, cuda)
+    before = {n: getattr(gpu, n).clone() for n in NAMES}
+    taken = gpu.build_coo_block_index()[:, 0].tolist()
+    for rep in ([[0, 0, 20]], [[0, 0, -1]], [[8, 0, 0]], [[0, -1, 0]], [[taken[0], taken[1], 1]]):
+        with pytest.raises(Exception, match="block_replacements"):
+            gpu.block_replace(torch.tensor(rep, device=cuda))
+        assert all(torch.equal(getattr(gpu, n), before[n]) for n in NAMES)
+
+
+def test_broken_buffers_give_the_message_of_the_host(cuda):
+    host, gpu = _pair(40, 33, 300, cuda)
+    ends = host.row_start_ends_a.tolist()
+    e0 = next(ends[r] for r in range(40) if ends[r + 1] - ends[r] >= 2)
+    nnz = 300
+    changes = [("row_start_ends_a", 0, 1), ("row_start_ends_a", 3, nnz + 1), ("row_start_ends_a", 40, nnz + 5), ("col_start_ends_b", 2, -4),
+               ("col_start_ends_b", 33, nnz - 1), ("cols_a", (0, 0), 33), ("rows_b", (5, 0), -1), ("cols_a", (7, 1), nnz), ("rows_b", (0, 1), int(host.rows_b[1, 1])),
+               ("blocks", 0, 1000), ("blocks", 1, 39 if int(host.blocks[1]) != 39 else 0), ("cols_a", (e0 + 1, 0), int(host.cols_a[e0, 0]))]
+    for name, at, value in changes:
+        messages = []
+        for m in (host, gpu):
+            t = getattr(m, name)
+            keep = t[at].clone()
+            t[at] = value
+            with pytest.raises(Exception) as e:
+                m.validate_indices()
+            messages.append(str(e.value))
+            t[at] = keep
+            m.validate_indices()
+        assert messages[0] == messages[1], (name, at, value)
