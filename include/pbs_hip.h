@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 5
+#define PBS_ABI_VERSION 6
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -192,10 +192,10 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
  *   Every token is accumulated (the reference drops tokens % 32 when tokens > 32).
  *   `out` need not be zeroed.
  *
- * When the tile grid alone cannot fill the GPU the token range is split over
- * workgroups and the fp32 partial blocks are summed in a fixed order by a second
- * kernel; that needs `workspace` of pbs_blocksparse_matmul_back_workspace_bytes()
- * bytes (16-byte aligned device memory; may be NULL when that returns 0).
+ * When the blocks alone cannot fill the GPU the token range is split over workgroups and the fp32
+ * partial blocks are summed in a fixed order by a second kernel; they and the unit table (below) lie
+ * in `workspace`: pbs_blocksparse_matmul_back_workspace_bytes() bytes of 16-byte aligned device memory
+ * (may be NULL when that returns 0).
  */
 size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_features, int in_features,
                                                    int nnz, int dtype);
@@ -204,6 +204,30 @@ int pbs_blocksparse_matmul_back(const void* dense_a, const void* dense_b,
                                 void* data_out,
                                 int64_t tokens, int out_features, int in_features, int nnz,
                                 int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * The same product, and the bias gradient bias_out[n] = sum_t dense_a[t][n] (NULL: not wanted) from the same pass over
+ * dense_a, for a caller that keeps what depends on the pattern alone.  No counterpart in the reference, which
+ * sums the bias gradient on its own (block_sparse_linear.py:28-47).
+ *
+ *   units   the table of the work of the pattern's rows, made by pbs_blocksparse_matmul_back_units in
+ *           pbs_blocksparse_matmul_back_units_bytes() bytes of 16-byte aligned device memory.  It depends on the
+ *           pattern only and serves every number of tokens and both dtypes.  ..._units_bytes returns 0 for problems whose kernel uses
+ *           none (units may then be NULL); those do not take bias_out either (PBS_ERR_BAD_SHAPE).
+ *   workspace: pbs_blocksparse_matmul_back_bias_workspace_bytes() bytes, may be NULL when that is 0.
+ *
+ * nnz may be 0 with a bias_out; data_out may then be NULL.
+ */
+size_t pbs_blocksparse_matmul_back_units_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype);
+int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int32_t* cols_a, int out_features, int in_features,
+                                      int nnz, void* units, size_t units_bytes, void* stream);
+size_t pbs_blocksparse_matmul_back_bias_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz,
+                                                        int dtype);
+int pbs_blocksparse_matmul_back_bias(const void* dense_a, const void* dense_b,
+                                     const int32_t* row_start_ends_a, const int32_t* cols_a, const void* units,
+                                     void* data_out, void* bias_out,
+                                     int64_t tokens, int out_features, int in_features, int nnz,
+                                     int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * The same product with the arguments of the reference's entry point blocksparse_matmul_back_cutlass
@@ -235,14 +259,14 @@ int pbs_blocksparse_matmul_back_blocks(const void* dense_a, int a_row_major, con
 /*
  * pbs_blocksparse_matmul_back for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
- * reference.  Same arguments, same kernels and bit-identical results as pbs_blocksparse_matmul_back,
- * without the workspace pair: the fp32 partial sums of a split token range go to a device array of
+ * reference.  Same arguments and kernels as pbs_blocksparse_matmul_back, and where that one's workspace would fit the array bit-identical
+ * results, without the workspace pair: the fp32 partial sums of a split token range go to a device array of
  * PBS_NOALLOC_SCRATCH_BYTES (64 MiB) that is part of the library (every GPU the library is used on
  * holds its own copy until the process ends).  The call makes no hipMalloc/hipFree and calls no
  * allocating routine.
  *
- *   - A problem whose pbs_blocksparse_matmul_back_workspace_bytes() exceeds the array is rejected
- *     with PBS_ERR_SCRATCH before anything is launched (4096 x 4096 at density 0.25 with 16384
+ *   - A problem of the row kernel whose pbs_blocksparse_matmul_back_workspace_bytes() exceeds the array runs with fewer slices
+ *     of the tokens; one of the rectangle kernel is rejected with PBS_ERR_SCRATCH before anything is launched (4096 x 4096 at density 0.25 with 16384
  *     tokens in bf16 needs exactly 64 MiB and fits).
  *   - Nothing in the array has to be cleared between calls: every word the reduction kernel reads
  *     is written by the product kernel of the same call first.
@@ -271,7 +295,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
  * the device.  The Python layer checks it after every product when PBS_DEBUG is set and raises.
  *
  * pbs_blocksparse_matmul_kernel_name / ..._back_kernel_name: which kernel(s) a call with these sizes runs
- * ("stream_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_seg_kernel", "sdd_kernel", "sdd_bf16_kernel", with
+ * ("stream_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel", "sdd_bf16_kernel", with
  * " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
  */

@@ -71,21 +71,6 @@ static __device__ __forceinline__ int acc_row(int v, int h) { return 8 * (v >> 2
 // pointer array then selects wrong entries instead of reading outside the entry list.
 static __device__ __forceinline__ int clamp_entry(int v, int nnz) { return v < 0 ? 0 : (v > nnz ? nnz : v); }
 
-static __device__ __forceinline__ uint4 ldg16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
-
-// Two 16-byte rows of 8 bf16 (row k even, row k odd, same 8 columns) -> 8 words, word n holding
-// (row_even[n] low half, row_odd[n] high half): the k-pair packing the bf16 MFMA operands want.
-static __device__ __forceinline__ void interleave_bf16_rows(const uint4& r0, const uint4& r1, uint4& lo, uint4& hi) {
-    lo.x = (r0.x & 0xffffu) | (r1.x << 16);
-    lo.y = (r0.x >> 16) | (r1.x & 0xffff0000u);
-    lo.z = (r0.y & 0xffffu) | (r1.y << 16);
-    lo.w = (r0.y >> 16) | (r1.y & 0xffff0000u);
-    hi.x = (r0.z & 0xffffu) | (r1.z << 16);
-    hi.y = (r0.z >> 16) | (r1.z & 0xffff0000u);
-    hi.z = (r0.w & 0xffffu) | (r1.w << 16);
-    hi.w = (r0.w >> 16) | (r1.w & 0xffff0000u);
-}
-
 // ds_read_b64_tr_b16: within each group of 16 lanes, lane s passes the LDS address of 4 consecutive
 // 16-bit elements (row s/4 of a 4 x 16 tile, columns 4*(s%4)..+3) and lane j receives column j of
 // the tile: the 4 rows' elements, in row order.

@@ -15,7 +15,7 @@
 #include "pbs_index.h"
 #include "pbs_sdd.h"
 #include "pbs_sdd_bf16.h"
-#include "pbs_sdd_seg.h"
+#include "pbs_sdd_row.h"
 
 namespace pbs {
 
@@ -389,38 +389,23 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
 }
 
 // ---- sparse-output product ----
-// fp32: equal shares of the blocks of a band of 16 block rows, 16-token chunks by DMA (pbs_sdd_seg.h); rectangles
-// of 8 x 8 block positions staged through registers (pbs_sdd.h) where that kernel does not apply.
-// bf16: 16 x 16 rectangles, 32-token chunks by DMA.
-struct SddShapeF32 {
-    int SR, SC, QW;
-};
-constexpr int SDD_F32_NSHAPES = 1;
-constexpr SddShapeF32 SDD_F32_SHAPES[SDD_F32_NSHAPES] = {{8, 8, 8}};
-constexpr int SDD_F32_NW = 8, SDD_F32_TC = 16;
+// Two kernels: up to four blocks of a block row per workgroup (pbs_sdd_row.h), which serves fp32 altogether and
+// bf16 while the operands are small enough, and for large bf16 problems rectangles of 16 x 16 block positions
+// (pbs_sdd_bf16.h).
 struct SddShapeBf16 {
     static constexpr int SR = 16, SC = 16, QW = 10, TC = 32, NS = 2, NW = 8;
 };
-
 struct SddPlan {
     int tiles_r, tiles_c, nsplit, tokens_per_split;
-    int shape;   // fp32: index into SDD_F32_SHAPES, or SDD_F32_SEGMENTS
-    int segs;    // segment kernel: shares per row band
 };
-constexpr int SDD_F32_SEGMENTS = SDD_F32_NSHAPES;
-constexpr int SEG_SR = 16, SEG_QW = 9;
-constexpr int SEG_NSC = 2;
-constexpr int SEG_SC[SEG_NSC] = {16, 20};   // X panel widths of the two builds of the segment kernel
-
-static SddPlan plan_sdd(long long M, int N, int K, int SR, int SC, int TC) {
+static SddPlan plan_sdd(long long M, int N, int K) {
+    constexpr int SR = SddShapeBf16::SR, SC = SddShapeBf16::SC, TC = SddShapeBf16::TC;
     SddPlan p;
-    p.shape = 0;
-    p.segs = 0;
     p.tiles_r = (N / 32 + SR - 1) / SR;
     p.tiles_c = (K / 32 + SC - 1) / SC;
     const long long tiles = (long long)p.tiles_r * p.tiles_c;
     const long long chunks = (M + TC - 1) / TC;
-    // Aim at one workgroup per CU and never slightly more (the kernels' registers and LDS allow one
+    // Aim at one workgroup per CU and never slightly more (the kernel's registers and LDS allow one
     // workgroup per CU, so 257 workgroups take twice as long as 256); keep at least 8 chunks per slice.
     long long want = 256 / tiles;
     long long cap = chunks / 8;
@@ -433,141 +418,167 @@ static SddPlan plan_sdd(long long M, int N, int K, int SR, int SC, int TC) {
     p.tokens_per_split = (int)(chunks_per * TC);
     return p;
 }
-// fp32: which kernel, and how the work is cut.  A workgroup's time per chunk of tokens is set by its busiest
-// wave, i.e. by rounds = ceil(blocks of the workgroup / 8), and the launch ends with its slowest workgroup.  The
-// estimate for either kernel is chunks per workgroup x (rounds + a half for the chunk's staging and barriers).
-// Rectangles: the fullest of the rectangles expected under a uniform pattern of the given density (33 blocks
-// on 8 waves cost 5 rounds for 4.1 rounds of work).
-static SddPlan plan_sdd_f32(long long M, int N, int K, long long nnz) {
-    const SddShapeF32 sh = SDD_F32_SHAPES[0];
-    SddPlan best = plan_sdd(M, N, K, sh.SR, sh.SC, SDD_F32_TC);
-    const double positions = (double)(N / 32) * (double)(K / 32);
-    const double d = positions > 0 ? (double)nnz / positions : 0.0;
-    double best_cost;
-    {
-        const int sr = N / 32 < sh.SR ? N / 32 : sh.SR, sc = K / 32 < sh.SC ? K / 32 : sh.SC;
-        const double mean = sr * sc * d;
-        const double full = (double)((N / 32) / sh.SR > 0 ? (N / 32) / sh.SR : 1) * ((K / 32) / sh.SC > 0 ? (K / 32) / sh.SC : 1);
-        const double spread = std::sqrt(mean * (1.0 - d)) * std::sqrt(2.0 * std::log(full < 2.0 ? 2.0 : full));
-        double fullest = mean + spread;
-        if (fullest > sr * sc) fullest = sr * sc;
-        double rounds = std::ceil(fullest / SDD_F32_NW);
-        if (rounds < 1.0) rounds = 1.0;
-        if (fullest > sh.QW * SDD_F32_NW) rounds *= 2.0;   // a second pass over the tokens
-        best_cost = (double)best.tokens_per_split / SDD_F32_TC * (rounds + 0.5);
-    }
-    // Equal shares of each row band's blocks (pbs_sdd_seg.h): every workgroup does `rounds` products per chunk.
-    // A share of 8 x rounds blocks spans about that many / (rows x density) block columns, which must fit the
-    // kernel's X panel; bands differ a little in their block counts, so the shares are sized for a band two
-    // standard deviations above the mean.  Of the feasible rounds the one with the smallest chunks x rounds wins.
-    const int nblk_r = N / 32, ncols = K / 32;
-    for (int v = 0; v < SEG_NSC; ++v) {
-        // the histogram of a band's block columns borrows the stage buffers
-        const int max_cols = 2 * 16 * (SEG_SR + SEG_SC[v]) * 128 / 4 - 64;
-        if (ncols > max_cols || nnz <= 0 || d <= 0.0) continue;
-        const int bands = (nblk_r + SEG_SR - 1) / SEG_SR;
-        const int rows_per_band = (nblk_r + bands - 1) / bands;
-        const double n_band = (double)nnz * rows_per_band / nblk_r;
-        const double heavy = n_band + (bands > 1 ? 2.0 * std::sqrt(n_band * (1.0 - d)) : 0.0);
-        const long long chunks = (M + SDD_F32_TC - 1) / SDD_F32_TC;
-        for (int q = 1; q <= SEG_QW; ++q) {
-            const double share = 8.0 * q;
-            if (share / (rows_per_band * d) + 2.0 > SEG_SC[v]) break;   // wider than the X panel
-            long long segs = (long long)std::ceil(heavy / share);
-            if (segs < 1) segs = 1;
-            const long long wgs1 = (long long)bands * segs;
-            long long want = 256 / wgs1, cap = chunks / 8;
-            if (cap < 1) cap = 1;
-            if (want > cap) want = cap;
-            if (want < 1) want = 1;
-            const long long chunks_per = (chunks + want - 1) / want;
-            const long long nsplit = (chunks + chunks_per - 1) / chunks_per;
-            const double waves_of_wgs = std::ceil((double)(wgs1 * nsplit) / 256.0);
-            const double rounds = std::ceil(n_band / segs / 8.0);
-            // the wider panel costs a few per cent (more bytes staged per chunk)
-            const double cost = (double)chunks_per * (rounds + 0.5) * waves_of_wgs * (1.0 + 0.04 * v);
-            if (cost < best_cost) {
-                best_cost = cost;
-                best.shape = SDD_F32_SEGMENTS + v;
-                best.tiles_r = bands;
-                best.tiles_c = 1;
-                best.segs = (int)segs;
-                best.nsplit = (int)nsplit;
-                best.tokens_per_split = (int)(chunks_per * SDD_F32_TC);
-            }
+// Estimated time in us, fitted to 60 measured problems (128 .. 4096 features, 64 .. 16384 tokens, densities 0.05 .. 0.75;
+// the choices made by it were 3.5 % slower than the best of all slice counts on average): launch, reduction of the slices,
+// chunks x blocks of a wave of the slowest workgroup, at the rate of a full chip or, below 32 workgroups per XCD, of
+// a wave alone, and what each round of workgroups on the chip costs besides.
+static double row_us(int dtype, long long M, int N, int nnz, int slices) {
+    struct Model {
+        double launch, reduce, per_slice, busy, alone, round;
+        int resident;   // workgroups per XCD
+    };
+    const Model m = dtype == PBS_DTYPE_F32 ? Model{3.34, 6.57, 0.0, 0.523, 0.058, 2.34, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
+    const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
+    const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows;
+    const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
+    const double tasks = std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices)) * blocks;
+    const double busy = std::ceil(tasks / 32) * wave * m.busy, alone = wave * m.alone;
+    return m.launch + (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) + (busy > alone ? busy : alone) +
+           std::ceil(tasks / m.resident) * m.round;
+}
+static double rectangle_us(long long M, int N, int K, int nnz) {
+    const SddPlan p = plan_sdd(M, N, K);
+    const double tiles = (double)p.tiles_r * p.tiles_c, blocks = nnz / tiles;
+    const double rounds = std::ceil(tiles * p.nsplit / 256), passes = std::ceil(blocks / (SddShapeBf16::QW * SddShapeBf16::NW));
+    return 15.1 + rounds * (p.tokens_per_split / SddShapeBf16::TC) * (0.4903 * passes + 0.1019 * blocks / 8) +
+           (p.nsplit > 1 ? 3.65 + 1.45 * p.nsplit * nnz / 1000.0 : 0.0);
+}
+// The kernel and, for the row kernel, the number of token slices (0: rectangles).
+static int choose_row_slices(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
+    constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
+    const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
+    // Workgroups of different rows read the same columns of X: they find them in the caches while the operands (fp32: a slice
+    // of them) are about the size of the L2s.  bf16 beyond that size: 250 us where the rectangles, which read
+    // every panel once per 16 rows, take 216.
+    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return 0;
+    const long long chunks = (M + ROW_TC - 1) / ROW_TC;
+    const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
+    int best = 1;
+    double best_us = 0.0;
+    for (const int s : CANDIDATES) {
+        if (s > 1 && (s > chunks / 4 || ((double)nnz * 1024 + N) * sizeof(float) * s > (double)workspace_limit)) break;
+        const double us = row_us(dtype, M, N, nnz, s);
+        if (s == 1 || best < at_least || us < best_us) {
+            best = s;
+            best_us = us;
         }
     }
-    return best;
+    return dtype == PBS_DTYPE_BF16 && rectangle_us(M, N, K, nnz) < best_us ? 0 : best;
 }
-static SddPlan plan_sdd_for(int dtype, long long M, int N, int K, long long nnz) {
-    if (dtype == PBS_DTYPE_F32) return plan_sdd_f32(M, N, K, nnz);
-    return plan_sdd(M, N, K, SddShapeBf16::SR, SddShapeBf16::SC, SddShapeBf16::TC);
+struct BackPlan {
+    int slices;   // row kernel; 0: rectangles
+    int chunks_per_slice;
+    SddPlan rect;
+    size_t partial_bytes;
+};
+static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit = ~(size_t)0) {
+    BackPlan p;
+    p.slices = choose_row_slices(dtype, M, N, K, nnz, workspace_limit);
+    p.rect = plan_sdd(M, N, K);
+    int n = p.rect.nsplit;
+    if (p.slices > 0) {
+        const long long chunks = (M + ROW_TC - 1) / ROW_TC;
+        p.chunks_per_slice = (int)((chunks + p.slices - 1) / p.slices);
+        p.slices = n = (int)((chunks + p.chunks_per_slice - 1) / p.chunks_per_slice);
+    }
+    // fp32 sums of each slice (row kernel: blocks, then bias columns)
+    p.partial_bytes = n > 1 ? ((size_t)nnz * 1024 + (p.slices > 0 ? N : 0)) * sizeof(float) * n : 0;
+    return p;
 }
 
-template <int SHAPE>
-static int launch_sdd_f32(const SddArgs& a, long long wgs, hipStream_t stream) {
-    constexpr SddShapeF32 S = SDD_F32_SHAPES[SHAPE];
-    using C = SddCfg<float, S.SR, S.SC, S.QW, SDD_F32_NW>;
-    static_assert(C::TC == SDD_F32_TC, "plan and kernel must agree on the chunk size");
-    static std::atomic<uint64_t> done{0};
-    auto kernel = sdd_kernel<float, S.SR, S.SC, S.QW, SDD_F32_NW>;
-    if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
-    return (int)hipGetLastError();
-}
+struct BackArgs {
+    const void *g, *x;       // [M, N] grad_output, [M, K] input
+    const int32_t *ptr, *idx;
+    const void* units;       // nullptr: built in the workspace
+    void* out;               // [nnz*32, 32]
+    void* bias_out;          // nullptr or [N]
+    int M, N, K, nnz;
+};
 
-template <int V>
-static int launch_sdd_seg(const SddArgs& a, long long wgs, hipStream_t stream) {
-    using C = SddSegCfg<SEG_SR, SEG_SC[V], SEG_QW, SDD_F32_NW>;
-    static_assert(C::MAX_COLS == 2 * 16 * (SEG_SR + SEG_SC[V]) * 128 / 4 - 64, "the plan's column limit is the kernel's");
-    static_assert(C::TC == SDD_F32_TC, "plan and kernel must agree on the chunk size");
-    static std::atomic<uint64_t> done{0};
-    auto kernel = sdd_seg_kernel<SEG_SR, SEG_SC[V], SEG_QW, SDD_F32_NW>;
-    if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
+static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int nnz, void* table, hipStream_t stream) {
+    const long long units = unit_bound(N, nnz);
+    int* t = static_cast<int*>(table);
+    int* before = nullptr;
+    if (unit_prefix_bytes(N)) {
+        before = t + 16 + units * UNIT_INTS;
+        hipLaunchKernelGGL(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, before);
+    }
+    hipLaunchKernelGGL(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, ptr, idx, nnz, N / 32, K / 32, before,
+                       (int)units, t);
     return (int)hipGetLastError();
 }
 
 template <typename T>
-static int launch_sdd(SddArgs a, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    const SddPlan p = plan_sdd_for(dtype, a.M, a.N, a.K, a.nnz);
+static int launch_reduce(const float* partial, void* out, size_t n, void* bias_out, size_t nbias, size_t stride, int nsplit, hipStream_t stream) {
+    const size_t total = n + (bias_out ? nbias : 0);
+    hipLaunchKernelGGL(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(out), n,
+                       static_cast<T*>(bias_out), total, stride, nsplit);
+    return (int)hipGetLastError();
+}
+
+template <typename T>
+static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const size_t need = p.partial_bytes + (a.units ? 0 : unit_table_bytes(a.N, a.nnz));
+    if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
+    const long long grid = NUM_XCD * (long long)p.slices * ((unit_bound(a.N, a.nnz) + NUM_XCD - 1) / NUM_XCD);
+    if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    SddRowArgs r;
+    r.g = a.g;
+    r.x = a.x;
+    r.table = static_cast<const int*>(a.units);
+    if (!a.units) {
+        void* table = static_cast<unsigned char*>(workspace) + p.partial_bytes;
+        if (int rc = build_units(a.ptr, a.idx, a.N, a.K, a.nnz, table, stream)) return rc;
+        r.table = static_cast<const int*>(table);
+    }
+    r.out = a.out;
+    r.bias_out = a.bias_out;
+    r.partial = p.partial_bytes ? static_cast<float*>(workspace) : nullptr;
+    r.M = a.M;
+    r.N = a.N;
+    r.K = a.K;
+    r.nnz = a.nnz;
+    r.slices = p.slices;
+    r.chunks_per_slice = p.chunks_per_slice;
+    hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
+    if (int rc = (int)hipGetLastError()) return rc;
+    const size_t n = (size_t)a.nnz * 1024;
+    return p.partial_bytes ? launch_reduce<T>(r.partial, a.out, n, a.bias_out, a.N, n + a.N, p.slices, stream) : PBS_OK;
+}
+
+static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    const SddPlan& p = plan.rect;
+    SddArgs a;
+    a.g = b.g;
+    a.x = b.x;
+    a.ptr = b.ptr;
+    a.idx = b.idx;
+    a.out = b.out;
+    a.partial = nullptr;
+    a.M = b.M;
+    a.N = b.N;
+    a.K = b.K;
+    a.nnz = b.nnz;
     a.tiles_r = p.tiles_r;
     a.tiles_c = p.tiles_c;
     a.nsplit = p.nsplit;
     a.tokens_per_split = p.tokens_per_split;
-    a.segs = p.segs;
-    a.partial = nullptr;
     const size_t n = (size_t)a.nnz * 1024;
     if (p.nsplit > 1) {
-        const size_t need = n * sizeof(float) * p.nsplit;
-        if (!workspace || workspace_bytes < need || !aligned16(workspace)) return PBS_ERR_WORKSPACE;
+        if (!workspace || workspace_bytes < plan.partial_bytes || !aligned16(workspace)) return PBS_ERR_WORKSPACE;
         a.partial = static_cast<float*>(workspace);
     }
-    const long long wgs = (long long)p.tiles_r * (p.segs > 0 ? p.segs : p.tiles_c) * p.nsplit;
+    const long long wgs = (long long)p.tiles_r * p.tiles_c * p.nsplit;
     if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    if constexpr (sizeof(T) == 4) {
-        const int rc = p.shape == SDD_F32_SEGMENTS ? launch_sdd_seg<0>(a, wgs, stream)
-                       : p.shape == SDD_F32_SEGMENTS + 1 ? launch_sdd_seg<1>(a, wgs, stream)
-                                                         : launch_sdd_f32<0>(a, wgs, stream);
-        if (rc) return rc;
-    } else {
-        using S = SddShapeBf16;
-        using C = SddBf16Cfg<S::QW, S::TC, S::NS, S::NW>;
-        static_assert(C::TC == S::TC && C::SR == S::SR && C::SC == S::SC, "plan and kernel must agree");
-        static std::atomic<uint64_t> done{0};
-        auto kernel = sdd_bf16_kernel<S::QW, S::TC, S::NS, S::NW>;
-        if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
-        hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
-    }
-    int rc = (int)hipGetLastError();
-    if (rc) return rc;
-    if (p.nsplit > 1) {
-        const unsigned grid = (unsigned)((n / 4 + 255) / 256);
-        hipLaunchKernelGGL(sdd_reduce_kernel<T>, dim3(grid), dim3(256), 0, stream, a.partial, static_cast<T*>(a.out), n,
-                           p.nsplit);
-        rc = (int)hipGetLastError();
-    }
-    return rc;
+    using S = SddShapeBf16;
+    using C = SddBf16Cfg<S::QW, S::TC, S::NS, S::NW>;
+    static_assert(C::TC == S::TC && C::SR == S::SR && C::SC == S::SC, "plan and kernel must agree");
+    static std::atomic<uint64_t> done{0};
+    auto kernel = sdd_bf16_kernel<S::QW, S::TC, S::NS, S::NW>;
+    if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
+    if (int rc = (int)hipGetLastError()) return rc;
+    return p.nsplit > 1 ? launch_reduce<bf16_t>(a.partial, a.out, n, nullptr, 0, n, p.nsplit, stream) : PBS_OK;
 }
 
 // ---- scratch of the entry point that allocates nothing ----
@@ -776,50 +787,79 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
                      : dispatch_dds<bf16_t, 1>(g, nullptr, 0, s);
 }
 
+static bool back_sizes_ok(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    return tokens > 0 && out_features > 0 && in_features > 0 && nnz >= 0 && out_features % 32 == 0 && in_features % 32 == 0 &&
+           (dtype == PBS_DTYPE_F32 || dtype == PBS_DTYPE_BF16);
+}
+
+size_t pbs_blocksparse_matmul_back_units_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
+    return plan_back(dtype, tokens, out_features, in_features, nnz).slices > 0 ? unit_table_bytes(out_features, nnz) : 0;
+}
+
+int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int32_t* cols_a, int out_features, int in_features,
+                                      int nnz, void* units, size_t units_bytes, void* stream) {
+    if (out_features <= 0 || in_features <= 0 || nnz < 0 || (out_features % 32) || (in_features % 32)) return PBS_ERR_BAD_SHAPE;
+    if ((long long)nnz > (long long)(out_features / 32) * (in_features / 32)) return PBS_ERR_TOO_LARGE;
+    if (!row_start_ends_a || (nnz > 0 && !cols_a) || !units) return PBS_ERR_NULL_POINTER;
+    if (!aligned16(units)) return PBS_ERR_MISALIGNED;
+    if (units_bytes < unit_table_bytes(out_features, nnz)) return PBS_ERR_WORKSPACE;
+    return build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, units, static_cast<hipStream_t>(stream));
+}
+
+size_t pbs_blocksparse_matmul_back_bias_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
+    return plan_back(dtype, tokens, out_features, in_features, nnz).partial_bytes;
+}
+
 size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz,
                                                    int dtype) {
-    if (tokens <= 0 || out_features <= 0 || in_features <= 0 || nnz <= 0) return 0;
-    if ((out_features % 32) || (in_features % 32)) return 0;
-    if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return 0;
-    const SddPlan p = plan_sdd_for(dtype, tokens, out_features, in_features, nnz);
-    if (p.nsplit <= 1) return 0;
-    return (size_t)nnz * 1024 * sizeof(float) * p.nsplit;
+    if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype) || nnz == 0) return 0;
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz);
+    return p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz) : 0);
+}
+
+static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,
+                size_t workspace_limit = ~(size_t)0) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return PBS_ERR_BAD_DTYPE;
+    if (tokens < 0 || a.N <= 0 || a.K <= 0 || a.nnz < 0 || (a.N % 32) || (a.K % 32)) return PBS_ERR_BAD_SHAPE;
+    if (tokens > (1ll << 30) || (long long)a.nnz > (long long)(a.N / 32) * (a.K / 32)) return PBS_ERR_TOO_LARGE;
+    if (a.nnz == 0 && !a.bias_out) return PBS_OK;
+    if (!a.ptr || (a.nnz > 0 && (!a.idx || !a.out))) return PBS_ERR_NULL_POINTER;
+    if (tokens > 0 && (!a.g || !a.x)) return PBS_ERR_NULL_POINTER;
+    if (!aligned16(a.g) || !aligned16(a.x) || !aligned16(a.out) || !aligned16(a.bias_out) || !aligned16(a.units)) return PBS_ERR_MISALIGNED;
+    if (tokens == 0) {
+        const size_t esz = dtype == PBS_DTYPE_F32 ? 4 : 2;
+        auto zero = [&](void* p, size_t values) {
+            const size_t nwords = values * esz / 4;
+            hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s, static_cast<uint32_t*>(p), nwords);
+            return (int)hipGetLastError();
+        };
+        if (a.nnz > 0)
+            if (int rc = zero(a.out, (size_t)a.nnz * 1024)) return rc;
+        return a.bias_out ? zero(a.bias_out, a.N) : PBS_OK;
+    }
+    const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, workspace_limit);
+    if (p.slices == 0) return a.bias_out ? PBS_ERR_BAD_SHAPE : launch_rectangles(a, p, workspace, workspace_bytes, s);
+    return dtype == PBS_DTYPE_F32 ? launch_row<float>(a, p, workspace, workspace_bytes, s) : launch_row<bf16_t>(a, p, workspace, workspace_bytes, s);
 }
 
 int pbs_blocksparse_matmul_back(const void* dense_a, const void* dense_b, const int32_t* row_start_ends_a,
                                 const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                 int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
                                 void* stream) {
-    if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return PBS_ERR_BAD_DTYPE;
-    if (tokens < 0 || out_features <= 0 || in_features <= 0 || nnz < 0 || (out_features % 32) || (in_features % 32))
-        return PBS_ERR_BAD_SHAPE;
-    if (tokens > (1ll << 30) || (long long)nnz > (long long)(out_features / 32) * (in_features / 32))
-        return PBS_ERR_TOO_LARGE;
-    if (nnz == 0) return PBS_OK;
-    if (!row_start_ends_a || !cols_a || !data_out) return PBS_ERR_NULL_POINTER;
-    if (tokens > 0 && (!dense_a || !dense_b)) return PBS_ERR_NULL_POINTER;
-    if (!aligned16(dense_a) || !aligned16(dense_b) || !aligned16(data_out)) return PBS_ERR_MISALIGNED;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (tokens == 0) {
-        const size_t nwords = (size_t)nnz * 1024 * (dtype == PBS_DTYPE_F32 ? 4 : 2) / 4;
-        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s,
-                           static_cast<uint32_t*>(data_out), nwords);
-        return (int)hipGetLastError();
-    }
-    SddArgs a;
-    a.g = dense_a;
-    a.x = dense_b;
-    a.ptr = row_start_ends_a;
-    a.idx = cols_a;
-    a.out = data_out;
-    a.partial = nullptr;
-    a.M = (int)tokens;
-    a.N = out_features;
-    a.K = in_features;
-    a.nnz = nnz;
-    a.tiles_r = a.tiles_c = a.nsplit = a.tokens_per_split = a.segs = 0;
-    if (dtype == PBS_DTYPE_F32) return launch_sdd<float>(a, dtype, workspace, workspace_bytes, s);
-    return launch_sdd<bf16_t>(a, dtype, workspace, workspace_bytes, s);
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    return back(a, tokens, dtype, workspace, workspace_bytes, stream);
+}
+
+int pbs_blocksparse_matmul_back_bias(const void* dense_a, const void* dense_b, const int32_t* row_start_ends_a,
+                                     const int32_t* cols_a, const void* units, void* data_out, void* bias_out, int64_t tokens,
+                                     int out_features, int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
+                                     void* stream) {
+    if (!units && pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, dtype) > 0) return PBS_ERR_NULL_POINTER;
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, units, data_out, bias_out, (int)tokens, out_features, in_features, nnz};
+    return back(a, tokens, dtype, workspace, workspace_bytes, stream);
 }
 
 // ---- the reference's own signature of the sparse-output product ----
@@ -917,15 +957,21 @@ int pbs_blocksparse_matmul_back_noalloc_init(void) {
 int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b, const int32_t* row_start_ends_a,
                                         const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                         int in_features, int nnz, int dtype, void* stream) {
-    // what pbs_blocksparse_matmul_back would ask the caller for (0 for arguments it is going to reject itself)
-    const size_t need = pbs_blocksparse_matmul_back_workspace_bytes(tokens, out_features, in_features, nnz, dtype);
+    // the array limits the number of slices of the row kernel; the rectangles' is fixed
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    size_t need = 0, limit = 0;
+    if (back_sizes_ok(tokens, out_features, in_features, nnz, dtype) && nnz > 0) {
+        const size_t table = unit_table_bytes(out_features, nnz);
+        limit = (size_t)PBS_NOALLOC_SCRATCH_BYTES > table ? (size_t)PBS_NOALLOC_SCRATCH_BYTES - table : 0;
+        const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, limit);
+        need = p.partial_bytes + (p.slices > 0 ? table : 0);
+    }
     if (need > (size_t)PBS_NOALLOC_SCRATCH_BYTES) return PBS_ERR_SCRATCH;
     void* ws = nullptr;
     if (need > 0) {
         if (int rc = scratch_of_current_device(&ws)) return rc;
     }
-    return pbs_blocksparse_matmul_back(dense_a, dense_b, row_start_ends_a, cols_a, data_out, tokens, out_features,
-                                       in_features, nnz, dtype, ws, need, stream);
+    return back(a, tokens, dtype, ws, need, stream, limit);
 }
 
 int pbs_protocol_failures(unsigned* count) {
@@ -944,10 +990,9 @@ const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_feat
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || out_features <= 0 || in_features <= 0 ||
         nnz <= 0 || (out_features % 32) || (in_features % 32))
         return "";
-    const SddPlan p = plan_sdd_for(dtype, tokens, out_features, in_features, nnz);
-    if (dtype == PBS_DTYPE_BF16) return p.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";
-    if (p.shape >= SDD_F32_SEGMENTS) return p.nsplit > 1 ? "sdd_seg_kernel + sdd_reduce_kernel" : "sdd_seg_kernel";
-    return p.nsplit > 1 ? "sdd_kernel + sdd_reduce_kernel" : "sdd_kernel";
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz);
+    if (p.slices > 0) return p.slices > 1 ? "sdd_row_kernel + sdd_reduce_kernel" : "sdd_row_kernel";
+    return p.rect.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";
 }
 
 }  // extern "C"

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(INDEX_THREADS) void csr_from_owner_kernel(const int
 // One workgroup, five short phases over the data blocks instead of scans over the grid: every block sets its bit in a bitmap
 // of its row and in one of its column; a row's (column's) start is the sum of the popcounts before it, and a block's place within it
 // the popcount of the bits below its own.  No sort, no search; the bitmaps sit in LDS while they fit (16 K positions take
-// 4 KB, 24 x 96 positions and 1152 blocks 6 us in all, where building a mask, sorting the positions and the two scans of
+// 4 KB, 24 x 96 positions and 1152 blocks 7 us in all, where building a mask, sorting the positions and the two scans of
 // build_indices_kernel took 150 us in a dozen launches).
 constexpr int REPLACE_LDS_WORDS = 12 * 1024;
 enum ReplaceError { REPLACE_BAD_ID = 1, REPLACE_BAD_POSITION = 2, REPLACE_TAKEN = 4 };

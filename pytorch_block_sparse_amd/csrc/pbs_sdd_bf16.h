@@ -240,7 +240,7 @@ template <int QW, int TC_, int NS_, int NW_ = 8>
 __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
     using C = SddBf16Cfg<QW, TC_, NS_, NW_>;
     constexpr int NS = C::NS;
-    constexpr int SR = C::SR, SC = C::SC, NW = C::NW, TC = C::TC;
+    constexpr int SR = C::SR, NW = C::NW, TC = C::TC;
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     int* s_blk = reinterpret_cast<int*>(smem + NS * C::STAGE_BYTES);                  // [LIST_MAX] data block

@@ -1,0 +1,447 @@
+// dense^T x dense -> block-sparse (weight gradient on the sparse support), and with it the bias gradient:
+//   out[32b + j][i] = sum_t G[t][32r + i] * X[t][32c + j]   for every data block b at (r, c),   bias[n] = sum_t G[t][n].
+//
+// A workgroup takes a unit, up to four blocks of one block row of W, over one slice of the tokens; each of its four waves
+// every fourth chunk of 32 tokens, with all accumulators of the unit (64 registers), so that nothing is shared until the
+// waves' sums meet in LDS at the end: no barrier and no wait for another wave in the loop, any shape of pattern makes
+// units of one size, and small problems have many workgroups.  A G fragment is read once for four products.
+//
+// What bounds it: the texture path that copies memory to LDS (a KB costs it 23 cycles in 128-byte rows, 35 in 64-byte ones)
+// and the matrix pipe.  fp32: 256 cycles of products per block and chunk against 4 + 4 / NB copies of 23 each: near the matrix rate
+// if copies and products overlap, so every copy is issued between two products (issued in a burst, all waves of a CU
+// copy together, then compute together: twice the time).  A piece of LDS (32 tokens x 32 features) is refilled as soon as
+// its fragments are in registers, and the registers as soon as their product is issued: five pieces per wave hold one
+// to four blocks of copies in flight.  bf16: 32 cycles of products against 2 x 35 of copies: bound by the copies, still
+// better than rectangles until the operands outgrow the L2s.
+// Fragments: fp32 as float2 of two features (the two 16-feature halves of a product are the even and the odd features: one
+// 8-byte read serves both); bf16 through transposing reads, the halves chosen so that eight result columns meet in a lane.
+//
+// Measured, us, against the kernels it replaced (fp32: equal shares of bands of 16 rows, barriers; bf16: rectangles):
+//   fp32 768 -> 3072 density 0.5, 4096 tokens 123 -> 96, 1024 tokens 56 -> 33;  3072 -> 768 density 0.25 with uneven rows, 4096 tokens
+//   78 -> 50;  768 -> 768 density 0.5, 16384 tokens 122 -> 98;  4096 -> 4096 density 0.25, 16384 tokens 1250 -> 1129 (122 of
+//   155 TFLOP/s);  3072 -> 768 density 0.5, 101 tokens 23 -> 8.7.
+//   bf16 768 -> 3072 density 0.5, 2317 tokens 48 -> 34;  4096 -> 4096 density 0.25, 509 tokens 38 -> 29, 64 tokens 21 -> 8.3.
+#pragma once
+#include <type_traits>
+
+#include "pbs_common.h"
+#include "pbs_stream.h"
+
+namespace pbs {
+
+constexpr int ROW_NB = 4;       // blocks of a unit, at most
+constexpr int ROW_NW = 4;       // waves of a workgroup: every ROW_NW-th chunk of tokens each
+constexpr int ROW_TC = 32;      // tokens per chunk
+constexpr int ROW_PARTS = 4;
+constexpr int ROW_PIECES = 5;   // LDS of a wave, in pieces of 32 tokens x 32 features
+
+// ---- unit table: what the workgroups of a pattern do ----
+// A unit is up to ROW_NB blocks of one block row: {row, blocks, number within the row, 0, columns [4], data blocks [4]} in 16
+// ints.  A row of n blocks has ceil(n / ROW_NB) units of equal size (+- 1), an empty row one without blocks (for the bias
+// gradient).  Order: (quarter of the row's units, row, unit): units that run at the same time then read neighbouring columns of
+// X from a common L2.  The table starts with the number of units, padded to 16 ints.
+constexpr int UNIT_INTS = 16;
+constexpr int UNIT_LDS_ROWS = 1024;
+static inline long long unit_bound(int N, int nnz) { return (long long)nnz / ROW_NB + N / 32; }   // ceil(n / 4) <= n / 4 + 3 / 4
+static inline size_t unit_prefix_bytes(int N) { return N / 32 > UNIT_LDS_ROWS ? ((size_t)ROW_PARTS * (N / 32) + 1) * sizeof(int) : 0; }
+static inline size_t unit_table_bytes(int N, int nnz) { return 64 + (size_t)unit_bound(N, nnz) * UNIT_INTS * sizeof(int) + unit_prefix_bytes(N); }
+static __device__ __forceinline__ int row_entries(const int32_t* __restrict__ ptr, int nnz, int r, int* lo) {
+    const int a = clamp_entry(ptr[r], nnz), b = clamp_entry(ptr[r + 1], nnz);
+    *lo = a;
+    return b > a ? b - a : 0;
+}
+static __device__ __forceinline__ int row_units(int n) { return n > 0 ? (n + ROW_NB - 1) / ROW_NB : 1; }
+static __device__ __forceinline__ int part_lo(int nu, int h) { return (h * nu + ROW_PARTS - 1) / ROW_PARTS; }   // first unit of quarter h
+static __device__ __forceinline__ int unit_entry(int n, int nu, int j) { return (int)((long long)n * j / nu); }
+
+// units before (quarter, row), into before [ROW_PARTS * rows + 1]; all threads of the workgroup
+template <int NT>
+static __device__ void unit_prefix(const int32_t* __restrict__ ptr, int nnz, int rows, int* before, int* s_wave) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int carry = 0;
+    for (int base = 0; base < ROW_PARTS * rows; base += NT) {
+        const int i = base + tid;
+        int v = 0, lo;
+        if (i < ROW_PARTS * rows) {
+            const int h = i / rows, nu = row_units(row_entries(ptr, nnz, i - h * rows, &lo));
+            v = part_lo(nu, h + 1) - part_lo(nu, h);
+        }
+        int incl = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        __syncthreads();
+        if (lane == 63) s_wave[wave] = incl;
+        __syncthreads();
+        int add = carry;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) {
+            if (w < wave) add += s_wave[w];
+            carry += s_wave[w];
+        }
+        if (i < ROW_PARTS * rows) before[i] = add + incl - v;
+    }
+    if (tid == 0) before[ROW_PARTS * rows] = carry;
+    __threadfence_block();
+    __syncthreads();
+}
+__global__ __launch_bounds__(1024) void unit_prefix_kernel(const int32_t* __restrict__ ptr, int nnz, int rows, int* before) {
+    __shared__ int s_wave[16];
+    unit_prefix<1024>(ptr, nnz, rows, before, s_wave);
+}
+// one unit per thread; global_before (unit_prefix_kernel) for patterns whose prefix does not fit LDS
+__global__ __launch_bounds__(256) void unit_table_kernel(const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx, int nnz, int rows,
+                                                         int cols, const int* global_before, int bound, int* table) {
+    __shared__ int s_before[ROW_PARTS * UNIT_LDS_ROWS + 1];
+    __shared__ int s_wave[4];
+    if (!global_before) unit_prefix<256>(ptr, nnz, rows, s_before, s_wave);
+    const int* before = global_before ? global_before : s_before;
+    const int total = before[ROW_PARTS * rows] < bound ? before[ROW_PARTS * rows] : bound;   // (a corrupt pointer array may ask for more)
+    const int u = blockIdx.x * 256 + threadIdx.x;
+    if (u == 0) table[0] = total;
+    if (u >= total) return;
+    int lo = 0, hi = ROW_PARTS * rows - 1;   // the place that holds unit u
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (before[mid + 1] <= u) lo = mid + 1; else hi = mid;
+    }
+    const int h = lo / rows, row = lo - h * rows;
+    int first;
+    const int n = row_entries(ptr, nnz, row, &first), nu = row_units(n);
+    const int j0 = part_lo(nu, h), j = j0 + u - before[lo];
+    const int e0 = unit_entry(n, nu, j), e1 = unit_entry(n, nu, j + 1);
+    int* o = table + 16 + (size_t)u * UNIT_INTS;
+    o[0] = row;
+    o[1] = e1 - e0;
+    o[2] = j;
+    o[3] = 0;
+#pragma unroll
+    for (int b = 0; b < ROW_NB; ++b) {
+        int c = 0, d = -1;
+        if (b < e1 - e0) {
+            c = idx[2 * (size_t)(first + e0 + b)];
+            d = idx[2 * (size_t)(first + e0 + b) + 1];
+            c = c < 0 ? 0 : (c >= cols ? cols - 1 : c);
+            d = d < 0 || d >= nnz ? -1 : d;
+        }
+        o[4 + b] = c;
+        o[8 + b] = d;
+        o[12 + b] = 0;
+    }
+}
+
+struct SddRowArgs {
+    const void* g;           // [M, N] grad_output
+    const void* x;           // [M, K] input
+    const int* table;        // unit_table_kernel
+    void* out;               // [nnz*32, 32]
+    void* bias_out;          // nullptr or [N]
+    float* partial;
+    int M, N, K, nnz;
+    int slices, chunks_per_slice;   // every unit in this many slices of the tokens
+};
+// What a lane holds of a piece, and the products of two pieces (4 x STEPS matrix instructions).  A lane's accumulators of a block
+// are d[a][b][v], column i = COL(q, a, v) of row j = FEAT(r, b): eight consecutive columns per row.
+template <typename T>
+struct RowFrag;
+template <>
+struct RowFrag<float> {
+    static constexpr int STEPS = 8;
+    static constexpr int DMA = 4;          // DMA instructions per piece
+    float2 v[STEPS];                       // step s: token 4 s + q, features 2 r and 2 r + 1
+    static __device__ __forceinline__ int feature(int r, int a) { return 2 * r + a; }
+    static __device__ __forceinline__ int place(int a, int v) { return 2 * v + a; }   // of column i among the eight
+    __device__ __forceinline__ void read(const unsigned char* piece, int s, int lane) {
+        v[s] = *reinterpret_cast<const float2*>(piece + s * 512 + lane * 8);
+    }
+    // the piece straight from memory, tokens from `end` on as zeros
+    __device__ __forceinline__ void fetch(const unsigned char* base, size_t stride, int end, int lane) {
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int t = 4 * s + (lane >> 4);
+            v[s] = t < end ? *reinterpret_cast<const float2*>(base + (size_t)t * stride + (lane & 15) * 8) : make_float2(0.f, 0.f);
+        }
+    }
+    __device__ __forceinline__ void sum(float (&o)[2]) const {
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            o[0] += v[s].x;
+            o[1] += v[s].y;
+        }
+    }
+    static __device__ __forceinline__ void mma(f32x4 (&d)[2][2], const RowFrag& g, const RowFrag& x, int s) {
+        d[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.v[s].x, x.v[s].x, d[0][0], 0, 0, 0);
+        d[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.v[s].y, x.v[s].x, d[1][0], 0, 0, 0);
+        d[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.v[s].x, x.v[s].y, d[0][1], 0, 0, 0);
+        d[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.v[s].y, x.v[s].y, d[1][1], 0, 0, 0);
+    }
+};
+template <>
+struct RowFrag<bf16_t> {
+    static constexpr int STEPS = 1;
+    static constexpr int DMA = 2;
+    uint4 v[2];                            // half a: tokens 8 q .. 8 q + 7 of one feature
+    static __device__ __forceinline__ int feature(int r, int a) { return 8 * (r >> 2) + 4 * a + (r & 3); }
+    static __device__ __forceinline__ int place(int a, int v) { return 4 * a + v; }
+    __device__ __forceinline__ void read(const unsigned char* piece, int, int lane) {
+        const int r = lane & 15, q = lane >> 4;
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const unsigned char* p = piece + (8 * q + (r >> 2)) * 64 + (r & 3) * 16 + 8 * a;
+            const uint2 lo = tr16_b64(p), hi = tr16_b64(p + 256);
+            v[a] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        }
+    }
+    __device__ __forceinline__ void fetch(const unsigned char* base, size_t stride, int end, int lane) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            uint32_t w[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const int tok = 8 * (lane >> 4) + t;
+                w[t] = tok < end ? *reinterpret_cast<const uint16_t*>(base + (size_t)tok * stride + feature(lane & 15, a) * 2) : 0u;
+            }
+            v[a] = make_uint4(w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16);
+        }
+    }
+    __device__ __forceinline__ void sum(float (&o)[2]) const {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+            for (const uint32_t w : {v[a].x, v[a].y, v[a].z, v[a].w}) o[a] += __uint_as_float(w << 16) + __uint_as_float(w & 0xffff0000u);
+    }
+    static __device__ __forceinline__ void mma(f32x4 (&d)[2][2], const RowFrag& g, const RowFrag& x, int) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+                d[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, g.v[a]), __builtin_bit_cast(bf16x8, x.v[b]), d[a][b], 0, 0, 0);
+    }
+};
+
+template <typename T>
+struct SddRowCfg {
+    static constexpr int PIECE = 1024 * Elem<T>::ESZ;
+    static constexpr int WAVE_LDS = ROW_PIECES * PIECE;
+    static constexpr int RED = ROW_NW * 2 * 4 * 1024 + ROW_NW * 32 * 4;   // the waves' sums of two blocks, and of the bias columns
+    static constexpr int LDS = ROW_NW * WAVE_LDS > RED ? ROW_NW * WAVE_LDS : RED;
+    static constexpr int WPE = sizeof(T) == 4 ? 2 : 3;   // waves per SIMD: LDS allows the former, registers the latter
+};
+
+// Chunks c_lo .. c_hi - 1 of a unit of NB blocks.
+template <typename T, int NB>
+static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const int* __restrict__ unit, int c_lo, int c_hi, float* partial,
+                                                    unsigned char* smem, int lane, int wave) {
+    using E = Elem<T>;
+    using F = RowFrag<T>;
+    using C = SddRowCfg<T>;
+    constexpr int ESZ = E::ESZ, PIECE = C::PIECE, D = F::DMA, CPR = 32 * ESZ / 16, RPI = 64 / CPR;
+    constexpr int NBX = NB > 0 ? NB : 1;
+    const int r = lane & 15, q = lane >> 4;
+    const int row = unit[0];
+    int cblk[NBX], bblk[NBX];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        cblk[b] = unit[4 + b];
+        bblk[b] = unit[8 + b];
+    }
+    const bool sums = a.bias_out && unit[2] == 0;
+
+    const int whole = a.M / ROW_TC;              // chunks below this one are whole
+    const int full_hi = whole < c_hi ? whole : c_hi;
+    const size_t gs = (size_t)a.N * ESZ, xs = (size_t)a.K * ESZ;   // row strides
+    const unsigned char* G = static_cast<const unsigned char*>(a.g) + (size_t)row * (32 * ESZ);
+    const unsigned char* X = static_cast<const unsigned char*>(a.x);
+    // A wave's LDS: one G piece and the rest X pieces in turn; one or two blocks per row need their G pieces faster and
+    // have two of them.
+    constexpr int GS = NB == 1 || NB == 2 ? 2 : 1, XS = ROW_PIECES - GS;
+    unsigned char* mem = smem + wave * C::WAVE_LDS;
+    const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)mem);
+    // DMA instruction i of a piece: tokens RPI i + lane / CPR, 16 bytes per lane
+    const unsigned gv = (unsigned)((lane / CPR) * (a.N * ESZ) + (lane % CPR) * 16), xv = (unsigned)((lane / CPR) * (a.K * ESZ) + (lane % CPR) * 16);
+    auto dma_g = [&](int slot, int chunk, int i) __attribute__((always_inline)) {
+        dma16(lds + slot * PIECE + i * 1024, uniform_ptr(G + ((size_t)chunk * ROW_TC + RPI * i) * gs), gv);
+    };
+    auto dma_x = [&](int slot, int chunk, int c, int i) __attribute__((always_inline)) {
+        dma16(lds + (GS + slot) * PIECE + i * 1024, uniform_ptr(X + ((size_t)chunk * ROW_TC + RPI * i) * xs + (size_t)c * (32 * ESZ)), xv);
+    };
+
+    f32x4 acc[NBX][2][2];
+#pragma unroll
+    for (int b = 0; b < NBX; ++b)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum[2] = {0.f, 0.f};
+
+    int chunk = c_lo + wave;
+    if (chunk < full_hi) {
+        const int last = chunk + (full_hi - 1 - chunk) / ROW_NW * ROW_NW;   // this wave's last whole chunk
+        auto after = [&](int c, int n) { return c + n * ROW_NW <= last ? c + n * ROW_NW : last; };   // (past the end: the last one again)
+        F gf, xf;
+        // piece k is block k % NB of chunk k / NB
+#pragma unroll
+        for (int t = 0; t < GS; ++t)
+#pragma unroll
+            for (int i = 0; i < D; ++i) dma_g(t, after(chunk, t), i);
+        if constexpr (NB > 0) {
+#pragma unroll
+            for (int k = 0; k < XS; ++k)
+#pragma unroll
+                for (int i = 0; i < D; ++i) dma_x(k, after(chunk, k / NBX), cblk[k % NBX], i);
+        }
+        wait_dma(NB > 0 ? (XS - 1) * D : 0);
+#pragma unroll
+        for (int s = 0; s < F::STEPS; ++s) {
+            gf.read(mem, s, lane);
+            if constexpr (NB > 0) xf.read(mem + GS * PIECE, s, lane);
+        }
+        int xat = 0, gat = 0;   // slots of the pieces in xf and gf
+        for (;; chunk += ROW_NW) {
+            if (sums) gf.sum(bsum);
+            if constexpr (NB == 0) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < D; ++i) dma_g(0, after(chunk, 1), i);
+                wait_dma(0);
+#pragma unroll
+                for (int s = 0; s < F::STEPS; ++s) gf.read(mem, s, lane);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                // Read below: the next block's piece, asked for XS - 1 blocks ago, and in the chunk's last block the next chunk's
+                // G piece.  The tables have the number of younger DMA instructions, for the orders of issue below.
+                constexpr int YOUNGER4[5][4] = {{0, 0, 0, 0}, {1, 0, 0, 0}, {4, 8, 0, 0}, {8, 12, 5, 0}, {8, 12, 12, 8}};
+                constexpr int YOUNGER2[5][4] = {{0, 0, 0, 0}, {2, 0, 0, 0}, {2, 4, 0, 0}, {4, 6, 4, 0}, {4, 6, 6, 4}};
+                wait_dma(D == 4 ? YOUNGER4[NB][b] : YOUNGER2[NB][b]);
+                const int xnext = xat + 1 == XS ? 0 : xat + 1;
+                const int kb = (b + XS) % NBX;       // the piece that takes this block's slot
+                const int cn = after(chunk, (b + XS) / NBX), gn = after(chunk, GS);
+                const int gnext = GS == 2 ? gat ^ 1 : 0;
+#pragma unroll
+                for (int s = 0; s < F::STEPS; ++s) {
+                    F::mma(acc[b], gf, xf, s);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (F::STEPS == 8) {
+                        // instruction i overwrites what steps 2 i and 2 i + 1 have read: their products are under way
+                        if (b == 0 && (s & 1)) dma_g(gat, gn, s >> 1);
+                        if (b == 0 ? s > 0 && !(s & 1) : (s & 1)) dma_x(xat, cn, cblk[kb], b == 0 ? s / 2 - 1 : s >> 1);
+                        if (b == 0 && s == 7) dma_x(xat, cn, cblk[kb], 3);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < D; ++i)
+                            if (b == 0) dma_g(gat, gn, i);
+#pragma unroll
+                        for (int i = 0; i < D; ++i) dma_x(xat, cn, cblk[kb], i);
+                    }
+                    xf.read(mem + (GS + xnext) * PIECE, s, lane);
+                    if (b == NB - 1) gf.read(mem + gnext * PIECE, s, lane);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                xat = xnext;
+                if (b == NB - 1) gat = gnext;
+            }
+            if (chunk >= last) break;
+        }
+        wait_dma(0);   // the sums below use the same space
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    // the ragged last chunk of the matrix
+    if (whole * ROW_TC < a.M && whole >= c_lo && whole < c_hi && (whole - c_lo) % ROW_NW == wave) {
+        const int end = a.M - whole * ROW_TC;
+        F gf, xf;
+        gf.fetch(G + (size_t)whole * ROW_TC * gs, gs, end, lane);
+        if (sums) gf.sum(bsum);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            xf.fetch(X + (size_t)whole * ROW_TC * xs + (size_t)cblk[b] * (32 * ESZ), xs, end, lane);
+#pragma unroll
+            for (int s = 0; s < F::STEPS; ++s) F::mma(acc[b], gf, xf, s);
+        }
+    }
+
+    // ---- the waves' sums meet in LDS, two blocks at a time: wave 2 k + jj stores rows FEAT(r, jj) of block k ----
+    f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int b0 = 0; b0 < NB; b0 += 2) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (b0 + k < NB)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) red[((wave * 2 + k) * 4 + i) * 64 + lane] = acc[(b0 + k) % NBX][i >> 1][i & 1];
+        __syncthreads();
+        const int k = wave >> 1, jj = wave & 1;
+        const int at = k == 0 ? bblk[b0] : bblk[(b0 + 1) % NBX];
+        if (b0 + k < NB && at >= 0) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                f32x4 s = red[(k * 4 + 2 * i + jj) * 64 + lane];
+#pragma unroll
+                for (int w = 1; w < ROW_NW; ++w) s += red[((w * 2 + k) * 4 + 2 * i + jj) * 64 + lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[F::place(i, e)] = s[e];
+            }
+            const size_t o = (size_t)at * 1024 + F::feature(r, jj) * 32 + 8 * q;
+            if (partial || ESZ == 4) {
+                float* p = (partial ? partial : static_cast<float*>(a.out)) + o;
+                reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
+                reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
+            } else {
+                uint32_t w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[e] = (uint32_t)Elem<bf16_t>::from_f32(v[2 * e]).bits | ((uint32_t)Elem<bf16_t>::from_f32(v[2 * e + 1]).bits << 16);
+                *reinterpret_cast<uint4*>(static_cast<uint16_t*>(a.out) + o) = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+    }
+    if (sums) {
+        float* s = reinterpret_cast<float*>(smem + ROW_NW * 2 * 4 * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            bsum[i] += __shfl_xor(bsum[i], 16, 64);
+            bsum[i] += __shfl_xor(bsum[i], 32, 64);
+            if (lane < 16) s[wave * 32 + F::feature(lane, i)] = bsum[i];
+        }
+        __syncthreads();
+        if (wave == 0 && lane < 32) {
+            float v = s[lane];
+#pragma unroll
+            for (int w = 1; w < ROW_NW; ++w) v += s[w * 32 + lane];
+            if (partial) partial[(size_t)a.nnz * 1024 + row * 32 + lane] = v;
+            else static_cast<T*>(a.bias_out)[row * 32 + lane] = E::from_f32(v);
+        }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel(SddRowArgs a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[SddRowCfg<T>::LDS];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // an XCD takes a run of units and goes through them for one token slice after the other
+    const int units = a.table[0];
+    const int xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD;
+    const int u_lo = (int)((long long)units * xcd / NUM_XCD), n_u = (int)((long long)units * (xcd + 1) / NUM_XCD) - u_lo;
+    if (local >= n_u * a.slices) return;
+    const int slice = local / n_u;
+    const int* unit = a.table + 16 + (size_t)(u_lo + local - slice * n_u) * UNIT_INTS;
+    const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
+    const int c_lo = slice * a.chunks_per_slice;
+    const int c_hi = c_lo + a.chunks_per_slice < chunks ? c_lo + a.chunks_per_slice : chunks;
+    float* partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + a.N) : nullptr;
+    switch (unit[1]) {
+        case 4: sdd_row_body<T, 4>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
+        case 3: sdd_row_body<T, 3>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
+        case 2: sdd_row_body<T, 2>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
+        case 1: sdd_row_body<T, 1>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
+        default:
+            if (a.bias_out) sdd_row_body<T, 0>(a, unit, c_lo, c_hi, partial, smem, lane, wave);
+            break;
+    }
+}
+
+}  // namespace pbs

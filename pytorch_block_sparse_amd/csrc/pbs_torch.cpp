@@ -93,6 +93,7 @@ struct Pattern {
     std::mutex lock;
     Tensor plan[2];      // [transpose]
     int parts[2] = {0, 0};
+    Tensor units;        // of the weight gradient
 
     bool still(const Tensor& rp, const Tensor& c, const Tensor& cp, const Tensor& r) const {
         return row_ptr.still(rp) && cols.still(c) && col_ptr.still(cp) && rows.still(r);
@@ -113,6 +114,20 @@ struct Pattern {
             parts[transpose] |= part;
         }
         return plan[transpose].const_data_ptr();
+    }
+    const void* units_for(int64_t tokens, int code, void* stream) {
+        const size_t bytes = pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, code);
+        if (!bytes) return nullptr;
+        std::lock_guard<std::mutex> hold(lock);
+        if (!units.defined()) {
+            TORCH_CHECK(row_ptr.t.is_cuda() && cols.t.is_cuda(), "the index buffers are not on the GPU");
+            Tensor t = at::empty({(int64_t)bytes}, row_ptr.t.options().dtype(at::kByte));
+            check(pbs_blocksparse_matmul_back_units(row_ptr.t.const_data_ptr<int>(), nnz ? cols.t.const_data_ptr<int>() : nullptr, out_features,
+                                                    in_features, nnz, t.mutable_data_ptr(), bytes, stream),
+                  "pbs_blocksparse_matmul_back_units");
+            units = t;
+        }
+        return units.const_data_ptr();
     }
 };
 using PatternPtr = std::shared_ptr<Pattern>;
@@ -156,8 +171,9 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     return out;
 }
 
-// packed blocks of a^T b on the pattern, into `out`
-void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out) {
+// packed blocks of a^T b on the pattern, into `out`; and, if the kernel for this problem can, the sums of a's columns, into `sums`
+// (made here when wanted)
+void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out, Tensor* sums = nullptr) {
     check_gpu(a_any);
     check_gpu(b_any);
     check_gpu(out);
@@ -172,14 +188,17 @@ void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Ten
     const int64_t tokens = a.numel() / p.out_features;
     TORCH_CHECK(b.numel() / p.in_features == tokens, "Invalid matrices sizes ", a.sizes(), "^T x ", b.sizes());
     c10::DeviceGuard guard(a.device());
-    const size_t ws_bytes = pbs_blocksparse_matmul_back_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
+    void* stream = current_stream(a);
+    const void* units = p.units_for(tokens, code, stream);
+    if (sums && units) *sums = at::empty({p.out_features}, a.options());
+    const size_t ws_bytes = pbs_blocksparse_matmul_back_bias_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
-    check(pbs_blocksparse_matmul_back(data_or_null(a), data_or_null(b), p.row_ptr.t.const_data_ptr<int>(),
-                                      static_cast<const int*>(data_or_null(p.cols.t)), out.numel() ? out.mutable_data_ptr() : nullptr, tokens,
-                                      p.out_features, p.in_features, p.nnz, code, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes,
-                                      current_stream(a)),
-          "pbs_blocksparse_matmul_back");
+    check(pbs_blocksparse_matmul_back_bias(data_or_null(a), data_or_null(b), p.row_ptr.t.const_data_ptr<int>(),
+                                           static_cast<const int*>(data_or_null(p.cols.t)), units, out.numel() ? out.mutable_data_ptr() : nullptr,
+                                           sums && units ? sums->mutable_data_ptr() : nullptr, tokens, p.out_features, p.in_features, p.nnz, code,
+                                           ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
+          "pbs_blocksparse_matmul_back_bias");
 }
 
 // y = x W^T + bias.  Backward: dx = dy W, dW on the pattern's blocks, dbias = sum of dy over the tokens.
@@ -203,9 +222,9 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
         if (task_should_compute_output(1)) {
             const Tensor xs = x.unpack(shared_from_this());
             out[1] = at::empty({(int64_t)pattern->nnz * 32, 32}, xs.options());
-            matmul_back(*pattern, dy, xs, out[1]);
+            matmul_back(*pattern, dy, xs, out[1], has_bias && task_should_compute_output(2) ? &out[2] : nullptr);
         }
-        if (has_bias && task_should_compute_output(2)) out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
+        if (has_bias && task_should_compute_output(2) && !out[2].defined()) out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
         return out;
     }
 };

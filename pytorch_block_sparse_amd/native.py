@@ -48,6 +48,13 @@ _PROTOTYPES = {
         _i32,
         [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp],
     ),
+    "pbs_blocksparse_matmul_back_units_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_matmul_back_units": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
+    "pbs_blocksparse_matmul_back_bias_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_matmul_back_bias": (
+        _i32,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp],
+    ),
     "pbs_blocksparse_matmul_back_blocks_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul_back_blocks": (
         _i32,

@@ -1,0 +1,45 @@
+"""The weight-gradient kernel with up to four blocks of a block row per workgroup, and the bias gradient that comes with it,
+against float64: token counts around the 32-token chunk, rows of 0 to 13 blocks, more block rows than the table kernel keeps in
+LDS, one and several token slices."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import block_sparse_oracle as O
+from pytorch_block_sparse_amd import BlockSparseMatrix, native
+from tests.helpers import assert_close, to64
+
+pytestmark = pytest.mark.gpu
+ROWS = [0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13]   # blocks of a block row
+
+
+def _layer(out_f, in_f, counts, dtype, device, seed):
+    rng = np.random.RandomState(seed)
+    blocks = [(r, int(c)) for r in range(out_f // 32) for c in rng.choice(in_f // 32, counts[r % len(counts)], replace=False)]
+    return BlockSparseMatrix.zeros((out_f, in_f), blocks=blocks, device=device, dtype=dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,out_f,in_f,counts,slices", [
+    (1, 384, 416, ROWS, False), (31, 384, 416, ROWS, False), (32, 384, 416, ROWS, False), (33, 384, 416, ROWS, False),
+    (97, 384, 416, ROWS, False), (160, 384, 416, ROWS, False), (161, 384, 416, [13], False), (2317, 384, 416, ROWS, True),
+    (4096, 32, 64, [2], True), (16415, 64, 32, [0, 1], True), (45, 32 * 1030, 64, [2, 0, 1], False),
+])
+def test_row_kernel(cuda, dtype, tokens, out_f, in_f, counts, slices):
+    m = _layer(out_f, in_f, counts, dtype, cuda, 3)
+    nnz = m.cols_a.shape[0]
+    name = native.matmul_back_kernel_name(tokens, out_f, in_f, nnz, dtype)
+    print(name, tokens, out_f, in_f, nnz, dtype, flush=True)
+    assert name.startswith("sdd_row_kernel") and name.endswith("sdd_reduce_kernel") == slices, name
+    g = torch.Generator().manual_seed(tokens)
+    x, dy = (torch.randn((tokens, f), generator=g).to(dtype) for f in (in_f, out_f))
+    coo = m.build_coo_block_index().cpu().numpy()
+    ref = O.matmul_with_output_sparse_support(to64(dy), to64(x), coo, (out_f, in_f))
+    xd, dyd = x.to(cuda), dy.to(cuda)
+    got = m.matmul_with_output_sparse_support(dyd, xd)
+    assert_close(got, ref, dtype, "weight gradient")
+
+    data, bias = m.data.detach().clone().requires_grad_(), torch.zeros(out_f, dtype=dtype, device=cuda, requires_grad=True)
+    native.torch_path().linear(xd, data, bias, m._buffers, m.schedule()).backward(dyd)
+    assert torch.equal(data.grad, got)   # with the bias gradient: the same sums
+    assert_close(bias.grad, to64(dy).sum(0), dtype, "bias gradient")
