@@ -213,7 +213,7 @@ int pbs_blocksparse_matmul_back(const void* dense_a, const void* dense_b,
  *   units   the table of the work of the pattern's rows, made by pbs_blocksparse_matmul_back_units in
  *           pbs_blocksparse_matmul_back_units_bytes() bytes of 16-byte aligned device memory.  It depends on the
  *           pattern only and serves every number of tokens and both dtypes.  ..._units_bytes returns 0 for problems whose kernel uses
- *           none (units may then be NULL); those do not take bias_out either (PBS_ERR_BAD_SHAPE).
+ *           none (units may then be NULL).
  *   workspace: pbs_blocksparse_matmul_back_bias_workspace_bytes() bytes, may be NULL when that is 0.
  *
  * nnz may be 0 with a bias_out; data_out may then be NULL.

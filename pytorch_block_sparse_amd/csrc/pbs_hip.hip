@@ -471,7 +471,7 @@ struct BackPlan {
     SddPlan rect;
     size_t partial_bytes;
 };
-static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit = ~(size_t)0) {
+static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ~(size_t)0) {
     BackPlan p;
     p.slices = choose_row_slices(dtype, M, N, K, nnz, workspace_limit);
     p.rect = plan_sdd(M, N, K);
@@ -481,8 +481,7 @@ static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, size_t 
         p.chunks_per_slice = (int)((chunks + p.slices - 1) / p.slices);
         p.slices = n = (int)((chunks + p.chunks_per_slice - 1) / p.chunks_per_slice);
     }
-    // fp32 sums of each slice (row kernel: blocks, then bias columns)
-    p.partial_bytes = n > 1 ? ((size_t)nnz * 1024 + (p.slices > 0 ? N : 0)) * sizeof(float) * n : 0;
+    p.partial_bytes = n > 1 ? ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * n : 0;   // fp32 sums of each slice: blocks, bias columns
     return p;
 }
 
@@ -509,10 +508,10 @@ static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int
 }
 
 template <typename T>
-static int launch_reduce(const float* partial, void* out, size_t n, void* bias_out, size_t nbias, size_t stride, int nsplit, hipStream_t stream) {
-    const size_t total = n + (bias_out ? nbias : 0);
-    hipLaunchKernelGGL(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(out), n,
-                       static_cast<T*>(bias_out), total, stride, nsplit);
+static int launch_reduce(const float* partial, const BackArgs& a, int nsplit, hipStream_t stream) {
+    const size_t n = (size_t)a.nnz * 1024, total = n + (a.bias_out ? a.N : 0);
+    hipLaunchKernelGGL(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(a.out), n,
+                       static_cast<T*>(a.bias_out), total, nsplit);
     return (int)hipGetLastError();
 }
 
@@ -542,8 +541,7 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     r.chunks_per_slice = p.chunks_per_slice;
     hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
     if (int rc = (int)hipGetLastError()) return rc;
-    const size_t n = (size_t)a.nnz * 1024;
-    return p.partial_bytes ? launch_reduce<T>(r.partial, a.out, n, a.bias_out, a.N, n + a.N, p.slices, stream) : PBS_OK;
+    return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;
 }
 
 static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -554,6 +552,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     a.ptr = b.ptr;
     a.idx = b.idx;
     a.out = b.out;
+    a.bias_out = b.bias_out;
     a.partial = nullptr;
     a.M = b.M;
     a.N = b.N;
@@ -563,7 +562,6 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     a.tiles_c = p.tiles_c;
     a.nsplit = p.nsplit;
     a.tokens_per_split = p.tokens_per_split;
-    const size_t n = (size_t)a.nnz * 1024;
     if (p.nsplit > 1) {
         if (!workspace || workspace_bytes < plan.partial_bytes || !aligned16(workspace)) return PBS_ERR_WORKSPACE;
         a.partial = static_cast<float*>(workspace);
@@ -578,7 +576,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
     hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
     if (int rc = (int)hipGetLastError()) return rc;
-    return p.nsplit > 1 ? launch_reduce<bf16_t>(a.partial, a.out, n, nullptr, 0, n, p.nsplit, stream) : PBS_OK;
+    return p.nsplit > 1 ? launch_reduce<bf16_t>(a.partial, b, p.nsplit, stream) : PBS_OK;
 }
 
 // ---- scratch of the entry point that allocates nothing ----
@@ -794,7 +792,7 @@ static bool back_sizes_ok(int64_t tokens, int out_features, int in_features, int
 
 size_t pbs_blocksparse_matmul_back_units_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
-    return plan_back(dtype, tokens, out_features, in_features, nnz).slices > 0 ? unit_table_bytes(out_features, nnz) : 0;
+    return plan_back(dtype, tokens, out_features, in_features, nnz, false).slices > 0 ? unit_table_bytes(out_features, nnz) : 0;
 }
 
 int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int32_t* cols_a, int out_features, int in_features,
@@ -809,13 +807,13 @@ int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int
 
 size_t pbs_blocksparse_matmul_back_bias_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
-    return plan_back(dtype, tokens, out_features, in_features, nnz).partial_bytes;
+    return plan_back(dtype, tokens, out_features, in_features, nnz, true).partial_bytes;
 }
 
 size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz,
                                                    int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype) || nnz == 0) return 0;
-    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz);
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
     return p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz) : 0);
 }
 
@@ -840,8 +838,8 @@ static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, s
             if (int rc = zero(a.out, (size_t)a.nnz * 1024)) return rc;
         return a.bias_out ? zero(a.bias_out, a.N) : PBS_OK;
     }
-    const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, workspace_limit);
-    if (p.slices == 0) return a.bias_out ? PBS_ERR_BAD_SHAPE : launch_rectangles(a, p, workspace, workspace_bytes, s);
+    const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, a.bias_out != nullptr, workspace_limit);
+    if (p.slices == 0) return launch_rectangles(a, p, workspace, workspace_bytes, s);
     return dtype == PBS_DTYPE_F32 ? launch_row<float>(a, p, workspace, workspace_bytes, s) : launch_row<bf16_t>(a, p, workspace, workspace_bytes, s);
 }
 
@@ -963,7 +961,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
     if (back_sizes_ok(tokens, out_features, in_features, nnz, dtype) && nnz > 0) {
         const size_t table = unit_table_bytes(out_features, nnz);
         limit = (size_t)PBS_NOALLOC_SCRATCH_BYTES > table ? (size_t)PBS_NOALLOC_SCRATCH_BYTES - table : 0;
-        const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, limit);
+        const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, limit);
         need = p.partial_bytes + (p.slices > 0 ? table : 0);
     }
     if (need > (size_t)PBS_NOALLOC_SCRATCH_BYTES) return PBS_ERR_SCRATCH;
@@ -990,7 +988,7 @@ const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_feat
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || out_features <= 0 || in_features <= 0 ||
         nnz <= 0 || (out_features % 32) || (in_features % 32))
         return "";
-    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz);
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
     if (p.slices > 0) return p.slices > 1 ? "sdd_row_kernel + sdd_reduce_kernel" : "sdd_row_kernel";
     return p.rect.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";
 }

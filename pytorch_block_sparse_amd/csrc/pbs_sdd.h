@@ -13,7 +13,8 @@ struct SddArgs {
     const int32_t* ptr;      // row_start_ends_a [N/32 + 1]
     const int32_t* idx;      // cols_a [nnz][2] = (block col, data block)
     void* out;               // [nnz*32, 32] (T) when nsplit == 1
-    float* partial;          // [nsplit][nnz*1024] fp32 when nsplit > 1
+    void* bias_out;          // nullptr or [N] (T)
+    float* partial;          // [nsplit][nnz*1024, then N] fp32 when nsplit > 1
     int M, N, K, nnz;
     int tiles_r, tiles_c, nsplit;
     int tokens_per_split;    // multiple of TC
@@ -76,10 +77,10 @@ static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__
 }
 
 // Sums of the token slices, in slice order: n values of the blocks and, behind them, total - n of the bias (both multiples
-// of 4), `stride` apart from slice to slice.  Bound by the bytes of the partial sums; eight loads of a thread in flight
+// of 4).  Bound by the bytes of the partial sums; eight loads of a thread in flight
 // (one at a time: 16 slices of 256 blocks 9.9 us instead of 7.3).
 template <typename T>
-__global__ __launch_bounds__(256) void sdd_reduce_kernel(const float* partial, T* out, size_t n, T* bias_out, size_t total, size_t stride, int nsplit) {
+__global__ __launch_bounds__(256) void sdd_reduce_kernel(const float* partial, T* out, size_t n, T* bias_out, size_t total, int nsplit) {
     using E = Elem<T>;
     const size_t i4 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i4 >= total) return;
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(256) void sdd_reduce_kernel(const float* partial, T
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     f32x4 s = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(partial + i4));
 #pragma unroll 8
-    for (int k = 1; k < nsplit; ++k) s += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(partial + (size_t)k * stride + i4));
+    for (int k = 1; k < nsplit; ++k) s += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(partial + (size_t)k * total + i4));
     T* o = i4 < n ? out + i4 : bias_out + (i4 - n);
     o[0] = E::from_f32(s.x);
     o[1] = E::from_f32(s.y);

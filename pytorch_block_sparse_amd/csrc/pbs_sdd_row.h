@@ -432,7 +432,7 @@ __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel
     const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
     const int c_lo = slice * a.chunks_per_slice;
     const int c_hi = c_lo + a.chunks_per_slice < chunks ? c_lo + a.chunks_per_slice : chunks;
-    float* partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + a.N) : nullptr;
+    float* partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + (a.bias_out ? a.N : 0)) : nullptr;
     switch (unit[1]) {
         case 4: sdd_row_body<T, 4>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
         case 3: sdd_row_body<T, 3>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;

@@ -171,9 +171,8 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     return out;
 }
 
-// packed blocks of a^T b on the pattern, into `out`; and, if the kernel for this problem can, the sums of a's columns, into `sums`
-// (made here when wanted)
-void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out, Tensor* sums = nullptr) {
+// packed blocks of a^T b on the pattern, into `out`, and the sums of a's columns, into `sums` (if defined)
+void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out, const Tensor& sums = Tensor()) {
     check_gpu(a_any);
     check_gpu(b_any);
     check_gpu(out);
@@ -190,13 +189,12 @@ void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Ten
     c10::DeviceGuard guard(a.device());
     void* stream = current_stream(a);
     const void* units = p.units_for(tokens, code, stream);
-    if (sums && units) *sums = at::empty({p.out_features}, a.options());
     const size_t ws_bytes = pbs_blocksparse_matmul_back_bias_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
     check(pbs_blocksparse_matmul_back_bias(data_or_null(a), data_or_null(b), p.row_ptr.t.const_data_ptr<int>(),
                                            static_cast<const int*>(data_or_null(p.cols.t)), units, out.numel() ? out.mutable_data_ptr() : nullptr,
-                                           sums && units ? sums->mutable_data_ptr() : nullptr, tokens, p.out_features, p.in_features, p.nnz, code,
+                                           sums.defined() ? sums.mutable_data_ptr() : nullptr, tokens, p.out_features, p.in_features, p.nnz, code,
                                            ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
           "pbs_blocksparse_matmul_back_bias");
 }
@@ -222,9 +220,11 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
         if (task_should_compute_output(1)) {
             const Tensor xs = x.unpack(shared_from_this());
             out[1] = at::empty({(int64_t)pattern->nnz * 32, 32}, xs.options());
-            matmul_back(*pattern, dy, xs, out[1], has_bias && task_should_compute_output(2) ? &out[2] : nullptr);
+            if (has_bias && task_should_compute_output(2)) out[2] = at::empty({pattern->out_features}, xs.options());
+            matmul_back(*pattern, dy, xs, out[1], out[2]);
+        } else if (has_bias && task_should_compute_output(2)) {
+            out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
         }
-        if (has_bias && task_should_compute_output(2) && !out[2].defined()) out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
         return out;
     }
 };

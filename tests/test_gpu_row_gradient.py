@@ -43,3 +43,24 @@ def test_row_kernel(cuda, dtype, tokens, out_f, in_f, counts, slices):
     native.torch_path().linear(xd, data, bias, m._buffers, m.schedule()).backward(dyd)
     assert torch.equal(data.grad, got)   # with the bias gradient: the same sums
     assert_close(bias.grad, to64(dy).sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("tokens,out_f,in_f,counts", [
+    (16391, 1600, 512, [7, 0, 3, 16]),     # one rectangle per band sums all 16 rows; the last band has two
+    (17000, 1024, 544, [9, 1]),            # two rectangles share the rows, the second with a single column
+    (13007, 1056, 1056, [30, 2, 2, 2]),    # uneven rows are dealt to the bands; three rectangles: 6, 6 and 4 rows
+    (2600, 64, 10240, [90]),               # more rectangles than rows
+    (16384, 1024, 1024, [0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2]),   # rectangles without blocks
+])
+def test_bias_gradient_of_rectangles(cuda, tokens, out_f, in_f, counts):
+    dtype = torch.bfloat16
+    m = _layer(out_f, in_f, counts, dtype, cuda, 7)
+    name = native.matmul_back_kernel_name(tokens, out_f, in_f, m.cols_a.shape[0], dtype)
+    print(name, tokens, out_f, in_f, flush=True)
+    assert name.startswith("sdd_bf16_kernel")
+    g = torch.Generator().manual_seed(tokens)
+    x, dy = (torch.randn((tokens, f), generator=g).to(dtype).to(cuda) for f in (in_f, out_f))
+    data, bias = m.data.detach().clone().requires_grad_(), torch.zeros(out_f, dtype=dtype, device=cuda, requires_grad=True)
+    native.torch_path().linear(x, data, bias, m._buffers, m.schedule()).backward(dy)
+    assert_close(bias.grad, to64(dy).sum(0), dtype, "bias gradient")
+    assert torch.equal(data.grad, m.matmul_with_output_sparse_support(dy, x))   # (checked against the oracle without it)
