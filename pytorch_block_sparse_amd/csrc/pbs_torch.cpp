@@ -84,50 +84,98 @@ struct Seen {
     }
 };
 
+bool capturing(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status);
+    TORCH_CHECK(e == hipSuccess, "hipStreamIsCapturing: ", hipGetErrorString(e));
+    return status != hipStreamCaptureStatusNone;
+}
+
+// A buffer that kernels on one stream fill and products on any stream read: each other stream waits for the filling once, and
+// the allocator learns of it.  A stream that is being captured cannot wait for work outside its graph: whoever captures
+// has the earlier work finished first (torch.cuda.graph waits for the device).
+struct Derived {
+    Tensor t;
+    void* filled_on = nullptr;
+    hipEvent_t event = nullptr;
+    c10::SmallVector<void*, 4> waited;
+
+    Derived() = default;
+    Derived(const Derived&) = delete;
+    Derived& operator=(const Derived&) = delete;
+    ~Derived() {
+        if (event) (void)hipEventDestroy(event);
+    }
+    void use_on(void* stream) {
+        if (!t.defined() || stream == filled_on || capturing(stream)) return;
+        for (void* w : waited)
+            if (w == stream) return;
+        const hipError_t e = hipStreamWaitEvent(static_cast<hipStream_t>(stream), event, 0);
+        TORCH_CHECK(e == hipSuccess, "hipStreamWaitEvent: ", hipGetErrorString(e));
+        t.record_stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).unwrap());
+        waited.push_back(stream);
+    }
+    // after the kernels that fill `now` were launched on `stream`, which has waited for what was in it before
+    void filled(const Tensor& now, void* stream) {
+        hipError_t e = event ? hipSuccess : hipEventCreateWithFlags(&event, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(event, static_cast<hipStream_t>(stream));
+        TORCH_CHECK(e == hipSuccess, "hipEventRecord: ", hipGetErrorString(e));
+        t = now;
+        filled_on = stream;
+        waited.clear();
+    }
+};
+
 // One pattern: its index arrays and the plans of both directions.  Never changed once made, except that parts of
 // the plans are added when a product first needs them; a matrix whose index arrays change gets a new one, and autograd
-// nodes keep the one of their forward product.
+// nodes keep the one of their forward product.  A part that is first needed while a graph is captured exists only
+// when the graph has run: it is built inside the graph, for the graph, and not kept.
 struct Pattern {
     Seen row_ptr, cols, col_ptr, rows;
     int out_features = 0, in_features = 0, nnz = 0;
     std::mutex lock;
-    Tensor plan[2];      // [transpose]
+    Derived plan[2];     // [transpose]
     int parts[2] = {0, 0};
-    Tensor units;        // of the weight gradient
+    Derived units;       // of the weight gradient
 
     bool still(const Tensor& rp, const Tensor& c, const Tensor& cp, const Tensor& r) const {
         return row_ptr.still(rp) && cols.still(c) && col_ptr.still(cp) && rows.still(r);
     }
 
-    const void* plan_for(bool transpose, int n, int k, int part, void* stream) {
+    Tensor plan_for(bool transpose, int n, int k, int part, void* stream) {
         std::lock_guard<std::mutex> hold(lock);
+        Derived& kept = plan[transpose];
+        kept.use_on(stream);
         part |= PBS_PLAN_LIST;
-        if ((parts[transpose] & part) != part) {
-            const Tensor& ptr = transpose ? row_ptr.t : col_ptr.t;
-            const Tensor& idx = transpose ? cols.t : rows.t;
-            TORCH_CHECK(ptr.is_cuda() && idx.is_cuda(), "the index buffers are not on the GPU");
-            const size_t bytes = pbs_blocksparse_matmul_plan_bytes(n, k);
-            if (!plan[transpose].defined()) plan[transpose] = at::empty({(int64_t)bytes}, ptr.options().dtype(at::kByte));
-            check(pbs_blocksparse_matmul_plan_part(ptr.const_data_ptr<int>(), idx.const_data_ptr<int>(), n, k, nnz, part & ~parts[transpose],
-                                                   plan[transpose].mutable_data_ptr(), bytes, stream),
-                  "pbs_blocksparse_matmul_plan_part");
+        if ((parts[transpose] & part) == part) return kept.t;
+        const Tensor& ptr = transpose ? row_ptr.t : col_ptr.t;
+        const Tensor& idx = transpose ? cols.t : rows.t;
+        TORCH_CHECK(ptr.is_cuda() && idx.is_cuda(), "the index buffers are not on the GPU");
+        const bool keep = !capturing(stream);
+        const size_t bytes = pbs_blocksparse_matmul_plan_bytes(n, k);
+        const Tensor t = keep && kept.t.defined() ? kept.t : at::empty({(int64_t)bytes}, ptr.options().dtype(at::kByte));
+        check(pbs_blocksparse_matmul_plan_part(ptr.const_data_ptr<int>(), idx.const_data_ptr<int>(), n, k, nnz,
+                                               keep ? part & ~parts[transpose] : part, t.mutable_data_ptr(), bytes, stream),
+              "pbs_blocksparse_matmul_plan_part");
+        if (keep) {
+            kept.filled(t, stream);
             parts[transpose] |= part;
         }
-        return plan[transpose].const_data_ptr();
+        return t;
     }
-    const void* units_for(int64_t tokens, int code, void* stream) {
+    Tensor units_for(int64_t tokens, int code, void* stream) {
         const size_t bytes = pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, code);
-        if (!bytes) return nullptr;
+        if (!bytes) return Tensor();
         std::lock_guard<std::mutex> hold(lock);
-        if (!units.defined()) {
-            TORCH_CHECK(row_ptr.t.is_cuda() && cols.t.is_cuda(), "the index buffers are not on the GPU");
-            Tensor t = at::empty({(int64_t)bytes}, row_ptr.t.options().dtype(at::kByte));
-            check(pbs_blocksparse_matmul_back_units(row_ptr.t.const_data_ptr<int>(), nnz ? cols.t.const_data_ptr<int>() : nullptr, out_features,
-                                                    in_features, nnz, t.mutable_data_ptr(), bytes, stream),
-                  "pbs_blocksparse_matmul_back_units");
-            units = t;
-        }
-        return units.const_data_ptr();
+        units.use_on(stream);
+        if (units.t.defined()) return units.t;
+        TORCH_CHECK(row_ptr.t.is_cuda() && cols.t.is_cuda(), "the index buffers are not on the GPU");
+        const Tensor t = at::empty({(int64_t)bytes}, row_ptr.t.options().dtype(at::kByte));
+        check(pbs_blocksparse_matmul_back_units(row_ptr.t.const_data_ptr<int>(), nnz ? cols.t.const_data_ptr<int>() : nullptr, out_features,
+                                                in_features, nnz, t.mutable_data_ptr(), bytes, stream),
+              "pbs_blocksparse_matmul_back_units");
+        if (!capturing(stream)) units.filled(t, stream);
+        return t;
     }
 };
 using PatternPtr = std::shared_ptr<Pattern>;
@@ -159,12 +207,12 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     Tensor out = at::empty(sizes, a.options());
     if (tokens == 0) return out;
     const int part = pbs_blocksparse_matmul_part(tokens, n, k, p.nnz, transpose, code, 1);
-    const void* plan = p.plan_for(transpose, n, k, part, stream);
+    const Tensor plan = p.plan_for(transpose, n, k, part, stream);
     // the transposed copy of the blocks that the bf16 column kernel's forward product works from
     const size_t ws_bytes = transpose && part == PBS_PLAN_COLUMN ? pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, p.nnz, 1, code) : 0;
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
-    check(pbs_blocksparse_matmul_ws(a.const_data_ptr(), data_or_null(data), plan, data_or_null(bias), out.mutable_data_ptr(), tokens, n, k,
+    check(pbs_blocksparse_matmul_ws(a.const_data_ptr(), data_or_null(data), plan.const_data_ptr(), data_or_null(bias), out.mutable_data_ptr(), tokens, n, k,
                                     p.nnz, transpose, code, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
           "pbs_blocksparse_matmul_ws");
     check_protocol("pbs_blocksparse_matmul_ws", a.device().index());
@@ -188,12 +236,12 @@ void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Ten
     TORCH_CHECK(b.numel() / p.in_features == tokens, "Invalid matrices sizes ", a.sizes(), "^T x ", b.sizes());
     c10::DeviceGuard guard(a.device());
     void* stream = current_stream(a);
-    const void* units = p.units_for(tokens, code, stream);
+    const Tensor units = p.units_for(tokens, code, stream);
     const size_t ws_bytes = pbs_blocksparse_matmul_back_bias_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
     check(pbs_blocksparse_matmul_back_bias(data_or_null(a), data_or_null(b), p.row_ptr.t.const_data_ptr<int>(),
-                                           static_cast<const int*>(data_or_null(p.cols.t)), units, out.numel() ? out.mutable_data_ptr() : nullptr,
+                                           static_cast<const int*>(data_or_null(p.cols.t)), data_or_null(units), out.numel() ? out.mutable_data_ptr() : nullptr,
                                            sums.defined() ? sums.mutable_data_ptr() : nullptr, tokens, p.out_features, p.in_features, p.nnz, code,
                                            ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
           "pbs_blocksparse_matmul_back_bias");
