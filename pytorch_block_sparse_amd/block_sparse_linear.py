@@ -111,7 +111,8 @@ class BlockSparseLinear(nn.Module):
 
     def forward(self, x):
         weight = self.weight
-        if isinstance(weight, BlockSparseMatrix):
+        # (torch.jit.trace can record the autograd function, but not see into the native call)
+        if isinstance(weight, BlockSparseMatrix) and not torch.jit.is_tracing():
             return native.torch_path().linear(x, weight.data, self.bias, weight._buffers, weight.schedule())
         return self.fn(x, self.weight.get_differentiable_data(), self.weight, self.bias)
 

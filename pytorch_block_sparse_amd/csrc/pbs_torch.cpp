@@ -262,15 +262,20 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
         torch::autograd::variable_list out(3);
         const Tensor& g = grads[0];
         if (!g.defined()) return out;
+        // under create_graph the sum of dy is recorded, as the operator it is; the products have no second derivative
+        const bool record = c10::GradMode::is_enabled() && has_bias && task_should_compute_output(2);
+        if (record) out[2] = g.reshape({-1, g.size(-1)}).sum(0);
+        const bool sums = has_bias && !record && task_should_compute_output(2);
         at::NoGradGuard no_grad;
         const Tensor dy = g.is_contiguous() ? g : g.contiguous();
         if (task_should_compute_output(0)) out[0] = matmul(*pattern, dy, data.unpack(shared_from_this()), Tensor(), false);
         if (task_should_compute_output(1)) {
             const Tensor xs = x.unpack(shared_from_this());
             out[1] = at::empty({(int64_t)pattern->nnz * 32, 32}, xs.options());
-            if (has_bias && task_should_compute_output(2)) out[2] = at::empty({pattern->out_features}, xs.options());
-            matmul_back(*pattern, dy, xs, out[1], out[2]);
-        } else if (has_bias && task_should_compute_output(2)) {
+            Tensor db;
+            if (sums) out[2] = db = at::empty({pattern->out_features}, xs.options());
+            matmul_back(*pattern, dy, xs, out[1], db);
+        } else if (sums) {
             out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
         }
         return out;
@@ -278,6 +283,8 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
 };
 
 Tensor linear(const PatternPtr& p, const Tensor& x, const Tensor& data, const Tensor& bias) {
+    for (const Tensor* t : {&x, &data, &bias})
+        TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), "the block-sparse linear layer has no forward-mode derivative");
     Tensor y;
     {
         at::NoGradGuard no_grad;
