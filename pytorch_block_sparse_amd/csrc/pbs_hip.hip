@@ -11,6 +11,7 @@
 #include "pbs_common.h"
 #include "pbs_dds16.h"
 #include "pbs_ddsc.h"
+#include "pbs_panel.h"
 #include "pbs_stream.h"
 #include "pbs_index.h"
 #include "pbs_sdd.h"
@@ -339,6 +340,41 @@ static int launch_stream(const DdsArgs& g, hipStream_t stream) {
     return PBS_ERR_TOO_LARGE;
 }
 
+// ---- bf16, the token tile in LDS ----
+// Estimated time in us and the number of workgroups per token tile: launch; per round of workgroups over the chip (one per CU) its
+// start, the tile, the blocks of the wave with the most, the stores; and what memory takes for the dense operands.  Fitted to 90
+// problems (K 256 to 1024, results 256 to 4096 wide, 200 to 16384 tokens, densities 0.1 to 0.75, 1 to 16 workgroups per tile),
+// met within 6 % on average; the number it picks is never more than 1.2 % slower than the best one.
+struct PanelChoice {
+    int splits;   // 0: the kernel cannot run the problem
+    double us;
+};
+static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
+    PanelChoice best{0, 0.0};
+    const int cols = n / 32;
+    // (below 1024 tokens, or with fewer columns than waves, it was the faster one nowhere)
+    if (k > PANEL_MAX_K || nnz < 1 || M < 1024 || cols < PANEL_NW) return best;
+    const double tiles = (double)((M + 16 * PANEL_TT - 1) / (16 * PANEL_TT));
+    for (int s = 1; s <= 16 && s <= cols; ++s) {
+        const int mine = (cols + s - 1) / s, turns = (mine + PANEL_NW - 1) / PANEL_NW;
+        const double us = 2.13 + std::ceil(tiles * s / 256) * (0.656 + 0.051 * (k / 32) + 0.33 * turns * nnz / cols + 0.133 * mine) +
+                          0.09e-6 * 2.0 * (double)M * (n + k);
+        if (best.splits == 0 || us < best.us) best = PanelChoice{s, us};
+    }
+    return best;
+}
+template <int TRANS>
+static int launch_panel(const DdsArgs& g, int splits, hipStream_t stream) {
+    static std::atomic<uint64_t> done{0};
+    auto kernel = panel_kernel<TRANS>;
+    const PanelArgs a{g.a, g.data, g.plan, g.bias, g.out, g.M, g.N, g.K, splits};
+    const long long wgs = (long long)((g.M + 16 * PANEL_TT - 1) / (16 * PANEL_TT)) * splits;
+    if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), panel_lds(g.K), stream, a);
+    return (int)hipGetLastError();
+}
+
 // ---- which kernel runs a product ----
 enum MatmulPart { PART_LIST = PBS_PLAN_LIST, PART_WIDE = PBS_PLAN_WIDE, PART_COLUMN = PBS_PLAN_COLUMN };   // and so which part of the plan it reads
 
@@ -354,27 +390,38 @@ static double column_us(long long M, int n, int k, int nnz, bool copy) {
     const ColumnLaunch c = column_launch(M, n);
     return (double)((c.m_tiles + c.wg_per_group - 1) / c.wg_per_group) * (0.262 * (k / 64) + 0.429 * nnz / (n / 32) + 12.2) + (copy ? 0.0031 * nnz : 0.0);
 }
-// The column kernel where column_kernel_fits: from 8192 tokens without further question (it is the faster one in nearly
-// all of that range and within a few us in the rest), below that where its estimate is the smallest.
-static int choose_part(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
-    if (esz == 4) return PART_LIST;
+// The column kernel where column_kernel_fits: from 8192 tokens against the others without further question (it is the
+// faster one in nearly all of that range and within a few us in the rest), otherwise the smallest estimate.
+struct ProductChoice {
+    int part;
+    int panel_splits;   // > 0: panel_kernel, which reads the list plan like stream_kernel
+};
+static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
+    if (esz == 4) return {PART_LIST, 0};
     const int wish = column_kernel_wish();
     const bool wide = wide_kernel_fits(M, n, k);
     const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz);
-    if (wish == 1 && column) return PART_COLUMN;
-    if (wish == 0 && wide) return PART_WIDE;
-    if (column && M >= 8192) return PART_COLUMN;
+    if (wish == 1 && column) return {PART_COLUMN, 0};
+    if (wish == 0 && wide) return {PART_WIDE, 0};
+    const PanelChoice panel = choose_panel(M, n, k, nnz);
+    // (where the estimates are within 6 % of each other the panel kernel was up to 5 % the slower one as often as the faster:
+    // 70 drawn problems, of which it takes 20 and is 1.02 to 1.8 times faster in them)
+    const double tp = panel.splits ? 1.06 * panel.us : 1e300;
+    const double tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
+    if (column && M >= 8192) return tp < tc ? ProductChoice{PART_LIST, panel.splits} : ProductChoice{PART_COLUMN, 0};
     const double ts = choose_stream(esz, M, n, k, nnz).us;
-    const double tw = wide ? wide_us(M, n, k, nnz) : 1e300, tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
-    if (tc < ts && tc < tw) return PART_COLUMN;
-    return tw < ts ? PART_WIDE : PART_LIST;
+    const double tw = wide ? wide_us(M, n, k, nnz) : 1e300;
+    if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel.splits};
+    if (tc < ts && tc < tw) return {PART_COLUMN, 0};
+    return {tw < ts ? PART_WIDE : PART_LIST, 0};
 }
 
 template <typename T, int TRANS>
 static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     if constexpr (sizeof(T) == 2) {
         const bool copy = workspace && workspace_bytes >= (size_t)g.nnz * 2048 && aligned16(workspace);
-        const int part = choose_part(2, g.M, g.N, g.K, g.nnz, !TRANS, copy);
+        const ProductChoice choice = choose_product(2, g.M, g.N, g.K, g.nnz, !TRANS, copy);
+        const int part = choice.part;
         if (part == PART_COLUMN && (reinterpret_cast<uintptr_t>(g.bias) & 3u) == 0) {   // (it reads the bias in words)
             // the kernel wants every block with k along its rows: as stored for TRANS, a transposed copy otherwise
             if constexpr (TRANS) return launch_ddsc<false>(g, g.data, stream);
@@ -384,6 +431,7 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
             return launch_ddsc<true>(g, workspace, stream);
         }
         if (part == PART_WIDE) return launch_dds16<TRANS>(g, stream);
+        if (choice.panel_splits) return launch_panel<TRANS>(g, choice.panel_splits, stream);
     }
     return launch_stream<T, TRANS>(g, stream);
 }
@@ -742,13 +790,13 @@ int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int 
 int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || nnz < 0 || (n % 32) || (k % 32))
         return PART_LIST;
-    return choose_part(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
+    return choose_product(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0).part;
 }
 
 size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype) {
     if (dtype != PBS_DTYPE_BF16 || !transpose || tokens <= 0 || n <= 0 || k <= 0 || nnz <= 0 || (n % 32) || (k % 32)) return 0;
     if ((long long)nnz > (long long)(n / 32) * (k / 32)) return 0;
-    return choose_part(2, tokens, n, k, nnz, 1, true) == PART_COLUMN ? (size_t)nnz * 2048 : 0;
+    return choose_product(2, tokens, n, k, nnz, 1, true).part == PART_COLUMN ? (size_t)nnz * 2048 : 0;
 }
 
 int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* plan, const void* bias, void* dense_out,
@@ -980,8 +1028,8 @@ int pbs_protocol_failures(unsigned* count) {
 const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int nnz, int transpose, int dtype,
                                                int with_workspace) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || (n % 32) || (k % 32)) return "";
-    const int part = pbs_blocksparse_matmul_part(tokens, n, k, nnz, transpose, dtype, with_workspace);
-    return part == PART_COLUMN ? "ddsc_kernel" : (part == PART_WIDE ? "dds16_kernel" : "stream_kernel");
+    const ProductChoice c = choose_product(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
+    return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (c.panel_splits ? "panel_kernel" : "stream_kernel"));
 }
 
 const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {

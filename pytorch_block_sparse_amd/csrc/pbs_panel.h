@@ -1,0 +1,206 @@
+// dense x block-sparse -> dense for bf16 with a short contraction (K <= 1024): the workgroup's token tile stays in LDS.
+//
+// A workgroup of 16 waves copies its 64 tokens, all K features of them, into LDS once, in whole rows; after one barrier each
+// wave multiplies block columns of its own, one after the other, and nothing is shared but the tile, which nobody writes any
+// more: no progress words, no further barrier, and a column costs what it holds.  A wave's block (2 KB) passes through LDS of
+// its own like in pbs_stream.h: DMA, fragments into registers, and the place takes the next block's DMA, of the next
+// column too.
+//
+// Why: the stream kernel fetches the token tile again for every block (10 KB per block and 128 tokens, in rows of 64 bytes, is
+// what bounds it), the wide kernel (pbs_dds16.h) moves panels through a ring and pays for every step of it.  Here a
+// block costs 2 KB of copies and 64 tokens' fragments from LDS, and four waves per SIMD keep the matrix cores near their rate
+// while they multiply: a block takes 128 cycles of a SIMD, which is what its matrix instructions take.  What is left around that:
+// launch, list and tile (4 to 6 us), and the stores, which bound wide results (768 -> 3072 at 16384 tokens writes 100 MB).
+// One block at a time per wave: a second place in the ring is 3 to 7 % slower (its LDS, and two loads in flight per wave
+// are not needed with four waves per SIMD); tiles of 32 tokens are 20 to 60 % slower from 2000 tokens (twice the copies).
+//
+// Measured, us, against what ran before: 768 -> 3072 density 0.5, 2317 tokens 22.9 -> 13.7 (stream), 4096 tokens 29.6 -> 19.5,
+// 16384 tokens 123 -> 53.5 (wide); 768 -> 3072 density 0.1, 16384 tokens 40 -> 28; 768 -> 768 density 0.5, 16384 tokens
+// 25.8 -> 20.6; 992 -> 2016 density 0.5, 16384 tokens 92 -> 46.  Below some thousand tokens, or with few columns, the stream
+// kernel is the faster one (768 -> 768, 2317 tokens 8.3 against 9.7).
+#pragma once
+#include "pbs_common.h"
+#include "pbs_stream.h"
+
+namespace pbs {
+
+constexpr int PANEL_NW = 16;          // waves of a workgroup
+constexpr int PANEL_TT = 4;           // token tile in units of 16
+constexpr int PANEL_MAX_K = 1024;     // 160 KB of LDS: the tile and a block per wave; a column's list fits half a wave
+
+struct PanelArgs {
+    const void* a;      // [M, K] row-major
+    const void* data;   // [nnz*32, 32]
+    const int* plan;    // the list plan
+    const void* bias;   // nullptr or [N]
+    void* out;          // [M, N] row-major
+    int M, N, K;
+    int splits;         // workgroups that share a token tile: every splits-th column of the ranking each
+};
+
+// a row of the tile in LDS, in 16-byte chunks: whole groups of 16 (256 bytes), so that the swizzle stays inside a group
+static inline __host__ __device__ int panel_chunks(int K) { return (K / 8 + 15) / 16 * 16; }
+static inline size_t panel_lds(int K) { return (size_t)16 * PANEL_TT * panel_chunks(K) * 16 + (size_t)PANEL_NW * 2048; }
+
+// TRANS as in stream_kernel.
+template <int TRANS>
+__global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_kernel(PanelArgs g) {
+    using E = Elem<bf16_t>;
+    constexpr int TT = PANEL_TT, BM = 16 * TT, NW = PANEL_NW;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int ncols = g.N >> 5;
+    const int tiles = (g.M + BM - 1) / BM;
+    const int id = xcd_tile_id(blockIdx.x, tiles * g.splits);
+    if (id < 0) return;
+    const int tile = id / g.splits, split = id - tile * g.splits;
+    const int m0 = tile * BM;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+
+    const int ckp = panel_chunks(g.K), pitch = ckp * 16;
+    const unsigned char* A = static_cast<const unsigned char*>(g.a) + (size_t)m0 * g.K * 2;
+    const unsigned char* D = static_cast<const unsigned char*>(g.data);
+    const unsigned lds0 = (unsigned)(uintptr_t)smem;
+    unsigned char* const place = smem + BM * pitch + wave * 2048;   // this wave's block
+    const unsigned lds_place = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)place);
+
+    // ---- the token tile: chunk p of row t holds chunk p ^ (t % 16) of the row, so that 16 rows' reads of one chunk meet no bank twice ----
+    {
+        const int rows = g.M - m0 < BM ? g.M - m0 : BM, last = g.K / 8 - 1;
+        for (int i = wave; i < BM * ckp / 64; i += NW) {
+            const int at = i * 64 + lane, t = at / ckp;
+            int c = (at - t * ckp) ^ (t & 15);
+            c = c < last ? c : last;
+            dma16(__builtin_amdgcn_readfirstlane(lds0 + i * 1024), A, (unsigned)((t < rows ? t : rows - 1) * (g.K * 2) + c * 16));
+        }
+    }
+
+    // ---- this wave's columns: of the workgroup's (ranked by length) one in each run of NW, the runs taken forth and back ----
+    const int nc = (ncols - split + g.splits - 1) / g.splits;
+    auto turn = [&](int i) { return i * NW + (i & 1 ? NW - 1 - wave : wave); };
+    int mine = nc / NW;
+    if (turn(mine) < nc) ++mine;
+    const int pairs = (mine + 1) / 2;
+    // two columns at a time, one per half of the wave: lane l has the half's column, its length, entry l % 32 and bias l % 32
+    struct Pair {
+        int n, col;
+        int2 e;
+        float b;
+    };
+    const int2* ent = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4);
+    auto load_pair = [&](int p) {
+        Pair o{0, 0, make_int2(0, 0), 0.f};
+        const int i = 2 * p + (lane >> 5), l = lane & 31;
+        if (i < mine) {
+            const int4 head = reinterpret_cast<const int4*>(g.plan)[split + g.splits * turn(i)];
+            o.n = head.z < 32 ? head.z : 32;
+            o.col = head.x;
+            if (o.n > 0) o.e = ent[head.y + (l < o.n ? l : o.n - 1)];
+            if (g.bias) o.b = E::to_f32(static_cast<const bf16_t*>(g.bias)[head.x * 32 + l]);
+        }
+        return o;
+    };
+    Pair cur = load_pair(0), nxt = load_pair(1);
+    float bias_of[2] = {cur.b, 0.f};   // by pair % 2
+
+    auto w_row_swz = [](int row) { return (row >> 3) & 3; };
+    unsigned w_voff[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int row = i * 16 + lane / 4;
+        w_voff[i] = TRANS ? row * 64 + ((lane & 3) ^ w_row_swz(row)) * 16 : i * 1024 + lane * 16;
+    }
+
+    // ---- the blocks in the order they are multiplied, asked for one ahead ----
+    constexpr int LAST = 1, EMPTY = 2, HALF = 4, ODD = 8, VALID = 16;
+    int kb = 0, col = 0, what = 0;   // the block asked for: k-block, block column, flags
+    int pair = 0, half = 0, idx = 0;
+    auto ask = [&]() __attribute__((always_inline)) {
+        what = 0;
+        if (pair >= pairs) return;
+        const int src = half * 32;
+        const int n = __builtin_amdgcn_readlane(cur.n, src);
+        col = __builtin_amdgcn_readlane(cur.col, src);
+        kb = __builtin_amdgcn_readlane(cur.e.x, src + idx);
+        // (a column without blocks asks for some block and does not multiply it)
+        const unsigned char* pw = uniform_ptr(D + (size_t)__builtin_amdgcn_readlane(cur.e.y, src + idx) * 2048);
+        dma16(lds_place, pw, w_voff[0]);
+        dma16(lds_place + 1024, pw, w_voff[1]);
+        const bool end = idx + 1 >= n;
+        what = VALID | (end ? LAST : 0) | (n == 0 ? EMPTY : 0) | (half ? HALF : 0) | (pair & 1 ? ODD : 0);
+        ++idx;
+        if (end) {
+            idx = 0;
+            ++half;
+            if (half == 2 || 2 * pair + half >= mine) {
+                half = 0;
+                ++pair;
+                cur = nxt;
+                nxt = load_pair(pair + 1);
+                if (pair & 1) bias_of[1] = cur.b;
+                else bias_of[0] = cur.b;
+            }
+        }
+    };
+    ask();
+
+    drain_barrier();   // the tile is there
+
+    f32x4 acc[TT][2];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned char* a_row = smem + r * pitch;
+    while (what & VALID) {
+        wait_dma(0);
+        uint4 fa[TT], fw[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if constexpr (TRANS) {
+                const int row = 8 * (r >> 2) + 4 * j + (r & 3);
+                fw[j] = *reinterpret_cast<const uint4*>(place + row * 64 + (q ^ w_row_swz(row)) * 16);
+            } else {
+                const unsigned char* p = place + (8 * q + (r >> 2)) * 64 + (r & 3) * 16 + 8 * j;
+                const uint2 lo = tr16_b64(p), hi = tr16_b64(p + 256);
+                fw[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            }
+        }
+        const unsigned char* as = a_row + (((kb * 4 + q) ^ r) * 16);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) fa[t] = *reinterpret_cast<const uint4*>(as + 16 * t * pitch);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const int now = what;
+        const size_t out_col = (size_t)col * 32 + 8 * q;
+        const float b = now & ODD ? bias_of[1] : bias_of[0];   // (before the next pair but one may replace it)
+        ask();
+        if (!(now & EMPTY)) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fw[j]), __builtin_bit_cast(bf16x8, fa[t]), acc[t][j], 0, 0, 0);
+        }
+        if (now & LAST) {
+            // a lane's eight results of a token: columns 8 q .. 8 q + 7, four of each parity
+            float bv[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) bv[i] = __shfl(b, (now & HALF ? 32 : 0) + 8 * q + i, 64);
+            uint16_t* out = static_cast<uint16_t*>(g.out) + out_col;
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const int row = m0 + 16 * t + r;
+                uint32_t w[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v0 = acc[t][i >> 1][2 * (i & 1)] + bv[2 * i], v1 = acc[t][i >> 1][2 * (i & 1) + 1] + bv[2 * i + 1];
+                    w[i] = (uint32_t)E::from_f32(v0).bits | ((uint32_t)E::from_f32(v1).bits << 16);
+                }
+                if (row < g.M) *reinterpret_cast<uint4*>(out + (size_t)row * g.N) = make_uint4(w[0], w[1], w[2], w[3]);
+                acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+    }
+}
+
+}  // namespace pbs
