@@ -348,9 +348,10 @@ static int launch_stream(const DdsArgs& g, hipStream_t stream) {
 struct PanelChoice {
     int splits;   // 0: the kernel cannot run the problem
     double us;
+    int turns;    // columns of a wave
 };
 static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
-    PanelChoice best{0, 0.0};
+    PanelChoice best{0, 0.0, 0};
     const int cols = n / 32;
     // (below 1024 tokens, or with fewer columns than waves, it was the faster one nowhere)
     if (k > PANEL_MAX_K || nnz < 1 || M < 1024 || cols < PANEL_NW) return best;
@@ -359,7 +360,7 @@ static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
         const int mine = (cols + s - 1) / s, turns = (mine + PANEL_NW - 1) / PANEL_NW;
         const double us = 2.13 + std::ceil(tiles * s / 256) * (0.656 + 0.051 * (k / 32) + 0.33 * turns * nnz / cols + 0.133 * mine) +
                           0.09e-6 * 2.0 * (double)M * (n + k);
-        if (best.splits == 0 || us < best.us) best = PanelChoice{s, us};
+        if (best.splits == 0 || us < best.us) best = PanelChoice{s, us, turns};
     }
     return best;
 }
@@ -390,8 +391,12 @@ static double column_us(long long M, int n, int k, int nnz, bool copy) {
     const ColumnLaunch c = column_launch(M, n);
     return (double)((c.m_tiles + c.wg_per_group - 1) / c.wg_per_group) * (0.262 * (k / 64) + 0.429 * nnz / (n / 32) + 12.2) + (copy ? 0.0031 * nnz : 0.0);
 }
-// The column kernel where column_kernel_fits: from 8192 tokens against the others without further question (it is the
-// faster one in nearly all of that range and within a few us in the rest), otherwise the smallest estimate.
+// The column kernel where column_kernel_fits: from 8192 tokens against the stream and the wide kernel without further question
+// (it is the faster one in nearly all of that range and within a few us in the rest), otherwise the smallest estimate.
+// The panel kernel against it: its estimate is up to 25 % short where a wave takes many full columns (the matrix cores, and
+// with them the power limit, are then what counts), the column kernel's is 4 us short for few steps and 12 % long for many; so
+// corrected, of 135 problems (K 512 to 1024, results 2048 to 4096 wide, densities 0.1 to 0.75, 4096 to 16384 tokens) the panel kernel
+// is given those in which it is 1.05 to 2.2 times the faster one, and the densest ones, where it is up to 13 % the slower one, are not.
 struct ProductChoice {
     int part;
     int panel_splits;   // > 0: panel_kernel, which reads the list plan like stream_kernel
@@ -408,7 +413,7 @@ static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz,
     // 70 drawn problems, of which it takes 20 and is 1.02 to 1.8 times faster in them)
     const double tp = panel.splits ? 1.06 * panel.us : 1e300;
     const double tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
-    if (column && M >= 8192) return tp < tc ? ProductChoice{PART_LIST, panel.splits} : ProductChoice{PART_COLUMN, 0};
+    if (column && M >= 8192) return panel.splits && (1.0 + 0.03 * panel.turns) * panel.us < 4.0 + 0.88 * tc ? ProductChoice{PART_LIST, panel.splits} : ProductChoice{PART_COLUMN, 0};
     const double ts = choose_stream(esz, M, n, k, nnz).us;
     const double tw = wide ? wide_us(M, n, k, nnz) : 1e300;
     if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel.splits};
