@@ -132,6 +132,16 @@ int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices,
 int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace);
 
 /*
+ * What a training step derives from a pattern, in one launch: the PBS_PLAN_LIST part of the plans of both directions (forward:
+ * of the transposed weight) and, if `units` is not NULL, the unit table of the weight gradient
+ * (pbs_blocksparse_matmul_back_units).  Same results, buffers and sizes as the calls that make them one by one.
+ */
+int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_a, const int32_t* col_start_ends_b,
+                           const int32_t* rows_b, int out_features, int in_features, int nnz, void* plan_forward,
+                           size_t plan_forward_bytes, void* plan_input, size_t plan_input_bytes, void* units,
+                           size_t units_bytes, void* stream);
+
+/*
  * dense x block-sparse -> dense.  Replaces blocksparse_matmul_cutlass
  * (native/block_sparse_native.cpp:6-16, launcher native/block_sparse_cutlass_kernel.cu:113-150)
  * as called by BlockSparseMatrixBase.reverse_matmul_ (block_sparse.py:496-578).

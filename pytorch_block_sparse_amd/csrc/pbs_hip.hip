@@ -555,8 +555,8 @@ static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int
         before = t + 16 + units * UNIT_INTS;
         hipLaunchKernelGGL(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, before);
     }
-    hipLaunchKernelGGL(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, ptr, idx, nnz, N / 32, K / 32, before,
-                       (int)units, t);
+    const UnitArgs a{ptr, idx, nnz, N / 32, K / 32, before, (int)units, t};
+    hipLaunchKernelGGL(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, a);
     return (int)hipGetLastError();
 }
 
@@ -749,9 +749,8 @@ int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices,
     hipStream_t s = static_cast<hipStream_t>(stream);
     unsigned char* base = static_cast<unsigned char*>(plan);
     if (part & PART_LIST) {
-        const long long work = (long long)nnz > 64ll * (n / 32) ? nnz : 64ll * (n / 32);
-        const unsigned grid = (unsigned)(work < 256 ? 1 : (work > 256ll * 1024 ? 1024 : (work + 255) / 256));
-        hipLaunchKernelGGL(list_plan_kernel, dim3(grid), dim3(256), 0, s, ptr, indices, n / 32, k / 32, nnz, reinterpret_cast<int*>(base));
+        const ListArgs a{ptr, indices, n / 32, k / 32, nnz, reinterpret_cast<int*>(base)};
+        hipLaunchKernelGGL(list_plan_kernel, dim3(list_plan_grid(n / 32, nnz)), dim3(256), 0, s, a);
         if (int rc = (int)hipGetLastError()) return rc;
     }
     if ((part & PART_WIDE) && wide_plan_bytes(n, k)) {
@@ -868,6 +867,29 @@ size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_featu
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype) || nnz == 0) return 0;
     const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
     return p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz) : 0);
+}
+
+int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_a, const int32_t* col_start_ends_b, const int32_t* rows_b,
+                           int out_features, int in_features, int nnz, void* plan_forward, size_t plan_forward_bytes, void* plan_input,
+                           size_t plan_input_bytes, void* units, size_t units_bytes, void* stream) {
+    if (int rc = plan_checks(row_start_ends_a, cols_a, out_features, in_features, nnz, plan_forward, plan_forward_bytes)) return rc;
+    if (int rc = plan_checks(col_start_ends_b, rows_b, in_features, out_features, nnz, plan_input, plan_input_bytes)) return rc;
+    if (units && !aligned16(units)) return PBS_ERR_MISALIGNED;
+    if (units && units_bytes < unit_table_bytes(out_features, nnz)) return PBS_ERR_WORKSPACE;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int N = out_features / 32, K = in_features / 32;
+    const bool with_units = units && !unit_prefix_bytes(out_features);   // (very tall matrices need a launch before that one)
+    DeriveArgs a;
+    a.list[0] = ListArgs{row_start_ends_a, cols_a, N, K, nnz, static_cast<int*>(plan_forward)};
+    a.list[1] = ListArgs{col_start_ends_b, rows_b, K, N, nnz, static_cast<int*>(plan_input)};
+    a.grid[0] = (int)list_plan_grid(N, nnz);
+    a.grid[1] = (int)list_plan_grid(K, nnz);
+    const long long bound = unit_bound(out_features, nnz);
+    a.units = UnitArgs{row_start_ends_a, cols_a, nnz, N, K, nullptr, (int)bound, with_units ? static_cast<int*>(units) : nullptr};
+    const long long grid = a.grid[0] + a.grid[1] + (with_units ? (bound + 255) / 256 : 0);
+    hipLaunchKernelGGL(derive_kernel, dim3((unsigned)grid), dim3(256), 0, s, a);
+    if (int rc = (int)hipGetLastError()) return rc;
+    return units && !with_units ? build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, units, s) : PBS_OK;
 }
 
 static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,

@@ -91,15 +91,26 @@ __global__ __launch_bounds__(1024) void unit_prefix_kernel(const int32_t* __rest
     __shared__ int s_wave[16];
     unit_prefix<1024>(ptr, nnz, rows, before, s_wave);
 }
-// one unit per thread; global_before (unit_prefix_kernel) for patterns whose prefix does not fit LDS
-__global__ __launch_bounds__(256) void unit_table_kernel(const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx, int nnz, int rows,
-                                                         int cols, const int* global_before, int bound, int* table) {
+struct UnitArgs {
+    const int32_t *ptr, *idx;
+    int nnz, rows, cols;
+    const int* global_before;   // of unit_prefix_kernel, for patterns whose prefix does not fit LDS
+    int bound;
+    int* table;
+};
+// one unit per thread; workgroup `block` (256 threads)
+static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) {
+    const int32_t* __restrict__ ptr = a.ptr;
+    const int32_t* __restrict__ idx = a.idx;
+    const int nnz = a.nnz, rows = a.rows, cols = a.cols, bound = a.bound;
+    const int* global_before = a.global_before;
+    int* table = a.table;
     __shared__ int s_before[ROW_PARTS * UNIT_LDS_ROWS + 1];
     __shared__ int s_wave[4];
     if (!global_before) unit_prefix<256>(ptr, nnz, rows, s_before, s_wave);
     const int* before = global_before ? global_before : s_before;
     const int total = before[ROW_PARTS * rows] < bound ? before[ROW_PARTS * rows] : bound;   // (a corrupt pointer array may ask for more)
-    const int u = blockIdx.x * 256 + threadIdx.x;
+    const int u = block * 256 + threadIdx.x;
     if (u == 0) table[0] = total;
     if (u >= total) return;
     int lo = 0, hi = ROW_PARTS * rows - 1;   // the place that holds unit u
@@ -130,6 +141,22 @@ __global__ __launch_bounds__(256) void unit_table_kernel(const int32_t* __restri
         o[8 + b] = d;
         o[12 + b] = 0;
     }
+}
+__global__ __launch_bounds__(256) void unit_table_kernel(UnitArgs a) { unit_table(a, blockIdx.x); }
+
+// What a training step derives from a pattern, in one launch: the lists of both directions and the units.  A pattern that
+// changes every step derives them every step, and each is a launch that the step's products wait for (3, 3 and 5 us and
+// the host's time for each; together they take 6).
+struct DeriveArgs {
+    ListArgs list[2];
+    UnitArgs units;      // table == nullptr: none
+    int grid[2];         // workgroups of the lists; the rest make units
+};
+__global__ __launch_bounds__(256) void derive_kernel(DeriveArgs a) {
+    const int b = blockIdx.x;
+    if (b < a.grid[0]) list_plan(a.list[0], b, a.grid[0]);
+    else if (b < a.grid[0] + a.grid[1]) list_plan(a.list[1], b - a.grid[0], a.grid[1]);
+    else unit_table(a.units, b - a.grid[0] - a.grid[1]);
 }
 
 struct SddRowArgs {

@@ -41,11 +41,23 @@ static inline size_t list_plan_bytes(int n, int k) { return (size_t)(n / 32) * (
 
 constexpr int LIST_RANK_MAX_COLS = 8192;   // ranking compares every pair of columns: beyond this, natural order
 
-// One thread per entry copies it, one wave per column ranks it.
-__global__ __launch_bounds__(256) void list_plan_kernel(const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx, int nblk_n,
-                                                        int KB, int nnz, int* __restrict__ plan) {
+struct ListArgs {
+    const int32_t *ptr, *idx;
+    int nblk_n, KB, nnz;
+    int* plan;
+};
+static inline unsigned list_plan_grid(int nblk_n, int nnz) {
+    const long long work = (long long)nnz > 64ll * nblk_n ? nnz : 64ll * nblk_n;
+    return (unsigned)(work < 256 ? 1 : (work > 256ll * 1024 ? 1024 : (work + 255) / 256));
+}
+// One thread per entry copies it, one wave per column ranks it; workgroup `block` of `blocks` (256 threads).
+static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, int blocks) {
+    const int32_t* __restrict__ ptr = a.ptr;
+    const int32_t* __restrict__ idx = a.idx;
+    const int nblk_n = a.nblk_n, KB = a.KB, nnz = a.nnz;
+    int* __restrict__ plan = a.plan;
     int2* ent = reinterpret_cast<int2*>(plan + (size_t)nblk_n * 4);
-    const int gid = blockIdx.x * 256 + threadIdx.x, total = gridDim.x * 256;
+    const int gid = block * 256 + threadIdx.x, total = blocks * 256;
     for (int e = gid; e < nnz; e += total) {
         const int kb = idx[2 * (size_t)e], b = idx[2 * (size_t)e + 1];
         ent[e] = make_int2(kb < 0 ? 0 : (kb >= KB ? KB - 1 : kb), b < 0 ? 0 : (b >= nnz ? nnz - 1 : b));
@@ -68,6 +80,7 @@ __global__ __launch_bounds__(256) void list_plan_kernel(const int32_t* __restric
         if (lane == 0) *reinterpret_cast<int4*>(plan + 4 * (size_t)rank) = make_int4(c, lo, n, 0);
     }
 }
+__global__ __launch_bounds__(256) void list_plan_kernel(ListArgs a) { list_plan(a, blockIdx.x, gridDim.x); }
 
 struct StreamArgs {
     const void* a;      // [M, K] row-major

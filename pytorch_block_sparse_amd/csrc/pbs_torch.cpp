@@ -163,6 +163,29 @@ struct Pattern {
         }
         return t;
     }
+    // a training step's plans in one launch, if there is none yet
+    void derive_all(int64_t tokens, int code, void* stream) {
+        std::lock_guard<std::mutex> hold(lock);
+        if (parts[0] || parts[1] || units.t.defined() || !row_ptr.t.is_cuda() || !cols.t.is_cuda() || !col_ptr.t.is_cuda() ||
+            !rows.t.is_cuda() || capturing(stream))
+            return;
+        const auto bytes = row_ptr.t.options().dtype(at::kByte);
+        const size_t forward_bytes = pbs_blocksparse_matmul_plan_bytes(out_features, in_features),
+                     input_bytes = pbs_blocksparse_matmul_plan_bytes(in_features, out_features),
+                     units_bytes = pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, code);
+        const Tensor forward = at::empty({(int64_t)forward_bytes}, bytes), input = at::empty({(int64_t)input_bytes}, bytes);
+        const Tensor table = units_bytes ? at::empty({(int64_t)units_bytes}, bytes) : Tensor();
+        const int* no_blocks = nullptr;
+        check(pbs_blocksparse_derive(row_ptr.t.const_data_ptr<int>(), nnz ? cols.t.const_data_ptr<int>() : no_blocks,
+                                     col_ptr.t.const_data_ptr<int>(), nnz ? rows.t.const_data_ptr<int>() : no_blocks, out_features, in_features,
+                                     nnz, forward.mutable_data_ptr(), forward_bytes, input.mutable_data_ptr(), input_bytes,
+                                     units_bytes ? table.mutable_data_ptr() : nullptr, units_bytes, stream),
+              "pbs_blocksparse_derive");
+        plan[1].filled(forward, stream);
+        plan[0].filled(input, stream);
+        parts[0] = parts[1] = PBS_PLAN_LIST;
+        if (units_bytes) units.filled(table, stream);
+    }
     Tensor units_for(int64_t tokens, int code, void* stream) {
         const size_t bytes = pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, code);
         if (!bytes) return Tensor();
@@ -182,8 +205,8 @@ using PatternPtr = std::shared_ptr<Pattern>;
 
 const void* data_or_null(const Tensor& t) { return t.defined() && t.numel() ? t.const_data_ptr() : nullptr; }
 
-// a [..., k] -> [..., n]
-Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose) {
+// a [..., k] -> [..., n]; `training`: the products of a backward pass will follow
+Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose, bool training = false) {
     check_gpu(a_any);
     check_gpu(data);
     check_gpu(bias);
@@ -206,6 +229,7 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     sizes.back() = n;
     Tensor out = at::empty(sizes, a.options());
     if (tokens == 0) return out;
+    if (training) p.derive_all(tokens, code, stream);
     const int part = pbs_blocksparse_matmul_part(tokens, n, k, p.nnz, transpose, code, 1);
     const Tensor plan = p.plan_for(transpose, n, k, part, stream);
     // the transposed copy of the blocks that the bf16 column kernel's forward product works from
@@ -285,12 +309,13 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
 Tensor linear(const PatternPtr& p, const Tensor& x, const Tensor& data, const Tensor& bias) {
     for (const Tensor* t : {&x, &data, &bias})
         TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), "the block-sparse linear layer has no forward-mode derivative");
+    const bool training = torch::autograd::compute_requires_grad(x, data, bias);
     Tensor y;
     {
         at::NoGradGuard no_grad;
-        y = matmul(*p, x, data, bias, true);
+        y = matmul(*p, x, data, bias, true, training && x.requires_grad() && data.requires_grad());
     }
-    if (torch::autograd::compute_requires_grad(x, data, bias)) {
+    if (training) {
         auto node = std::shared_ptr<BlockSparseLinearBackward>(new BlockSparseLinearBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(x, data, bias));
         node->pattern = p;

@@ -36,6 +36,10 @@ _PROTOTYPES = {
     "pbs_blocksparse_matmul_plan_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "pbs_blocksparse_matmul_plan": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "pbs_blocksparse_matmul_plan_part": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
+    "pbs_blocksparse_derive": (
+        _i32,
+        [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp],
+    ),
     "pbs_blocksparse_matmul_part": (_i32, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp]),
     "pbs_blocksparse_matmul_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i32]),
