@@ -112,6 +112,7 @@ int pbs_validate_indices(const int32_t* cols_a, const int32_t* row_start_ends_a,
  *
  *   transpose = 1 (forward):        ptr = row_start_ends_a, indices = cols_a, n = out, k = in
  *   transpose = 0 (input gradient): ptr = col_start_ends_b, indices = rows_b, n = in,  k = out
+ *   (the coordinates increase within each list, as pbs_build_indices writes them)
  *   plan: 16-byte aligned device buffer of pbs_blocksparse_matmul_plan_bytes(n, k) bytes
  */
 size_t pbs_blocksparse_matmul_plan_bytes(int n, int k);
@@ -305,8 +306,8 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
  * the device.  The Python layer checks it after every product when PBS_DEBUG is set and raises.
  *
  * pbs_blocksparse_matmul_kernel_name / ..._back_kernel_name: which kernel(s) a call with these sizes runs
- * ("stream_kernel", "panel_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel", "sdd_bf16_kernel", with
- * " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
+ * ("stream_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel",
+ * "sdd_bf16_kernel", with " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
  */
 int pbs_protocol_failures(unsigned* count);

@@ -349,18 +349,33 @@ struct PanelChoice {
     int splits;   // 0: the kernel cannot run the problem
     double us;
     int turns;    // columns of a wave
+    int ways;     // 0: the whole contraction in LDS; else panel_chunk_kernel with so many waves per column
 };
 static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
-    PanelChoice best{0, 0.0, 0};
+    PanelChoice best{0, 0.0, 0, 0};
     const int cols = n / 32;
     // (below 1024 tokens, or with fewer columns than waves, it was the faster one nowhere)
-    if (k > PANEL_MAX_K || nnz < 1 || M < 1024 || cols < PANEL_NW) return best;
+    if (nnz < 1 || M < 1024 || cols < PANEL_NW) return best;
     const double tiles = (double)((M + 16 * PANEL_TT - 1) / (16 * PANEL_TT));
+    if (k > PANEL_MAX_K) {
+        if (nnz < 5 * cols) return best;   // (shorter columns pay for chunks they do not use: 4 to 13 % slower than the stream kernel at 3 to 4 blocks)
+        // the same in chunks, fitted to 90 problems (K 1056 to 4096, results 512 to 4096 wide, 509 to 16384 tokens, densities 0.08 to
+        // 0.75; within 9 % on average, its number of waves per column at most 9 % slower than the best): rounds x (start, chunks,
+        // blocks of a wave, which a full chip slows down), memory, and the tile once per workgroup that shares it
+        for (int ways = 4; ways >= 1; ways /= 2) {
+            const int s = (cols + PANEL_NW / ways - 1) / (PANEL_NW / ways);
+            const double wgs = tiles * s, full = wgs < 256 ? wgs / 256 : 1.0;
+            const double us = 1.68 + std::ceil(wgs / 256) * (1.17 + 0.814 * ((k + PANEL_KC - 1) / PANEL_KC) + (0.359 + 0.221 * full) * nnz / cols / ways) +
+                              1e-6 * 2.0 * (double)M * (0.0283 * (n + k) + 0.1363 / 8 * k * s);
+            if (best.splits == 0 || us < best.us) best = PanelChoice{s, us, 1, ways};
+        }
+        return best;
+    }
     for (int s = 1; s <= 16 && s <= cols; ++s) {
         const int mine = (cols + s - 1) / s, turns = (mine + PANEL_NW - 1) / PANEL_NW;
         const double us = 2.13 + std::ceil(tiles * s / 256) * (0.656 + 0.051 * (k / 32) + 0.33 * turns * nnz / cols + 0.133 * mine) +
                           0.09e-6 * 2.0 * (double)M * (n + k);
-        if (best.splits == 0 || us < best.us) best = PanelChoice{s, us, turns};
+        if (best.splits == 0 || us < best.us) best = PanelChoice{s, us, turns, 0};
     }
     return best;
 }
@@ -373,6 +388,18 @@ static int launch_panel(const DdsArgs& g, int splits, hipStream_t stream) {
     if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
     hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), panel_lds(g.K), stream, a);
+    return (int)hipGetLastError();
+}
+
+template <int TRANS, int S>
+static int launch_panel_chunks(const DdsArgs& g, int splits, hipStream_t stream) {
+    static std::atomic<uint64_t> done{0};
+    auto kernel = panel_chunk_kernel<TRANS, S>;
+    const PanelArgs a{g.a, g.data, g.plan, g.bias, g.out, g.M, g.N, g.K, splits};
+    const long long wgs = (long long)((g.M + 16 * PANEL_TT - 1) / (16 * PANEL_TT)) * splits;
+    if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), PANEL_CHUNK_LDS, stream, a);
     return (int)hipGetLastError();
 }
 
@@ -399,26 +426,30 @@ static double column_us(long long M, int n, int k, int nnz, bool copy) {
 // is given those in which it is 1.05 to 2.2 times the faster one, and the densest ones, where it is up to 13 % the slower one, are not.
 struct ProductChoice {
     int part;
-    int panel_splits;   // > 0: panel_kernel, which reads the list plan like stream_kernel
+    PanelChoice panel;   // splits > 0: panel_kernel or panel_chunk_kernel, which read the list plan like stream_kernel
 };
+constexpr PanelChoice NO_PANEL{0, 0.0, 0, 0};
 static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
-    if (esz == 4) return {PART_LIST, 0};
+    if (esz == 4) return {PART_LIST, NO_PANEL};
     const int wish = column_kernel_wish();
     const bool wide = wide_kernel_fits(M, n, k);
     const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz);
-    if (wish == 1 && column) return {PART_COLUMN, 0};
-    if (wish == 0 && wide) return {PART_WIDE, 0};
+    if (wish == 1 && column) return {PART_COLUMN, NO_PANEL};
+    if (wish == 0 && wide) return {PART_WIDE, NO_PANEL};
     const PanelChoice panel = choose_panel(M, n, k, nnz);
-    // (where the estimates are within 6 % of each other the panel kernel was up to 5 % the slower one as often as the faster:
-    // 70 drawn problems, of which it takes 20 and is 1.02 to 1.8 times faster in them)
-    const double tp = panel.splits ? 1.06 * panel.us : 1e300;
     const double tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
-    if (column && M >= 8192) return panel.splits && (1.0 + 0.03 * panel.turns) * panel.us < 4.0 + 0.88 * tc ? ProductChoice{PART_LIST, panel.splits} : ProductChoice{PART_COLUMN, 0};
+    if (column && M >= 8192) {
+        const bool panel_first = panel.splits && !panel.ways && (1.0 + 0.03 * panel.turns) * panel.us < 4.0 + 0.88 * tc;
+        return panel_first ? ProductChoice{PART_LIST, panel} : ProductChoice{PART_COLUMN, NO_PANEL};
+    }
+    // (where the estimates are within 6 % of each other panel_kernel was up to 5 % the slower one as often as the faster: 70 drawn
+    // problems, of which it takes 20 and is 1.02 to 1.8 times faster in them; panel_chunk_kernel's is up to 15 % short)
+    const double tp = panel.splits ? (panel.ways ? 1.1 : 1.06) * panel.us : 1e300;
     const double ts = choose_stream(esz, M, n, k, nnz).us;
     const double tw = wide ? wide_us(M, n, k, nnz) : 1e300;
-    if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel.splits};
-    if (tc < ts && tc < tw) return {PART_COLUMN, 0};
-    return {tw < ts ? PART_WIDE : PART_LIST, 0};
+    if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel};
+    if (tc < ts && tc < tw) return {PART_COLUMN, NO_PANEL};
+    return {tw < ts ? PART_WIDE : PART_LIST, NO_PANEL};
 }
 
 template <typename T, int TRANS>
@@ -436,7 +467,13 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
             return launch_ddsc<true>(g, workspace, stream);
         }
         if (part == PART_WIDE) return launch_dds16<TRANS>(g, stream);
-        if (choice.panel_splits) return launch_panel<TRANS>(g, choice.panel_splits, stream);
+        switch (choice.panel.splits ? choice.panel.ways : -1) {
+            case 0: return launch_panel<TRANS>(g, choice.panel.splits, stream);
+            case 1: return launch_panel_chunks<TRANS, 1>(g, choice.panel.splits, stream);
+            case 2: return launch_panel_chunks<TRANS, 2>(g, choice.panel.splits, stream);
+            case 4: return launch_panel_chunks<TRANS, 4>(g, choice.panel.splits, stream);
+            default: break;
+        }
     }
     return launch_stream<T, TRANS>(g, stream);
 }
@@ -1056,7 +1093,7 @@ const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int
                                                int with_workspace) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || (n % 32) || (k % 32)) return "";
     const ProductChoice c = choose_product(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
-    return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (c.panel_splits ? "panel_kernel" : "stream_kernel"));
+    return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (!c.panel.splits ? "stream_kernel" : (c.panel.ways ? "panel_chunk_kernel" : "panel_kernel")));
 }
 
 const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {

@@ -203,4 +203,157 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_kernel(PanelArgs g) {
     }
 }
 
+// The same for contractions that do not fit: the tile passes through LDS in chunks of 512 features, two buffers, the next chunk on its way
+// while this one is multiplied, one barrier per chunk.  A column belongs to S waves (every S-th of its blocks each), whose sums meet
+// in LDS at the end; one column per wave, so the accumulators stay where they are from chunk to chunk.  S = 4, 2, 1 make 4, 8, 16 columns per
+// workgroup: few tokens need many workgroups, many tokens fewer that share a tile.  The lists are sorted by k-block (as the kernels
+// with merged lists need them too).
+//
+// What bounds it: a chunk's copy, 64 KB at the texture path's rate (1.5 k cycles) and its latency behind the barrier (0.8 us per chunk in all).
+// Measured, us, against the stream kernel: 3072 -> 768 density 0.5, 2317 tokens 21.8 -> 16.5, 4096 tokens 27.8 -> 22.7; 4096 -> 4096
+// density 0.25, 1024 tokens 30.3 -> 24.1; 4096 -> 1024 density 0.75, 4096 tokens 69.8 -> 36.7; 1536 -> 2976 density 0.4, 2317 tokens
+// 31.8 -> 20.1.  Below 1024 tokens it is the slower one (3072 -> 768, 509 tokens 7.6 against 12.2).
+constexpr int PANEL_KC = 512;         // features of a chunk: 64 rows of 1 KB
+constexpr int PANEL_CHUNK_LDS = 2 * 16 * PANEL_TT * 1024 + PANEL_NW * 2048;
+template <int TRANS, int S>
+__global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_chunk_kernel(PanelArgs g) {
+    using E = Elem<bf16_t>;
+    constexpr int TT = PANEL_TT, BM = 16 * TT, NW = PANEL_NW, BUF = BM * 1024, KBC = PANEL_KC / 32;
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    const int ncols = g.N >> 5;
+    const int tiles = (g.M + BM - 1) / BM;
+    const int id = xcd_tile_id(blockIdx.x, tiles * g.splits);
+    if (id < 0) return;
+    const int tile = id / g.splits, split = id - tile * g.splits;
+    const int m0 = tile * BM;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int s = wave % S;
+    const int rank = split + g.splits * (wave / S);
+
+    const unsigned char* A = static_cast<const unsigned char*>(g.a) + (size_t)m0 * g.K * 2;
+    const unsigned char* D = static_cast<const unsigned char*>(g.data);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem);
+    unsigned char* const place = smem + 2 * BUF + wave * 2048;   // this wave's block
+    const unsigned lds_place = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)place);
+
+    const int rows = g.M - m0 < BM ? g.M - m0 : BM, last_chunk = g.K / 8 - 1;
+    const int nchunks = (g.K + PANEL_KC - 1) / PANEL_KC;
+    // place p of row t of a chunk holds 16-byte piece p ^ (t % 16)
+    auto stage = [&](int ci) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < BM / NW; ++k) {
+            const int t = wave + k * NW;
+            int c = ci * (PANEL_KC / 8) + (lane ^ (t & 15));
+            c = c < last_chunk ? c : last_chunk;
+            dma16(lds0 + (ci & 1) * BUF + t * 1024, A, (unsigned)((t < rows ? t : rows - 1) * (g.K * 2) + c * 16));
+        }
+    };
+    stage(0);
+
+    int4 head = make_int4(0, 0, 0, 0);
+    if (rank < ncols) head = reinterpret_cast<const int4*>(g.plan)[rank];
+    const int n = __builtin_amdgcn_readfirstlane(head.z);
+    const int col = __builtin_amdgcn_readfirstlane(head.x) * 32;
+    const int2* ent = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4) + __builtin_amdgcn_readfirstlane(head.y) + s;
+    const int mine = n > s ? (n - s + S - 1) / S : 0;
+    auto load64 = [&](int i) { return ent[(size_t)(i + lane < mine ? i + lane : mine - 1) * S]; };
+    int2 ev = make_int2(0, 0);
+    if (mine > 0) ev = load64(0);
+    float bv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bv[i] = g.bias ? E::to_f32(static_cast<const bf16_t*>(g.bias)[col + 8 * q + i]) : 0.f;
+
+    auto w_row_swz = [](int row) { return (row >> 3) & 3; };
+    unsigned w_voff[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int row = i * 16 + lane / 4;
+        w_voff[i] = TRANS ? row * 64 + ((lane & 3) ^ w_row_swz(row)) * 16 : i * 1024 + lane * 16;
+    }
+    int kb = 1 << 30;   // k-block of the block asked for; none: past every chunk
+    auto ask = [&](int i) __attribute__((always_inline)) {
+        kb = 1 << 30;
+        if (i >= mine) return;
+        if (i > 0 && (i & 63) == 0) ev = load64(i);
+        kb = __builtin_amdgcn_readlane(ev.x, i & 63);
+        const unsigned char* pw = uniform_ptr(D + (size_t)__builtin_amdgcn_readlane(ev.y, i & 63) * 2048);
+        dma16(lds_place, pw, w_voff[0]);
+        dma16(lds_place + 1024, pw, w_voff[1]);
+    };
+    int i = 0;
+    ask(0);
+
+    f32x4 acc[TT][2];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[t][0] = acc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ci = 0; ci < nchunks; ++ci) {
+        drain_barrier();   // chunk ci and this wave's block are there, and every wave has left the other buffer
+        if (ci + 1 < nchunks) stage(ci + 1);
+        const unsigned char* a_row = smem + (ci & 1) * BUF + r * 1024;
+        for (bool first = true; kb < (ci + 1) * KBC; first = false) {
+            if (!first) wait_dma(0);
+            uint4 fa[TT], fw[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if constexpr (TRANS) {
+                    const int row = 8 * (r >> 2) + 4 * j + (r & 3);
+                    fw[j] = *reinterpret_cast<const uint4*>(place + row * 64 + (q ^ w_row_swz(row)) * 16);
+                } else {
+                    const unsigned char* p = place + (8 * q + (r >> 2)) * 64 + (r & 3) * 16 + 8 * j;
+                    const uint2 lo = tr16_b64(p), hi = tr16_b64(p + 256);
+                    fw[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                }
+            }
+            const unsigned char* as = a_row + ((((kb - ci * KBC) * 4 + q) ^ r) * 16);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) fa[t] = *reinterpret_cast<const uint4*>(as + 16 * t * 1024);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            ask(++i);
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fw[j]), __builtin_bit_cast(bf16x8, fa[t]), acc[t][j], 0, 0, 0);
+        }
+    }
+
+    auto store = [&](int t, const f32x4& v0, const f32x4& v1) __attribute__((always_inline)) {
+        const int row = m0 + 16 * t + r;
+        if (row >= g.M || rank >= ncols) return;
+        uint32_t w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const f32x4& v = e < 2 ? v0 : v1;
+            w[e] = (uint32_t)E::from_f32(v[2 * (e & 1)] + bv[2 * e]).bits | ((uint32_t)E::from_f32(v[2 * (e & 1) + 1] + bv[2 * e + 1]).bits << 16);
+        }
+        *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.out) + (size_t)row * g.N + col + 8 * q) = make_uint4(w[0], w[1], w[2], w[3]);
+    };
+    if constexpr (S == 1) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) store(t, acc[t][0], acc[t][1]);
+    } else {
+        f32x4* red = reinterpret_cast<f32x4*>(smem);   // [wave][t][j][lane]: the two buffers
+        static_assert(NW * TT * 2 * 1024 <= 2 * BUF, "the sums fit the buffers");
+        drain_barrier();
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) red[((wave * TT + t) * 2 + j) * 64 + lane] = acc[t][j];
+        lds_barrier();
+        for (int t = s; t < TT; t += S) {
+            f32x4 v[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                v[j] = red[(((wave - s) * TT + t) * 2 + j) * 64 + lane];
+#pragma unroll
+                for (int w = 1; w < S; ++w) v[j] += red[(((wave - s + w) * TT + t) * 2 + j) * 64 + lane];
+            }
+            store(t, v[0], v[1]);
+        }
+    }
+}
+
 }  // namespace pbs
