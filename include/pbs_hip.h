@@ -206,7 +206,8 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
  * When the blocks alone cannot fill the GPU the token range is split over workgroups and the fp32
  * partial blocks are summed in a fixed order by a second kernel; they and the unit table (below) lie
  * in `workspace`: pbs_blocksparse_matmul_back_workspace_bytes() bytes of 16-byte aligned device memory
- * (may be NULL when that returns 0).
+ * (may be NULL when that returns 0).  In fp32 the partial blocks take at most 64 MiB, whatever the problem's size: ranges of
+ * the tokens whose slices do not fit are added by further launches.
  */
 size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_features, int in_features,
                                                    int nnz, int dtype);
@@ -277,7 +278,7 @@ int pbs_blocksparse_matmul_back_blocks(const void* dense_a, int a_row_major, con
  * allocating routine.
  *
  *   - A problem of the row kernel whose pbs_blocksparse_matmul_back_workspace_bytes() exceeds the array runs with fewer slices
- *     of the tokens; one of the rectangle kernel is rejected with PBS_ERR_SCRATCH before anything is launched (4096 x 4096 at density 0.25 with 16384
+ *     of the tokens and more launches (the last bits of its sums may differ); one of the rectangle kernel is rejected with PBS_ERR_SCRATCH before anything is launched (4096 x 4096 at density 0.25 with 16384
  *     tokens in bf16 needs exactly 64 MiB and fits).
  *   - Nothing in the array has to be cleared between calls: every word the reduction kernel reads
  *     is written by the product kernel of the same call first.

@@ -512,7 +512,7 @@ static SddPlan plan_sdd(long long M, int N, int K) {
 // the choices made by it were 3.5 % slower than the best of all slice counts on average): launch, reduction of the slices,
 // chunks x blocks of a wave of the slowest workgroup, at the rate of a full chip or, below 32 workgroups per XCD, of
 // a wave alone, and what each round of workgroups on the chip costs besides.
-static double row_us(int dtype, long long M, int N, int nnz, int slices) {
+static double row_us(int dtype, long long M, int N, int nnz, int slices, int passes) {
     struct Model {
         double launch, reduce, per_slice, busy, alone, round;
         int resident;   // workgroups per XCD
@@ -521,10 +521,10 @@ static double row_us(int dtype, long long M, int N, int nnz, int slices) {
     const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
     const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows;
     const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
-    const double tasks = std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices)) * blocks;
+    const double tasks = std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices * (double)passes)) * blocks;
     const double busy = std::ceil(tasks / 32) * wave * m.busy, alone = wave * m.alone;
-    return m.launch + (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) + (busy > alone ? busy : alone) +
-           std::ceil(tasks / m.resident) * m.round;
+    return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) +
+           passes * (m.launch + (busy > alone ? busy : alone) + std::ceil(tasks / m.resident) * m.round);
 }
 static double rectangle_us(long long M, int N, int K, int nnz) {
     const SddPlan p = plan_sdd(M, N, K);
@@ -533,43 +533,59 @@ static double rectangle_us(long long M, int N, int K, int nnz) {
     return 15.1 + rounds * (p.tokens_per_split / SddShapeBf16::TC) * (0.4903 * passes + 0.1019 * blocks / 8) +
            (p.nsplit > 1 ? 3.65 + 1.45 * p.nsplit * nnz / 1000.0 : 0.0);
 }
-// The kernel and, for the row kernel, the number of token slices (0: rectangles).
-static int choose_row_slices(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
+// The kernel and, for the row kernel, the number of token slices of a launch (0: rectangles) and of launches, one behind the
+// other over consecutive ranges of the tokens.
+//
+// fp32 wants slices of about 64 MB of the operands: workgroups of different rows read the same columns of X and find them in the
+// last-level cache while a slice is about that size (4096 -> 4096 density 0.25, 16384 tokens: 1398 us in one slice, 1333 in four,
+// 1233 in eight).  But every slice of a launch is a copy of the gradient in the workspace, so a launch has at most as many as
+// fit ROW_WORKSPACE_BYTES, and further launches add to the sums that are there.  Slices x launches, us, against eight slices and more
+// in one launch (whose workspace is 128 MB for the first and grows with tokens and features): 4096 -> 4096, 16384 tokens, density 0.25
+// 4 x 2 1199 against 1222, 0.5 2 x 4 2258 against 2347, 1 1 x 8 4131 against 4297; 65536 tokens, density 1 1 x 33 16538 against
+// 16998; 8192 -> 8192, 16384 tokens, density 0.25 1 x 16 4805 against 5211, 0.5 9264 against 10299.
+constexpr size_t ROW_WORKSPACE_BYTES = 64u << 20;
+struct RowChoice {
+    int slices, passes;
+};
+static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
     constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
     const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
-    // Workgroups of different rows read the same columns of X: they find them in the caches while the operands (fp32: a slice
-    // of them) are about the size of the L2s.  bf16 beyond that size: 250 us where the rectangles, which read
-    // every panel once per 16 rows, take 216.
-    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return 0;
+    // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 216.
+    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return {0, 1};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
-    int best = 1;
+    RowChoice best{1, 1};
     double best_us = 0.0;
     for (const int s : CANDIDATES) {
-        if (s > 1 && (s > chunks / 4 || ((double)nnz * 1024 + N) * sizeof(float) * s > (double)workspace_limit)) break;
-        const double us = row_us(dtype, M, N, nnz, s);
-        if (s == 1 || best < at_least || us < best_us) {
-            best = s;
+        if (s > 1 && (s > chunks / 4 || (size_t)nnz * 4096 * s > workspace_limit)) break;
+        const int passes = at_least > s ? (int)std::ceil(at_least / s) : 1;
+        const double us = row_us(dtype, M, N, nnz, s, passes);
+        if (s == 1 || us < best_us) {
+            best = {s, passes};
             best_us = us;
         }
     }
-    return dtype == PBS_DTYPE_BF16 && rectangle_us(M, N, K, nnz) < best_us ? 0 : best;
+    if (dtype == PBS_DTYPE_BF16 && rectangle_us(M, N, K, nnz) < best_us) best.slices = 0;
+    return best;
 }
 struct BackPlan {
     int slices;   // row kernel; 0: rectangles
-    int chunks_per_slice;
+    int passes, chunks_per_slice;
     SddPlan rect;
     size_t partial_bytes;
 };
-static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ~(size_t)0) {
+static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
     BackPlan p;
-    p.slices = choose_row_slices(dtype, M, N, K, nnz, workspace_limit);
+    const RowChoice row = choose_row(dtype, M, N, K, nnz, workspace_limit);
+    p.slices = row.slices;
     p.rect = plan_sdd(M, N, K);
     int n = p.rect.nsplit;
     if (p.slices > 0) {
-        const long long chunks = (M + ROW_TC - 1) / ROW_TC;
-        p.chunks_per_slice = (int)((chunks + p.slices - 1) / p.slices);
-        p.slices = n = (int)((chunks + p.chunks_per_slice - 1) / p.chunks_per_slice);
+        const long long chunks = (M + ROW_TC - 1) / ROW_TC, shares = (long long)row.slices * row.passes;
+        p.chunks_per_slice = (int)((chunks + shares - 1) / shares);
+        const long long filled = (chunks + p.chunks_per_slice - 1) / p.chunks_per_slice;   // slices with tokens
+        p.slices = n = (int)(filled < row.slices ? filled : row.slices);
+        p.passes = (int)((filled + n - 1) / n);   // (the last launch may have slices without tokens, which add nothing)
     }
     p.partial_bytes = n > 1 ? ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * n : 0;   // fp32 sums of each slice: blocks, bias columns
     return p;
@@ -629,8 +645,12 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     r.nnz = a.nnz;
     r.slices = p.slices;
     r.chunks_per_slice = p.chunks_per_slice;
-    hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
-    if (int rc = (int)hipGetLastError()) return rc;
+    for (int pass = 0; pass < p.passes; ++pass) {
+        r.chunk0 = pass * p.slices * p.chunks_per_slice;
+        r.add = pass > 0;
+        hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
+        if (int rc = (int)hipGetLastError()) return rc;
+    }
     return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;
 }
 
@@ -930,7 +950,7 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
 }
 
 static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,
-                size_t workspace_limit = ~(size_t)0) {
+                size_t workspace_limit = ROW_WORKSPACE_BYTES) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return PBS_ERR_BAD_DTYPE;
     if (tokens < 0 || a.N <= 0 || a.K <= 0 || a.nnz < 0 || (a.N % 32) || (a.K % 32)) return PBS_ERR_BAD_SHAPE;

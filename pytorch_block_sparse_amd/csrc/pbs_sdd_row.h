@@ -1,7 +1,8 @@
 // dense^T x dense -> block-sparse (weight gradient on the sparse support), and with it the bias gradient:
 //   out[32b + j][i] = sum_t G[t][32r + i] * X[t][32c + j]   for every data block b at (r, c),   bias[n] = sum_t G[t][n].
 //
-// A workgroup takes a unit, up to four blocks of one block row of W, over one slice of the tokens; each of its four waves
+// A workgroup takes a unit, up to four blocks of one block row of W, over one slice of the tokens (in fp32, where the slices do not
+// fit the workspace, of a launch's range of them: a later launch adds to what it finds); each of its four waves
 // every fourth chunk of 32 tokens, with all accumulators of the unit (64 registers), so that nothing is shared until the
 // waves' sums meet in LDS at the end: no barrier and no wait for another wave in the loop, any shape of pattern makes
 // units of one size, and small problems have many workgroups.  A G fragment is read once for four products.
@@ -168,6 +169,8 @@ struct SddRowArgs {
     float* partial;
     int M, N, K, nnz;
     int slices, chunks_per_slice;   // every unit in this many slices of the tokens
+    int chunk0;              // the pass starts here
+    bool add;                // fp32: a pass behind the first adds to the sums that are there
 };
 // What a lane holds of a piece, and the products of two pieces (4 x STEPS matrix instructions).  A lane's accumulators of a block
 // are d[a][b][v], column i = COL(q, a, v) of row j = FEAT(r, b): eight consecutive columns per row.
@@ -449,6 +452,12 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
             const size_t o = (size_t)at * 1024 + F::feature(r, jj) * 32 + 8 * q;
             if (partial || ESZ == 4) {
                 float* p = (partial ? partial : static_cast<float*>(a.out)) + o;
+                if (ESZ == 4 && a.add) {
+                    const float4 lo = reinterpret_cast<const float4*>(p)[0], hi = reinterpret_cast<const float4*>(p)[1];
+                    const float w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] += w[e];
+                }
                 reinterpret_cast<float4*>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
                 reinterpret_cast<float4*>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
             } else {
@@ -472,8 +481,14 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
             float v = s[lane];
 #pragma unroll
             for (int w = 1; w < ROW_NW; ++w) v += s[w * 32 + lane];
-            if (partial) partial[(size_t)a.nnz * 1024 + row * 32 + lane] = v;
-            else static_cast<T*>(a.bias_out)[row * 32 + lane] = E::from_f32(v);
+            if constexpr (ESZ == 4) {
+                float* p = (partial ? partial + (size_t)a.nnz * 1024 : static_cast<float*>(a.bias_out)) + row * 32 + lane;
+                *p = a.add ? *p + v : v;
+            } else if (partial) {
+                partial[(size_t)a.nnz * 1024 + row * 32 + lane] = v;
+            } else {
+                static_cast<T*>(a.bias_out)[row * 32 + lane] = E::from_f32(v);
+            }
         }
     }
 }
@@ -491,7 +506,7 @@ __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel
     const int slice = local / n_u;
     const int* unit = a.table + 16 + (size_t)(u_lo + local - slice * n_u) * UNIT_INTS;
     const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
-    const int c_lo = slice * a.chunks_per_slice;
+    const int c_lo = a.chunk0 + slice * a.chunks_per_slice;
     const int c_hi = c_lo + a.chunks_per_slice < chunks ? c_lo + a.chunks_per_slice : chunks;
     float* partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + (a.bias_out ? a.N : 0)) : nullptr;
     switch (unit[1]) {
