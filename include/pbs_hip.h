@@ -112,7 +112,8 @@ int pbs_validate_indices(const int32_t* cols_a, const int32_t* row_start_ends_a,
  *
  *   transpose = 1 (forward):        ptr = row_start_ends_a, indices = cols_a, n = out, k = in
  *   transpose = 0 (input gradient): ptr = col_start_ends_b, indices = rows_b, n = in,  k = out
- *   (the coordinates increase within each list, as pbs_build_indices writes them)
+ *   (the coordinates increase within each list, as pbs_build_indices writes them; an entry whose coordinate or data
+ *   block is outside its range is left out, and of several with one coordinate one is taken)
  *   plan: 16-byte aligned device buffer of pbs_blocksparse_matmul_plan_bytes(n, k) bytes
  */
 size_t pbs_blocksparse_matmul_plan_bytes(int n, int k);

@@ -807,7 +807,7 @@ int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices,
     unsigned char* base = static_cast<unsigned char*>(plan);
     if (part & PART_LIST) {
         const ListArgs a{ptr, indices, n / 32, k / 32, nnz, reinterpret_cast<int*>(base)};
-        hipLaunchKernelGGL(list_plan_kernel, dim3(list_plan_grid(n / 32, nnz)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(list_plan_kernel, dim3(list_plan_grid(n / 32)), dim3(256), 0, s, a);
         if (int rc = (int)hipGetLastError()) return rc;
     }
     if ((part & PART_WIDE) && wide_plan_bytes(n, k)) {
@@ -939,8 +939,8 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
     DeriveArgs a;
     a.list[0] = ListArgs{row_start_ends_a, cols_a, N, K, nnz, static_cast<int*>(plan_forward)};
     a.list[1] = ListArgs{col_start_ends_b, rows_b, K, N, nnz, static_cast<int*>(plan_input)};
-    a.grid[0] = (int)list_plan_grid(N, nnz);
-    a.grid[1] = (int)list_plan_grid(K, nnz);
+    a.grid[0] = (int)list_plan_grid(N);
+    a.grid[1] = (int)list_plan_grid(K);
     const long long bound = unit_bound(out_features, nnz);
     a.units = UnitArgs{row_start_ends_a, cols_a, nnz, N, K, nullptr, (int)bound, with_units ? static_cast<int*>(units) : nullptr};
     const long long grid = a.grid[0] + a.grid[1] + (with_units ? (bound + 255) / 256 : 0);

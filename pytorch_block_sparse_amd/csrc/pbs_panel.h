@@ -206,8 +206,7 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_kernel(PanelArgs g) {
 // The same for contractions that do not fit: the tile passes through LDS in chunks of 512 features, two buffers, the next chunk on its way
 // while this one is multiplied, one barrier per chunk.  A column belongs to S waves (every S-th of its blocks each), whose sums meet
 // in LDS at the end; one column per wave, so the accumulators stay where they are from chunk to chunk.  S = 4, 2, 1 make 4, 8, 16 columns per
-// workgroup: few tokens need many workgroups, many tokens fewer that share a tile.  The lists are sorted by k-block (as the kernels
-// with merged lists need them too).
+// workgroup: few tokens need many workgroups, many tokens fewer that share a tile.  The lists are by k-block (list_plan).
 //
 // What bounds it: a chunk's copy, 64 KB at the texture path's rate (1.5 k cycles) and its latency behind the barrier (0.8 us per chunk in all).
 // Measured, us, against the stream kernel: 3072 -> 768 density 0.5, 2317 tokens 21.8 -> 16.5, 4096 tokens 27.8 -> 22.7; 4096 -> 4096
@@ -306,7 +305,8 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_chunk_kernel(PanelArgs
                     fw[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
                 }
             }
-            const unsigned char* as = a_row + ((((kb - ci * KBC) * 4 + q) ^ r) * 16);
+            const int at = kb > ci * KBC ? kb - ci * KBC : 0;   // (inside the chunk whatever the list holds)
+            const unsigned char* as = a_row + (((at * 4 + q) ^ r) * 16);
 #pragma unroll
             for (int t = 0; t < TT; ++t) fa[t] = *reinterpret_cast<const uint4*>(as + 16 * t * 1024);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -135,7 +135,7 @@ static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) 
         if (b < e1 - e0) {
             c = idx[2 * (size_t)(first + e0 + b)];
             d = idx[2 * (size_t)(first + e0 + b) + 1];
-            c = c < 0 ? 0 : (c >= cols ? cols - 1 : c);
+            if (c < 0 || c >= cols) c = 0, d = -1;   // (an entry outside the range gets no result)
             d = d < 0 || d >= nnz ? -1 : d;
         }
         o[4 + b] = c;

@@ -28,8 +28,8 @@
 // eight consecutive columns of a token and stores them with 16-byte stores, 128 (64) contiguous bytes per token.
 //
 // Work list ("list plan", list_plan_kernel), per pattern and direction: per block column, in order of falling block
-// count, {column, first entry, entries, 0}, then the entries {k-block, data block} with every value inside its range.
-// Long columns are so started first.
+// count, {column, first entry, entries, 0}, then the entries {k-block, data block}, by k-block, with every value inside its
+// range.  Long columns are so started first.
 #pragma once
 #include "pbs_common.h"
 
@@ -46,24 +46,21 @@ struct ListArgs {
     int nblk_n, KB, nnz;
     int* plan;
 };
-static inline unsigned list_plan_grid(int nblk_n, int nnz) {
-    const long long work = (long long)nnz > 64ll * nblk_n ? nnz : 64ll * nblk_n;
-    return (unsigned)(work < 256 ? 1 : (work > 256ll * 1024 ? 1024 : (work + 255) / 256));
-}
-// One thread per entry copies it, one wave per column ranks it; workgroup `block` of `blocks` (256 threads).
+static inline unsigned list_plan_grid(int nblk_n) { return (unsigned)(nblk_n > 4 * 1024 ? 1024 : (nblk_n + 3) / 4); }
+// One wave per column copies its entries and ranks it; workgroup `block` of `blocks` (256 threads).  Entries as the host layer keeps
+// them (by k-block, every value in its range) are copied as they are; of any other list the entries outside the range and all but the first
+// entry of a k-block are dropped and the rest is sorted, like in the plans of pbs_dds16.h and pbs_ddsc.h: panel_chunk_kernel goes
+// through a column by k-block, and panel_kernel has room for one entry per k-block.
 static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, int blocks) {
     const int32_t* __restrict__ ptr = a.ptr;
     const int32_t* __restrict__ idx = a.idx;
     const int nblk_n = a.nblk_n, KB = a.KB, nnz = a.nnz;
     int* __restrict__ plan = a.plan;
     int2* ent = reinterpret_cast<int2*>(plan + (size_t)nblk_n * 4);
-    const int gid = block * 256 + threadIdx.x, total = blocks * 256;
-    for (int e = gid; e < nnz; e += total) {
-        const int kb = idx[2 * (size_t)e], b = idx[2 * (size_t)e + 1];
-        ent[e] = make_int2(kb < 0 ? 0 : (kb >= KB ? KB - 1 : kb), b < 0 ? 0 : (b >= nnz ? nnz - 1 : b));
-    }
+    auto entry = [&](int i) { return make_int2(idx[2 * (size_t)i], idx[2 * (size_t)i + 1]); };
+    auto good = [&](int2 e) { return e.x >= 0 && e.x < KB && e.y >= 0 && e.y < nnz; };
     const int lane = threadIdx.x & 63;
-    for (int c = gid >> 6; c < nblk_n; c += total >> 6) {
+    for (int c = block * 4 + (threadIdx.x >> 6); c < nblk_n; c += blocks * 4) {
         const int lo = clamp_entry(ptr[c], nnz), hi = clamp_entry(ptr[c + 1], nnz);
         const int n = hi > lo ? hi - lo : 0;
         int rank = c;
@@ -77,7 +74,35 @@ static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, i
 #pragma unroll
             for (int d = 32; d; d >>= 1) rank += __shfl_xor(rank, d, 64);
         }
-        if (lane == 0) *reinterpret_cast<int4*>(plan + 4 * (size_t)rank) = make_int4(c, lo, n, 0);
+        bool as_it_is = true;
+#pragma unroll 4
+        for (int i = lane; i < n; i += 64) {
+            const int2 e = entry(lo + i);
+            if (!good(e) || (i > 0 && entry(lo + i - 1).x >= e.x)) as_it_is = false;
+            ent[lo + i] = make_int2(e.x < 0 ? 0 : (e.x >= KB ? KB - 1 : e.x), e.y < 0 ? 0 : (e.y >= nnz ? nnz - 1 : e.y));
+        }
+        int kept = n;
+        if (__any(!as_it_is)) {   // the smallest k-block that is left, and of its entries the first, n times over
+            int last = -1;
+            for (kept = 0; kept < n; ++kept) {
+                long long least = 1ll << 62;
+                for (int i = lane; i < n; i += 64) {
+                    const int2 e = entry(lo + i);
+                    const long long key = (long long)e.x << 32 | i;
+                    if (good(e) && e.x > last && key < least) least = key;
+                }
+#pragma unroll
+                for (int d = 32; d; d >>= 1) {
+                    const long long o = __shfl_xor(least, d, 64);
+                    least = o < least ? o : least;
+                }
+                if (least == 1ll << 62) break;
+                last = (int)(least >> 32);
+                // (by the lane that has written this place above)
+                if (lane == (kept & 63)) ent[lo + kept] = make_int2(last, entry(lo + (int)(least & 0xffffffffll)).y);
+            }
+        }
+        if (lane == 0) *reinterpret_cast<int4*>(plan + 4 * (size_t)rank) = make_int4(c, lo, kept, 0);
     }
 }
 __global__ __launch_bounds__(256) void list_plan_kernel(ListArgs a) { list_plan(a, blockIdx.x, gridDim.x); }
