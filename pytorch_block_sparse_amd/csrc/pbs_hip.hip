@@ -654,6 +654,7 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;
 }
 
+template <bool BIAS>
 static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     const SddPlan& p = plan.rect;
     SddArgs a;
@@ -682,7 +683,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     using C = SddBf16Cfg<S::QW, S::TC, S::NS, S::NW>;
     static_assert(C::TC == S::TC && C::SR == S::SR && C::SC == S::SC, "plan and kernel must agree");
     static std::atomic<uint64_t> done{0};
-    auto kernel = sdd_bf16_kernel<S::QW, S::TC, S::NS, S::NW>;
+    auto kernel = sdd_bf16_kernel<BIAS, S::QW, S::TC, S::NS, S::NW>;
     if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
     hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
     if (int rc = (int)hipGetLastError()) return rc;
@@ -971,7 +972,7 @@ static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, s
         return a.bias_out ? zero(a.bias_out, a.N) : PBS_OK;
     }
     const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, a.bias_out != nullptr, workspace_limit);
-    if (p.slices == 0) return launch_rectangles(a, p, workspace, workspace_bytes, s);
+    if (p.slices == 0) return a.bias_out ? launch_rectangles<true>(a, p, workspace, workspace_bytes, s) : launch_rectangles<false>(a, p, workspace, workspace_bytes, s);
     return dtype == PBS_DTYPE_F32 ? launch_row<float>(a, p, workspace, workspace_bytes, s) : launch_row<bf16_t>(a, p, workspace, workspace_bytes, s);
 }
 
