@@ -43,6 +43,9 @@ class BlockSparseLinearFunction(torch.autograd.Function):
         return grad_input, grad_weight, None, grad_bias
 
 
+_APPLY = BlockSparseLinearFunction.apply
+
+
 class BlockSparseLinear(nn.Module):
     """reference: block_sparse_linear.py:157-233."""
 
@@ -111,8 +114,10 @@ class BlockSparseLinear(nn.Module):
 
     def forward(self, x):
         weight = self.weight
-        # (torch.jit.trace can record the autograd function, but not see into the native call)
-        if isinstance(weight, BlockSparseMatrix) and not torch.jit.is_tracing():
+        # The native call does what the autograd function does with a BlockSparseMatrix.  The function itself where there may be more
+        # to do: a subclass of the matrix may have products of its own, `fn` may have been replaced, and torch.jit.trace can
+        # record the function but not see into the native call.
+        if type(weight) is BlockSparseMatrix and self.fn == _APPLY and not torch.jit.is_tracing():
             return native.torch_path().linear(x, weight.data, self.bias, weight._buffers, weight.schedule())
         return self.fn(x, self.weight.get_differentiable_data(), self.weight, self.bias)
 
