@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <memory>
 #include <mutex>
+#include <unordered_map>
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -22,6 +23,8 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
+#include <torch/library.h>
 
 #include "../../include/pbs_hip.h"
 
@@ -137,7 +140,9 @@ struct Pattern {
     Derived plan[2];     // [transpose]
     int parts[2] = {0, 0};
     Derived units;       // of the weight gradient
+    int64_t number = 0;  // that graphs of torch know it by (pattern_number)
 
+    ~Pattern();
     bool still(const Tensor& rp, const Tensor& c, const Tensor& cp, const Tensor& r) const {
         return row_ptr.still(rp) && cols.still(c) && col_ptr.still(cp) && rows.still(r);
     }
@@ -271,7 +276,77 @@ void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Ten
           "pbs_blocksparse_matmul_back_bias");
 }
 
-// y = x W^T + bias.  Backward: dx = dy W, dW on the pattern's blocks, dbias = sum of dy over the tokens.
+// The gradients of x (dx = dy W), of the blocks and of the bias (the sum of dy over the tokens) that are wanted, others undefined.
+std::array<Tensor, 3> linear_backward(Pattern& p, const Tensor& dy_any, const Tensor& x, const Tensor& data, std::array<bool, 3> wanted) {
+    at::NoGradGuard no_grad;
+    std::array<Tensor, 3> out;
+    const Tensor dy = dy_any.is_contiguous() ? dy_any : dy_any.contiguous();
+    if (wanted[0]) out[0] = matmul(p, dy, data, Tensor(), false);
+    if (wanted[1]) {
+        out[1] = at::empty({(int64_t)p.nnz * 32, 32}, x.options());
+        if (wanted[2]) out[2] = at::empty({p.out_features}, x.options());
+        matmul_back(p, dy, x, out[1], out[2]);
+    } else if (wanted[2]) {
+        out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
+    }
+    return out;
+}
+
+// Patterns that graphs of torch refer to, by a number that is never given out again; a graph does not keep its pattern.
+std::mutex numbered_lock;
+std::unordered_map<int64_t, std::weak_ptr<Pattern>>& numbered() {   // (outlives every pattern)
+    static auto* all = new std::unordered_map<int64_t, std::weak_ptr<Pattern>>();
+    return *all;
+}
+int64_t pattern_number(const PatternPtr& p) {
+    static int64_t last = 0;
+    std::lock_guard<std::mutex> hold(numbered_lock);
+    if (!p->number) {
+        p->number = ++last;
+        numbered()[p->number] = p;
+    }
+    return p->number;
+}
+PatternPtr numbered_pattern(int64_t number) {
+    std::lock_guard<std::mutex> hold(numbered_lock);
+    const auto at = numbered().find(number);
+    const PatternPtr p = at == numbered().end() ? nullptr : at->second.lock();
+    TORCH_CHECK(p, "the block-sparse pattern of this graph does not exist any more");
+    return p;
+}
+Pattern::~Pattern() {
+    if (!number) return;
+    std::lock_guard<std::mutex> hold(numbered_lock);
+    numbered().erase(number);
+}
+
+// The same as an operator that a graph of torch can hold, for compiled autograd, which calls the node below with tensors that have no
+// data.  Returns the wanted gradients alone.
+std::vector<Tensor> linear_backward_op(const Tensor& dy, const std::optional<Tensor>& x, const std::optional<Tensor>& data, int64_t pattern, bool dx,
+                                       bool dw, bool db) {
+    std::vector<Tensor> out;
+    for (Tensor& t : linear_backward(*numbered_pattern(pattern), dy, x.value_or(Tensor()), data.value_or(Tensor()), {dx, dw, db}))
+        if (t.defined()) out.push_back(std::move(t));
+    return out;
+}
+std::vector<Tensor> linear_backward_shapes(const Tensor& dy, const std::optional<Tensor>&, const std::optional<Tensor>&, int64_t pattern, bool dx,
+                                           bool dw, bool db) {
+    const PatternPtr p = numbered_pattern(pattern);
+    std::vector<Tensor> out;
+    auto sizes = dy.sym_sizes().vec();
+    sizes.back() = p->in_features;
+    if (dx) out.push_back(at::empty_symint(sizes, dy.options()));
+    if (dw) out.push_back(at::empty({(int64_t)p->nnz * 32, 32}, dy.options()));
+    if (db) out.push_back(at::empty({p->out_features}, dy.options()));
+    return out;
+}
+TORCH_LIBRARY(pytorch_block_sparse_amd, m) {
+    m.def("linear_backward(Tensor dy, Tensor? x, Tensor? data, int pattern, bool dx, bool dw, bool db) -> Tensor[]");
+}
+TORCH_LIBRARY_IMPL(pytorch_block_sparse_amd, CUDA, m) { m.impl("linear_backward", linear_backward_op); }
+TORCH_LIBRARY_IMPL(pytorch_block_sparse_amd, Meta, m) { m.impl("linear_backward", linear_backward_shapes); }
+
+// y = x W^T + bias
 struct BlockSparseLinearBackward : public torch::autograd::Node {
     PatternPtr pattern;
     torch::autograd::SavedVariable x, data;
@@ -286,23 +361,50 @@ struct BlockSparseLinearBackward : public torch::autograd::Node {
         torch::autograd::variable_list out(3);
         const Tensor& g = grads[0];
         if (!g.defined()) return out;
+        std::array<bool, 3> wanted = wants();
         // under create_graph the sum of dy is recorded, as the operator it is; the products have no second derivative
-        const bool record = c10::GradMode::is_enabled() && has_bias && task_should_compute_output(2);
-        if (record) out[2] = g.reshape({-1, g.size(-1)}).sum(0);
-        const bool sums = has_bias && !record && task_should_compute_output(2);
-        at::NoGradGuard no_grad;
-        const Tensor dy = g.is_contiguous() ? g : g.contiguous();
-        if (task_should_compute_output(0)) out[0] = matmul(*pattern, dy, data.unpack(shared_from_this()), Tensor(), false);
-        if (task_should_compute_output(1)) {
-            const Tensor xs = x.unpack(shared_from_this());
-            out[1] = at::empty({(int64_t)pattern->nnz * 32, 32}, xs.options());
-            Tensor db;
-            if (sums) out[2] = db = at::empty({pattern->out_features}, xs.options());
-            matmul_back(*pattern, dy, xs, out[1], db);
-        } else if (sums) {
-            out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
+        if (c10::GradMode::is_enabled() && wanted[2]) {
+            out[2] = g.reshape({-1, g.size(-1)}).sum(0);
+            wanted[2] = false;
         }
+        auto made = linear_backward(*pattern, g, wanted[1] ? x.unpack(shared_from_this()) : Tensor(), wanted[0] ? data.unpack(shared_from_this()) : Tensor(),
+                                    wanted);
+        for (int i = 0; i < 3; ++i)
+            if (wanted[i]) out[i] = std::move(made[i]);
         return out;
+    }
+
+    void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override {
+        args.collect(x, false);
+        args.collect(data, false);
+        args.collect(has_bias);
+        args.collect(pattern_number(pattern));   // a graph is made for one pattern
+    }
+    torch::autograd::variable_list apply_with_saved(const torch::autograd::variable_list& grads, torch::dynamo::autograd::SwapSavedVariables& saved) override {
+        saved.before(x);
+        saved.before(data);
+        torch::autograd::variable_list out(3);
+        if (grads[0].defined()) {
+            static const auto op = c10::Dispatcher::singleton()
+                                       .findSchemaOrThrow("pytorch_block_sparse_amd::linear_backward", "")
+                                       .typed<std::vector<Tensor>(const Tensor&, const std::optional<Tensor>&, const std::optional<Tensor>&, int64_t, bool, bool, bool)>();
+            const std::array<bool, 3> wanted = wants();
+            const auto maybe = [&](bool want, torch::autograd::SavedVariable& v) {
+                return want ? std::optional<Tensor>(v.unpack(shared_from_this())) : std::nullopt;
+            };
+            auto made = op.call(grads[0], maybe(wanted[1], x), maybe(wanted[0], data), pattern_number(pattern), wanted[0], wanted[1], wanted[2]);
+            size_t at = 0;
+            for (int i = 0; i < 3; ++i)
+                if (wanted[i]) out[i] = std::move(made[at++]);
+        }
+        saved.after(x);
+        saved.after(data);
+        return out;
+    }
+
+  private:
+    std::array<bool, 3> wants() const {
+        return {task_should_compute_output(0), task_should_compute_output(1), has_bias && task_should_compute_output(2)};
     }
 };
 
