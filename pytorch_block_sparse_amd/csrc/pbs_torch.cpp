@@ -624,7 +624,22 @@ PyObject* py_validate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {{"replace_blocks", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_replace_blocks)), METH_FASTCALL, nullptr},
+// check_protocol(what): with PBS_DEBUG set, raise if a bounded wait has run out on the current device since the last check
+PyObject* py_check_protocol(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    need(n, 1, "check_protocol");
+    const char* what = PyUnicode_AsUTF8(args[0]);
+    if (!what) return nullptr;
+    {
+        NoGil no_gil;
+        check_protocol(what, c10::hip::current_device());
+    }
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {{"check_protocol", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_check_protocol)), METH_FASTCALL, nullptr},
+                         {"replace_blocks", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_replace_blocks)), METH_FASTCALL, nullptr},
                          {"validate", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_validate)), METH_FASTCALL, nullptr},
                          {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_linear)), METH_FASTCALL, nullptr},
                          {"matmul", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_matmul)), METH_FASTCALL, nullptr},

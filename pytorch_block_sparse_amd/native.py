@@ -126,6 +126,14 @@ def _check(code, what):
         raise RuntimeError(f"{what} failed with code {code}: {error_string(code)}")
 
 
+def check_protocol(what):
+    """With PBS_DEBUG set: raise if a bounded wait of a barrier-free kernel has run out on the current device since the last check
+    (the kernel marks the affected results NaN and counts the event; without this the call reports success).  The products of
+    ``torch_path()`` check by themselves."""
+    if os.environ.get("PBS_DEBUG"):
+        torch_path().check_protocol(what)
+
+
 def matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace=True):
     """Which kernel pbs_blocksparse_matmul_ws runs for these sizes (for benchmark labels)."""
     return load().pbs_blocksparse_matmul_kernel_name(
@@ -203,3 +211,53 @@ def blocksparse_matmul_plan(ptr, indices, n, k):
         )
     _check(code, "pbs_blocksparse_matmul_plan")
     return plan
+
+
+def _dtype_code(t):
+    code = DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise RuntimeError(f"unsupported dtype {t.dtype}; supported: {SUPPORTED_DTYPES}")
+    return code
+
+
+def blocksparse_matmul(dense_a, data, plan, n, k, nnz, transpose, bias=None, out=None):
+    """out[tokens, n] = dense_a[tokens, k] . W^T (transpose) or . W (not transpose), with a plan of blocksparse_matmul_plan."""
+    lib = load()
+    _require_cuda(dense_a, data, plan, bias)
+    code_dtype = _dtype_code(dense_a)
+    if data.dtype != dense_a.dtype:
+        raise RuntimeError(f"dense operand is {dense_a.dtype} but the block data is {data.dtype}")
+    if bias is not None and bias.dtype != dense_a.dtype:
+        raise RuntimeError(f"bias is {bias.dtype}, expected {dense_a.dtype}")
+    tokens, tr = dense_a.shape[0], 1 if transpose else 0
+    if out is None:
+        out = torch.empty((tokens, n), dtype=dense_a.dtype, device=dense_a.device)
+    # the transposed copy of the blocks that the forward bf16 kernel for dense patterns works from (made by the library)
+    ws_bytes = lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, code_dtype)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dense_a.device)
+    with torch.cuda.device(dense_a.device):
+        code = lib.pbs_blocksparse_matmul_ws(
+            _ptr(dense_a), _ptr(data), _ptr(plan), _ptr(bias), _ptr(out), tokens, n, k, nnz, tr, code_dtype, _ptr(ws), ws_bytes, _stream(),
+        )
+        _check(code, "pbs_blocksparse_matmul_ws")
+        check_protocol("pbs_blocksparse_matmul_ws")
+    return out
+
+
+def blocksparse_matmul_back(dense_a, dense_b, row_start_ends_a, cols_a, out):
+    """out (packed [nnz*32, 32]) = blocks of dense_a^T . dense_b on the pattern's support."""
+    lib = load()
+    _require_cuda(dense_a, dense_b, row_start_ends_a, cols_a, out)
+    code_dtype = _dtype_code(dense_a)
+    if dense_b.dtype != dense_a.dtype or out.dtype != dense_a.dtype:
+        raise RuntimeError("operands and result must share one dtype")
+    tokens, out_features = dense_a.shape
+    sizes = (tokens, out_features, dense_b.shape[1], cols_a.shape[0], code_dtype)
+    ws_bytes = lib.pbs_blocksparse_matmul_back_workspace_bytes(*sizes)
+    ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dense_a.device)
+    with torch.cuda.device(dense_a.device):
+        code = lib.pbs_blocksparse_matmul_back(
+            _ptr(dense_a), _ptr(dense_b), _ptr(row_start_ends_a), _ptr(cols_a), _ptr(out), *sizes, _ptr(ws), ws_bytes, _stream(),
+        )
+    _check(code, "pbs_blocksparse_matmul_back")
+    return out
