@@ -27,9 +27,19 @@ def build(verbose=True):
         )]
         for j in jobs:
             j.result()
+    _link_torch(verbose)
+    return LIB
+
+
+def build_torch(verbose=True):
+    """_pbs_torch.so alone, next to a libpbs_hip.so that is there (the Makefile's way)."""
+    _run(_torch_command(compile_only=True), verbose)
+    _link_torch(verbose)
+
+
+def _link_torch(verbose):
     _run(_torch_command(compile_only=False), verbose)   # links against libpbs_hip.so
     os.remove(TORCH_EXT + ".o")
-    return LIB
 
 
 def _hip_command(lib, defines):
@@ -79,5 +89,5 @@ def _run(cmd, verbose):
 
 
 if __name__ == "__main__":
-    build()
+    build_torch() if "--torch-only" in sys.argv else build()
     sys.exit(0)

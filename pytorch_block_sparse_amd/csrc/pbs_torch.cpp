@@ -650,6 +650,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pbs_torch", nullptr, -1, methods}
 }  // namespace
 
 PyMODINIT_FUNC PyInit__pbs_torch() {
+    if (pbs_abi_version() != PBS_ABI_VERSION)
+        return PyErr_Format(PyExc_ImportError, "_pbs_torch.so was built for version %d of libpbs_hip.so, which is version %d: build both again",
+                            PBS_ABI_VERSION, pbs_abi_version());
     ScheduleType.tp_name = "pytorch_block_sparse_amd.csrc._pbs_torch.Schedule";
     ScheduleType.tp_basicsize = sizeof(Schedule);
     ScheduleType.tp_flags = Py_TPFLAGS_DEFAULT;

@@ -16,6 +16,8 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libpbs_hip.so")
 
+ABI_VERSION = 6   # PBS_ABI_VERSION of the header that the prototypes below restate
+
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
 SUPPORTED_DTYPES = tuple(DTYPE_CODES)
 
@@ -94,6 +96,8 @@ def load():
         fn = getattr(lib, name)
         fn.restype = restype
         fn.argtypes = argtypes
+    if lib.pbs_abi_version() != ABI_VERSION:
+        raise NativeLibraryMissing(f"{LIB_PATH} is version {lib.pbs_abi_version()}, expected {ABI_VERSION}: build it again")
     _lib = lib
     return lib
 
