@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 6
+#define PBS_ABI_VERSION 7
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -125,10 +125,13 @@ int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int 
  * (PBS_PLAN_LIST, one launch) is all that fp32 and small bf16 products need.  `part` is a sum of PBS_PLAN_*;
  * pbs_blocksparse_matmul_part() tells which part a product of these sizes reads, given whether the call has a
  * workspace.  PBS_PLAN_LIST has to be there in any case.  pbs_blocksparse_matmul_plan builds everything.
+ * Such a plan takes pbs_blocksparse_matmul_plan_part_bytes(n, k) bytes, about half of pbs_blocksparse_matmul_plan_bytes(n, k)
+ * (a larger buffer will do as well).
  */
 #define PBS_PLAN_LIST 1
 #define PBS_PLAN_WIDE 2
 #define PBS_PLAN_COLUMN 4
+size_t pbs_blocksparse_matmul_plan_part_bytes(int n, int k);
 int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, int part,
                                      void* plan, size_t plan_bytes, void* stream);
 int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace);
@@ -136,7 +139,8 @@ int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int trans
 /*
  * What a training step derives from a pattern, in one launch: the PBS_PLAN_LIST part of the plans of both directions (forward:
  * of the transposed weight) and, if `units` is not NULL, the unit table of the weight gradient
- * (pbs_blocksparse_matmul_back_units).  Same results, buffers and sizes as the calls that make them one by one.
+ * (pbs_blocksparse_matmul_back_units).  Same results and buffers as the calls that make them one by one; the plans take
+ * pbs_blocksparse_matmul_plan_part_bytes.
  */
 int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_a, const int32_t* col_start_ends_b,
                            const int32_t* rows_b, int out_features, int in_features, int nnz, void* plan_forward,

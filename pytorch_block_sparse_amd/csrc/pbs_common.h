@@ -12,30 +12,13 @@ struct bf16_t {
     uint16_t bits;
 };
 
-// Per element type: bytes, and how one 32x32x32 block product is issued on the matrix cores.
-//
-// A "fragment" is what one lane holds of a 32(rows) x 32(k) operand tile: lane l serves row
-// (l & 31) and the 16 consecutive k values 16*(l >> 5) .. +15, kept as NQ 16-byte registers
-// quads.  Both operands of a product use the same assignment of k to (lane half, register),
-// so any operand whose k runs contiguously in memory is loaded with plain 16-byte reads.
+// Per element type: bytes, and the conversions from and to float.
 template <typename T>
 struct Elem;
 
 template <>
 struct Elem<float> {
     static constexpr int ESZ = 4;
-    static constexpr int NQ = 4;  // 16 floats per lane
-    // v_mfma_f32_32x32x2_f32: lane half h supplies k = h of each 2-wide step; here step
-    // (q, e) contracts the k pair {4q+e, 16+4q+e}.
-    static __device__ __forceinline__ void mma(f32x16& acc, const uint4* a, const uint4* b) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[q].x), __uint_as_float(b[q].x), acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[q].y), __uint_as_float(b[q].y), acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[q].z), __uint_as_float(b[q].z), acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[q].w), __uint_as_float(b[q].w), acc, 0, 0, 0);
-        }
-    }
     static __device__ __forceinline__ float from_f32(float v) { return v; }
     static __device__ __forceinline__ float to_f32(float v) { return v; }
 };
@@ -43,16 +26,6 @@ struct Elem<float> {
 template <>
 struct Elem<bf16_t> {
     static constexpr int ESZ = 2;
-    static constexpr int NQ = 2;  // 16 bf16 per lane
-    // v_mfma_f32_32x32x16_bf16: lane half h supplies 8 consecutive k of each 16-wide step;
-    // here step q contracts k in {8q..8q+7} u {16+8q..16+8q+7}.
-    static __device__ __forceinline__ void mma(f32x16& acc, const uint4* a, const uint4* b) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[q]),
-                                                          __builtin_bit_cast(bf16x8, b[q]), acc, 0, 0, 0);
-        }
-    }
     // round to nearest even, NaN kept quiet: the hardware conversion (v_cvt_pk_bf16_f32, two values per
     // instruction where the compiler can pair them)
     static __device__ __forceinline__ bf16_t from_f32(float v) {

@@ -52,11 +52,11 @@ struct DdsArgs {
 };
 
 // ---- plan buffer ----
-// [work list, pbs_stream.h][wide plan, pbs_dds16.h][block column tables][column plan, pbs_ddsc.h].  Its size and the
-// places of its parts are those callers of the C ABI have sized and read it by since plans held records for groups of
-// 8, 7, 6 and 5 block columns: per width an area of 64-byte records and a table of the block column in each of a group's
-// 8 places.  The work list fills the area of the first width exactly; the tables are still written (they tell
-// which columns exist), the other widths' records are not.
+// [work list, pbs_stream.h][wide plan, pbs_dds16.h][column plan, pbs_ddsc.h], which is what the products read and
+// pbs_blocksparse_matmul_plan_part_bytes counts.  pbs_blocksparse_matmul_plan_bytes counts, behind that, what plans held when the first
+// area was records for groups of 8 block columns: per width of 8, 7, 6 and 5 a table of the block column in each of a group's 8 places
+// (written by pbs_blocksparse_matmul_plan alone; it tells which columns exist), and for the last three an area of records, not
+// written any more.
 constexpr int PLAN_NWIDTHS = 4;
 constexpr int PLAN_WIDTHS[PLAN_NWIDTHS] = {8, 7, 6, 5};
 constexpr int PLAN_PLACES = 8;
@@ -69,20 +69,7 @@ static inline size_t wide_plan_bytes(int n, int k) {
     const size_t groups = ((size_t)(n / 32) + D16_NB - 1) / D16_NB;
     return (groups * dds16_plan_group_ints(k / 32) + D16_SEQ_INTS) * sizeof(int);
 }
-
-static inline size_t width_offset(int n, int k, int wi) {
-    if (wi == 0) return 0;
-    size_t off = list_area_bytes(n, k) + wide_plan_bytes(n, k) + slot_table_bytes_w(n, 0);
-    for (int i = 1; i < wi; ++i) off += width_bytes(n, k, i) + slot_table_bytes_w(n, i);
-    return off;
-}
-static inline size_t slot_table_offset(int n, int k, int wi) {
-    if (wi == 0) return list_area_bytes(n, k) + wide_plan_bytes(n, k);
-    return width_offset(n, k, wi) + width_bytes(n, k, wi);
-}
-static inline size_t column_plan_offset(int n, int k) {
-    return width_offset(n, k, PLAN_NWIDTHS - 1) + width_bytes(n, k, PLAN_NWIDTHS - 1) + slot_table_bytes_w(n, PLAN_NWIDTHS - 1);
-}
+static inline size_t column_plan_offset(int n, int k) { return list_area_bytes(n, k) + wide_plan_bytes(n, k); }
 static inline int column_groups(int n) { return (n / 32 + DC_NB - 1) / DC_NB; }
 static inline size_t column_table_bytes(int n) { return ((size_t)column_groups(n) * DC_NB * sizeof(int) + 63) / 64 * 64; }
 static inline size_t column_plan_bytes(int n, int k) {
@@ -90,7 +77,13 @@ static inline size_t column_plan_bytes(int n, int k) {
     if ((k % 64) || DC_NB * (k / 32) > DC_ITEMS_LDS) return 0;
     return column_table_bytes(n) + ((size_t)column_groups(n) * ddsc_plan_group_ints(k / 32) + DC_SEQ_INTS) * sizeof(int);
 }
-static inline size_t all_plan_bytes(int n, int k) { return column_plan_offset(n, k) + column_plan_bytes(n, k); }
+static inline size_t part_plan_bytes(int n, int k) { return column_plan_offset(n, k) + column_plan_bytes(n, k); }
+static inline size_t slot_table_offset(int n, int k, int wi) {
+    size_t off = part_plan_bytes(n, k);
+    for (int i = 1; i <= wi; ++i) off += slot_table_bytes_w(n, i - 1) + width_bytes(n, k, i);
+    return off;
+}
+static inline size_t all_plan_bytes(int n, int k) { return slot_table_offset(n, k, PLAN_NWIDTHS - 1) + slot_table_bytes_w(n, PLAN_NWIDTHS - 1); }
 
 // the block column in each of the 8 places of each group, one table per width: every column once, -1 elsewhere
 struct SlotTables {
@@ -793,11 +786,16 @@ size_t pbs_blocksparse_matmul_plan_bytes(int n, int k) {
     return all_plan_bytes(n, k);
 }
 
+size_t pbs_blocksparse_matmul_plan_part_bytes(int n, int k) {
+    if (n <= 0 || k <= 0 || (n % 32) || (k % 32)) return 0;
+    return part_plan_bytes(n, k);
+}
+
 static int plan_checks(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, const void* plan, size_t plan_bytes) {
     if (n <= 0 || k <= 0 || nnz < 0 || (n % 32) || (k % 32)) return PBS_ERR_BAD_SHAPE;
     if ((long long)nnz > (long long)(n / 32) * (k / 32) || k > (1 << 24)) return PBS_ERR_TOO_LARGE;
     if (!ptr || !plan || (nnz > 0 && !indices)) return PBS_ERR_NULL_POINTER;
-    if (!aligned16(plan) || plan_bytes < all_plan_bytes(n, k)) return PBS_ERR_WORKSPACE;
+    if (!aligned16(plan) || plan_bytes < part_plan_bytes(n, k)) return PBS_ERR_WORKSPACE;
     return PBS_OK;
 }
 
@@ -836,6 +834,8 @@ int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices,
 
 int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int n, int k, int nnz, void* plan,
                                 size_t plan_bytes, void* stream) {
+    if (int rc = plan_checks(ptr, indices, n, k, nnz, plan, plan_bytes)) return rc;
+    if (plan_bytes < all_plan_bytes(n, k)) return PBS_ERR_WORKSPACE;
     if (int rc = pbs_blocksparse_matmul_plan_part(ptr, indices, n, k, nnz, PART_LIST | PART_WIDE | PART_COLUMN, plan, plan_bytes, stream))
         return rc;
     SlotTables t;

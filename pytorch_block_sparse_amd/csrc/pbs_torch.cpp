@@ -157,7 +157,7 @@ struct Pattern {
         const Tensor& idx = transpose ? cols.t : rows.t;
         TORCH_CHECK(ptr.is_cuda() && idx.is_cuda(), "the index buffers are not on the GPU");
         const bool keep = !capturing(stream);
-        const size_t bytes = pbs_blocksparse_matmul_plan_bytes(n, k);
+        const size_t bytes = pbs_blocksparse_matmul_plan_part_bytes(n, k);
         const Tensor t = keep && kept.t.defined() ? kept.t : at::empty({(int64_t)bytes}, ptr.options().dtype(at::kByte));
         check(pbs_blocksparse_matmul_plan_part(ptr.const_data_ptr<int>(), idx.const_data_ptr<int>(), n, k, nnz,
                                                keep ? part & ~parts[transpose] : part, t.mutable_data_ptr(), bytes, stream),
@@ -175,8 +175,8 @@ struct Pattern {
             !rows.t.is_cuda() || capturing(stream))
             return;
         const auto bytes = row_ptr.t.options().dtype(at::kByte);
-        const size_t forward_bytes = pbs_blocksparse_matmul_plan_bytes(out_features, in_features),
-                     input_bytes = pbs_blocksparse_matmul_plan_bytes(in_features, out_features),
+        const size_t forward_bytes = pbs_blocksparse_matmul_plan_part_bytes(out_features, in_features),
+                     input_bytes = pbs_blocksparse_matmul_plan_part_bytes(in_features, out_features),
                      units_bytes = pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, code);
         const Tensor forward = at::empty({(int64_t)forward_bytes}, bytes), input = at::empty({(int64_t)input_bytes}, bytes);
         const Tensor table = units_bytes ? at::empty({(int64_t)units_bytes}, bytes) : Tensor();

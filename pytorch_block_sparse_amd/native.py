@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libpbs_hip.so")
 
-ABI_VERSION = 6   # PBS_ABI_VERSION of the header that the prototypes below restate
+ABI_VERSION = 7   # PBS_ABI_VERSION of the header that the prototypes below restate
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
 SUPPORTED_DTYPES = tuple(DTYPE_CODES)
@@ -37,6 +37,7 @@ _PROTOTYPES = {
     "pbs_validate_indices": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, ctypes.c_size_t, _vp]),
     "pbs_blocksparse_matmul_plan_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "pbs_blocksparse_matmul_plan": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
+    "pbs_blocksparse_matmul_plan_part_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "pbs_blocksparse_matmul_plan_part": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp]),
     "pbs_blocksparse_derive": (
         _i32,
