@@ -118,7 +118,7 @@ class BlockSparseLinear(nn.Module):
         # to do: a subclass of the matrix may have products of its own, `fn` may have been replaced, and torch.jit.trace can
         # record the function but not see into the native call.
         if type(weight) is BlockSparseMatrix and self.fn == _APPLY and not torch.jit.is_tracing():
-            return native.torch_path().linear(x, weight.data, self.bias, weight._buffers, weight.schedule())
+            return (native._torch_path or native.torch_path()).linear(x, weight.data, self.bias, weight._buffers, weight.schedule())
         return self.fn(x, self.weight.get_differentiable_data(), self.weight, self.bias)
 
     def extra_repr(self):
