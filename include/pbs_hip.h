@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 7
+#define PBS_ABI_VERSION 8
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -180,9 +180,15 @@ int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* pl
  * unspecified afterwards).  With workspace = NULL, or one that is too small, the call is
  * pbs_blocksparse_matmul: same results to the last bit of bf16 rounding of the same fp32 sums in a
  * different order, from a kernel that reads the data as stored.  ..._workspace_bytes() returns 0 when
- * no workspace would be used (fp32, the input-gradient direction, small or very sparse problems).
+ * no copy would be made (fp32, the input-gradient direction, small or very sparse problems).
+ *
+ * Larger fp32 products run on the bf16 matrix cores, which multiply 16 times as fast: every value as the sum of three bfloat16 values
+ * (without a rest), six of their nine products, sums in fp32; closer to the exact result than the fp32 instructions' chains are.  For that the
+ * call writes the parts of the blocks into a workspace of pbs_blocksparse_matmul_parts_bytes() bytes (6 KB per block; 0 where such a
+ * workspace would not be used: bf16, smaller or very sparse problems).  Without it, the product is made of fp32 instructions.
  */
 size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype);
+size_t pbs_blocksparse_matmul_parts_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype);
 int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void* plan,
                               const void* bias, void* dense_out,
                               int64_t tokens, int n, int k, int nnz,
@@ -305,14 +311,14 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
 /*
  * Diagnostics.  Neither has a counterpart in the reference.
  *
- * pbs_protocol_failures: the bf16 kernels for large problems (dds16_kernel, ddsc_kernel) synchronise their waves
+ * pbs_protocol_failures: the kernels for large problems (dds16_kernel, ddsc_kernel, split_kernel) synchronise their waves
  * through progress words in LDS with bounded waits instead of barriers.  A wait that runs into its bound means a
  * broken protocol; the kernel then writes NaN into the results it could not vouch for and counts the event in a
  * device word.  This call copies the current GPU's count (since the library was loaded) to *count; it synchronises
  * the device.  The Python layer checks it after every product when PBS_DEBUG is set and raises.
  *
  * pbs_blocksparse_matmul_kernel_name / ..._back_kernel_name: which kernel(s) a call with these sizes runs
- * ("stream_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel",
+ * ("stream_kernel", "split_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel",
  * "sdd_bf16_kernel", with " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
  */

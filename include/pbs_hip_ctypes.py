@@ -28,6 +28,7 @@ PROTOTYPES = {
     "pbs_blocksparse_matmul_plan": (_i, [_p, _p, _i, _i, _i, _p, _z, _p]),
     "pbs_blocksparse_matmul": (_i, [_p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p]),
     "pbs_blocksparse_matmul_workspace_bytes": (_z, [_l, _i, _i, _i, _i, _i]),
+    "pbs_blocksparse_matmul_parts_bytes": (_z, [_l, _i, _i, _i, _i, _i]),
     "pbs_blocksparse_matmul_ws": (_i, [_p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _i, _p, _z, _p]),
     "pbs_blocksparse_matmul_back_workspace_bytes": (_z, [_l, _i, _i, _i, _i]),
     "pbs_blocksparse_matmul_back": (_i, [_p, _p, _p, _p, _p, _l, _i, _i, _i, _i, _p, _z, _p]),
@@ -69,8 +70,9 @@ class PbsHip:
         """dense_a [tokens, k] row-major contiguous -> [tokens, n]; replaces the reference's call at block_sparse.py:562-574."""
         tokens, tr, dt = dense_a.shape[0], int(bool(transpose)), DTYPES[dense_a.dtype]
         out = torch.empty(tokens, n, dtype=dense_a.dtype, device=dense_a.device)
-        # room for the transposed copy of the blocks that the reference makes itself at block_sparse.py:541-544
-        nws = self.lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, dt)
+        # room for the transposed copy of the blocks that the reference makes itself at block_sparse.py:541-544, or for their bf16 parts
+        nws = (self.lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, dt)
+               or self.lib.pbs_blocksparse_matmul_parts_bytes(tokens, n, k, nnz, tr, dt))
         ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dense_a.device)
         with torch.cuda.device(dense_a.device):
             self._check(self.lib.pbs_blocksparse_matmul_ws(

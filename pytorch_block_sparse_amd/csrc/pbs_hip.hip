@@ -12,6 +12,7 @@
 #include "pbs_dds16.h"
 #include "pbs_ddsc.h"
 #include "pbs_panel.h"
+#include "pbs_split.h"
 #include "pbs_stream.h"
 #include "pbs_index.h"
 #include "pbs_sdd.h"
@@ -231,7 +232,8 @@ struct StreamShape {
 };
 // The shapes that are built, of the 15 with tt in {1, 2, 4, 8} and ks in {1, 2, 4, 8} that were timed on 140 problems (1 to
 // 16384 tokens, 256 to 4096 features, densities 0.05 to 0.75, even and Zipf columns).  In fp32 the number of waves
-// follows from the pattern alone, so that a token's result does not depend, to the last bit, on how many tokens share the call: four from 14
+// follows from the pattern alone, so that a token's result does not depend, to the last bit, on how many tokens share the call (among the
+// calls that run here: split_kernel_fits): four from 14
 // blocks per column (then within 1 to 4 % of the best on average), two below (within 5 %; four are 6 to 14 % slower there,
 // the sum of the waves' parts weighs more).
 constexpr StreamShape STREAM_F32[] = {{1, 2}, {2, 2}, {4, 2}, {1, 4}, {2, 4}, {4, 4}};
@@ -396,6 +398,90 @@ static int launch_panel_chunks(const DdsArgs& g, int splits, hipStream_t stream)
     return (int)hipGetLastError();
 }
 
+// ---- fp32 on the bf16 matrix cores ----
+// Which problems: products of 370 random problems (256 to 4096 features, 300 to 16384 tokens, densities 0.05 to 0.75, even and Zipf rows) were
+// timed with this kernel and with stream_kernel.  With a pattern of density 0.2 and more, groups of 8 columns that are filled to three quarters,
+// and 4.3 GFLOP (2^21 tokens x blocks) it takes 1.29 times less time on average and at most 1.1 times more; below, a panel is split for too few
+// products (density 0.15: 0.8 to 1.1 times as fast, 0.05: half as fast), waves have no column, or the launch that splits the blocks and the first
+// panels weigh too much (at 2^20 as often slower as faster; 1024 -> 2560, 700 tokens 14 us in stream_kernel, 20 here).
+// The line depends on the pattern and then on the number of tokens alone: a token's result does not depend, to the last bit, on
+// the others in the call among all calls of a pattern on the same side of it.
+static bool split_kernel_fits(long long M, int n, int k, int nnz) {
+    const long long cols = n / 32, groups = (cols + SP_NC - 1) / SP_NC;
+    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
+    // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
+    return k <= (1 << 16) && (M + 31) / 32 * groups < (1 << 28);
+}
+static inline size_t split_workspace_bytes(int nnz) { return (size_t)nnz * SP_BLOCK_BYTES; }
+
+// How many tiles of 64 tokens, the rest being low ones of 32: full tiles for as many whole rounds of units over the 256 CUs as is best, low ones
+// behind them (which a result's bits do not depend on).  A low unit takes 0.58 to 0.65 of a full one's time.  Against full tiles alone: 264 units
+// (4215 tokens 2784 -> 800) 73 -> 60 us, 128 units (512 tokens 4096 -> 4096) 52 -> 44, multiples of 256 the same.
+constexpr double SP_LOW = 0.62;
+static int split_full_tiles(long long M, int groups) {
+    const long long most = M / SP_BM, all = (M + SP_BM - 1) / SP_BM;
+    auto rounds = [&](long long full) {
+        const long long low = (M - full * SP_BM + 31) / 32;
+        const double f = (double)full * groups / 256, l = low > 0 ? (double)low * groups / 256 : 0.0;
+        // full rounds, then what is left of the full units beside the low ones
+        const double whole = std::floor(f), rest = f - whole;
+        if (rest == 0.0) return whole + SP_LOW * std::ceil(l);
+        const double beside = (1.0 - rest) * std::floor(1.0 / SP_LOW);   // low units that fit beside the rest
+        return whole + 1.0 + (l > beside ? SP_LOW * std::ceil(l - beside) : 0.0);
+    };
+    long long best = all;   // (the last one ragged)
+    double least = rounds(all);
+    for (long long r = 0; r <= most * groups / 256; ++r) {
+        const long long full = r * 256 / groups;
+        if (full <= most && rounds(full) < least - 1e-9) {
+            least = rounds(full);
+            best = full;
+        }
+    }
+    return (int)best;
+}
+
+template <int TRANS>
+static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
+    static std::atomic<uint64_t> done{0};
+    auto kernel = split_kernel<TRANS>;
+    if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
+    hipLaunchKernelGGL(split_blocks_kernel<TRANS>, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream, static_cast<const float*>(g.data),
+                       static_cast<unsigned char*>(workspace), g.nnz);
+    if (int rc = (int)hipGetLastError()) return rc;
+    SplitArgs a;
+    a.a = static_cast<const float*>(g.a);
+    a.data = static_cast<const float*>(g.data);
+    a.parts = static_cast<const unsigned char*>(workspace);
+    a.plan = g.plan;
+    a.bias = static_cast<const float*>(g.bias);
+    a.out = static_cast<float*>(g.out);
+    a.M = g.M;
+    a.N = g.N;
+    a.K = g.K;
+    a.groups = (g.N / 32 + SP_NC - 1) / SP_NC;
+    a.tiles = split_full_tiles(g.M, a.groups);
+    a.low_tiles = g.M > a.tiles * SP_BM ? (g.M - a.tiles * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
+    // the 32 workgroups of an XCD work on tile_block token tiles x 32 / tile_block groups: the split with the least to read per k-block
+    const double w_bytes = (double)SP_NC * SP_BLOCK_BYTES * g.nnz / ((double)(g.N / 32) * (g.K / 32)), x_bytes = SP_BM * 128.0;
+    double least = 0.0;
+    a.tile_block = 1;
+    for (int t = 1; t <= 32; t *= 2) {
+        const double groups = a.groups < 32 / t ? a.groups : 32 / t, bytes = t * x_bytes + groups * w_bytes;
+        if (groups * t >= 32 || t == 1)
+            if (least == 0.0 || bytes < least) {
+                least = bytes;
+                a.tile_block = t;
+            }
+    }
+    // one workgroup per CU; more where each would have more units than it keeps the heads of
+    const long long units = (long long)(a.tiles + a.low_tiles) * a.groups;
+    long long per_xcd = (units + NUM_XCD - 1) / NUM_XCD + 1;
+    if (per_xcd > 32) per_xcd = per_xcd > 32 * (SP_MAX_UNITS - 1) ? per_xcd / (SP_MAX_UNITS - 1) + 1 : 32;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(NUM_XCD * per_xcd)), dim3((SP_NC + SP_NP) * 64), SP_LDS, stream, a);
+    return (int)hipGetLastError();
+}
+
 // ---- which kernel runs a product ----
 enum MatmulPart { PART_LIST = PBS_PLAN_LIST, PART_WIDE = PBS_PLAN_WIDE, PART_COLUMN = PBS_PLAN_COLUMN };   // and so which part of the plan it reads
 
@@ -467,6 +553,10 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
             case 4: return launch_panel_chunks<TRANS, 4>(g, choice.panel.splits, stream);
             default: break;
         }
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (workspace && workspace_bytes >= split_workspace_bytes(g.nnz) && aligned16(workspace) && split_kernel_fits(g.M, g.N, g.K, g.nnz))
+            return launch_split<TRANS>(g, workspace, stream);
     }
     return launch_stream<T, TRANS>(g, stream);
 }
@@ -861,6 +951,12 @@ size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int 
     return choose_product(2, tokens, n, k, nnz, 1, true).part == PART_COLUMN ? (size_t)nnz * 2048 : 0;
 }
 
+size_t pbs_blocksparse_matmul_parts_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype) {
+    if (dtype != PBS_DTYPE_F32 || tokens <= 0 || n <= 0 || k <= 0 || nnz <= 0 || (n % 32) || (k % 32)) return 0;
+    if ((long long)nnz > (long long)(n / 32) * (k / 32)) return 0;
+    return split_kernel_fits(tokens, n, k, nnz) ? split_workspace_bytes(nnz) : 0;
+}
+
 int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* plan, const void* bias, void* dense_out,
                            int64_t tokens, int n, int k, int nnz, int transpose, int dtype, void* stream) {
     return pbs_blocksparse_matmul_ws(dense_a, data, plan, bias, dense_out, tokens, n, k, nnz, transpose, dtype, nullptr, 0,
@@ -889,7 +985,7 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
     g.nnz = nnz;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == PBS_DTYPE_F32) {
-        return transpose ? dispatch_dds<float, 0>(g, nullptr, 0, s) : dispatch_dds<float, 1>(g, nullptr, 0, s);
+        return transpose ? dispatch_dds<float, 0>(g, workspace, workspace_bytes, s) : dispatch_dds<float, 1>(g, workspace, workspace_bytes, s);
     }
     return transpose ? dispatch_dds<bf16_t, 0>(g, workspace, workspace_bytes, s)
                      : dispatch_dds<bf16_t, 1>(g, nullptr, 0, s);
@@ -1114,6 +1210,7 @@ const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int
                                                int with_workspace) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || (n % 32) || (k % 32)) return "";
     const ProductChoice c = choose_product(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
+    if (dtype == PBS_DTYPE_F32 && with_workspace && nnz > 0 && split_kernel_fits(tokens, n, k, nnz)) return "split_kernel";
     return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (!c.panel.splits ? "stream_kernel" : (c.panel.ways ? "panel_chunk_kernel" : "panel_kernel")));
 }
 

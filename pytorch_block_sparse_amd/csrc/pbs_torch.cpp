@@ -237,8 +237,10 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     if (training) p.derive_all(tokens, code, stream);
     const int part = pbs_blocksparse_matmul_part(tokens, n, k, p.nnz, transpose, code, 1);
     const Tensor plan = p.plan_for(transpose, n, k, part, stream);
-    // the transposed copy of the blocks that the bf16 column kernel's forward product works from
-    const size_t ws_bytes = transpose && part == PBS_PLAN_COLUMN ? pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, p.nnz, 1, code) : 0;
+    // the transposed copy of the blocks that the bf16 column kernel's forward product works from, or the blocks in bf16 parts for larger fp32 products
+    size_t ws_bytes = 0;
+    if (code == PBS_DTYPE_F32) ws_bytes = pbs_blocksparse_matmul_parts_bytes(tokens, n, k, p.nnz, transpose, code);
+    else if (transpose && part == PBS_PLAN_COLUMN) ws_bytes = pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, p.nnz, 1, code);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, a.options().dtype(at::kByte));
     check(pbs_blocksparse_matmul_ws(a.const_data_ptr(), data_or_null(data), plan.const_data_ptr(), data_or_null(bias), out.mutable_data_ptr(), tokens, n, k,

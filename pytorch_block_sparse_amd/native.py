@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libpbs_hip.so")
 
-ABI_VERSION = 7   # PBS_ABI_VERSION of the header that the prototypes below restate
+ABI_VERSION = 8   # PBS_ABI_VERSION of the header that the prototypes below restate
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
 SUPPORTED_DTYPES = tuple(DTYPE_CODES)
@@ -46,6 +46,7 @@ _PROTOTYPES = {
     "pbs_blocksparse_matmul_part": (_i32, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp]),
     "pbs_blocksparse_matmul_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_matmul_parts_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul_ws": (
         _i32,
         [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp],
@@ -237,8 +238,10 @@ def blocksparse_matmul(dense_a, data, plan, n, k, nnz, transpose, bias=None, out
     tokens, tr = dense_a.shape[0], 1 if transpose else 0
     if out is None:
         out = torch.empty((tokens, n), dtype=dense_a.dtype, device=dense_a.device)
-    # the transposed copy of the blocks that the forward bf16 kernel for dense patterns works from (made by the library)
-    ws_bytes = lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, code_dtype)
+    # the transposed copy of the blocks that the forward bf16 kernel for dense patterns works from, or the bf16 parts of the blocks that
+    # larger fp32 products are made of (both made by the library)
+    ws_bytes = (lib.pbs_blocksparse_matmul_workspace_bytes(tokens, n, k, nnz, tr, code_dtype)
+                or lib.pbs_blocksparse_matmul_parts_bytes(tokens, n, k, nnz, tr, code_dtype))
     ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dense_a.device)
     with torch.cuda.device(dense_a.device):
         code = lib.pbs_blocksparse_matmul_ws(
