@@ -18,6 +18,7 @@
 #include "pbs_sdd.h"
 #include "pbs_sdd_bf16.h"
 #include "pbs_sdd_row.h"
+#include "pbs_sdd_split.h"
 
 namespace pbs {
 
@@ -595,12 +596,15 @@ static SddPlan plan_sdd(long long M, int N, int K) {
 // the choices made by it were 3.5 % slower than the best of all slice counts on average): launch, reduction of the slices,
 // chunks x blocks of a wave of the slowest workgroup, at the rate of a full chip or, below 32 workgroups per XCD, of
 // a wave alone, and what each round of workgroups on the chip costs besides.
-static double row_us(int dtype, long long M, int N, int nnz, int slices, int passes) {
+enum RowKernel { ROW_F32, ROW_SPLIT, ROW_BF16 };   // sdd_row_kernel<float>, sdd_split_kernel, sdd_row_kernel<bf16_t>
+static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, int passes) {
     struct Model {
         double launch, reduce, per_slice, busy, alone, round;
         int resident;   // workgroups per XCD
     };
-    const Model m = dtype == PBS_DTYPE_F32 ? Model{3.34, 6.57, 0.0, 0.523, 0.058, 2.34, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
+    // (ROW_SPLIT: 90 problems of 2^20 tokens x blocks and more, within 12 %, its choices 2.8 % slower than the best on average)
+    const Model m = kernel == ROW_F32 ? Model{3.34, 6.57, 0.0, 0.523, 0.058, 2.34, 64}
+                  : kernel == ROW_SPLIT ? Model{7.0, 11.27, -2.643, 0.4487, 0.540, 5.186, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
     const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
     const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows;
     const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
@@ -627,32 +631,42 @@ static double rectangle_us(long long M, int N, int K, int nnz) {
 // 4 x 2 1199 against 1222, 0.5 2 x 4 2258 against 2347, 1 1 x 8 4131 against 4297; 65536 tokens, density 1 1 x 33 16538 against
 // 16998; 8192 -> 8192, 16384 tokens, density 0.25 1 x 16 4805 against 5211, 0.5 9264 against 10299.
 constexpr size_t ROW_WORKSPACE_BYTES = 64u << 20;
+// fp32 on the bf16 matrix cores (sdd_split_kernel) from 2^22 tokens x blocks where its estimate is the smaller one: of those 30 of the problems it
+// is 1.1 times faster on average, 1.0 to 1.29 and twice 0.95; at 2^21 as often slower as faster (768 x 3072 with Zipf rows, 4096 tokens 52 -> 48 us,
+// 4926 tokens 4064 -> 352 48 -> 58), at 2^20 mostly slower: a wave starts by splitting its first pieces, and the code is larger.
+constexpr long long SPLIT_BACK_WORK = 1ll << 22;
 struct RowChoice {
     int slices, passes;
+    bool split;
 };
 static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
     constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
     const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
     // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 216.
-    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return {0, 1};
+    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return {0, 1, false};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
-    RowChoice best{1, 1};
-    double best_us = 0.0;
+    RowChoice best{1, 1, false};
+    double best_us = -1.0;
     for (const int s : CANDIDATES) {
         if (s > 1 && (s > chunks / 4 || (size_t)nnz * 4096 * s > workspace_limit)) break;
         const int passes = at_least > s ? (int)std::ceil(at_least / s) : 1;
-        const double us = row_us(dtype, M, N, nnz, s, passes);
-        if (s == 1 || us < best_us) {
-            best = {s, passes};
-            best_us = us;
-        }
+        auto consider = [&](RowKernel kernel) {
+            const double us = row_us(kernel, M, N, nnz, s, passes);
+            if (best_us < 0.0 || us < best_us) {
+                best = {s, passes, kernel == ROW_SPLIT};
+                best_us = us;
+            }
+        };
+        consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16);
+        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK) consider(ROW_SPLIT);
     }
     if (dtype == PBS_DTYPE_BF16 && rectangle_us(M, N, K, nnz) < best_us) best.slices = 0;
     return best;
 }
 struct BackPlan {
     int slices;   // row kernel; 0: rectangles
+    bool split;   // fp32 in parts
     int passes, chunks_per_slice;
     SddPlan rect;
     size_t partial_bytes;
@@ -661,6 +675,7 @@ static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bi
     BackPlan p;
     const RowChoice row = choose_row(dtype, M, N, K, nnz, workspace_limit);
     p.slices = row.slices;
+    p.split = row.split;
     p.rect = plan_sdd(M, N, K);
     int n = p.rect.nsplit;
     if (p.slices > 0) {
@@ -731,7 +746,8 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     for (int pass = 0; pass < p.passes; ++pass) {
         r.chunk0 = pass * p.slices * p.chunks_per_slice;
         r.add = pass > 0;
-        hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
+        if (sizeof(T) == 4 && p.split) hipLaunchKernelGGL(sdd_split_kernel, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
+        else hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
         if (int rc = (int)hipGetLastError()) return rc;
     }
     return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;
@@ -1219,6 +1235,7 @@ const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_feat
         nnz <= 0 || (out_features % 32) || (in_features % 32))
         return "";
     const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
+    if (p.slices > 0 && p.split) return p.slices > 1 ? "sdd_split_kernel + sdd_reduce_kernel" : "sdd_split_kernel";
     if (p.slices > 0) return p.slices > 1 ? "sdd_row_kernel + sdd_reduce_kernel" : "sdd_row_kernel";
     return p.rect.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";
 }

@@ -493,29 +493,41 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     }
 }
 
+// What a workgroup does: a unit, and its chunks of the tokens.
+struct RowTask {
+    const int* unit;
+    int c_lo, c_hi;
+    float* partial;
+};
+static __device__ __forceinline__ bool row_task(const SddRowArgs& a, RowTask& t) {
+    // an XCD takes a run of units and goes through them for one token slice after the other
+    const int units = a.table[0];
+    const int xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD;
+    const int u_lo = (int)((long long)units * xcd / NUM_XCD), n_u = (int)((long long)units * (xcd + 1) / NUM_XCD) - u_lo;
+    if (local >= n_u * a.slices) return false;
+    const int slice = local / n_u;
+    t.unit = a.table + 16 + (size_t)(u_lo + local - slice * n_u) * UNIT_INTS;
+    const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
+    t.c_lo = a.chunk0 + slice * a.chunks_per_slice;
+    t.c_hi = t.c_lo + a.chunks_per_slice < chunks ? t.c_lo + a.chunks_per_slice : chunks;
+    t.partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + (a.bias_out ? a.N : 0)) : nullptr;
+    return true;
+}
+
 template <typename T>
 __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel(SddRowArgs a) {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SddRowCfg<T>::LDS];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // an XCD takes a run of units and goes through them for one token slice after the other
-    const int units = a.table[0];
-    const int xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD;
-    const int u_lo = (int)((long long)units * xcd / NUM_XCD), n_u = (int)((long long)units * (xcd + 1) / NUM_XCD) - u_lo;
-    if (local >= n_u * a.slices) return;
-    const int slice = local / n_u;
-    const int* unit = a.table + 16 + (size_t)(u_lo + local - slice * n_u) * UNIT_INTS;
-    const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
-    const int c_lo = a.chunk0 + slice * a.chunks_per_slice;
-    const int c_hi = c_lo + a.chunks_per_slice < chunks ? c_lo + a.chunks_per_slice : chunks;
-    float* partial = a.slices > 1 ? a.partial + (size_t)slice * ((size_t)a.nnz * 1024 + (a.bias_out ? a.N : 0)) : nullptr;
-    switch (unit[1]) {
-        case 4: sdd_row_body<T, 4>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
-        case 3: sdd_row_body<T, 3>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
-        case 2: sdd_row_body<T, 2>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
-        case 1: sdd_row_body<T, 1>(a, unit, c_lo, c_hi, partial, smem, lane, wave); break;
+    RowTask t;
+    if (!row_task(a, t)) return;
+    switch (t.unit[1]) {
+        case 4: sdd_row_body<T, 4>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 3: sdd_row_body<T, 3>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 2: sdd_row_body<T, 2>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 1: sdd_row_body<T, 1>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         default:
-            if (a.bias_out) sdd_row_body<T, 0>(a, unit, c_lo, c_hi, partial, smem, lane, wave);
+            if (a.bias_out) sdd_row_body<T, 0>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave);
             break;
     }
 }

@@ -54,9 +54,12 @@ static_assert(SP_RS % SP_NP == 0 && SP_LDS <= 160 * 1024, "a slot has one writer
 
 // two values into their three parts, packed in pairs
 static __device__ __forceinline__ void split2(float a0, float a1, uint32_t& h, uint32_t& m, uint32_t& l) {
-    auto pack = [](float x, float y) __attribute__((always_inline)) {   // (as a vector: one instruction, where two conversions and an or take four)
+    // as a vector: one instruction, where two conversions and an or take four; and opaque, or every part is converted again to be taken off
+    auto pack = [](float x, float y) __attribute__((always_inline)) {
         typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(x), static_cast<__bf16>(y)});
+        uint32_t p = __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(x), static_cast<__bf16>(y)});
+        asm("" : "+v"(p));
+        return p;
     };
     auto rest = [](float& x, float& y, uint32_t p) __attribute__((always_inline)) {   // exact
         x -= __uint_as_float(p << 16);
