@@ -4,6 +4,7 @@ import copy
 import numpy as np
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 from pytorch_block_sparse_amd import BlockSparseLinear, BlockSparseMatrix
 
@@ -52,3 +53,24 @@ def test_copies_keep_the_native_path(cuda, monkeypatch):
     calls = []
     monkeypatch.setattr(BlockSparseMatrix, "reverse_matmul", lambda *a, **k: calls.append(a))
     assert layer(torch.randn(5, 96, device=cuda)).shape == (5, 64) and not calls
+
+
+@pytest.mark.gpu
+def test_tensors_that_are_not_in_the_dicts(cuda):
+    """A parametrized bias, one kept as a plain attribute, and swapped tensors reach the product."""
+    np.random.seed(1)
+    x = torch.randn(5, 96, device=cuda)
+
+    def plain(layer):
+        return x @ layer.weight.to_dense().t()
+
+    layer = BlockSparseLinear(96, 64, density=0.5, device=cuda)
+    torch.nn.utils.parametrize.register_parametrization(layer, "bias", type("One", (torch.nn.Module,), {"forward": lambda self, b: b + 1})())
+    assert torch.allclose(layer(x), plain(layer) + 1, atol=1e-5)
+    layer = BlockSparseLinear(96, 64, density=0.5, device=cuda)
+    del layer.bias
+    layer.bias = torch.full((64,), 3.0, device=cuda)
+    assert torch.allclose(layer(x), plain(layer) + 3, atol=1e-5)
+    layer = BlockSparseLinear(96, 64, density=0.5, device=cuda)
+    swapped = {"bias": torch.full((64,), 2.0, device=cuda), "weight.data": layer.weight.data.detach() * 2}
+    assert torch.allclose(torch.func.functional_call(layer, swapped, (x,)), 2 * plain(layer) + 2, atol=1e-5)
