@@ -86,6 +86,14 @@ static __device__ __forceinline__ void dma16(unsigned lds_base_uniform, const un
                  : "memory");
 }
 
+// 16 bytes per lane from `off` on in a buffer of `bytes` bytes (both below 2^31; base and bytes wave-uniform); zeros, and no memory
+// access, where off lies behind its end
+static __device__ __forceinline__ uint4 buffer16(const unsigned char* base_uniform, unsigned bytes, unsigned off) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(base_uniform), 0, bytes, 0x00020000);
+    return __builtin_bit_cast(uint4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+}
+
 // wait until at most n (wave-uniform) of this wave's DMA loads are outstanding, make this wave's
 // LDS accesses complete, and meet the other waves.  Loads retire in order, so a smaller n than
 // necessary is only slower, never wrong.

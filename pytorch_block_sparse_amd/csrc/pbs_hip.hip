@@ -564,18 +564,16 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
 
 // ---- sparse-output product ----
 // Two kernels: up to four blocks of a block row per workgroup (pbs_sdd_row.h), which serves fp32 altogether and
-// bf16 while the operands are small enough, and for large bf16 problems rectangles of 16 x 16 block positions
+// bf16 while the operands are small enough, and for large bf16 problems rectangles of 16 x 16 or 8 x 16 block positions
 // (pbs_sdd_bf16.h).
-struct SddShapeBf16 {
-    static constexpr int SR = 16, SC = 16, QW = 10, TC = 32, NS = 2, NW = 8;
-};
 struct SddPlan {
-    int tiles_r, tiles_c, nsplit, tokens_per_split;
+    int rows, tiles_r, tiles_c, nsplit, tokens_per_split;   // rows: block rows of a rectangle, 16 or 8
 };
-static SddPlan plan_sdd(long long M, int N, int K) {
-    constexpr int SR = SddShapeBf16::SR, SC = SddShapeBf16::SC, TC = SddShapeBf16::TC;
+static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
+    constexpr int SC = SddBf16Cfg<16>::SC, TC = SddBf16Cfg<16>::TC;
     SddPlan p;
-    p.tiles_r = (N / 32 + SR - 1) / SR;
+    p.rows = rows;
+    p.tiles_r = (N / 32 + rows - 1) / rows;
     p.tiles_c = (K / 32 + SC - 1) / SC;
     const long long tiles = (long long)p.tiles_r * p.tiles_c;
     const long long chunks = (M + TC - 1) / TC;
@@ -613,12 +611,22 @@ static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, 
     return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) +
            passes * (m.launch + (busy > alone ? busy : alone) + std::ceil(tasks / m.resident) * m.round);
 }
-static double rectangle_us(long long M, int N, int K, int nnz) {
-    const SddPlan p = plan_sdd(M, N, K);
+// Launch; per round of workgroups and chunk what a pass costs and what the blocks of a wave cost; reduction of the slices (75 problems, 256 .. 16384
+// tokens, 256 .. 4096 features, densities 0.05 .. 0.95, one in seven with uneven rows: within 11 % for 16 rows and 9 % for 8).
+static double rectangle_us(const SddPlan& p, int nnz) {
+    using C = SddBf16Cfg<16>;
     const double tiles = (double)p.tiles_r * p.tiles_c, blocks = nnz / tiles;
-    const double rounds = std::ceil(tiles * p.nsplit / 256), passes = std::ceil(blocks / (SddShapeBf16::QW * SddShapeBf16::NW));
-    return 15.1 + rounds * (p.tokens_per_split / SddShapeBf16::TC) * (0.4903 * passes + 0.1019 * blocks / 8) +
-           (p.nsplit > 1 ? 3.65 + 1.45 * p.nsplit * nnz / 1000.0 : 0.0);
+    const double rounds = std::ceil(tiles * p.nsplit / 256), passes = std::ceil(blocks / C::QMAX), chunks = p.tokens_per_split / C::TC;
+    const double reduce = p.nsplit * (nnz / 1000.0);
+    if (p.rows == 16) return 9.84 + rounds * (3.57 + chunks * (0.709 * passes + 0.1114 * blocks / 8)) + (p.nsplit > 1 ? 1.20 + 1.15 * reduce : 0.0);
+    return 10.1 + rounds * chunks * (0.738 * passes + 0.0713 * blocks / 8) + (p.nsplit > 1 ? 3.20 + 1.24 * reduce : 0.0);
+}
+// Rectangles of eight block rows read X once per eight rows but need one pass where sixteen rows hold more blocks than the accumulators, and half the
+// slices: 4096 -> 4096, 16384 tokens, density 0.25 198 us with sixteen rows and 265 with eight, 0.5 383 and 339; 768 -> 3072 density 0.5 103 and 77.
+// Of the 75 problems the estimates pick the faster one or one within 2 %.
+static SddPlan plan_sdd(long long M, int N, int K, int nnz) {
+    const SddPlan tall = plan_rectangles(M, N, K, 16), flat = plan_rectangles(M, N, K, 8);
+    return rectangle_us(flat, nnz) < rectangle_us(tall, nnz) ? flat : tall;
 }
 // The kernel and, for the row kernel, the number of token slices of a launch (0: rectangles) and of launches, one behind the
 // other over consecutive ranges of the tokens.
@@ -642,8 +650,10 @@ struct RowChoice {
 static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
     constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
     const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
-    // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 216.
-    if (dtype == PBS_DTYPE_BF16 && bytes > 52e6) return {0, 1, false};
+    // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 198.
+    // (rectangles count the bytes of a chunk in 31 bits)
+    const bool rectangles = dtype == PBS_DTYPE_BF16 && N < (1 << 25) && K < (1 << 25);
+    if (rectangles && bytes > 52e6) return {0, 1, false};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
     RowChoice best{1, 1, false};
@@ -661,7 +671,8 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_
         consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16);
         if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK) consider(ROW_SPLIT);
     }
-    if (dtype == PBS_DTYPE_BF16 && rectangle_us(M, N, K, nnz) < best_us) best.slices = 0;
+    const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
+    if (rectangles && fits && rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
     return best;
 }
 struct BackPlan {
@@ -676,8 +687,10 @@ static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bi
     const RowChoice row = choose_row(dtype, M, N, K, nnz, workspace_limit);
     p.slices = row.slices;
     p.split = row.split;
-    p.rect = plan_sdd(M, N, K);
-    int n = p.rect.nsplit;
+    p.rect = plan_sdd(M, N, K, nnz);
+    // (the workspace of sixteen rows also where eight need less: what an entry point without one refuses does not follow the estimates)
+    const int tall = plan_rectangles(M, N, K, 16).nsplit;
+    int n = tall > p.rect.nsplit ? tall : p.rect.nsplit;
     if (p.slices > 0) {
         const long long chunks = (M + ROW_TC - 1) / ROW_TC, shares = (long long)row.slices * row.passes;
         p.chunks_per_slice = (int)((chunks + shares - 1) / shares);
@@ -768,6 +781,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     a.N = b.N;
     a.K = b.K;
     a.nnz = b.nnz;
+    a.rows = p.rows;
     a.tiles_r = p.tiles_r;
     a.tiles_c = p.tiles_c;
     a.nsplit = p.nsplit;
@@ -778,11 +792,9 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     }
     const long long wgs = (long long)p.tiles_r * p.tiles_c * p.nsplit;
     if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    using S = SddShapeBf16;
-    using C = SddBf16Cfg<S::QW, S::TC, S::NS, S::NW>;
-    static_assert(C::TC == S::TC && C::SR == S::SR && C::SC == S::SC, "plan and kernel must agree");
+    using C = SddBf16Cfg<16>;   // (the buffers of both)
     static std::atomic<uint64_t> done{0};
-    auto kernel = sdd_bf16_kernel<BIAS, S::QW, S::TC, S::NS, S::NW>;
+    auto kernel = sdd_bf16_kernel<BIAS>;
     if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
     hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
     if (int rc = (int)hipGetLastError()) return rc;

@@ -1,48 +1,51 @@
-// bf16 weight gradient on the sparse support, DMA + transposing-read version.
+// bf16 weight gradient on the sparse support.
 //
 //   out[32b + j][i] = sum_t G[t][32r + i] * X[t][32c + j]   for every data block b at (r, c).
 //
-// One workgroup (8 waves) owns a 16 x 16 rectangle of block positions of W and one slice of the
+// One workgroup (8 waves) owns a rectangle of 16 x 16 or 8 x 16 block positions of W and one slice of the
 // tokens.  The blocks present in the rectangle are listed row-major and dealt to the waves in equal
 // contiguous runs (at most QW accumulators per wave; denser rectangles take further passes).
 //
-// Tokens are streamed in chunks of 32.  A chunk is 32 token rows of G (16 block rows = 1 KB per
-// token) and of X (16 block columns = 1 KB per token): each row is one DMA instruction
-// (global_load_lds_dwordx4, contiguous in global memory) into one of NS chunk buffers, so that NS - 1
-// chunks of loads are in flight while one is consumed (the operands come from HBM; a single chunk in
-// flight does not cover that latency).  The rows stay
-// token-major in LDS; both MFMA operands need 8 consecutive tokens per lane, which
-// ds_read_b64_tr_b16 gathers from 4 consecutive token rows.  One such read takes 64 bytes from each of
-// 4 consecutive token rows per half wave; to put those on different banks the 16-byte chunks of token
-// row t are stored at chunk position c ^ ((t & 3) << 2), i.e. shifted by multiples of 64 bytes.
+// Tokens are streamed in chunks of 32.  A chunk is 32 token rows of G (16 or 8 block rows, 1 KB or 512 bytes per
+// token) and of X (16 block columns, 1 KB per token).  Both matrix operands need 8 consecutive tokens of a feature
+// per lane, the rows hold consecutive features of a token.  So a lane loads the same eight features of eight token
+// rows into registers, turns them there (a byte permutation per pair of values) and writes them to one of two chunk
+// buffers as the operands themselves: a wave reads an operand with two ds_read_b128 of 1 KB each, at one address that an
+// exclusive or makes from the block's place.  The loads are a chunk ahead of their writes, in two groups of four rows, so the texture path
+// and the LDS's writes are busy in turn through the whole chunk.  Tokens past the slice's end are zeros by the loads' own
+// bounds check.
+//
+// What it replaced copied the rows to the LDS as they are (one DMA instruction each) and read them with ds_read_b64_tr_b16, twice the LDS
+// instructions at two thirds of their rate, in a loop of 60 instructions per block (12 now: no branch around a copied operand, no address
+// arithmetic).  4096 -> 4096, 16384 tokens, with the reduction: density 0.25 216 -> 198 us, 0.5 (8 rows now) 428 -> 339; 768 -> 3072 density 0.5 112 -> 77;
+// 2048 -> 2048 density 0.5 146 -> 105.  Of a chunk's 2500 cycles (16 rows, density 0.25) the matrix cores have 1024, the LDS 1300, the texture path
+// 1450; the phases of the two waves of a SIMD overlap in part.  The chip is at its power limit (1.9 GHz): a build with 6 % fewer cycles took
+// the same time.  Tried and not faster: the upper four waves two slots behind the lower four (210 us; 188 against 134 with few blocks: the waves no longer
+// read a row of memory together), two barriers in the middle of a chunk instead of one at its start (212), eight rows of loads in one group
+// (201), token-major rows through registers (228).
 //
 // The bias gradient (the sums of G's columns) comes out of the G panels in LDS: the rectangles of a band share the band's
-// 16 block rows among themselves.  4096 -> 4096 density 0.25, 16384 tokens: 216 us without, 222 with it, a reduction of its own
+// block rows among themselves.  4096 -> 4096 density 0.25, 16384 tokens: 3 us; a reduction of its own
 // over G took 43 (the 134 MB of G once more).
 //
-// Consecutive blocks of a wave mostly share their block row, so the G fragment is reloaded only
-// when the row changes.  Tokens past the end are zero rows written by the waves themselves.
+// Consecutive blocks of a wave mostly share their block row, so the G operand is reloaded only when the row changes.
 #pragma once
 #include "pbs_common.h"
 #include "pbs_sdd.h"
 
 namespace pbs {
 
-template <int QW, int TC_, int NS_, int NW_ = 8>
+template <int SR_>
 struct SddBf16Cfg {
-    static constexpr int SR = 16, SC = 16, NW = NW_, NT = NW * 64;
-    static constexpr int TC = TC_;                           // tokens per chunk (16 or 32)
-    static constexpr int NS = NS_;                           // chunk buffers: NS - 1 chunks of loads in flight
-    static constexpr int ROW_BYTES = 1024;                   // one token row of a panel: 16 blocks x 32 x 2 B
-    static constexpr int PANEL_BYTES = TC * ROW_BYTES;
-    static constexpr int STAGE_BYTES = 2 * PANEL_BYTES;      // G panel, then X panel
+    static constexpr int SR = SR_, SC = 16, NW = 8, NT = NW * 64, QW = 9;
+    static constexpr int TC = 32;                            // tokens per chunk
+    static constexpr int BLOCK_BYTES = TC * 64;              // a block row or column of a chunk
+    static constexpr int X_PANEL = 32768, STAGE = 65536;     // offset of the X panel in a buffer, of the second buffer (powers of two: added by xor)
     static constexpr int LIST_MAX = SR * SC;
     static constexpr int QMAX = QW * NW;
-    static constexpr int LDS_BYTES = NS * STAGE_BYTES + LIST_MAX * 4 + LIST_MAX * 2 + (2 * SR + SC / 2 + 4) * 4;
-    static constexpr int ROWS_PER_WAVE = TC / NW;            // token rows of each panel a wave copies per chunk
-    static_assert(TC_ == 16 || TC_ == 32, "one or two 16-token matrix steps per chunk");
-    static_assert(NS_ >= 2 && NS_ <= 4, "chunk buffers");
-    static_assert(QW >= ROWS_PER_WAVE, "a wave issues its token rows between its block products");
+    static constexpr int TABLE_BYTES = LIST_MAX * 4 + LIST_MAX * 2 + (2 * SR + SC / 2 + 4) * 4;
+    static constexpr int LDS_BYTES = 2 * STAGE + TABLE_BYTES;
+    static_assert(SR == 16 || SR == 8, "a G panel of 32 or 16 KB for four waves");
 };
 
 // The rectangle's rows, columns and block list, built by all threads of the workgroup (NT threads, of
@@ -52,17 +55,17 @@ struct SddBf16Cfg {
 // W in each row place or -1, s_gu[SC / 2] = column unit (pair of block columns) in each place or -1.
 constexpr int SDD_BF16_EMAX = 8192, SDD_BF16_UMAX = 1024;
 constexpr int SDD_BF16_PROLOGUE_BYTES = (2 * 16 + 1 + 2 * SDD_BF16_EMAX + 2 * SDD_BF16_UMAX + 2 * SDD_BALANCE_MAX_ROWS + 3) * 4;
-template <int NT>
+template <int NT, int SR, typename Known>
 static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int tile, unsigned char* smem, int* s_blk,
-                                                         unsigned short* s_pos, int* s_rowoff, int* s_rowid, int* s_gu) {
-    constexpr int SR = 16, SC = 16, NW = 8;
+                                                         unsigned short* s_pos, int* s_rowoff, int* s_rowid, int* s_gu, Known&& known) {
+    constexpr int SC = 16, NW = 8;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c0 = (tile % a.tiles_c) * SC;
     const int nblk_r = a.N / 32;
     // ---- which rows and columns of W this rectangle covers, and the list of its blocks (row-major) ----
-    // Rows: the band's 16 block rows (sdd_band_rows).  Columns: normally the band's columns c0 .. c0+15.
+    // Rows: the band's SR block rows (sdd_band_rows).  Columns: normally the band's columns c0 .. c0+15.
     // When the band's entries fit in LDS the columns of the band are instead dealt to the band's
     // rectangles by block count, in units of two adjacent columns (one 128-byte piece of an X row):
     // the units are ranked by their number of blocks in this band and handed out in serpentine order.
@@ -125,7 +128,7 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
             s_eblk[i] = e.y;
         }
         if (dealt)
-            for (int u = tid; u < nunits; u += NT) s_cnt[u] = 0;
+            for (int u = tid; u < nunits; u += NT) s_cnt[u] = s_ug[u] = 0;
         __syncthreads();
         if (dealt) {
             for (int i = tid; i < nent; i += NT) {
@@ -133,13 +136,21 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
                 if (c >= 0 && c < nblk_c) atomicAdd(&s_cnt[c >> 1], 1);
             }
             __syncthreads();
-            for (int u = tid; u < nunits; u += NT) {
-                const int n = s_cnt[u];
+            // (the units that precede a unit, counted by several threads)
+            const int parts = nunits < NT ? NT / nunits : 1, part = (nunits + parts - 1) / parts;
+            for (int i = tid; i < parts * nunits; i += NT) {
+                const int u = i % nunits, n = s_cnt[u], o0 = i / nunits * part, o1 = o0 + part < nunits ? o0 + part : nunits;
                 int rank = 0;
-                for (int o = 0; o < nunits; ++o) {
+#pragma unroll 4
+                for (int o = o0; o < o1; ++o) {
                     const int m = s_cnt[o];
                     rank += (m > n || (m == n && o < u)) ? 1 : 0;
                 }
+                if (rank) atomicAdd(&s_ug[u], rank);
+            }
+            __syncthreads();
+            for (int u = tid; u < nunits; u += NT) {
+                const int rank = s_ug[u];
                 const int place = rank / a.tiles_c;   // < SC / 2: there are at most 8 units per rectangle
                 int gsel = rank % a.tiles_c;
                 if (place & 1) gsel = a.tiles_c - 1 - gsel;
@@ -151,6 +162,7 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
             s_gu[tid] = u < nunits ? u : -1;
         }
         __syncthreads();
+        known();
         // rows 2*wave and 2*wave + 1: first count this rectangle's blocks, then (below) place them
         auto mine_of = [&](int c) -> int {   // place (0..15) of block column c in this rectangle, or -1
             if (c < 0 || c >= nblk_c) return -1;
@@ -174,6 +186,8 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
             const int u = grp * (SC / 2) + tid;
             s_gu[tid] = u < nunits ? u : -1;
         }
+        __syncthreads();
+        known();
         if (tid < SR) {
             const int r = s_rowid[tid];
             if (r >= 0) {
@@ -240,20 +254,17 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
     __syncthreads();
 }
 
-// BIAS: with the bias gradient (bias_out given).  The build without it spares layers without a bias the bookkeeping of the sums (110
-// spilled scalar registers instead of 69): with the reduction, 4096 -> 4096 at 16384 tokens density 0.25 209.7 -> 206.8 us, 0.5
-// 391 -> 380; 2048 -> 2048 density 0.25 79.0 -> 77.0.
-template <bool BIAS, int QW, int TC_, int NS_, int NW_ = 8>
-__global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
-    using C = SddBf16Cfg<QW, TC_, NS_, NW_>;
-    constexpr int NS = C::NS;
-    constexpr int SR = C::SR, NW = C::NW, TC = C::TC;
+// BIAS: with the bias gradient (bias_out given).  The build without it spares layers without a bias the bookkeeping of the sums (18
+// spilled scalar registers instead of none).
+template <bool BIAS, int SR>
+static __device__ __forceinline__ void sdd_rectangle(const SddArgs& a) {
+    using C = SddBf16Cfg<SR>;
+    constexpr int NW = C::NW, TC = C::TC, QW = C::QW;
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    int* s_blk = reinterpret_cast<int*>(smem + NS * C::STAGE_BYTES);                  // [LIST_MAX] data block
+    int* s_blk = reinterpret_cast<int*>(smem + 2 * C::STAGE);                       // [LIST_MAX] data block
     unsigned short* s_pos = reinterpret_cast<unsigned short*>(s_blk + C::LIST_MAX);  // [LIST_MAX] (rl << 8) | cl
     int* s_rowoff = reinterpret_cast<int*>(s_pos + C::LIST_MAX);                     // [SR + 1]
-    const unsigned lds0 = (unsigned)(uintptr_t)smem;
 
     const int ntiles = a.tiles_r * a.tiles_c;
     const int wg = xcd_tile_id(blockIdx.x, ntiles * a.nsplit);
@@ -269,97 +280,95 @@ __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
     // ---- which rows and columns of W this rectangle covers, and the list of its blocks (row-major) ----
     int* s_rowid = s_rowoff + SR + 2;   // [SR] block row of W in each place of this rectangle's band, or -1
     int* s_gu = s_rowid + SR;           // [SC / 2] column unit in each place of this rectangle, or -1
-    static_assert(SDD_BF16_PROLOGUE_BYTES <= NS * C::STAGE_BYTES, "scratch fits in the chunk buffers");
+    static_assert(SDD_BF16_PROLOGUE_BYTES <= 2 * C::STAGE, "scratch fits in the chunk buffers");
     const int nblk_c = a.K / 32;
-    sdd_bf16_prologue<C::NT>(a, tile, smem, s_blk, s_pos, s_rowoff, s_rowid, s_gu);
+    const int t_begin = __builtin_amdgcn_readfirstlane(sp * a.tokens_per_split);
+    const int t_end = t_begin + a.tokens_per_split < a.M ? t_begin + a.tokens_per_split : a.M;
+    const int nchunks = t_begin < t_end ? (t_end - t_begin + TC - 1) / TC : 0;
+
+    // ---- this wave's share of a chunk: the 16 bytes (eight features) at chunk position `pc` of eight token rows of G or of X in every
+    //      lane, transposed in registers to eight tokens of each feature ----
+    // Waves 0 to 3 copy X, a group of eight tokens each; the others G: with SR = 16 a group as well, with SR = 8 half of two groups.
+    const bool of_g = wave >= NW / 2, whole = SR == 16 || !of_g;
+    constexpr int G_LANES = SR * 4;
+    const int pc = of_g ? lane % G_LANES : lane, place = pc >> 2;
+    const int tg = SR == 16 || !of_g ? wave & 3 : (wave & 2) + lane / G_LANES;   // group of eight tokens
+    const unsigned row_bytes = (unsigned)(of_g ? a.N : a.K) * 2;
+    // Four rows at a time: in every other pair of places the last four of the eight first, so that the lanes that write together fill
+    // whole 16-byte places of the LDS.
+    const int half = ((place >> 1) ^ (whole ? 0 : wave)) & 1;
+    unsigned voff = (unsigned)(8 * tg + 4 * half) * row_bytes;
+    auto find_source = [&]() {
+        // The 64 bytes of a place come from its block row of W, or block column (two adjacent columns per unit); a place without one
+        // fetches any valid address; nothing reads it.
+        int src;
+        if (of_g) {
+            src = s_rowid[place];
+        } else {
+            const int unit = s_gu[place >> 1];
+            src = unit >= 0 ? unit * 2 + (place & 1) : -1;
+            if (src >= nblk_c) src = -1;
+        }
+        if (src >= 0) voff += (unsigned)(src * 64 + (pc & 3) * 16);
+    };
+    // the chunk being loaded, as a buffer that ends with the slice: a load behind the end gives zeros and reads nothing
+    const unsigned char* ld_base = nullptr;
+    int ld_left = 0, ld_bytes = 0;   // tokens from the chunk being loaded to the end of the slice; bytes of its rows
+    uint4 st[8];
+    auto load_reset = [&]() {
+        ld_base = static_cast<const unsigned char*>(of_g ? a.g : a.x) + (size_t)t_begin * row_bytes;
+        ld_left = t_end - t_begin;
+        ld_bytes = (ld_left < 0 ? 0 : (ld_left < TC ? ld_left : TC)) * row_bytes;
+    };
+    auto load_next = [&]() {
+        ld_base = uniform_ptr(ld_base + (size_t)TC * row_bytes);   // (kept in scalar registers: each load is a loop otherwise)
+        ld_left -= TC;
+        ld_bytes = __builtin_amdgcn_readfirstlane((ld_left < 0 ? 0 : (ld_left < TC ? ld_left : TC)) * row_bytes);
+    };
+    const unsigned second = half ? 0u - 4 * row_bytes : 4 * row_bytes;
+    auto load_row = [&](int k) {   // 0..3: the lane's first four rows, 4..7: the others
+        unsigned step = (k & 3) * row_bytes;
+        asm volatile("" : "+s"(step));   // (the offsets of all rows kept in vector registers spill)
+        st[k] = buffer16(ld_base, k < 4 || whole ? ld_bytes : 0, voff + step + (k < 4 ? 0u : second));   // (no branch: the waits count loads)
+    };
+    // LDS: a block of a panel is its two matrix operands of 16 tokens, 1 KB each: 512 bytes for the first eight tokens, 512 for the
+    // others, 16 per feature.  Bits 4..7 of an address are swizzled by bits of the lane that writes it: the lanes that write together
+    // would otherwise meet in two places of 16 bytes, mod 256.
+    const int write_at = (of_g ? 0 : C::X_PANEL) + place * C::BLOCK_BYTES + (tg >> 1) * 1024 + (tg & 1) * 512 +
+                         (((pc & 3) * 128 + (pc & 3) * 16) ^ (place & 3) << 6) + half * 8;
+    auto write_features = [&](int four, int d, int stage) {   // features 2d and 2d + 1 of the lane's first (0) or other (1) four rows
+        const uint32_t r[4] = {(&st[4 * four].x)[d], (&st[4 * four + 1].x)[d], (&st[4 * four + 2].x)[d], (&st[4 * four + 3].x)[d]};
+        const int at = write_at ^ stage ^ four << 3;
+        *reinterpret_cast<uint2*>(smem + (at ^ (2 * d) << 4)) =
+            make_uint2(__builtin_amdgcn_perm(r[1], r[0], 0x05040100u), __builtin_amdgcn_perm(r[3], r[2], 0x05040100u));
+        *reinterpret_cast<uint2*>(smem + (at ^ (2 * d + 1) << 4)) =
+            make_uint2(__builtin_amdgcn_perm(r[1], r[0], 0x07060302u), __builtin_amdgcn_perm(r[3], r[2], 0x07060302u));
+    };
+
+    // ---- fragment addresses: lane l serves feature l & 31 of the block; lane half h tokens 8h .. 8h + 7 of each 16-token matrix step ----
+    const int read_at = h * 512 + (lrow & 24) * 16 + (((lrow & 7) ^ (lrow >> 3)) << 4);
+
+    auto load_first = [&]() {
+        load_reset();
+#pragma unroll
+        for (int k = 0; k < 8; ++k) load_row(k);
+        load_next();
+    };
+    // (the first loads are on their way while the blocks are listed: with the row counts and ranks above 29000 -> 13500 cycles to the first product)
+    sdd_bf16_prologue<C::NT, SR>(a, tile, smem, s_blk, s_pos, s_rowoff, s_rowid, s_gu, [&]() {
+        find_source();
+        load_first();
+    });
     const int nq = __builtin_amdgcn_readfirstlane(s_rowoff[SR]);
-    // bias gradient: places sum_p0 .. sum_p0 + sum_rows - 1 of the band are this rectangle's.  A thread sums 16 bytes of a token row
-    // (eight features), of every sum_step-th token.
+    // bias gradient: places sum_p0 .. sum_p0 + sum_rows - 1 of the band are this rectangle's.  A thread sums one feature, over every
+    // sum_step-th group of eight tokens.
     const int sum_share = (SR + a.tiles_c - 1) / a.tiles_c, sum_p0 = (tile % a.tiles_c) * sum_share;
     const int sum_rows = !BIAS || sum_p0 >= SR ? 0 : (sum_p0 + sum_share < SR ? sum_share : SR - sum_p0);
     if (nq == 0 && sum_rows == 0) return;
-    const int sum_width = sum_rows > 0 ? 4 * sum_rows : 1, sum_step = C::NT / sum_width < TC ? C::NT / sum_width : TC;
-    const int sum_chunk = 4 * sum_p0 + tid % sum_width, sum_t0 = tid / sum_width;
+    const int sum_width = sum_rows > 0 ? 32 * sum_rows : 1, sum_step = C::NT / sum_width < 4 ? C::NT / sum_width : 4;
+    const int sum_t0 = tid / sum_width, sum_place = sum_p0 + tid % sum_width / 32, sum_f = tid % 32;
     const bool sum_mine = sum_rows > 0 && sum_t0 < sum_step;
-    float sums[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sums[e] = 0.f;
-
-    const int t_begin = sp * a.tokens_per_split;
-    int t_end = t_begin + a.tokens_per_split;
-    if (t_end > a.M) t_end = a.M;
-    const int nchunks = t_begin < t_end ? (t_end - t_begin + TC - 1) / TC : 0;
-
-    // ---- DMA address pattern: this wave copies token rows wave, wave + 8, ... of both panels; the
-    //      chunk swizzle of those rows is the same ((wave & 3) << 2) ----
-    const unsigned char* G = static_cast<const unsigned char*>(a.g);
-    const unsigned char* X = static_cast<const unsigned char*>(a.x);
-    const int pc = lane ^ ((wave & 3) << 2);   // panel chunk fetched by this lane
-    // G: the 64 bytes of place pc / 4 of the band come from that place's block row (a place without a
-    // row fetches any valid address; nothing reads it)
-    const int g_rid = s_rowid[pc >> 2];
-    const unsigned g_voff = g_rid >= 0 ? (unsigned)(g_rid * 64 + (pc & 3) * 16) : 0u;
-    // X: the 64 bytes of place pc / 4 come from that place's block column (two adjacent columns per unit)
-    const int x_unit = s_gu[pc >> 3];
-    const int x_cid = x_unit >= 0 ? x_unit * 2 + ((pc >> 2) & 1) : -1;
-    const unsigned x_voff = (x_cid >= 0 && x_cid < nblk_c) ? (unsigned)(x_cid * 64 + (pc & 3) * 16) : 0u;
-    const size_t g_row_bytes = (size_t)a.N * 2, x_row_bytes = (size_t)a.K * 2;
-
-    // DMA issue state: chunks are issued in order; the addresses of the chunk being issued are kept and
-    // advanced by constant strides (a 64-bit multiply per row and panel cost more scalar instructions per
-    // chunk than all the rest of the chunk's bookkeeping).
-    const size_t g_kstep = (size_t)NW * g_row_bytes, x_kstep = (size_t)NW * x_row_bytes;   // between this wave's rows
-    const size_t g_cstep = (size_t)TC * g_row_bytes, x_cstep = (size_t)TC * x_row_bytes;   // between chunks
-    int iss_t = 0;                       // token of this wave's first row in the chunk being issued
-    unsigned iss_stage = 0;              // LDS address of that row in the chunk's buffer
-    const unsigned char* iss_g = G;      // global address of that row, G panel
-    const unsigned char* iss_x = X;
-    auto issue_reset = [&]() {
-        iss_t = t_begin + wave;
-        iss_stage = lds0 + wave * C::ROW_BYTES;
-        iss_g = uniform_ptr(G + (size_t)iss_t * g_row_bytes);
-        iss_x = uniform_ptr(X + (size_t)iss_t * x_row_bytes);
-    };
-    // token row number k of this wave's ROWS_PER_WAVE, both panels, of the chunk being issued; returns the DMA count
-    auto issue_row = [&](int k) -> int {
-        const int t = iss_t + k * NW;
-        const unsigned stage = iss_stage + k * NW * C::ROW_BYTES;
-        if (t < t_end) {
-            dma16(stage, iss_g + k * g_kstep, g_voff);
-            dma16(stage + C::PANEL_BYTES, iss_x + k * x_kstep, x_voff);
-            return 2;
-        }
-        // tokens past the end contribute nothing
-        unsigned char* p = smem + (stage - lds0) + lane * 16;
-        *reinterpret_cast<uint4*>(p) = make_uint4(0, 0, 0, 0);
-        *reinterpret_cast<uint4*>(p + C::PANEL_BYTES) = make_uint4(0, 0, 0, 0);
-        return 0;
-    };
-    auto issue_next = [&]() {   // the next chunk goes to the next buffer
-        iss_t += TC;
-        iss_g += g_cstep;
-        iss_x += x_cstep;
-        iss_stage += C::STAGE_BYTES;
-        if (iss_stage >= lds0 + NS * C::STAGE_BYTES) iss_stage -= NS * C::STAGE_BYTES;
-    };
-    auto issue_chunk = [&]() -> int {
-        int n = 0;
-#pragma unroll
-        for (int k = 0; k < C::ROWS_PER_WAVE; ++k) n += issue_row(k);
-        issue_next();
-        return n;
-    };
-
-    // ---- per-lane part of the fragment addresses ----
-    // transposing read: within 16 lanes, lane s addresses 4 consecutive features of token row s/4 and
-    // receives, for its own feature, the 4 token rows as 4 consecutive k.  Lane l serves feature
-    // (l & 31) of the block; lane half h serves tokens 8h..8h+7 of each 16-token MFMA step.
-    const int l16 = lane & 15;
-    const int trow = 8 * h + (l16 >> 2);                              // + 16u + 4v
-    const int cb = 2 * ((lane >> 4) & 1) + ((l16 & 3) >> 1);          // 16-byte chunk inside the block's 64 bytes
-    const int xr = ((l16 >> 2) & 3) << 2;                             // swizzle of token row trow (+ multiples of 4)
-    const int lane_const = trow * C::ROW_BYTES + (l16 & 1) * 8;
-    auto frag_off = [&](int blk16) -> int { return lane_const + (((blk16 * 4 + cb) ^ xr) * 16); };
+    float sum = 0.f;
 
     bf16_t* out = static_cast<bf16_t*>(a.out);
     float* part = a.partial ? a.partial + (size_t)sp * ((size_t)a.nnz * 1024 + (BIAS ? a.N : 0)) : nullptr;
@@ -373,15 +382,16 @@ __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
         const int w_lo = q0 + wave * per + (wave < rem ? wave : rem);
         const int w_n = per + (wave < rem ? 1 : 0);
 
-        // per accumulator slot: fragment offsets of its X block (A operand) and G block (B operand)
-        int a_off[QW], b_off[QW], rl_of[QW], blk_of[QW];
+        // per accumulator slot: where its G block and X block are, with the part of x that is theirs, and whether the G block is another
+        // than the slot's before
+        int g_at[QW], x_at[QW];
+        unsigned turns = 1;
 #pragma unroll
         for (int q = 0; q < QW; ++q) {
-            const int pos = q < w_n ? __builtin_amdgcn_readfirstlane((int)s_pos[w_lo + q]) : 0;
-            rl_of[q] = pos >> 8;
-            a_off[q] = C::PANEL_BYTES + frag_off(pos & 255);
-            b_off[q] = frag_off(pos >> 8);
-            blk_of[q] = q < w_n ? __builtin_amdgcn_readfirstlane(s_blk[w_lo + q]) : -1;
+            const int pos = q < w_n ? __builtin_amdgcn_readfirstlane((int)s_pos[w_lo + q]) : 0, r = pos >> 8, c = pos & 255;
+            g_at[q] = r * C::BLOCK_BYTES | (r & 3) << 6;
+            x_at[q] = C::X_PANEL | c * C::BLOCK_BYTES | (c & 3) << 6;
+            if (q > 0 && g_at[q] != g_at[q - 1]) turns |= 1u << q;
         }
 
         f32x16 acc[QW];
@@ -391,118 +401,67 @@ __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
             for (int v = 0; v < 16; ++v) acc[q][v] = 0.f;
 
         constexpr int NU = TC / 16;   // 16-token matrix steps per chunk
-        auto load_frag = [&](uint4 (&f)[NU], const unsigned char* p) {
+        auto load_frag = [&](uint4 (&f)[NU], int at) {
 #pragma unroll
-            for (int u = 0; u < NU; ++u) {
-                const uint2 lo = tr16_b64(p + (16 * u) * C::ROW_BYTES);
-                const uint2 hi = tr16_b64(p + (16 * u + 4) * C::ROW_BYTES);
-                f[u] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-            }
-        };
-        // products of chunk ci, and this wave's share of the DMA of the next chunk to issue (if do_issue): in the lower
-        // four waves one token row of both panels after each of the first blocks, so that the texture path works
-        // while the matrix cores do (issued in one go ahead of the products, the copy instructions hold a wave for as
-        // long as the texture path needs for them, and its products only start after that: what the upper four waves do
-        // on purpose, see below).  Returns the number of DMA instructions issued.
-        auto compute_chunk = [&](int ci, bool do_issue) -> int {
-            const unsigned char* stage = smem + (ci % NS) * C::STAGE_BYTES;
-            int n_dma = 0;
-            // The fragments of block q + 1 are fetched before the products of block q are issued, so that the
-            // LDS round trip of one block runs under the matrix instructions of the one before it (fetched
-            // right before their own products, the eight or so round trips of a chunk added up to twice the
-            // matrix time).  The loop is unrolled: the two fragment sets alternate by name, not by copying.
-            uint4 fa[2][NU], fb[2][NU];
-            if (w_n > 0) {
-                load_frag(fb[0], stage + b_off[0]);
-                load_frag(fa[0], stage + a_off[0]);
-            }
-            // The two waves of a SIMD copy at different times: the upper four waves issue their token rows in one go
-            // ahead of their products (and are held by the texture path meanwhile), the lower four between their
-            // first products, so that a SIMD has one wave computing while the other is held (all eight issuing
-            // between their products stalled in step: 0.246 -> 0.238 ms).
-            const bool early = wave >= NW / 2;
-            if (early && do_issue) {
-#pragma unroll
-                for (int k = 0; k < C::ROWS_PER_WAVE; ++k) n_dma += issue_row(k);
-            }
-            const bool do_issue_between = do_issue && !early;
-#pragma unroll
-            for (int q = 0; q < QW; ++q) {
-                if (q >= w_n && q < C::ROWS_PER_WAVE && do_issue_between) n_dma += issue_row(q);   // fewer blocks than rows to copy
-                if (q < w_n) {
-                    constexpr int cur = 0, nxt = 1;
-                    uint4(&fa_c)[NU] = fa[(q & 1) ? nxt : cur];
-                    uint4(&fb_c)[NU] = fb[(q & 1) ? nxt : cur];
-                    uint4(&fa_n)[NU] = fa[(q & 1) ? cur : nxt];
-                    uint4(&fb_n)[NU] = fb[(q & 1) ? cur : nxt];
-                    if (q + 1 < QW && q + 1 < w_n) {
-                        load_frag(fa_n, stage + a_off[q + 1]);
-                        if (rl_of[q + 1] != rl_of[q]) {
-                            load_frag(fb_n, stage + b_off[q + 1]);
-                        } else {
-#pragma unroll
-                            for (int u = 0; u < NU; ++u) fb_n[u] = fb_c[u];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < NU; ++u)
-                        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa_c[u]),
-                                                                         __builtin_bit_cast(bf16x8, fb_c[u]), acc[q], 0, 0, 0);
-                    if (q < C::ROWS_PER_WAVE && do_issue_between) n_dma += issue_row(q);
-                }
-            }
-            if (do_issue) issue_next();
-            return n_dma;
+            for (int u = 0; u < NU; ++u) f[u] = *reinterpret_cast<const uint4*>(smem + at + u * 1024);
         };
 
-        if (nchunks > 0) {
-            // DMA counts of the chunks in flight, oldest (the one computed next) first
-            int pend[NS];
+        if (q0 > 0) load_first();
 #pragma unroll
-            for (int k = 0; k < NS; ++k) pend[k] = 0;
-            issue_reset();
+        for (int d = 0; d < 8; ++d)
+            if (d < 4 || whole) write_features(d >> 2, d & 3, 0);
 #pragma unroll
-            for (int k = 0; k < NS - 1; ++k)
-                if (k < nchunks) pend[k] = issue_chunk();
-            for (int ci = 0; ci < nchunks; ++ci) {
-                // chunk ci has landed for every wave, and every wave is done reading chunk ci - 1
-                if constexpr (NS == 2) {
-                    drain_barrier();   // with two buffers nothing younger than chunk ci is in flight
-                } else {
-                    int later = 0;
+        for (int k = 0; k < 8; ++k) load_row(k);
+        load_next();
+        for (int ci = 0; ci < nchunks; ++ci) {
+            // chunk ci is in its buffer for every wave, and every wave is done reading chunk ci - 1
+            lds_barrier();
+            const int stage = (ci & 1) * C::STAGE, other = stage ^ C::STAGE;
+            int read = read_at ^ stage;
+            asm volatile("" : "+v"(read));   // (the addresses of all of a wave's blocks kept in vector registers spill)
+            // The X fragment of block q + 1 is fetched before the products of block q are issued, that of G where it changes.  The
+            // loop is unrolled: the two fragment sets alternate by name, not by copying.
+            uint4 fa[2][NU], fb[NU];
+            if (w_n > 0) load_frag(fa[0], read ^ x_at[0]);
 #pragma unroll
-                    for (int k = 1; k < NS; ++k) later += pend[k];
-                    wait_dma_and_barrier(later);
+            for (int q = 0; q < QW; ++q) {
+                if (q < w_n) {
+                    if (turns >> q & 1) load_frag(fb, read ^ g_at[q]);
+                    if (q + 1 < QW) load_frag(fa[(q + 1) & 1], read ^ x_at[q + 1 < QW ? q + 1 : q]);
+#pragma unroll
+                    for (int u = 0; u < NU; ++u)
+                        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[q & 1][u]),
+                                                                         __builtin_bit_cast(bf16x8, fb[u]), acc[q], 0, 0, 0);
                 }
-#pragma unroll
-                for (int k = 0; k + 1 < NS; ++k) pend[k] = pend[k + 1];
-                pend[NS - 1] = 0;
-                // chunk ci + NS - 1 goes into the buffer of chunk ci - 1, which every wave has left
-                pend[NS - 2] = compute_chunk(ci, ci + NS - 1 < nchunks);
-                if (sum_mine && q0 == 0) {
-                    const unsigned char* stage = smem + (ci % NS) * C::STAGE_BYTES;
-                    for (int t = sum_t0; t < TC; t += sum_step) {
-                        const uint4 v = *reinterpret_cast<const uint4*>(stage + t * C::ROW_BYTES + ((sum_chunk ^ ((t & 3) << 2)) * 16));
-                        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            sums[2 * e] += __uint_as_float(w[e] << 16);
-                            sums[2 * e + 1] += __uint_as_float(w[e] & 0xffff0000u);
-                        }
-                    }
+                // this wave's share of chunk ci + 1, loaded during the chunk before, to its buffer; then that of chunk ci + 2 from memory
+                if (q < 2 || ((q == 4 || q == 5) && whole)) {
+                    write_features(q >> 2, (2 * q) & 3, other);
+                    write_features(q >> 2, (2 * q + 1) & 3, other);
+                }
+                if (q == 2 || q == 3 || q == 6 || q == 7) {
+                    load_row((q & 4) + 2 * (q & 1));
+                    load_row((q & 4) + 2 * (q & 1) + 1);
                 }
             }
-            lds_barrier();   // the next pass refills the buffers
+            load_next();
+            if (sum_mine && q0 == 0) {
+                for (int t = sum_t0; t < TC / 8; t += sum_step) {
+                    const int at = sum_place * C::BLOCK_BYTES + (t >> 1) * 1024 + (t & 1) * 512 +
+                                   (((sum_f & 24) * 16 + (((sum_f & 7) ^ (sum_f >> 3)) << 4)) ^ (sum_place & 3) << 6);
+                    const uint4 v = *reinterpret_cast<const uint4*>(smem + stage + at);
+                    auto pair = [](uint32_t w) { return __uint_as_float(w << 16) + __uint_as_float(w & 0xffff0000u); };
+                    sum += (pair(v.x) + pair(v.y)) + (pair(v.z) + pair(v.w));
+                }
+            }
         }
+        lds_barrier();   // the next pass, or the sums of the bias, take the buffers
         if (sum_rows > 0 && q0 == 0) {
-            float* s_sum = reinterpret_cast<float*>(smem);   // [sum_step][sum_width * 8]
-            if (sum_mine)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) s_sum[tid * 8 + e] = sums[e];
+            float* s_sum = reinterpret_cast<float*>(smem);   // [sum_step][sum_width]
+            if (sum_mine) s_sum[tid] = sum;
             lds_barrier();
-            if (tid < sum_width * 8) {
+            if (tid < sum_width) {
                 float v = 0.f;
-                for (int t = 0; t < sum_step; ++t) v += s_sum[t * sum_width * 8 + tid];
+                for (int t = 0; t < sum_step; ++t) v += s_sum[t * sum_width + tid];
                 const int row = s_rowid[sum_p0 + tid / 32];
                 if (row >= 0) {
                     if (part) part[(size_t)a.nnz * 1024 + row * 32 + tid % 32] = v;
@@ -515,10 +474,11 @@ __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
         // ---- store: result row j (X feature), column i (G feature) ----
 #pragma unroll
         for (int q = 0; q < QW; ++q) {
-            if (q < w_n && blk_of[q] >= 0) {
+            const int blk = q < w_n ? __builtin_amdgcn_readfirstlane(s_blk[w_lo + q]) : -1;
+            if (blk >= 0) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
-                    const size_t o = (size_t)blk_of[q] * 1024 + acc_row(v, h) * 32 + lrow;
+                    const size_t o = (size_t)blk * 1024 + acc_row(v, h) * 32 + lrow;
                     // (partial sums are written once and read once, by sdd_reduce_kernel: stored and loaded non-temporally
                     // they leave the operands of the next product in the last-level cache)
                     if (part) __builtin_nontemporal_store(acc[q][v], part + o);
@@ -527,6 +487,12 @@ __global__ __launch_bounds__(NW_ * 64) void sdd_bf16_kernel(SddArgs a) {
             }
         }
     }
+}
+
+template <bool BIAS>
+__global__ __launch_bounds__(512) void sdd_bf16_kernel(SddArgs a) {
+    if (a.rows == 8) sdd_rectangle<BIAS, 8>(a);
+    else sdd_rectangle<BIAS, 16>(a);
 }
 
 }  // namespace pbs
