@@ -600,9 +600,10 @@ static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, 
         double launch, reduce, per_slice, busy, alone, round;
         int resident;   // workgroups per XCD
     };
-    // (ROW_SPLIT: 90 problems of 2^20 tokens x blocks and more, within 12 %, its choices 2.8 % slower than the best on average)
+    // (ROW_SPLIT: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted without
+    // a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
     const Model m = kernel == ROW_F32 ? Model{3.34, 6.57, 0.0, 0.523, 0.058, 2.34, 64}
-                  : kernel == ROW_SPLIT ? Model{7.0, 11.27, -2.643, 0.4487, 0.540, 5.186, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
+                  : kernel == ROW_SPLIT ? Model{7.03, 3.02, 0.0, 0.454, 0.540, 4.5, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
     const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
     const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows;
     const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
