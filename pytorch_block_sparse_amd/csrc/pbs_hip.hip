@@ -590,8 +590,8 @@ static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
     p.tokens_per_split = (int)(chunks_per * TC);
     return p;
 }
-// Estimated time in us, fitted to 60 measured problems (128 .. 4096 features, 64 .. 16384 tokens, densities 0.05 .. 0.75;
-// the choices made by it were 3.5 % slower than the best of all slice counts on average): launch, reduction of the slices,
+// Estimated time in us, fitted to problems of 256 .. 4096 features, 64 .. 16384 tokens, densities 0.05 .. 0.75 at ten slice counts (fp32 80 below 2^22 tokens x
+// blocks, its choices 2.4 % slower than the best on average, 8.9 % by constants from before the tasks were dealt as they are; bf16 85, 2.0 %): launch, reduction of the slices,
 // chunks x blocks of a wave of the slowest workgroup, at the rate of a full chip or, below 32 workgroups per XCD, of
 // a wave alone, and what each round of workgroups on the chip costs besides.
 enum RowKernel { ROW_F32, ROW_SPLIT, ROW_BF16 };   // sdd_row_kernel<float>, sdd_split_kernel, sdd_row_kernel<bf16_t>
@@ -602,12 +602,12 @@ static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, 
     };
     // (ROW_SPLIT: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted without
     // a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
-    const Model m = kernel == ROW_F32 ? Model{3.34, 6.57, 0.0, 0.523, 0.058, 2.34, 64}
+    const Model m = kernel == ROW_F32 ? Model{2.22, 3.75, 0.033, 0.577, 0.608, 2.67, 64}
                   : kernel == ROW_SPLIT ? Model{7.03, 3.02, 0.0, 0.454, 0.540, 4.5, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
     const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
-    const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows;
+    const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
     const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
-    const double tasks = std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices * (double)passes)) * blocks;
+    const double tasks = units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices * (double)passes)) * blocks;
     const double busy = std::ceil(tasks / 32) * wave * m.busy, alone = wave * m.alone;
     return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) +
            passes * (m.launch + (busy > alone ? busy : alone) + std::ceil(tasks / m.resident) * m.round);
