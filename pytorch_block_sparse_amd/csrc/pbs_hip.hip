@@ -460,15 +460,16 @@ static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
     a.M = g.M;
     a.N = g.N;
     a.K = g.K;
-    a.groups = (g.N / 32 + SP_NC - 1) / SP_NC;
-    a.tiles = split_full_tiles(g.M, a.groups);
+    const int groups_even = (g.N / 32 + SP_NC - 1) / SP_NC;   // (the kernel takes up to half as many again where columns are uneven)
+    a.heavy = (int)(2ll * g.nnz / (g.N / 32));
+    a.tiles = split_full_tiles(g.M, groups_even);
     a.low_tiles = g.M > a.tiles * SP_BM ? (g.M - a.tiles * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
     // the 32 workgroups of an XCD work on tile_block token tiles x 32 / tile_block groups: the split with the least to read per k-block
     const double w_bytes = (double)SP_NC * SP_BLOCK_BYTES * g.nnz / ((double)(g.N / 32) * (g.K / 32)), x_bytes = SP_BM * 128.0;
     double least = 0.0;
     a.tile_block = 1;
     for (int t = 1; t <= 32; t *= 2) {
-        const double groups = a.groups < 32 / t ? a.groups : 32 / t, bytes = t * x_bytes + groups * w_bytes;
+        const double groups = groups_even < 32 / t ? groups_even : 32 / t, bytes = t * x_bytes + groups * w_bytes;
         if (groups * t >= 32 || t == 1)
             if (least == 0.0 || bytes < least) {
                 least = bytes;
@@ -476,7 +477,7 @@ static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
             }
     }
     // one workgroup per CU; more where each would have more units than it keeps the heads of
-    const long long units = (long long)(a.tiles + a.low_tiles) * a.groups;
+    const long long units = (long long)(a.tiles + a.low_tiles) * (groups_even + groups_even / 2 + 1);
     long long per_xcd = (units + NUM_XCD - 1) / NUM_XCD + 1;
     if (per_xcd > 32) per_xcd = per_xcd > 32 * (SP_MAX_UNITS - 1) ? per_xcd / (SP_MAX_UNITS - 1) + 1 : 32;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(NUM_XCD * per_xcd)), dim3((SP_NC + SP_NP) * 64), SP_LDS, stream, a);

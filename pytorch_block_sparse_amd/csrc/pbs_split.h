@@ -111,7 +111,7 @@ struct SplitArgs {
     float* out;                   // [M, N] row-major
     int M, N, K;
     int tiles, low_tiles;         // of 64 tokens, and behind them of 32
-    int groups;
+    int heavy;                    // columns of more blocks than this take two waves
     int tile_block;               // units are ordered by blocks of this many token tiles, then groups, then tiles
 };
 
@@ -128,12 +128,31 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KB = g.K >> 5, ncols = g.N >> 5;
 
+    // A column of many more blocks than the others keeps its wave busy when all others are done.  So the columns of more than twice the average are
+    // taken by two waves, 32 tokens of a tile each, in more groups if need be (3072 -> 768 with Zipf rows, 96 blocks of 24 on average, 4096 tokens: 66 -> 54 us
+    // with the launch that splits the blocks).  Splitting more of them, or wherever a sum of rounds and longest stays says so, costs even patterns up to
+    // 40 % (another group is another time that the panels are split).
+    // Place v of the dealing: below 2 * heavy half v % 2 of column v / 2 of the ranking, else column v - heavy.
+    int heavy = 0;
+    {
+        const int4* ranked = reinterpret_cast<const int4*>(g.plan);
+        bool more = true;
+        for (int c0 = 0; more && c0 < ncols; c0 += 64) {   // (the first 64 and no more in even patterns)
+            const int c = c0 + lane;
+            const unsigned long long not_heavy = __ballot(c >= ncols || ranked[c < ncols ? c : 0].z <= g.heavy);
+            more = not_heavy == 0;
+            heavy += more ? 64 : __builtin_ctzll(not_heavy);
+        }
+        heavy = __builtin_amdgcn_readfirstlane(heavy < ncols / 2 ? heavy : ncols / 2);   // (more only where a list holds more entries than there are blocks)
+    }
+    const int groups = (ncols + heavy + SP_NC - 1) / SP_NC;
+
     // The units of this XCD: its share of the tiles x groups, then of the low tiles x groups.  Its workgroups take them in turn, every other round
     // from the other end: who has started with one of the first, which hold the longest columns, does not get the odd one at the end as well.
     const int xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD, peers = gridDim.x / NUM_XCD;
     auto share = [&](int units, int x) __attribute__((always_inline)) { return (int)((long long)units * x / NUM_XCD); };
-    const int full0 = share(g.tiles * g.groups, xcd), n_full = share(g.tiles * g.groups, xcd + 1) - full0;
-    const int low0 = share(g.low_tiles * g.groups, xcd), n_low = share(g.low_tiles * g.groups, xcd + 1) - low0;
+    const int full0 = share(g.tiles * groups, xcd), n_full = share(g.tiles * groups, xcd + 1) - full0;
+    const int low0 = share(g.low_tiles * groups, xcd), n_low = share(g.low_tiles * groups, xcd + 1) - low0;
     const int rounds = (n_full + n_low) / peers;
     const int mine = rounds + ((rounds & 1 ? peers - 1 - local : local) < (n_full + n_low) % peers ? 1 : 0);
     if (mine == 0) return;
@@ -142,7 +161,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         const int w = j * peers + (j & 1 ? peers - 1 - local : local);
         low = w >= n_full;
         const int v = low ? low0 + w - n_full : full0 + w, of = low ? g.low_tiles : g.tiles;
-        const int tb = v / (g.tile_block * g.groups), rem = v - tb * (g.tile_block * g.groups);
+        const int tb = v / (g.tile_block * groups), rem = v - tb * (g.tile_block * groups);
         int tiles = of - tb * g.tile_block;
         tiles = tiles < g.tile_block ? tiles : g.tile_block;
         group = rem / tiles;
@@ -257,7 +276,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     const int r = lane & 31, h = lane >> 5;
     const int band = wave < 4 ? wave : 11 - wave;   // waves w and w + 4 share a SIMD: a long column and a short one
     const int2* const all_entries = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4);
-    // block column of the result, its first entry, its entries, and first token | (1 for a low tile), of this workgroup's units
+    // block column of the result, its first entry, its entries, and first token | (1: the first 32 tokens alone, 2: the second), of this workgroup's units
     struct Head {
         int col, lo, n, row;
     };
@@ -266,10 +285,12 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         int group, row0;
         bool low;
         unit_of(lane, group, row0, low);
-        const int rank = band * g.groups + ((band & 1) ? g.groups - 1 - group : group);
+        const int v = band * groups + ((band & 1) ? groups - 1 - group : group);
+        const int rank = v < 2 * heavy ? v >> 1 : v - heavy;
+        const int tokens = v >= 2 * heavy ? (low ? 1 : 0) : (v & 1) ? 2 : 1;
         int4 head = make_int4(-1, 0, 0, 0);
-        if (rank < ncols) head = reinterpret_cast<const int4*>(g.plan)[rank];
-        head.w = row0 | (low ? 1 : 0);
+        if (rank < ncols && !(low && tokens == 2)) head = reinterpret_cast<const int4*>(g.plan)[rank];
+        head.w = row0 | tokens;
         heads[lane] = head;
     }
     auto head_of = [&](int j) __attribute__((always_inline)) {
@@ -304,7 +325,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     };
     // results of a unit, a token's 16 values per lane: columns 8 q + 4 h + e of token 32 t + r
     auto epilogue = [&](const Head& unit) __attribute__((always_inline)) {
-        const int col = unit.col, row0 = unit.row & ~1;
+        const int col = unit.col, row0 = unit.row & ~3;
         if (col < 0) return;
         const bool failed = gave_up || __builtin_amdgcn_readfirstlane(lds_peek(s_fail)) != 0;
         float b[16];   // (word by word: a bias need not be aligned to more)
@@ -312,7 +333,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         for (int v = 0; v < 16; ++v) b[v] = g.bias ? g.bias[col * 32 + 8 * (v >> 2) + 4 * h + (v & 3)] : 0.f;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            if (t == 1 && (unit.row & 1)) break;
+            if (unit.row & (2 >> t)) continue;
             float off = 0.f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -384,7 +405,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         const int n = unit.n, u0 = j * KB;
         ev2 = window(head_of(j + 2), 0);
         if (n > 0) {
-            const bool low = unit.row & 1;
+            const bool first = unit.row & 1, second = unit.row & 2;
             int kb = __builtin_amdgcn_readlane(ev.x, 0);
             publish(u0 + kb);
             slot = slot_of(u0 + kb);
@@ -405,7 +426,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                 const unsigned char* p0 = x_base + slot * SLOT;
                 const unsigned char* p1 = p0 + x_other;
                 u32x4 x[2][3];
-                auto read = [&](int s) __attribute__((always_inline)) {   // s = 2 * (half of k) + 32 tokens (of a low tile the second are not used)
+                auto read = [&](int s) __attribute__((always_inline)) {   // s = 2 * (half of k) + 32 tokens (not used where the wave has the other 32)
 #pragma unroll
                     for (int i = 0; i < 3; ++i) x[s & 1][i] = *reinterpret_cast<const u32x4*>((s >> 1 ? p1 : p0) + i * PLANE + (s & 1) * 2048);
                 };
@@ -424,7 +445,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                     auto mma = [&](int pw, int px, f32x16& c) __attribute__((always_inline)) {
                         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[s & 1][px]), c, 0, 0, 0);
                     };
-                    if (t == 0 || !low) {
+                    if (t == 0 ? !second : !first) {
                         mma(0, 2, lo[t]);
                         mma(1, 1, lo[t]);
                         mma(2, 0, lo[t]);

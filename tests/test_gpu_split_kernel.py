@@ -58,6 +58,8 @@ CASES = [
     (4096, 4096, 512, 4096),       # low tiles alone
     (256, 32, 1040039, 8),         # one k-block, more units than the heads of one workgroup hold
     (768, 3072, 4096, zipf_positions(24, 96, 576, seed=3)),
+    (800, 3072, 4127, zipf_positions(25, 96, 600, seed=4)),   # columns of two waves in a group more, low tiles
+    (2560, 1600, 1300, [r * 50 + c for r in range(80) for c in range(50) if r < 30 or (r + c) % 10 == 0]),   # as many of them as there can be
     (768, 3072, 4096, [r * 96 + c for r in range(24) for c in range(96) if r % 3 and (r + c) % 2]),   # every third column empty
 ]
 
