@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <mutex>
+#include <tuple>
 
 #include "pbs_common.h"
 #include "pbs_dds16.h"
@@ -23,6 +24,19 @@
 namespace pbs {
 
 static inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Launches a kernel; the call that the triple brackets end in, without the way through the thread's launch configuration and the last error (2.8 us of a
+// launch's host time -> 2.6).  An error is returned and does not stay behind for the next runtime call to report.
+template <typename... P, typename... A>
+static int launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, const A&... args) {
+    std::tuple<P...> values{static_cast<P>(args)...};
+    const hipError_t e = std::apply([&](P&... v) {
+        void* at[] = {&v...};
+        return hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, at, lds, stream);
+    }, values);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return (int)e;
+}
 
 // Zero fill as a kernel (callers may capture the stream into a graph).
 __global__ __launch_bounds__(256) void fill_zero_kernel(uint32_t* p, size_t nwords) {
@@ -146,8 +160,7 @@ static int launch_dds16(const DdsArgs& g, hipStream_t stream) {
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
     const long long grid = 8ll * a.n_groups * ((P + 7) / 8);
     if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::NT), lds, stream, a);
-    return (int)hipGetLastError();
+    return launch(kernel, dim3((unsigned)grid), dim3(C::NT), lds, stream, a);
 }
 
 // ---- bf16 kernel with one block column per wave ----
@@ -223,8 +236,7 @@ static int launch_ddsc(const DdsArgs& g, const void* data_nk, hipStream_t stream
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
     const long long grid = 8ll * a.n_groups * ((c.wg_per_group + 7) / 8);
     if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, a);
-    return (int)hipGetLastError();
+    return launch(kernel, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, a);
 }
 
 // ---- one block column per workgroup ----
@@ -317,8 +329,7 @@ static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
     a.group = fit < 1.0 ? 1 : (fit > a.m_tiles ? a.m_tiles : (int)fit);
     const long long grid = NUM_XCD * (((long long)a.m_tiles + a.xcd_t - 1) / a.xcd_t) * ((cols + NUM_XCD / a.xcd_t - 1) / (NUM_XCD / a.xcd_t));
     if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    hipLaunchKernelGGL((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)grid), dim3(KS * 64), 0, stream, a);
-    return (int)hipGetLastError();
+    return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)grid), dim3(KS * 64), 0, stream, a);
 }
 
 template <typename T, int TRANS>
@@ -383,8 +394,7 @@ static int launch_panel(const DdsArgs& g, int splits, hipStream_t stream) {
     const long long wgs = (long long)((g.M + 16 * PANEL_TT - 1) / (16 * PANEL_TT)) * splits;
     if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), panel_lds(g.K), stream, a);
-    return (int)hipGetLastError();
+    return launch(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), panel_lds(g.K), stream, a);
 }
 
 template <int TRANS, int S>
@@ -395,8 +405,7 @@ static int launch_panel_chunks(const DdsArgs& g, int splits, hipStream_t stream)
     const long long wgs = (long long)((g.M + 16 * PANEL_TT - 1) / (16 * PANEL_TT)) * splits;
     if (wgs > (1ll << 30)) return PBS_ERR_TOO_LARGE;
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), PANEL_CHUNK_LDS, stream, a);
-    return (int)hipGetLastError();
+    return launch(kernel, dim3(xcd_grid((int)wgs)), dim3(PANEL_NW * 64), PANEL_CHUNK_LDS, stream, a);
 }
 
 // ---- fp32 on the bf16 matrix cores ----
@@ -447,9 +456,8 @@ static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
     static std::atomic<uint64_t> done{0};
     auto kernel = split_kernel<TRANS>;
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    hipLaunchKernelGGL(split_blocks_kernel<TRANS>, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream, static_cast<const float*>(g.data),
-                       static_cast<unsigned char*>(workspace), g.nnz);
-    if (int rc = (int)hipGetLastError()) return rc;
+    if (int rc = launch(split_blocks_kernel<TRANS>, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream, static_cast<const float*>(g.data),
+                        static_cast<unsigned char*>(workspace), g.nnz)) return rc;
     SplitArgs a;
     a.a = static_cast<const float*>(g.a);
     a.data = static_cast<const float*>(g.data);
@@ -480,8 +488,7 @@ static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
     const long long units = (long long)(a.tiles + a.low_tiles) * (groups_even + groups_even / 2 + 1);
     long long per_xcd = (units + NUM_XCD - 1) / NUM_XCD + 1;
     if (per_xcd > 32) per_xcd = per_xcd > 32 * (SP_MAX_UNITS - 1) ? per_xcd / (SP_MAX_UNITS - 1) + 1 : 32;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(NUM_XCD * per_xcd)), dim3((SP_NC + SP_NP) * 64), SP_LDS, stream, a);
-    return (int)hipGetLastError();
+    return launch(kernel, dim3((unsigned)(NUM_XCD * per_xcd)), dim3((SP_NC + SP_NP) * 64), SP_LDS, stream, a);
 }
 
 // ---- which kernel runs a product ----
@@ -542,9 +549,8 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
         if (part == PART_COLUMN && (reinterpret_cast<uintptr_t>(g.bias) & 3u) == 0) {   // (it reads the bias in words)
             // the kernel wants every block with k along its rows: as stored for TRANS, a transposed copy otherwise
             if constexpr (TRANS) return launch_ddsc<false>(g, g.data, stream);
-            hipLaunchKernelGGL(transpose_blocks_kernel, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream,
-                               static_cast<const uint16_t*>(g.data), static_cast<uint16_t*>(workspace), g.nnz);
-            if (int rc = (int)hipGetLastError()) return rc;
+            if (int rc = launch(transpose_blocks_kernel, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream,
+                                static_cast<const uint16_t*>(g.data), static_cast<uint16_t*>(workspace), g.nnz)) return rc;
             return launch_ddsc<true>(g, workspace, stream);
         }
         if (part == PART_WIDE) return launch_dds16<TRANS>(g, stream);
@@ -601,9 +607,11 @@ static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, 
         double launch, reduce, per_slice, busy, alone, round;
         int resident;   // workgroups per XCD
     };
+    // (ROW_F32: the fit has 3.75 for the reduction.  It is a launch and an allocation more, 4 us of host time, and a program that waits for the host loses
+    // them: two training steps that move blocks, 768 -> 3072 at 1024 tokens, 281 us without and 287 with it, for 2.5 us less of the GPU each.)
     // (ROW_SPLIT: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted without
     // a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
-    const Model m = kernel == ROW_F32 ? Model{2.22, 3.75, 0.033, 0.577, 0.608, 2.67, 64}
+    const Model m = kernel == ROW_F32 ? Model{2.22, 6.3, 0.033, 0.577, 0.608, 2.67, 64}
                   : kernel == ROW_SPLIT ? Model{7.03, 3.02, 0.0, 0.454, 0.540, 4.5, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
     const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
     const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
@@ -719,19 +727,17 @@ static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int
     int* before = nullptr;
     if (unit_prefix_bytes(N)) {
         before = t + 16 + units * UNIT_INTS;
-        hipLaunchKernelGGL(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, before);
+        if (int rc = launch(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, before)) return rc;
     }
     const UnitArgs a{ptr, idx, nnz, N / 32, K / 32, before, (int)units, t};
-    hipLaunchKernelGGL(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, a);
-    return (int)hipGetLastError();
+    return launch(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, a);
 }
 
 template <typename T>
 static int launch_reduce(const float* partial, const BackArgs& a, int nsplit, hipStream_t stream) {
     const size_t n = (size_t)a.nnz * 1024, total = n + (a.bias_out ? a.N : 0);
-    hipLaunchKernelGGL(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(a.out), n,
-                       static_cast<T*>(a.bias_out), total, nsplit);
-    return (int)hipGetLastError();
+    return launch(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(a.out), n,
+                  static_cast<T*>(a.bias_out), total, nsplit);
 }
 
 template <typename T>
@@ -761,9 +767,8 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     for (int pass = 0; pass < p.passes; ++pass) {
         r.chunk0 = pass * p.slices * p.chunks_per_slice;
         r.add = pass > 0;
-        if (sizeof(T) == 4 && p.split) hipLaunchKernelGGL(sdd_split_kernel, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
-        else hipLaunchKernelGGL(sdd_row_kernel<T>, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r);
-        if (int rc = (int)hipGetLastError()) return rc;
+        const auto kernel = sizeof(T) == 4 && p.split ? sdd_split_kernel : sdd_row_kernel<T>;
+        if (int rc = launch(kernel, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r)) return rc;
     }
     return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;
 }
@@ -798,8 +803,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     static std::atomic<uint64_t> done{0};
     auto kernel = sdd_bf16_kernel<BIAS>;
     if (int rc = raise_lds_limit(kernel, C::LDS_BYTES, done)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a);
-    if (int rc = (int)hipGetLastError()) return rc;
+    if (int rc = launch(kernel, dim3(xcd_grid((int)wgs)), dim3(C::NT), C::LDS_BYTES, stream, a)) return rc;
     return p.nsplit > 1 ? launch_reduce<bf16_t>(a.partial, b, p.nsplit, stream) : PBS_OK;
 }
 
@@ -863,9 +867,8 @@ int pbs_build_indices(const uint8_t* mask, const int64_t* block_ptr, int X, int 
     if ((long long)X * Y > (1ll << 30)) return PBS_ERR_TOO_LARGE;
     if (!mask || !row_start_ends_a || !col_start_ends_b || !status) return PBS_ERR_NULL_POINTER;
     if (nnz > 0 && (!cols_a || !rows_b || !blocks)) return PBS_ERR_NULL_POINTER;
-    hipLaunchKernelGGL(build_indices_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), mask,
-                       block_ptr, X, Y, nnz, cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks, status);
-    return (int)hipGetLastError();
+    return launch(build_indices_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), mask,
+                  block_ptr, X, Y, nnz, cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks, status);
 }
 
 size_t pbs_replace_blocks_workspace_bytes(int X, int Y, int nnz) {
@@ -881,9 +884,8 @@ int pbs_replace_blocks(const int32_t* old_blocks, const int64_t* moves, int n_mo
     if (nnz > 0 && (!old_blocks || !cols_a || !rows_b || !blocks)) return PBS_ERR_NULL_POINTER;
     const size_t need = replace_ws_bytes(X, Y, nnz);
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
-    hipLaunchKernelGGL(replace_blocks_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), old_blocks, moves, n_moves, X,
-                       Y, nnz, cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks, status, static_cast<int*>(workspace));
-    return (int)hipGetLastError();
+    return launch(replace_blocks_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), old_blocks, moves, n_moves, X,
+                  Y, nnz, cols_a, row_start_ends_a, rows_b, col_start_ends_b, blocks, status, static_cast<int*>(workspace));
 }
 
 size_t pbs_validate_indices_workspace_bytes(int nnz) { return nnz < 0 ? 0 : validate_ws_bytes(nnz); }
@@ -896,9 +898,8 @@ int pbs_validate_indices(const int32_t* cols_a, const int32_t* row_start_ends_a,
     if (!row_start_ends_a || !col_start_ends_b || !status || (nnz > 0 && (!cols_a || !rows_b || !blocks))) return PBS_ERR_NULL_POINTER;
     const size_t need = validate_ws_bytes(nnz);
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
-    hipLaunchKernelGGL(validate_indices_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), cols_a, row_start_ends_a,
-                       rows_b, col_start_ends_b, blocks, X, Y, nnz, status, static_cast<int*>(workspace));
-    return (int)hipGetLastError();
+    return launch(validate_indices_kernel, dim3(1), dim3(INDEX_THREADS), 0, static_cast<hipStream_t>(stream), cols_a, row_start_ends_a,
+                  rows_b, col_start_ends_b, blocks, X, Y, nnz, status, static_cast<int*>(workspace));
 }
 
 size_t pbs_blocksparse_matmul_plan_bytes(int n, int k) {
@@ -926,28 +927,23 @@ int pbs_blocksparse_matmul_plan_part(const int32_t* ptr, const int32_t* indices,
     unsigned char* base = static_cast<unsigned char*>(plan);
     if (part & PART_LIST) {
         const ListArgs a{ptr, indices, n / 32, k / 32, nnz, reinterpret_cast<int*>(base)};
-        hipLaunchKernelGGL(list_plan_kernel, dim3(list_plan_grid(n / 32)), dim3(256), 0, s, a);
-        if (int rc = (int)hipGetLastError()) return rc;
+        if (int rc = launch(list_plan_kernel, dim3(list_plan_grid(n / 32)), dim3(256), 0, s, a)) return rc;
     }
     if ((part & PART_WIDE) && wide_plan_bytes(n, k)) {
         const int groups16 = (n / 32 + D16_NB - 1) / D16_NB;
         int* wide = reinterpret_cast<int*>(base + list_area_bytes(n, k));
-        hipLaunchKernelGGL(dds16_plan_kernel, dim3(groups16), dim3(256), 0, s, ptr, indices, n / 32, k / 32, nnz, wide,
-                           (int)dds16_plan_group_ints(k / 32), wide + (size_t)groups16 * dds16_plan_group_ints(k / 32));
-        if (int rc = (int)hipGetLastError()) return rc;
+        if (int rc = launch(dds16_plan_kernel, dim3(groups16), dim3(256), 0, s, ptr, indices, n / 32, k / 32, nnz, wide,
+                            (int)dds16_plan_group_ints(k / 32), wide + (size_t)groups16 * dds16_plan_group_ints(k / 32))) return rc;
     }
     if ((part & PART_COLUMN) && column_plan_bytes(n, k)) {
         const int groups = column_groups(n);
         const int group_ints = (int)ddsc_plan_group_ints(k / 32);
         int* cols = reinterpret_cast<int*>(base + column_plan_offset(n, k));
         int* lists = reinterpret_cast<int*>(base + column_plan_offset(n, k) + column_table_bytes(n));
-        hipLaunchKernelGGL(ddsc_cols_kernel, dim3(1), dim3(256), 0, s, ptr, n / 32, groups, nnz, cols);
-        if (int rc = (int)hipGetLastError()) return rc;
-        hipLaunchKernelGGL(ddsc_plan_kernel, dim3(groups), dim3(256), 0, s, ptr, indices, cols, n / 32, k / 32, nnz, lists,
-                           group_ints, lists + (size_t)groups * group_ints);
-        if (int rc = (int)hipGetLastError()) return rc;
-        hipLaunchKernelGGL(ddsc_plan_ahead_kernel, dim3(groups), dim3(64), 0, s, k / 32, lists, group_ints);
-        if (int rc = (int)hipGetLastError()) return rc;
+        if (int rc = launch(ddsc_cols_kernel, dim3(1), dim3(256), 0, s, ptr, n / 32, groups, nnz, cols)) return rc;
+        if (int rc = launch(ddsc_plan_kernel, dim3(groups), dim3(256), 0, s, ptr, indices, cols, n / 32, k / 32, nnz, lists,
+                            group_ints, lists + (size_t)groups * group_ints)) return rc;
+        if (int rc = launch(ddsc_plan_ahead_kernel, dim3(groups), dim3(64), 0, s, k / 32, lists, group_ints)) return rc;
     }
     return PBS_OK;
 }
@@ -964,9 +960,8 @@ int pbs_blocksparse_matmul_plan(const int32_t* ptr, const int32_t* indices, int 
         t.groups[wi] = (int)width_groups(n, wi);
     }
     const int places = t.groups[PLAN_NWIDTHS - 1] * PLAN_PLACES;
-    hipLaunchKernelGGL(slot_tables_kernel, dim3((unsigned)(places < 16384 ? (places + 255) / 256 : 64)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), t, n / 32);
-    return (int)hipGetLastError();
+    return launch(slot_tables_kernel, dim3((unsigned)(places < 16384 ? (places + 255) / 256 : 64)), dim3(256), 0,
+                  static_cast<hipStream_t>(stream), t, n / 32);
 }
 
 int pbs_blocksparse_matmul_part(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace) {
@@ -1071,8 +1066,7 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
     const long long bound = unit_bound(out_features, nnz);
     a.units = UnitArgs{row_start_ends_a, cols_a, nnz, N, K, nullptr, (int)bound, with_units ? static_cast<int*>(units) : nullptr};
     const long long grid = a.grid[0] + a.grid[1] + (with_units ? (bound + 255) / 256 : 0);
-    hipLaunchKernelGGL(derive_kernel, dim3((unsigned)grid), dim3(256), 0, s, a);
-    if (int rc = (int)hipGetLastError()) return rc;
+    if (int rc = launch(derive_kernel, dim3((unsigned)grid), dim3(256), 0, s, a)) return rc;
     return units && !with_units ? build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, units, s) : PBS_OK;
 }
 
@@ -1090,8 +1084,7 @@ static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, s
         const size_t esz = dtype == PBS_DTYPE_F32 ? 4 : 2;
         auto zero = [&](void* p, size_t values) {
             const size_t nwords = values * esz / 4;
-            hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s, static_cast<uint32_t*>(p), nwords);
-            return (int)hipGetLastError();
+            return launch(fill_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s, static_cast<uint32_t*>(p), nwords);
         };
         if (a.nnz > 0)
             if (int rc = zero(a.out, (size_t)a.nnz * 1024)) return rc;
@@ -1175,20 +1168,17 @@ int pbs_blocksparse_matmul_back_blocks(const void* dense_a, int a_row_major, con
     int32_t* cols_a = reinterpret_cast<int32_t*>(ws + l.cols_a);
     int* owner = reinterpret_cast<int*>(ws + l.owner);
     const long long positions = (long long)X * Y;
-    hipLaunchKernelGGL(blocks_owner_clear_kernel, dim3((unsigned)((positions + 255) / 256)), dim3(256), 0, s, owner, positions);
-    hipLaunchKernelGGL(blocks_owner_kernel, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, s, blocks, nnz, X, Y, owner);
-    hipLaunchKernelGGL(csr_from_owner_kernel, dim3(1), dim3(INDEX_THREADS), 0, s, owner, X, Y, cols_a, row_ptr);
-    if (int rc = (int)hipGetLastError()) return rc;
+    if (int rc = launch(blocks_owner_clear_kernel, dim3((unsigned)((positions + 255) / 256)), dim3(256), 0, s, owner, positions)) return rc;
+    if (int rc = launch(blocks_owner_kernel, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, s, blocks, nnz, X, Y, owner)) return rc;
+    if (int rc = launch(csr_from_owner_kernel, dim3(1), dim3(INDEX_THREADS), 0, s, owner, X, Y, cols_a, row_ptr)) return rc;
     // an operand given with the tokens along its rows' direction ([features, tokens]) is brought to [tokens, features]
     auto to_row_major = [&](const void* src, size_t off, int features) -> int {
         const dim3 grid((unsigned)((tokens + 31) / 32), (unsigned)((features + 31) / 32));
         if (dtype == PBS_DTYPE_F32)
-            hipLaunchKernelGGL(transpose_dense_kernel<uint32_t>, grid, dim3(256), 0, s, static_cast<const uint32_t*>(src),
-                               reinterpret_cast<uint32_t*>(ws + off), (long long)features, (long long)tokens);
-        else
-            hipLaunchKernelGGL(transpose_dense_kernel<uint16_t>, grid, dim3(256), 0, s, static_cast<const uint16_t*>(src),
-                               reinterpret_cast<uint16_t*>(ws + off), (long long)features, (long long)tokens);
-        return (int)hipGetLastError();
+            return launch(transpose_dense_kernel<uint32_t>, grid, dim3(256), 0, s, static_cast<const uint32_t*>(src),
+                          reinterpret_cast<uint32_t*>(ws + off), (long long)features, (long long)tokens);
+        return launch(transpose_dense_kernel<uint16_t>, grid, dim3(256), 0, s, static_cast<const uint16_t*>(src),
+                      reinterpret_cast<uint16_t*>(ws + off), (long long)features, (long long)tokens);
     };
     const void* a = dense_a;
     const void* b = dense_b;
