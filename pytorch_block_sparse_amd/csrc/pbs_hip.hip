@@ -649,9 +649,9 @@ static SddPlan plan_sdd(long long M, int N, int K, int nnz) {
 // 4 x 2 1199 against 1222, 0.5 2 x 4 2258 against 2347, 1 1 x 8 4131 against 4297; 65536 tokens, density 1 1 x 33 16538 against
 // 16998; 8192 -> 8192, 16384 tokens, density 0.25 1 x 16 4805 against 5211, 0.5 9264 against 10299.
 constexpr size_t ROW_WORKSPACE_BYTES = 64u << 20;
-// fp32 on the bf16 matrix cores (sdd_split_kernel) from 2^22 tokens x blocks where its estimate is the smaller one: of those 30 of the problems it
-// is 1.1 times faster on average, 1.0 to 1.29 and twice 0.95; at 2^21 as often slower as faster (768 x 3072 with Zipf rows, 4096 tokens 52 -> 48 us,
-// 4926 tokens 4064 -> 352 48 -> 58), at 2^20 mostly slower: a wave starts by splitting its first pieces, and the code is larger.
+// fp32 on the bf16 matrix cores (sdd_split_kernel) from 2^22 tokens x blocks where its estimate is the smaller one (2048 -> 2048 density 0.25, 4096 tokens
+// 98 -> 86 us, 4096 -> 4096 density 0.25, 16384 tokens 1267 -> 1091).  Between 2^21 and 2^22 its time is 0.7 to 1.24 of the fp32 kernel's and the estimates do not tell which
+// (25 problems, 0.95 on average; 3072 -> 768 with Zipf rows 52 and 48 us, 2016 -> 1408 at 2779 tokens 51 and 63), below 2^21 the same on average.
 constexpr long long SPLIT_BACK_WORK = 1ll << 22;
 struct RowChoice {
     int slices, passes;
