@@ -376,10 +376,15 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         }
     };
 
-    // the entries i0 .. i0 + 63 of a unit's column, one per lane (of a column without blocks, or behind the last unit: anything)
+    // the entries i0 .. i0 + 63 of a unit's column, one per lane.  Of a column without blocks, or behind the last unit, the first k-block and block 0: both
+    // exist, no step of the ring that is still needed is given up for them, and nothing is read of the plan, whose entries no list may have written.
     auto window = [&](const Head& unit, int i0) __attribute__((always_inline)) {
-        const int l = i0 + lane;
-        return all_entries[unit.n > 0 ? unit.lo + (l < unit.n ? l : unit.n - 1) : 0];
+        int2 e = make_int2(0, 0);
+        if (unit.n > 0) {
+            const int l = i0 + lane;
+            e = all_entries[unit.lo + (l < unit.n ? l : unit.n - 1)];
+        }
+        return e;
     };
     auto arrived = [](int2& w) __attribute__((always_inline)) { asm volatile("" : "+v"(w.x), "+v"(w.y)); };
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));

@@ -91,3 +91,60 @@ def test_weight_gradient_of_entries_outside_the_range(cuda, dtype):
             r = e // per_row
             want[b] = x[:, 32 * c:32 * c + 32].double().cpu().t() @ dy[:, 32 * r:32 * r + 32].double().cpu()
     assert (got.double().cpu() - want).norm() / want.norm() < (1e-5 if dtype == F32 else 1e-2)
+
+
+def _split_product(a, data, ptr, entries, n, k, transpose):
+    """The product through the entry that takes a workspace, with a plan in memory that holds something else where no list has an entry."""
+    lib, cuda = native.load(), a.device
+    tokens, nnz = a.shape[0], len(entries)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ptr, entries = (torch.from_numpy(np.asarray(v).astype(np.int32)).to(cuda) for v in (ptr, entries))
+    plan = torch.full((lib.pbs_blocksparse_matmul_plan_part_bytes(n, k),), 0x7f, dtype=torch.uint8, device=cuda)
+    assert lib.pbs_blocksparse_matmul_plan_part(p(ptr), p(entries), n, k, nnz, 1, p(plan), plan.numel(), stream) == 0
+    code = native.DTYPE_CODES[F32]
+    size = lib.pbs_blocksparse_matmul_parts_bytes(tokens, n, k, nnz, int(transpose), code)
+    name = native.matmul_kernel_name(tokens, n, k, nnz, transpose, F32, True)
+    print(name, n, k, tokens, nnz, transpose, flush=True)
+    assert name == "split_kernel" and size > 0
+    ws = torch.empty(size, dtype=torch.uint8, device=cuda)
+    y = torch.full((tokens, n), float("nan"), device=cuda)
+    assert lib.pbs_blocksparse_matmul_ws(p(a), p(data), p(plan), None, p(y), tokens, n, k, nnz, int(transpose), code, p(ws), size, stream) == 0
+    return y
+
+
+@pytest.mark.parametrize("n, k, tokens, per_column, transpose", [(768, 3072, 4096, 48, True), (2048, 4384, 1100, 70, False)])
+def test_larger_fp32_products(cuda, n, k, tokens, per_column, transpose):
+    torch.manual_seed(n)
+    a, data = torch.randn(tokens, k, device=cuda), torch.randn(n // 32 * per_column * 32, 32, device=cuda)
+    out = [_split_product(a, data, ptr, entries, n, k, transpose) for ptr, entries in _lists(n, k, per_column, True, 7)]
+    assert torch.isfinite(out[1]).all() and torch.equal(*out)
+
+
+@pytest.mark.parametrize("first, counts", [
+    (1152, [0] * 24),                # no entries
+    (0, [0] * 24),
+    (1104, [0] * 23 + [48]),         # the last column's alone
+    (576, [0] * 12 + [48] * 12),
+    (336, [0, 48, 0] * 8),
+    (3, [90, 0, 0, 1, 0, 0, 0, 2, 0, 64, 65, 0] * 2),
+])
+def test_larger_fp32_products_of_short_lists(cuda, first, counts):
+    """Pointer arrays that start above 0 leave entries of the plan unwritten: columns without entries must not read one."""
+    n, k, tokens, nnz = 768, 3072, 4096, 1152
+    rng = np.random.RandomState(3)
+    ptr = np.cumsum([first] + counts)
+    entries = np.zeros((nnz, 2), dtype=np.int64)
+    entries[first:ptr[-1], 1] = rng.permutation(nnz)[:sum(counts)]
+    for c, count in enumerate(counts):
+        entries[ptr[c]:ptr[c + 1], 0] = np.sort(rng.permutation(k // 32)[:count])
+    torch.manual_seed(1)
+    a, data = torch.randn(tokens, k, device=cuda), torch.randn(nnz * 32, 32, device=cuda)
+    got = _split_product(a, data, ptr, entries, n, k, True)
+    want = torch.zeros(tokens, n, dtype=torch.float64, device=cuda)
+    for c in range(n // 32):
+        for x, b in entries[ptr[c]:ptr[c + 1]]:
+            want[:, 32 * c:32 * c + 32] += a[:, 32 * x:32 * x + 32].double() @ data[32 * b:32 * b + 32].double()
+    # as in tests/test_gpu_split_kernel.py: four roundings per block of the fullest column, and that of the result
+    limit = 0.35 * 2.0 ** -24 * (4 * max(counts)) ** 0.5 + 2.0 ** -25
+    assert (got.double() - want).norm() <= limit * want.norm()
