@@ -1,12 +1,20 @@
 // dense x block-sparse -> dense in fp32 on the bf16 matrix cores (forward and input gradient of larger problems).
 //
 // The fp32 matrix instruction multiplies at a sixteenth of the bf16 rate.  A float is the sum of three bfloat16 values without a rest
-// (24 bits of significand in three times 8), so a product of two floats is nine products of bfloat16 values, of which the three
-// smallest are below 2^-25 of the whole and are left out: six bf16 instructions do the work of an fp32 instruction that takes
-// 16 times as long.  Sums are float32 as before; the five small products have an accumulator of their own, so the large sums are
-// rounded once per 8 terms (what the measured errors say an instruction adds at a time).  Distance from float64 in units of 1e-7, here and in
-// the four chains of fp32 instructions of stream_kernel: 768 -> 3072 density 0.5 1.1 and 2.6, 3072 -> 768 2.3 and 3.6, 4096 -> 4096 density 0.25
-// 1.9 and 2.9.
+// (24 bits of significand in three times 8), so a product of two floats is nine products of bfloat16 values.  The three smallest, each
+// below 2^-25 of the whole and together at most 2^-24 of it, are left out: six bf16 instructions do the work of an fp32 instruction that takes
+// 16 times as long (G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision
+// computations", ARITH 2019).
+//
+// Sums are float32.  A block's twelve products (two halves of k) are summed by themselves, the small ones first, and join the column's total with
+// one rounding per block.  The matrix instruction cuts what is far below its largest term off, towards minus infinity (a mean error of -3e-8 of the
+// results' size at 48 blocks), so every other k-block is multiplied with the dense operand's sign changed and subtracted (mean error below 1e-9).
+// Distance from float64 in units of 1e-7, in the chains of fp32 instructions of stream_kernel, in one chain over the column here, and as it is:
+//   768 -> 3072 density 0.5   2.6  1.1  0.8      3072 -> 768 density 0.5   3.6  2.3  1.4      4096 -> 4096 density 0.25   2.9  1.9  1.1
+//   the same layers with operands between 0 and 1   1.5  1.1  0.6      1.5  2.1  1.1      1.3  1.7  0.9
+// and of products of a single value, which no sum averages, 0.25 and 0.35 (at most 0.6 and 1.6).
+// The sums by block cost 1 to 4 % of a product against the one chain (32 vector instructions per block and wave, in a kernel bound by power); blocks in
+// pairs would cost half of that, but leave the mean error: a pair has no sign of its own in panels that eight columns share.
 //
 // Range.  Operands are scaled by 2^30 when they are split, so that the third part of the smallest normal float is still a
 // normal bfloat16; the result is scaled back.  Whatever does not fit (an operand above 2^97, a result above 2^67, infinities and
@@ -18,8 +26,8 @@
 // many users: the blocks by a launch of their own (split_blocks_kernel, into a workspace, in the order the fragments are loaded in), the
 // dense operand once per 8 block columns, by waves that do nothing else.  What is left is mostly power: the matrix cores are busy 0.52 to 0.56 of
 // the time at 1.56 GHz (with zeros for operands the same cycles pass at 2.0 GHz).
-// us, stream_kernel -> here (with the launch that splits the blocks): 768 -> 3072 density 0.5, 4096 tokens 92 -> 63, 3072 -> 768 83 -> 65, 768 -> 768
-// density 0.5, 16384 tokens 92 -> 62, 4096 -> 4096 density 0.25, 16384 tokens 1216 -> 845.
+// us, stream_kernel -> here (with the launch that splits the blocks): 768 -> 3072 density 0.5, 4096 tokens 92 -> 65, 3072 -> 768 83 -> 66, 768 -> 768
+// density 0.5, 16384 tokens 92 -> 64, 4096 -> 4096 density 0.25, 16384 tokens 1216 -> 870.
 //
 // A workgroup takes 64 tokens x 8 block columns at a time.  Waves 0-7 multiply, one block column each: per block, 6 KB of fragments from
 // memory (asked for an item ahead) and 12 KB from the panel ring in LDS for 24 instructions of 32 cycles.  Waves 8-11 load the panel of a k-block
@@ -70,6 +78,13 @@ static __device__ __forceinline__ void split2(float a0, float a1, uint32_t& h, u
     m = pack(a0, a1);
     rest(a0, a1, m);
     l = pack(a0, a1);
+}
+
+// The sign bit of the dense operand in a k-block: the parity of the ones in its number, so that any regular choice of k-blocks has as many of either
+// kind.
+static __device__ __forceinline__ int block_sign(int kb) { return (__popc((unsigned)kb) & 1) << 31; }
+static __device__ __forceinline__ float with_sign(float v, int sign_uniform) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane((int)__float_as_uint(v) ^ sign_uniform));
 }
 
 // The blocks in parts, as fragments: block b = [half q of k][part][lane = 32 h + n][8 k values], k = 16 q + 8 h + e, 6 KB.  One wave
@@ -210,8 +225,10 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         set_tile(lj);
         float4 buf[2][8];
         bool buf_low[2];
-        auto load = [&](float4 (&v)[8], bool& v_low) __attribute__((always_inline)) {
+        float buf_scale[2];
+        auto load = [&](float4 (&v)[8], bool& v_low, float& v_scale) __attribute__((always_inline)) {
             v_low = low;
+            v_scale = with_sign(SP_SCALE, block_sign(lkb));
             const unsigned char* src = A + (base + (size_t)lkb * 128);
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const float4*>(src + voff[i]);
@@ -225,14 +242,14 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
             if (moved) set_tile(lj);
         };
         int s_at = p;   // the slot of the step being filled
-        auto fill = [&](int u, const float4 (&v)[8], bool v_low) __attribute__((always_inline)) {
+        auto fill = [&](int u, const float4 (&v)[8], bool v_low, float v_scale) __attribute__((always_inline)) {
             // split first: a slot that becomes free then only waits for the writes
             uint2 part[3][8];
             auto rows = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
                 for (int i = i0; i < i0 + 4; ++i) {
-                    split2(v[i].x * SP_SCALE, v[i].y * SP_SCALE, part[0][i].x, part[1][i].x, part[2][i].x);
-                    split2(v[i].z * SP_SCALE, v[i].w * SP_SCALE, part[0][i].y, part[1][i].y, part[2][i].y);
+                    split2(v[i].x * v_scale, v[i].y * v_scale, part[0][i].x, part[1][i].x, part[2][i].x);
+                    split2(v[i].z * v_scale, v[i].w * v_scale, part[0][i].y, part[1][i].y, part[2][i].y);
                 }
             };
             rows(0);
@@ -260,13 +277,13 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
             if (lane == 0) lds_poke(s_landed + s_at, u + 1);
             s_at = s_at + SP_NP < RS ? s_at + SP_NP : s_at + SP_NP - RS;
         };
-        if (p < steps) load(buf[0], buf_low[0]);
+        if (p < steps) load(buf[0], buf_low[0], buf_scale[0]);
         for (int u = p; u < steps; u += 2 * SP_NP) {
-            load(buf[1], buf_low[1]);   // (past the last step: the last tile again, never used)
-            fill(u, buf[0], buf_low[0]);
+            load(buf[1], buf_low[1], buf_scale[1]);   // (past the last step: the last tile again, never used)
+            fill(u, buf[0], buf_low[0], buf_scale[0]);
             if (u + SP_NP >= steps) break;
-            load(buf[0], buf_low[0]);
-            fill(u + SP_NP, buf[1], buf_low[1]);
+            load(buf[0], buf_low[0], buf_scale[0]);
+            fill(u + SP_NP, buf[1], buf_low[1], buf_scale[1]);
         }
         if (gave_up) count_protocol_failure();
         return;
@@ -299,12 +316,18 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         return Head{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y), __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w)};
     };
 
-    f32x16 hi[2], lo[2];
+    f32x16 total[2], part[2];   // of 32 tokens each: the column so far, and a block
+    int sign = 0;               // of the block in part[1]
+    auto join = [&](int t) __attribute__((always_inline)) {
+        const float one = with_sign(1.f, sign);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) total[t][v] = __builtin_fmaf(part[t][v], one, total[t][v]);
+    };
     auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) hi[t][v] = lo[t][v] = 0.f;
+            for (int v = 0; v < 16; ++v) total[t][v] = part[t][v] = 0.f;
     };
     clear();
 
@@ -327,48 +350,62 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     auto epilogue = [&](const Head& unit) __attribute__((always_inline)) {
         const int col = unit.col, row0 = unit.row & ~3;
         if (col < 0) return;
+        join(1);   // (of the last block)
+        int at = lane;   // (opaque: the addresses below are made here, not kept in registers while the column is multiplied)
+        asm volatile("" : "+v"(at));
+        const int r = at & 31, h = at >> 5;
         const bool failed = gave_up || __builtin_amdgcn_readfirstlane(lds_peek(s_fail)) != 0;
         float b[16];   // (word by word: a bias need not be aligned to more)
 #pragma unroll
         for (int v = 0; v < 16; ++v) b[v] = g.bias ? g.bias[col * 32 + 8 * (v >> 2) + 4 * h + (v & 3)] : 0.f;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            if (unit.row & (2 >> t)) continue;
+            if (t == 0 && unit.row & 3) continue;
             float off = 0.f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                hi[t][v] = (hi[t][v] + lo[t][v]) * SP_UNSCALE;
-                off = __builtin_fmaf(hi[t][v], 0.f, off);
+                total[t][v] *= SP_UNSCALE;
+                off = __builtin_fmaf(total[t][v], 0.f, off);
             }
-            const int row = row0 + 32 * t + r;
+            const int row = row0 + (t == 1 && !(unit.row & 1) ? 32 : 0) + r;
             if (__any(off != 0.f || off != off)) {
-                // again, with fp32 instructions and operands as they are: infinities, NaN, results beyond the scaled range
-                f32x16 s;
+                // again, with fp32 instructions and operands as they are, each block's products summed by themselves as well: infinities, NaN, results
+                // beyond the scaled range
+                unsigned bad = 0;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) s[v] = 0.f;
+                for (int v = 0; v < 16; ++v)
+                    if (total[t][v] - total[t][v] != 0.f) {
+                        bad |= 1u << v;
+                        total[t][v] = 0.f;
+                    }
                 const float* x = g.a + (size_t)(row < g.M ? row : g.M - 1) * g.K;
 #pragma unroll 1
                 for (int i = 0; i < unit.n; ++i) {
                     const int2 e = all_entries[unit.lo + i];
                     const float* w = g.data + (size_t)e.y * 1024 + (TRANS ? r * 32 + 16 * h : 16 * h * 32 + r);
-                    float wk[16], xk[16];   // k = 16 h + 0 .. 15, asked for together
+                    f32x16 s;
 #pragma unroll
-                    for (int k = 0; k < 16; ++k) {
-                        wk[k] = w[TRANS ? k : k * 32];
-                        xk[k] = x[e.x * 32 + 16 * h + k];
+                    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll 1
+                    for (int k0 = 0; k0 < 16; k0 += 8) {
+                        float wk[8], xk[8];   // k = 16 h + k0 + 0 .. 7, asked for together
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) {
+                            wk[k] = w[(k0 + k) * (TRANS ? 1 : 32)];
+                            xk[k] = x[e.x * 32 + 16 * h + k0 + k];
+                        }
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) s = __builtin_amdgcn_mfma_f32_32x32x2f32(wk[k], xk[k], s, 0, 0, 0);
                     }
 #pragma unroll
-                    for (int k = 0; k < 16; ++k) s = __builtin_amdgcn_mfma_f32_32x32x2f32(wk[k], xk[k], s, 0, 0, 0);
+                    for (int v = 0; v < 16; ++v) total[t][v] = bad >> v & 1 ? total[t][v] + s[v] : total[t][v];
                 }
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    if (hi[t][v] - hi[t][v] != 0.f) hi[t][v] = s[v];
             }
             if (row < g.M) {
                 float* o = g.out + (size_t)row * g.N + col * 32 + 4 * h;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    float4 v = make_float4(hi[t][4 * q] + b[4 * q], hi[t][4 * q + 1] + b[4 * q + 1], hi[t][4 * q + 2] + b[4 * q + 2], hi[t][4 * q + 3] + b[4 * q + 3]);
+                    float4 v = make_float4(total[t][4 * q] + b[4 * q], total[t][4 * q + 1] + b[4 * q + 1], total[t][4 * q + 2] + b[4 * q + 2], total[t][4 * q + 3] + b[4 * q + 3]);
                     if (failed) v.x = v.y = v.z = v.w = __builtin_nanf("");
                     *reinterpret_cast<float4*>(o + 8 * q) = v;
                 }
@@ -396,8 +433,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         for (int i = 0; i < 6; ++i) w[i] = *reinterpret_cast<const u32x4*>(src + i * 1024 + lane16);
     };
     // chunk c (8 values of k) of token row r at c ^ (r / 4 % 4): 16 rows' reads of one chunk meet no bank twice
-    const unsigned char* const x_base = smem + r * 64 + ((h ^ ((r >> 2) & 3)) * 16);
-    const int x_other = (h ^ ((r >> 2) & 3)) & 2 ? -32 : 32;   // to the other half of k
+    const unsigned x_at = r * 64 + ((h ^ ((r >> 2) & 3)) * 16);   // (the other half of k: ^ 32)
 
     // entries of this unit and the next, and those of the one after, on their way
     Head unit = head_of(0);
@@ -410,13 +446,16 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         const int n = unit.n, u0 = j * KB;
         ev2 = window(head_of(j + 2), 0);
         if (n > 0) {
-            const bool first = unit.row & 1, second = unit.row & 2;
+            // a wave with 32 tokens of the tile has them in total[1], part[1]: the block before joins its total while the operands come from LDS
+            const bool half = unit.row & 3;
+            const int x_second = unit.row & 1 ? 0 : 2048;
             int kb = __builtin_amdgcn_readlane(ev.x, 0);
             publish(u0 + kb);
             slot = slot_of(u0 + kb);
             // one item: w = its block, w_next takes the next one's (behind the last one the first of the next unit)
             auto item = [&](int i, u32x4 (&w)[6], u32x4 (&w_next)[6]) __attribute__((always_inline)) {
                 const int u = u0 + kb;
+                const int this_sign = block_sign(kb);
                 const bool last = i + 1 == n;
                 if (((i + 1) & 63) == 0 && !last) {
                     ev = window(unit, i + 1);
@@ -428,15 +467,16 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                 load_block(w_next, last ? b_out : b_in);
                 if (__builtin_expect(__builtin_amdgcn_readfirstlane(raw) <= u, 0)) wait_for(u);
                 asm volatile("" ::: "memory");
-                const unsigned char* p0 = x_base + slot * SLOT;
-                const unsigned char* p1 = p0 + x_other;
-                u32x4 x[2][3];
-                auto read = [&](int s) __attribute__((always_inline)) {   // s = 2 * (half of k) + 32 tokens (not used where the wave has the other 32)
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) x[s & 1][i] = *reinterpret_cast<const u32x4*>((s >> 1 ? p1 : p0) + i * PLANE + (s & 1) * 2048);
+                const unsigned char* p0 = smem + (x_at + slot * SLOT);
+                const unsigned char* p1 = smem + ((x_at ^ 32) + slot * SLOT);
+                u32x4 x[2][3];   // [half of k][part] of 32 tokens
+                auto read = [&](int t, int q, int p) __attribute__((always_inline)) {
+                    x[q][p] = *reinterpret_cast<const u32x4*>((q ? p1 : p0) + p * PLANE + (t ? x_second : 0));
                 };
-                read(0);
-                read(1);
+                if (!half) {
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) read(0, k / 3, 2 - k % 3);
+                }
                 slot = slot_of(u0 + kb);
                 auto reads_back = [&]() __attribute__((always_inline)) {   // every read of the slot
                     raw = landed(slot);
@@ -445,22 +485,50 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                 };
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int t = s & 1, q = s >> 1;
-                    auto mma = [&](int pw, int px, f32x16& c) __attribute__((always_inline)) {
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[s & 1][px]), c, 0, 0, 0);
+                for (int t = 0; t < 2; ++t) {
+                    const bool mine = t == 1 || !half;
+                    f32x16& c = part[t];
+                    auto mma = [&](int q, int pw, int px) __attribute__((always_inline)) {
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[q][px]), c, 0, 0, 0);
                     };
-                    if (t == 0 ? !second : !first) {
-                        mma(0, 2, lo[t]);
-                        mma(1, 1, lo[t]);
-                        mma(2, 0, lo[t]);
-                        mma(0, 1, lo[t]);
-                        mma(1, 0, lo[t]);
-                        mma(0, 0, hi[t]);
+                    auto small = [&](int q) __attribute__((always_inline)) {   // (first those whose operands are read first)
+                        mma(q, 0, 2);
+                        mma(q, 1, 1);
+                        mma(q, 0, 1);
+                        mma(q, 2, 0);
+                        mma(q, 1, 0);
+                    };
+                    if (mine) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) c[v] = 0.f;
+                        small(0);
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                    if (s < 2) read(s + 2);
-                    if (s == 1) reads_back();
+                    if (t == 0) {
+                        read(1, 0, 2);
+                        read(1, 0, 1);
+                    }
+                    if (t == 0 || !half) join(t ^ 1);   // t = 0: of the block before
+                    if (t == 0) sign = this_sign;
+                    asm volatile("" : "+v"(total[t ^ 1]));   // (here, where matrix instructions are under way, and not at the end)
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (mine) {
+                        small(1);
+                        mma(0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t == 0) {
+                        read(1, 0, 0);
+                        read(1, 1, 2);
+                        read(1, 1, 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (mine) mma(1, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t == 0) {
+                        read(1, 1, 0);
+                        reads_back();
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
