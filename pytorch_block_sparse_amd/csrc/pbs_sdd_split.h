@@ -268,31 +268,45 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
                 for (int e = 0; e < 4; ++e) off = __builtin_fmaf(v[i][e], 0.f, off);
             }
             if (__any(off != 0.f)) {
-                // again, with fp32 instructions: infinities, NaN, sums beyond the scaled range
-                f32x16 s;
+                // again, with fp32 instructions: infinities, NaN, sums beyond the scaled range.  A chunk's products by themselves, then what would be a
+                // wave's chunks, as in pbs_sdd_row.h.
+                f32x16 sum;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s[e] = 0.f;
+                for (int e = 0; e < 16; ++e) sum[e] = 0.f;
                 const float* g = static_cast<const float*>(a.g) + row * 32 + r;
                 const float* x = static_cast<const float*>(a.x) + (k == 0 ? cblk[b0] : cblk[(b0 + 1) % NB]) * 32 + r;
-                const int t_hi = c_hi * ROW_TC < a.M ? c_hi * ROW_TC : a.M;
 #pragma unroll 1
-                for (int t0 = c_lo * ROW_TC; t0 < t_hi; t0 += 16) {
-                    float gk[8], xk[8];
+                for (int w = 0; w < ROW_NW; ++w) {
+                    f32x16 of_wave;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int t = t0 + 2 * e + h, at = t < t_hi ? t : t_hi - 1;
-                        gk[e] = g[(size_t)at * a.N];
-                        xk[e] = x[(size_t)at * a.K];
-                        if (t >= t_hi) gk[e] = xk[e] = 0.f;
+                    for (int e = 0; e < 16; ++e) of_wave[e] = 0.f;
+#pragma unroll 1
+                    for (int c = c_lo + w; c < c_hi && c * ROW_TC < a.M; c += ROW_NW) {
+                        f32x16 s;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll 1
+                        for (int t0 = c * ROW_TC; t0 < (c + 1) * ROW_TC; t0 += 16) {
+                            float gk[8], xk[8];
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                const int t = t0 + 2 * e + h, at = t < a.M ? t : a.M - 1;
+                                gk[e] = g[(size_t)at * a.N];
+                                xk[e] = x[(size_t)at * a.K];
+                                if (t >= a.M) gk[e] = xk[e] = 0.f;
+                            }
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(gk[e], xk[e], s, 0, 0, 0);
+                        }
+                        of_wave += s;
                     }
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(gk[e], xk[e], s, 0, 0, 0);
+                    sum += of_wave;
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (v[i][e] - v[i][e] != 0.f) v[i][e] = jj == 0 ? s[4 * i + e] : s[8 + 4 * i + e];
+                        if (v[i][e] - v[i][e] != 0.f) v[i][e] = jj == 0 ? sum[4 * i + e] : sum[8 + 4 * i + e];
             }
 #pragma unroll
             for (int i = 0; i < 2; ++i) {

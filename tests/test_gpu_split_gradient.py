@@ -79,5 +79,7 @@ def test_values_that_have_no_parts(cuda):
         x, dy = torch.randn(tokens, 1024, device=cuda) * scale_x, torch.randn(tokens, 1024, device=cuda) * scale_dy
         want = _want(m, dy, x)
         got = m.matmul_with_output_sparse_support(dy, x).double()
-        # (the fp32 instructions' chains, and of results near 2^-119 what is left above 2^-149)
-        assert ((got - want).norm() / want.norm()).item() < 3e-6, (scale_x, scale_dy)
+        # (the fp32 instructions' chains of a chunk and of a wave's chunks; what products near 2^-120 lose below 2^-149 is far less)
+        distance = ((got - want).norm() / want.norm()).item()
+        print(scale_x, scale_dy, distance, flush=True)
+        assert distance <= 0.35 * 2.0 ** -24 * np.sqrt(32 + tokens / 128) + 2.0 ** -25, (scale_x, scale_dy)
