@@ -409,46 +409,61 @@ static int launch_panel_chunks(const DdsArgs& g, int splits, hipStream_t stream)
 }
 
 // ---- fp32 on the bf16 matrix cores ----
-// Which problems: products of 370 random problems (256 to 4096 features, 300 to 16384 tokens, densities 0.05 to 0.75, even and Zipf rows) were
-// timed with this kernel and with stream_kernel.  With a pattern of density 0.2 and more, groups of 8 columns that are filled to three quarters,
-// and 4.3 GFLOP (2^21 tokens x blocks) it takes 1.29 times less time on average and at most 1.1 times more; below, a panel is split for too few
-// products (density 0.15: 0.8 to 1.1 times as fast, 0.05: half as fast), waves have no column, or the launch that splits the blocks and the first
-// panels weigh too much (at 2^20 as often slower as faster; 1024 -> 2560, 700 tokens 14 us in stream_kernel, 20 here).
-// The line depends on the pattern and then on the number of tokens alone: a token's result does not depend, to the last bit, on
-// the others in the call among all calls of a pattern on the same side of it.
-static bool split_kernel_fits(long long M, int n, int k, int nnz) {
-    const long long cols = n / 32, groups = (cols + SP_NC - 1) / SP_NC;
-    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
-    // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
-    return k <= (1 << 16) && (M + 31) / 32 * groups < (1 << 28);
-}
 static inline size_t split_workspace_bytes(int nnz) { return (size_t)nnz * SP_BLOCK_BYTES; }
+static inline int split_groups(int n) { return (n / 32 + SP_NC - 1) / SP_NC; }   // (the kernel takes up to half as many again where columns are uneven)
 
 // How many tiles of 64 tokens, the rest being low ones of 32: full tiles for as many whole rounds of units over the 256 CUs as is best, low ones
 // behind them (which a result's bits do not depend on).  A low unit takes 0.58 to 0.65 of a full one's time.  Against full tiles alone: 264 units
 // (4215 tokens 2784 -> 800) 73 -> 60 us, 128 units (512 tokens 4096 -> 4096) 52 -> 44, multiples of 256 the same.
 constexpr double SP_LOW = 0.62;
-static int split_full_tiles(long long M, int groups) {
+struct SplitTiles {
+    int full;
+    double rounds;   // of full units over the chip, in time
+};
+static SplitTiles split_tiles(long long M, int groups) {
     const long long most = M / SP_BM, all = (M + SP_BM - 1) / SP_BM;
     auto rounds = [&](long long full) {
-        const long long low = (M - full * SP_BM + 31) / 32;
-        const double f = (double)full * groups / 256, l = low > 0 ? (double)low * groups / 256 : 0.0;
+        const long long low = M > full * SP_BM ? (M - full * SP_BM + 31) / 32 : 0;
+        const double f = (double)full * groups / 256, l = (double)low * groups / 256;
         // full rounds, then what is left of the full units beside the low ones
         const double whole = std::floor(f), rest = f - whole;
         if (rest == 0.0) return whole + SP_LOW * std::ceil(l);
         const double beside = (1.0 - rest) * std::floor(1.0 / SP_LOW);   // low units that fit beside the rest
         return whole + 1.0 + (l > beside ? SP_LOW * std::ceil(l - beside) : 0.0);
     };
-    long long best = all;   // (the last one ragged)
-    double least = rounds(all);
-    for (long long r = 0; r <= most * groups / 256; ++r) {
+    SplitTiles best{(int)all, rounds(all)};   // (the last one ragged)
+    const long long last = most * groups / 256;
+    for (long long r = last > 64 ? last - 64 : 0; r <= last; ++r) {
         const long long full = r * 256 / groups;
-        if (full <= most && rounds(full) < least - 1e-9) {
-            least = rounds(full);
-            best = full;
-        }
+        if (full <= most && rounds(full) < best.rounds - 1e-9) best = SplitTiles{(int)full, rounds(full)};
     }
-    return (int)best;
+    return best;
+}
+
+// Estimated time in us with the launch that splits the blocks: launches; splitting; per round of units over the chip what a step of the ring, a wave's
+// blocks (slower where the chip is full) and a unit's start and end cost.  Fitted to 821 products (256 to 4096 features, 512 to 16384 tokens, densities 0.2 to
+// 0.8, 2^21 to 2^25 tokens x blocks) whose fullest column holds less than 1.7 times the average; within 5 %.
+static double split_us(long long M, int n, int k, int nnz) {
+    const int groups = split_groups(n);
+    const double units = (double)M / SP_BM * groups / 256, full = units < 1.0 ? units : 1.0;
+    return 6.61 + 0.00319 * nnz + split_tiles(M, groups).rounds * (0.101 * (k / 32) + 1.07 * nnz / (n / 32) * (0.669 + 0.331 * full) + 2.48);
+}
+// Which problems: a density of 0.2 and more, groups of 8 columns that are filled to three quarters, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and an
+// estimate below stream_kernel's by 1.08.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05: half as fast); with
+// emptier groups waves have no column; with fewer tokens or products the launch that splits and the first panels weigh too much.  Of the 821 products
+// 706 are taken, 1.31 times faster on average, 3 of them slower (0.88, 0.97, 0.99 times as fast); the others are level on average (1.01), and without the
+// estimates 42 more than 2 % slower were taken (down to 0.69).  Columns that are more uneven than that are not known here: 278 of 312 such products (Zipf rows) are
+// taken, 1.12 times faster on average, but 64 of them more than 2 % slower, down to 0.57 times as fast where a full column among short ones meets a single round of
+// units (2186 tokens 3104 -> 1472, 1397 blocks 59 -> 105 us).
+// The choice depends on the pattern's sizes and then on the number of tokens alone: a token's result does not depend, to the last bit, on
+// the others in the call among all calls of a pattern that make the same choice.
+constexpr double SPLIT_MARGIN = 1.08;
+static bool split_kernel_fits(long long M, int n, int k, int nnz) {
+    const long long cols = n / 32, groups = split_groups(n);
+    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
+    // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
+    if (k > (1 << 16) || (M + 31) / 32 * groups >= (1 << 28)) return false;
+    return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us;
 }
 
 template <int TRANS>
@@ -468,9 +483,9 @@ static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
     a.M = g.M;
     a.N = g.N;
     a.K = g.K;
-    const int groups_even = (g.N / 32 + SP_NC - 1) / SP_NC;   // (the kernel takes up to half as many again where columns are uneven)
+    const int groups_even = split_groups(g.N);
     a.heavy = (int)(2ll * g.nnz / (g.N / 32));
-    a.tiles = split_full_tiles(g.M, groups_even);
+    a.tiles = split_tiles(g.M, groups_even).full;
     a.low_tiles = g.M > a.tiles * SP_BM ? (g.M - a.tiles * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
     // the 32 workgroups of an XCD work on tile_block token tiles x 32 / tile_block groups: the split with the least to read per k-block
     const double w_bytes = (double)SP_NC * SP_BLOCK_BYTES * g.nnz / ((double)(g.N / 32) * (g.K / 32)), x_bytes = SP_BM * 128.0;
