@@ -433,7 +433,8 @@ static SplitTiles split_tiles(long long M, int groups) {
     };
     SplitTiles best{(int)all, rounds(all)};   // (the last one ragged)
     const long long last = most * groups / 256;
-    for (long long r = last > 64 ? last - 64 : 0; r <= last; ++r) {
+    const int window = 2 + groups / 128;   // (fewer full rounds were the best nowhere)
+    for (long long r = last > window ? last - window : 0; r <= last; ++r) {
         const long long full = r * 256 / groups;
         if (full <= most && rounds(full) < best.rounds - 1e-9) best = SplitTiles{(int)full, rounds(full)};
     }
@@ -463,7 +464,16 @@ static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
     // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
     if (k > (1 << 16) || (M + 31) / 32 * groups >= (1 << 28)) return false;
-    return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us;
+    // (a product asks twice, for the size of its workspace and when it is launched: the last answer of a thread, by the sizes it follows from)
+    struct Answer {
+        long long M;
+        int n, k, nnz;
+        bool fits;
+    };
+    static thread_local Answer last{-1, 0, 0, 0, false};
+    if (last.M != M || last.n != n || last.k != k || last.nnz != nnz)
+        last = Answer{M, n, k, nnz, SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us};
+    return last.fits;
 }
 
 template <int TRANS>
@@ -703,9 +713,10 @@ struct BackPlan {
     bool split;   // fp32 in parts
     int passes, chunks_per_slice;
     SddPlan rect;
+    int partials;            // sums of this many slices in the workspace, or none
     size_t partial_bytes;
 };
-static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
+static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
     BackPlan p;
     const RowChoice row = choose_row(dtype, M, N, K, nnz, workspace_limit);
     p.slices = row.slices;
@@ -721,7 +732,24 @@ static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bi
         p.slices = n = (int)(filled < row.slices ? filled : row.slices);
         p.passes = (int)((filled + n - 1) / n);   // (the last launch may have slices without tokens, which add nothing)
     }
-    p.partial_bytes = n > 1 ? ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * n : 0;   // fp32 sums of each slice: blocks, bias columns
+    p.partials = n > 1 ? n : 0;
+    return p;
+}
+static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
+    // (a gradient asks three times, for the unit table, for the size of its workspace and when it is launched: the last answer of a thread, by the
+    // sizes it follows from)
+    struct Answer {
+        int dtype;
+        long long M;
+        int N, K, nnz;
+        size_t workspace_limit;
+        BackPlan plan;
+    };
+    static thread_local Answer last{-1, 0, 0, 0, 0, 0, {}};
+    if (last.dtype != dtype || last.M != M || last.N != N || last.K != K || last.nnz != nnz || last.workspace_limit != workspace_limit)
+        last = Answer{dtype, M, N, K, nnz, workspace_limit, plan_back_anew(dtype, M, N, K, nnz, workspace_limit)};
+    BackPlan p = last.plan;
+    p.partial_bytes = ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * p.partials;   // fp32 sums of each slice: blocks, bias columns
     return p;
 }
 

@@ -6,6 +6,7 @@ before the library touches the HIP runtime.
 import ctypes
 import os
 import re
+import threading
 
 import pytest
 
@@ -142,6 +143,27 @@ def test_fp32_products_by_estimate(lib, tokens, n, k, nnz, kernel):
 def test_slices_of_small_fp32_gradients_follow_the_fit(lib):
     """768 -> 3072, 1024 tokens: two slices and their reduction take less of the GPU's time than one (the host's time for the launch is not weighed)."""
     assert lib.pbs_blocksparse_matmul_back_kernel_name(1024, 3072, 768, 1152, 0) == b"sdd_row_kernel + sdd_reduce_kernel"
+
+
+def test_answers_do_not_depend_on_what_was_asked_before(lib):
+    """The last choice of kernels is kept, by every size that it follows from."""
+    sizes = [(2317, 3072, 768, 1152, 1), (2317, 3072, 768, 1152, 0), (4096, 3072, 768, 1152, 0), (4096, 768, 3072, 1152, 0), (4096, 768, 3072, 1151, 0),
+             (16384, 4096, 4096, 4096, 1), (600, 4096, 4096, 4096, 0)]
+
+    def ask(c):
+        return (lib.pbs_blocksparse_matmul_back_bias_workspace_bytes(*c), lib.pbs_blocksparse_matmul_back_workspace_bytes(*c),
+                lib.pbs_blocksparse_matmul_back_units_bytes(*c), lib.pbs_blocksparse_matmul_parts_bytes(*c[:4], 1, c[4]))
+
+    alone = {}
+    for c in sizes:
+        t = threading.Thread(target=lambda: alone.__setitem__(c, ask(c)))   # (a thread has asked nothing before)
+        t.start()
+        t.join()
+    for a in sizes:
+        for b in sizes:
+            ask(a)
+            assert ask(b) == alone[b], (a, b)
+    assert all(alone[c][0] >= alone[c][1] - alone[c][2] for c in sizes)
 
 
 def test_build_indices_argument_checks(lib):
