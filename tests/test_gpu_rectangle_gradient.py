@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
     (13007, 1056, 1056, [30, 2, 2, 2]),    # uneven rows are dealt to the bands
     (2600, 64, 10240, [90]),               # more rectangles than rows, 20 columns each
     (16391, 1600, 512, [7, 0, 3, 16]),
+    (800, 512, 33056, [1033, 1020, 1031]),  # eight rows, more entries in a band than its list in LDS holds
     (26001, 544, 544, [17, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0]),   # one row of a band has all the blocks, rectangles without blocks
 ])
 def test_rectangles(cuda, tokens, out_f, in_f, counts):

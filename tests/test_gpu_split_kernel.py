@@ -59,6 +59,7 @@ CASES = [
     (768, 3072, 2317, 1152),       # low tiles, the last one ragged
     (1632, 1024, 1501, 1468),      # 51 columns: waves without a column
     (256, 4384, 4701, 1000),       # lists over two windows
+    (2048, 65536, 2017, 26300),    # the longest contraction
     (2048, 2048, 797, 3072),       # low tiles alone
     (256, 32, 1040039, 8),         # one k-block, more units than the heads of one workgroup hold
     (768, 3072, 4096, zipf_positions(24, 96, 576, seed=3)),
