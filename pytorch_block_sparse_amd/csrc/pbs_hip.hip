@@ -449,16 +449,17 @@ static double split_us(long long M, int n, int k, int nnz) {
     const double units = (double)M / SP_BM * groups / 256, full = units < 1.0 ? units : 1.0;
     return 6.61 + 0.00319 * nnz + split_tiles(M, groups).rounds * (0.101 * (k / 32) + 1.07 * nnz / (n / 32) * (0.669 + 0.331 * full) + 2.48);
 }
-// Which problems: a density of 0.2 and more, groups of 8 columns that are filled to three quarters, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and an
-// estimate below stream_kernel's by 1.08.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05: half as fast); with
-// emptier groups waves have no column; with fewer tokens or products the launch that splits and the first panels weigh too much.  Of the 821 products
-// 706 are taken, 1.31 times faster on average, 3 of them slower (0.88, 0.97, 0.99 times as fast); the others are level on average (1.01), and without the
-// estimates 42 more than 2 % slower were taken (down to 0.69).  Columns that are more uneven than that are not known here: 278 of 312 such products (Zipf rows) are
-// taken, 1.12 times faster on average, but 64 of them more than 2 % slower, down to 0.57 times as fast where a full column among short ones meets a single round of
-// units (2186 tokens 3104 -> 1472, 1397 blocks 59 -> 105 us).
-// The choice depends on the pattern's sizes and then on the number of tokens alone: a token's result does not depend, to the last bit, on
-// the others in the call among all calls of a pattern that make the same choice.
-constexpr double SPLIT_MARGIN = 1.08;
+// Which problems: a density of 0.2 and more, groups of 8 columns that are filled to three quarters, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and not
+// where the estimates see stream_kernel ahead by a tenth.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05:
+// half as fast); with emptier groups waves have no column; with fewer tokens or products the launch that splits and the first panels weigh too much.
+// The tenth is for a result's bits: those of a token are the same, to the last bit, in all calls of a pattern that are served alike, and a line
+// at level estimates would part the calls of a 4096 -> 4096 layer of density 0.25 seven times between 512 and 2177 tokens.  Of the 821 products 802 are taken, 1.28
+// times faster on average (706 and 1.31 where the estimate has to be 1.08 below), 24 of them more than 2 % slower, the worst 0.83 times as fast, where
+// without the estimates 42 were, down to 0.69 (4096 -> 4096 density 0.25, 512 tokens 45 us in stream_kernel and 48 here, 1024 76 and 66, 1025 82 and 94, 2049 152 and 145).
+// Columns that are more uneven than that are not known here: 311 of 312 such products (Zipf rows) are taken, 1.10 times faster on average, but 80 of them more than
+// 2 % slower, down to 0.57 times as fast where a full column among short ones meets a single round of units (2186 tokens 3104 -> 1472, 1397 blocks
+// 59 -> 105 us).
+constexpr double SPLIT_MARGIN = 0.91;
 static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     const long long cols = n / 32, groups = split_groups(n);
     if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;

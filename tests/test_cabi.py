@@ -130,8 +130,8 @@ def test_back_argument_checks(lib):
 
 
 @pytest.mark.parametrize("tokens, n, k, nnz, kernel", [
-    # (measured: split_kernel 0.78 to 0.88 and 1.2 to 1.5 times as fast as stream_kernel)
-    (512, 2048, 4096, 6000, "stream_kernel"), (600, 4096, 4096, 4096, "stream_kernel"), (1025, 1152, 3104, 2285, "stream_kernel"),
+    # (measured: split_kernel 0.77 to 0.88 and 1.2 to 1.5 times as fast as stream_kernel)
+    (512, 2048, 4096, 6000, "stream_kernel"), (600, 4096, 4096, 4096, "stream_kernel"), (1025, 4096, 4096, 4096, "stream_kernel"),
     (4096, 3072, 768, 1152, "split_kernel"), (2048, 4096, 4096, 8192, "split_kernel"), (16384, 768, 768, 288, "split_kernel"),
     (1 << 24, 4096, 4096, 4096, "split_kernel"), (1 << 30, 4096, 4096, 4096, "stream_kernel"),   # (units have 32-bit numbers)
 ])
