@@ -183,9 +183,16 @@ int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* pl
  * no copy would be made (fp32, the input-gradient direction, small or very sparse problems).
  *
  * Larger fp32 products run on the bf16 matrix cores, which multiply 16 times as fast: every value as the sum of three bfloat16 values
- * (without a rest), six of their nine products, sums in fp32; closer to the exact result than the fp32 instructions' chains are.  For that the
- * call writes the parts of the blocks into a workspace of pbs_blocksparse_matmul_parts_bytes() bytes (6 KB per block; 0 where such a
- * workspace would not be used: bf16, smaller or very sparse problems).  Without it, the product is made of fp32 instructions.
+ * (without a rest), six of their nine products, sums in fp32.  The three products left out are at most 2^-24 of a product; a sum of many is closer to the
+ * exact result than with fp32 instructions (1.1e-7 against 2.9e-7 of its size at 4096 x 4096, density 0.25), one of few nonzero products up to 1.4 times further off
+ * (0.35e-7 against 0.25e-7).  For that the call writes the parts of the blocks into a workspace of pbs_blocksparse_matmul_parts_bytes() bytes (6 KB per block; 0
+ * where such a workspace would not be used: bf16, smaller or very sparse problems).  Without it, the product is made of fp32 instructions.
+ *
+ * Bits.  A token's fp32 result is the same, to the last bit, in all calls of a pattern and direction that take the same of these two ways, whatever other
+ * tokens share the call; between the two it differs by rounding.  Which way a call takes follows from its sizes: with the workspace the bf16 cores' from
+ * 512 tokens and 2^21 tokens x blocks on at densities of 0.2 and more, apart from token counts for which an estimate sees the fp32 instructions ahead by a tenth
+ * (pbs_blocksparse_matmul_parts_bytes() > 0 tells).  A caller who needs the same bits for requests batched in any way passes no workspace.  bf16
+ * results, and the gradient of the blocks in either dtype, may differ by rounding between calls of different numbers of tokens.
  */
 size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype);
 size_t pbs_blocksparse_matmul_parts_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype);
