@@ -140,11 +140,6 @@ def test_fp32_products_by_estimate(lib, tokens, n, k, nnz, kernel):
     assert lib.pbs_blocksparse_matmul_parts_bytes(tokens, n, k, nnz, 1, 0) == (nnz * 6144 if kernel == "split_kernel" else 0)
 
 
-def test_slices_of_small_fp32_gradients_follow_the_fit(lib):
-    """768 -> 3072, 1024 tokens: two slices and their reduction take less of the GPU's time than one (the host's time for the launch is not weighed)."""
-    assert lib.pbs_blocksparse_matmul_back_kernel_name(1024, 3072, 768, 1152, 0) == b"sdd_row_kernel + sdd_reduce_kernel"
-
-
 def test_answers_do_not_depend_on_what_was_asked_before(lib):
     """The last choice of kernels is kept, by every size that it follows from."""
     sizes = [(2317, 3072, 768, 1152, 1), (2317, 3072, 768, 1152, 0), (4096, 3072, 768, 1152, 0), (4096, 768, 3072, 1152, 0), (4096, 768, 3072, 1151, 0),
