@@ -88,15 +88,18 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_kernel(PanelArgs g) {
         int2 e;
         float b;
     };
-    const int2* ent = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4);
+    const int KB = g.K >> 5;
     auto load_pair = [&](int p) {
         Pair o{0, 0, make_int2(0, 0), 0.f};
         const int i = 2 * p + (lane >> 5), l = lane & 31;
         if (i < mine) {
-            const int4 head = reinterpret_cast<const int4*>(g.plan)[split + g.splits * turn(i)];
-            o.n = head.z < 32 ? head.z : 32;
+            // (the entry with the head: places behind the last one hold anything, and are not multiplied)
+            const int2* record = reinterpret_cast<const int2*>(g.plan) + list_record(KB, split + g.splits * turn(i));
+            const int2 head = record[0];
+            const int2 e = record[LIST_HEAD + (l < KB ? l : KB - 1)];
+            o.n = head.y < 32 ? head.y : 32;
             o.col = head.x;
-            if (o.n > 0) o.e = ent[head.y + (l < o.n ? l : o.n - 1)];
+            if (l < o.n) o.e = e;
             if (g.bias) o.b = E::to_f32(static_cast<const bf16_t*>(g.bias)[head.x * 32 + l]);
         }
         return o;
@@ -251,15 +254,16 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_chunk_kernel(PanelArgs
     };
     stage(0);
 
-    int4 head = make_int4(0, 0, 0, 0);
-    if (rank < ncols) head = reinterpret_cast<const int4*>(g.plan)[rank];
-    const int n = __builtin_amdgcn_readfirstlane(head.z);
-    const int col = __builtin_amdgcn_readfirstlane(head.x) * 32;
-    const int2* ent = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4) + __builtin_amdgcn_readfirstlane(head.y) + s;
+    const int KB = g.K >> 5;
+    const int2* const record = reinterpret_cast<const int2*>(g.plan) + list_record(KB, rank < ncols ? rank : 0);
+    const int2* const ent = record + LIST_HEAD + s;
+    const int room = (KB - 1 - s) / S;   // (the record's last place for an entry of this wave's: there are more than PANEL_MAX_K / 32 k-blocks)
+    int2 ev = ent[(size_t)(lane < room ? lane : room) * S];   // (with the head: places behind the last entry hold anything, and are not asked for)
+    const int2 head = record[0];
+    const int n = rank < ncols ? __builtin_amdgcn_readfirstlane(head.y) : 0;
+    const int col = rank < ncols ? __builtin_amdgcn_readfirstlane(head.x) * 32 : 0;
     const int mine = n > s ? (n - s + S - 1) / S : 0;
     auto load64 = [&](int i) { return ent[(size_t)(i + lane < mine ? i + lane : mine - 1) * S]; };
-    int2 ev = make_int2(0, 0);
-    if (mine > 0) ev = load64(0);
     float bv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) bv[i] = g.bias ? E::to_f32(static_cast<const bf16_t*>(g.bias)[col + 8 * q + i]) : 0.f;

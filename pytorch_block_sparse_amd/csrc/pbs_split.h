@@ -152,11 +152,11 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     // Place v of the dealing: below 2 * heavy half v % 2 of column v / 2 of the ranking, else column v - heavy.
     int heavy = 0;
     {
-        const int4* ranked = reinterpret_cast<const int4*>(g.plan);
+        const int2* ranked = reinterpret_cast<const int2*>(g.plan);
         bool more = true;
         for (int c0 = 0; more && c0 < ncols; c0 += 64) {   // (the first 64 and no more in even patterns)
             const int c = c0 + lane;
-            const unsigned long long not_heavy = __ballot(c >= ncols || ranked[c < ncols ? c : 0].z <= g.heavy);
+            const unsigned long long not_heavy = __ballot(c >= ncols || ranked[list_record(KB, c < ncols ? c : 0)].y <= g.heavy);
             more = not_heavy == 0;
             heavy += more ? 64 : __builtin_ctzll(not_heavy);
         }
@@ -294,10 +294,10 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     // ---------------- multiplying ----------------
     const int r = lane & 31, h = lane >> 5;
     const int band = wave < 4 ? wave : 11 - wave;   // waves w and w + 4 share a SIMD: a long column and a short one
-    const int2* const all_entries = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4);
-    // block column of the result, its first entry, its entries, and first token | (1: the first 32 tokens alone, 2: the second), of this workgroup's units
+    const int2* const records = reinterpret_cast<const int2*>(g.plan);
+    // block column of the result, its rank, its entries, and first token | (1: the first 32 tokens alone, 2: the second), of this workgroup's units
     struct Head {
-        int col, lo, n, row;
+        int col, rank, n, row;
     };
     int4* const heads = s_heads + wave * SP_MAX_UNITS;
     if (lane < mine) {
@@ -307,10 +307,9 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         const int v = band * groups + ((band & 1) ? groups - 1 - group : group);
         const int rank = v < 2 * heavy ? v >> 1 : v - heavy;
         const int tokens = v >= 2 * heavy ? (low ? 1 : 0) : (v & 1) ? 2 : 1;
-        int4 head = make_int4(-1, 0, 0, 0);
-        if (rank < ncols && !(low && tokens == 2)) head = reinterpret_cast<const int4*>(g.plan)[rank];
-        head.w = row0 | tokens;
-        heads[lane] = head;
+        int2 head = make_int2(-1, 0);
+        if (rank < ncols && !(low && tokens == 2)) head = records[list_record(KB, rank)];
+        heads[lane] = make_int4(head.x, rank < ncols ? rank : 0, head.y, row0 | tokens);
     }
     auto head_of = [&](int j) __attribute__((always_inline)) {
         int4 v = make_int4(-1, 0, 0, 0);
@@ -381,9 +380,10 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                         total[t][v] = 0.f;
                     }
                 const float* x = g.a + (size_t)(row < g.M ? row : g.M - 1) * g.K;
+                const int2* const entries = records + list_record(KB, unit.rank) + LIST_HEAD;
 #pragma unroll 1
                 for (int i = 0; i < unit.n; ++i) {
-                    const int2 e = all_entries[unit.lo + i];
+                    const int2 e = entries[i];
                     const float* w = g.data + (size_t)e.y * 1024 + (TRANS ? r * 32 + 16 * h : 16 * h * 32 + r);
                     f32x16 s;
 #pragma unroll
@@ -421,7 +421,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         int2 e = make_int2(0, 0);
         if (unit.n > 0) {
             const int l = i0 + lane;
-            e = all_entries[unit.lo + (l < unit.n ? l : unit.n - 1)];
+            e = records[list_record(KB, unit.rank) + LIST_HEAD + (l < unit.n ? l : unit.n - 1)];
         }
         return e;
     };

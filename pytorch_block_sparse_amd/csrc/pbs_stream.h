@@ -28,8 +28,9 @@
 // eight consecutive columns of a token and stores them with 16-byte stores, 128 (64) contiguous bytes per token.
 //
 // Work list ("list plan", list_plan_kernel), per pattern and direction: per block column, in order of falling block
-// count, {column, first entry, entries, 0}, then the entries {k-block, data block}, by k-block, with every value inside its
-// range.  Long columns are so started first.
+// count, a record {column, entries, 0, 0} and the entries {k-block, data block}, by k-block, with every value inside its
+// range.  Long columns are so started first.  A record has room for as many entries as there are k-blocks, so a wave asks for its first entries
+// together with the number of them: one round trip to memory before the first operands instead of two.
 #pragma once
 #include "pbs_common.h"
 
@@ -37,7 +38,9 @@ namespace pbs {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-static inline size_t list_plan_bytes(int n, int k) { return (size_t)(n / 32) * (16 + (size_t)(k / 32) * 8); }
+constexpr int LIST_HEAD = 2;   // of a record's KB + 2 pairs; {column, entries} is the first
+static __host__ __device__ __forceinline__ size_t list_record(int KB, int rank) { return (size_t)rank * (size_t)(KB + LIST_HEAD); }
+static inline size_t list_plan_bytes(int n, int k) { return list_record(k / 32, n / 32) * 8; }
 
 constexpr int LIST_RANK_MAX_COLS = 8192;   // ranking compares every pair of columns: beyond this, natural order
 
@@ -56,7 +59,6 @@ static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, i
     const int32_t* __restrict__ idx = a.idx;
     const int nblk_n = a.nblk_n, KB = a.KB, nnz = a.nnz;
     int* __restrict__ plan = a.plan;
-    int2* ent = reinterpret_cast<int2*>(plan + (size_t)nblk_n * 4);
     auto entry = [&](int i) { return make_int2(idx[2 * (size_t)i], idx[2 * (size_t)i + 1]); };
     auto good = [&](int2 e) { return e.x >= 0 && e.x < KB && e.y >= 0 && e.y < nnz; };
     const int lane = threadIdx.x & 63;
@@ -74,12 +76,14 @@ static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, i
 #pragma unroll
             for (int d = 32; d; d >>= 1) rank += __shfl_xor(rank, d, 64);
         }
+        int2* const record = reinterpret_cast<int2*>(plan) + list_record(KB, rank);
+        int2* const ent = record + LIST_HEAD;
         bool as_it_is = true;
 #pragma unroll 4
         for (int i = lane; i < n; i += 64) {
             const int2 e = entry(lo + i);
             if (!good(e) || (i > 0 && entry(lo + i - 1).x >= e.x)) as_it_is = false;
-            ent[lo + i] = make_int2(e.x < 0 ? 0 : (e.x >= KB ? KB - 1 : e.x), e.y < 0 ? 0 : (e.y >= nnz ? nnz - 1 : e.y));
+            if (i < KB) ent[i] = make_int2(e.x < 0 ? 0 : (e.x >= KB ? KB - 1 : e.x), e.y < 0 ? 0 : (e.y >= nnz ? nnz - 1 : e.y));
         }
         int kept = n;
         if (__any(!as_it_is)) {   // the smallest k-block that is left, and of its entries the first, n times over
@@ -99,10 +103,10 @@ static __device__ __forceinline__ void list_plan(const ListArgs& a, int block, i
                 if (least == 1ll << 62) break;
                 last = (int)(least >> 32);
                 // (by the lane that has written this place above)
-                if (lane == (kept & 63)) ent[lo + kept] = make_int2(last, entry(lo + (int)(least & 0xffffffffll)).y);
+                if (lane == (kept & 63)) ent[kept] = make_int2(last, entry(lo + (int)(least & 0xffffffffll)).y);
             }
         }
-        if (lane == 0) *reinterpret_cast<int4*>(plan + 4 * (size_t)rank) = make_int4(c, lo, kept, 0);
+        if (lane < LIST_HEAD) record[lane] = lane == 0 ? make_int2(c, kept) : make_int2(0, 0);
     }
 }
 __global__ __launch_bounds__(256) void list_plan_kernel(ListArgs a) { list_plan(a, blockIdx.x, gridDim.x); }
@@ -169,9 +173,14 @@ __global__ __launch_bounds__(KS * 64, WPE) void stream_kernel(StreamArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
 
-    const int4 head = reinterpret_cast<const int4*>(g.plan)[cr];
-    const int2* ent = reinterpret_cast<const int2*>(g.plan + (size_t)ncols * 4) + head.y;
-    const int n = head.z;
+    // this wave's entries are wave, wave + KS, ...: its next 64, one per lane, and with the first of them the number of all
+    const int2* const record = reinterpret_cast<const int2*>(g.plan) + list_record(g.K >> 5, cr);
+    const int2* const ent = record + LIST_HEAD + wave;
+    const int room = ((g.K >> 5) - 1 - wave) / KS;   // (a record's last place for an entry of this wave's; of a wave behind the last k-block 0, and not read)
+    int2 ev = make_int2(0, 0);
+    if (wave < g.K >> 5) ev = ent[(size_t)(lane < room ? lane : room) * KS];
+    const int2 head = record[0];
+    const int n = head.y;
     const int col = head.x * 32;
 
     const unsigned char* A = static_cast<const unsigned char*>(g.a) + (size_t)m0 * g.K * ESZ;
@@ -213,7 +222,6 @@ __global__ __launch_bounds__(KS * 64, WPE) void stream_kernel(StreamArgs g) {
 
     if (wave < n) {
         const int mine = (n - wave + KS - 1) / KS;   // entries wave, wave + KS, ...
-        ent += wave;
         auto a_src = [&](int2 e) { return uniform_ptr(A + (size_t)e.x * C::ROWB); };
         auto w_src = [&](int2 e) { return uniform_ptr(D + (size_t)e.y * (1024 * ESZ)); };
         constexpr int NISSUE = C::A_DMA + C::W_DMA;
@@ -273,8 +281,6 @@ __global__ __launch_bounds__(KS * 64, WPE) void stream_kernel(StreamArgs g) {
             }
         };
 
-        // this wave's next 64 entries, one per lane
-        int2 ev = ent[(size_t)(lane < mine ? lane : mine - 1) * KS];
         auto entry = [&](int i) __attribute__((always_inline)) {
             return make_int2(__builtin_amdgcn_readlane(ev.x, i & 63), __builtin_amdgcn_readlane(ev.y, i & 63));
         };
