@@ -94,6 +94,22 @@ static __device__ __forceinline__ uint4 buffer16(const unsigned char* base_unifo
     return __builtin_bit_cast(uint4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
 }
 
+// A buffer of `bytes` bytes (below 2^32) at a wave-uniform address, and the same from `voff` on in it: lanes whose 16 bytes lie behind its end
+// read nothing and put zeros in the LDS.  (All of an offset is in voff: what the instruction adds from a scalar register is no part of
+// its check.)
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ u32x4_t bounded_buffer(const unsigned char* base_uniform, unsigned bytes) {
+    const uint64_t at = reinterpret_cast<uint64_t>(base_uniform);
+    return u32x4_t{(unsigned)__builtin_amdgcn_readfirstlane((uint32_t)at), (unsigned)__builtin_amdgcn_readfirstlane((uint32_t)(at >> 32)),
+                   (unsigned)__builtin_amdgcn_readfirstlane(bytes), 0x00020000u};
+}
+static __device__ __forceinline__ void dma16_bounded(unsigned lds_base_uniform, u32x4_t buffer, unsigned voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\t"
+                 :
+                 : "s"(lds_base_uniform), "v"(voff), "s"(buffer)
+                 : "memory");
+}
+
 // wait until at most n (wave-uniform) of this wave's DMA loads are outstanding, make this wave's
 // LDS accesses complete, and meet the other waves.  Loads retire in order, so a smaller n than
 // necessary is only slower, never wrong.

@@ -680,6 +680,8 @@ constexpr size_t ROW_WORKSPACE_BYTES = 64u << 20;
 // 98 -> 86 us, 4096 -> 4096 density 0.25, 16384 tokens 1267 -> 1091).  Between 2^21 and 2^22 its time is 0.7 to 1.24 of the fp32 kernel's and the estimates do not tell which
 // (25 problems, 0.95 on average; 3072 -> 768 with Zipf rows 52 and 48 us, 2016 -> 1408 at 2779 tokens 51 and 63), below 2^21 the same on average.
 constexpr long long SPLIT_BACK_WORK = 1ll << 22;
+// a chunk of 32 tokens that has 4 GB or more: it is not addressed as one buffer
+static bool row_far(int esz, int N, int K) { return (long long)(N > K ? N : K) * esz * ROW_TC >= (1ll << 32); }
 struct RowChoice {
     int slices, passes;
     bool split;
@@ -706,7 +708,7 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_
             }
         };
         consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16);
-        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK) consider(ROW_SPLIT);
+        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK && !row_far(4, N, K)) consider(ROW_SPLIT);
     }
     const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
     if (rectangles && fits && rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
@@ -812,7 +814,7 @@ static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, siz
     for (int pass = 0; pass < p.passes; ++pass) {
         r.chunk0 = pass * p.slices * p.chunks_per_slice;
         r.add = pass > 0;
-        const auto kernel = sizeof(T) == 4 && p.split ? sdd_split_kernel : sdd_row_kernel<T>;
+        const auto kernel = sizeof(T) == 4 && p.split ? sdd_split_kernel : (row_far(sizeof(T), a.N, a.K) ? sdd_row_kernel<T, true> : sdd_row_kernel<T, false>);
         if (int rc = launch(kernel, dim3((unsigned)grid), dim3(ROW_NW * 64), 0, stream, r)) return rc;
     }
     return p.partial_bytes ? launch_reduce<T>(r.partial, a, p.slices, stream) : PBS_OK;

@@ -187,14 +187,6 @@ struct RowFrag<float> {
     __device__ __forceinline__ void read(const unsigned char* piece, int s, int lane) {
         v[s] = *reinterpret_cast<const float2*>(piece + s * 512 + lane * 8);
     }
-    // the piece straight from memory, tokens from `end` on as zeros
-    __device__ __forceinline__ void fetch(const unsigned char* base, size_t stride, int end, int lane) {
-#pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const int t = 4 * s + (lane >> 4);
-            v[s] = t < end ? *reinterpret_cast<const float2*>(base + (size_t)t * stride + (lane & 15) * 8) : make_float2(0.f, 0.f);
-        }
-    }
     __device__ __forceinline__ void sum(float (&o)[2]) const {   // (in pairs: an eighth of the additions to the running sum)
         static_assert(STEPS == 8, "three levels");
         o[0] += ((v[0].x + v[1].x) + (v[2].x + v[3].x)) + ((v[4].x + v[5].x) + (v[6].x + v[7].x));
@@ -223,18 +215,6 @@ struct RowFrag<bf16_t> {
             v[a] = make_uint4(lo.x, lo.y, hi.x, hi.y);
         }
     }
-    __device__ __forceinline__ void fetch(const unsigned char* base, size_t stride, int end, int lane) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            uint32_t w[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int tok = 8 * (lane >> 4) + t;
-                w[t] = tok < end ? *reinterpret_cast<const uint16_t*>(base + (size_t)tok * stride + feature(lane & 15, a) * 2) : 0u;
-            }
-            v[a] = make_uint4(w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16);
-        }
-    }
     __device__ __forceinline__ void sum(float (&o)[2]) const {
 #pragma unroll
         for (int a = 0; a < 2; ++a)
@@ -258,8 +238,28 @@ struct SddRowCfg {
     static constexpr int WPE = sizeof(T) == 4 ? 2 : 3;   // waves per SIMD: LDS allows the former, registers the latter
 };
 
+// The pieces of a matrix of M rows: D DMA instructions of ROWS rows each, zeros for rows behind the last one, so that a matrix's last chunk is one like
+// the others.  FAR: chunks of 4 GB and more, each instruction then has a buffer of its own.
+template <bool FAR, int D, int ROWS>
+struct RowSource {
+    const unsigned char* base;
+    size_t stride;
+    int M;
+    unsigned voff[FAR ? 1 : D];
+    __device__ __forceinline__ RowSource(const unsigned char* base, size_t stride, int M, int row, int place) : base(base), stride(stride), M(M) {
+#pragma unroll
+        for (int i = 0; i < (FAR ? 1 : D); ++i) voff[i] = (unsigned)(i * ROWS + row) * (unsigned)stride + place * 16;
+    }
+    __device__ __forceinline__ void dma(unsigned lds, int chunk, unsigned column_bytes, int i) const {
+        const int t0 = chunk * ROW_TC + (FAR ? i * ROWS : 0), rows = FAR ? ROWS : ROW_TC;
+        const int left = M - t0 < rows ? M - t0 : rows;
+        dma16_bounded(lds, bounded_buffer(base + (size_t)t0 * stride + (FAR ? column_bytes : 0), FAR && left < 0 ? 0u : (unsigned)left * (unsigned)stride),
+                      voff[FAR ? 0 : i] + (FAR ? 0 : column_bytes));
+    }
+};
+
 // Chunks c_lo .. c_hi - 1 of a unit of NB blocks.
-template <typename T, int NB>
+template <typename T, int NB, bool FAR>
 static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const int* __restrict__ unit, int c_lo, int c_hi, float* partial,
                                                     unsigned char* smem, int lane, int wave) {
     using E = Elem<T>;
@@ -277,8 +277,6 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     }
     const bool sums = a.bias_out && unit[2] == 0;
 
-    const int whole = a.M / ROW_TC;              // chunks below this one are whole
-    const int full_hi = whole < c_hi ? whole : c_hi;
     const size_t gs = (size_t)a.N * ESZ, xs = (size_t)a.K * ESZ;   // row strides
     const unsigned char* G = static_cast<const unsigned char*>(a.g) + (size_t)row * (32 * ESZ);
     const unsigned char* X = static_cast<const unsigned char*>(a.x);
@@ -287,13 +285,11 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     constexpr int GS = NB == 1 || NB == 2 ? 2 : 1, XS = ROW_PIECES - GS;
     unsigned char* mem = smem + wave * C::WAVE_LDS;
     const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)mem);
-    // DMA instruction i of a piece: tokens RPI i + lane / CPR, 16 bytes per lane
-    const unsigned gv = (unsigned)((lane / CPR) * (a.N * ESZ) + (lane % CPR) * 16), xv = (unsigned)((lane / CPR) * (a.K * ESZ) + (lane % CPR) * 16);
-    auto dma_g = [&](int slot, int chunk, int i) __attribute__((always_inline)) {
-        dma16(lds + slot * PIECE + i * 1024, uniform_ptr(G + ((size_t)chunk * ROW_TC + RPI * i) * gs), gv);
-    };
+    // DMA instruction i of a piece: tokens RPI i + lane / CPR, 16 bytes per lane; zeros for tokens behind the matrix's last one
+    RowSource<FAR, D, RPI> from_g(G, gs, a.M, lane / CPR, lane % CPR), from_x(X, xs, a.M, lane / CPR, lane % CPR);
+    auto dma_g = [&](int slot, int chunk, int i) __attribute__((always_inline)) { from_g.dma(lds + slot * PIECE + i * 1024, chunk, 0, i); };
     auto dma_x = [&](int slot, int chunk, int c, int i) __attribute__((always_inline)) {
-        dma16(lds + (GS + slot) * PIECE + i * 1024, uniform_ptr(X + ((size_t)chunk * ROW_TC + RPI * i) * xs + (size_t)c * (32 * ESZ)), xv);
+        from_x.dma(lds + (GS + slot) * PIECE + i * 1024, chunk, c * (32 * ESZ), i);
     };
 
     f32x4 acc[NBX][2][2];
@@ -328,8 +324,8 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     }
 
     int chunk = c_lo + wave;
-    if (chunk < full_hi) {
-        const int last = chunk + (full_hi - 1 - chunk) / ROW_NW * ROW_NW;   // this wave's last whole chunk
+    if (chunk < c_hi) {
+        const int last = chunk + (c_hi - 1 - chunk) / ROW_NW * ROW_NW;   // this wave's last chunk
         auto after = [&](int c, int n) { return c + n * ROW_NW <= last ? c + n * ROW_NW : last; };   // (past the end: the last one again)
         F gf, xf;
         // piece k is block k % NB of chunk k / NB
@@ -405,20 +401,6 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
         wait_dma(0);   // the sums below use the same space
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    // the ragged last chunk of the matrix
-    if (whole * ROW_TC < a.M && whole >= c_lo && whole < c_hi && (whole - c_lo) % ROW_NW == wave) {
-        const int end = a.M - whole * ROW_TC;
-        F gf, xf;
-        gf.fetch(G + (size_t)whole * ROW_TC * gs, gs, end, lane);
-        if (sums) gf.sum(bsum);
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            xf.fetch(X + (size_t)whole * ROW_TC * xs + (size_t)cblk[b] * (32 * ESZ), xs, end, lane);
-#pragma unroll
-            for (int s = 0; s < F::STEPS; ++s) F::mma(acc[b], gf, xf, s);
-        }
-    }
-
     if constexpr (TOTALS) {
 #pragma unroll
         for (int b = 0; b < NBX; ++b)
@@ -525,7 +507,7 @@ static __device__ __forceinline__ bool row_task(const SddRowArgs& a, RowTask& t)
     return true;
 }
 
-template <typename T>
+template <typename T, bool FAR>
 __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel(SddRowArgs a) {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[SddRowCfg<T>::LDS];
     const int lane = threadIdx.x & 63;
@@ -533,12 +515,12 @@ __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel
     RowTask t;
     if (!row_task(a, t)) return;
     switch (t.unit[1]) {
-        case 4: sdd_row_body<T, 4>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
-        case 3: sdd_row_body<T, 3>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
-        case 2: sdd_row_body<T, 2>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
-        case 1: sdd_row_body<T, 1>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 4: sdd_row_body<T, 4, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 3: sdd_row_body<T, 3, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 2: sdd_row_body<T, 2, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 1: sdd_row_body<T, 1, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         default:
-            if (a.bias_out) sdd_row_body<T, 0>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave);
+            if (a.bias_out) sdd_row_body<T, 0, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave);
             break;
     }
 }

@@ -28,14 +28,6 @@ struct HalfRaw {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const float*>(p + e * 256);
     }
-    // straight from memory, tokens from `end` on as zeros
-    __device__ __forceinline__ void fetch(const unsigned char* base, size_t stride, int kk, int end, int lane) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int t = 16 * kk + 2 * e + (lane >> 5);
-            v[e] = t < end ? *reinterpret_cast<const float*>(base + (size_t)t * stride + (lane & 31) * 4) : 0.f;
-        }
-    }
     __device__ __forceinline__ float sum() const { return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])); }
 };
 struct HalfParts {
@@ -75,19 +67,17 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
     }
     const bool sums = a.bias_out && unit[2] == 0;
 
-    const int whole = a.M / ROW_TC;              // chunks below this one are whole
-    const int full_hi = whole < c_hi ? whole : c_hi;
     const size_t gs = (size_t)a.N * 4, xs = (size_t)a.K * 4;   // row strides
     const unsigned char* G = static_cast<const unsigned char*>(a.g) + (size_t)row * 128;
     const unsigned char* X = static_cast<const unsigned char*>(a.x);
     unsigned char* mem = smem + wave * C::WAVE_LDS;   // GS pieces of G, XS of X
     const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)mem);
-    const unsigned gv = (unsigned)((lane / 8) * (a.N * 4) + (lane % 8) * 16), xv = (unsigned)((lane / 8) * (a.K * 4) + (lane % 8) * 16);
+    RowSource<false, 4, 8> from_g(G, gs, a.M, lane / 8, lane % 8), from_x(X, xs, a.M, lane / 8, lane % 8);
     auto dma_g = [&](int slot, int chunk, int i) __attribute__((always_inline)) {
-        dma16(lds + slot * PIECE + i * 1024, uniform_ptr(G + ((size_t)chunk * ROW_TC + 8 * i) * gs), gv);
+        from_g.dma(lds + slot * PIECE + i * 1024, chunk, 0, i);
     };
     auto dma_x = [&](int slot, int chunk, int c, int i) __attribute__((always_inline)) {
-        dma16(lds + (GS + slot) * PIECE + i * 1024, uniform_ptr(X + ((size_t)chunk * ROW_TC + 8 * i) * xs + (size_t)c * 128), xv);
+        from_x.dma(lds + (GS + slot) * PIECE + i * 1024, chunk, c * 128, i);
     };
 
     f32x16 total[NB], part[2];
@@ -100,8 +90,8 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
     float bsum = 0.f;
 
     int chunk = c_lo + wave;
-    if (chunk < full_hi) {
-        const int last = chunk + (full_hi - 1 - chunk) / ROW_NW * ROW_NW;   // this wave's last whole chunk
+    if (chunk < c_hi) {
+        const int last = chunk + (c_hi - 1 - chunk) / ROW_NW * ROW_NW;   // this wave's last chunk
         auto after = [&](int c, int n) { return c + n * ROW_NW <= last ? c + n * ROW_NW : last; };   // (past the end: the last one again)
         // X piece q is block q % NB of this wave's chunk q / NB, in slot q % XS
 #pragma unroll
@@ -211,33 +201,6 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
         wait_dma(0);   // the sums below use the same space
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    // the ragged last chunk of the matrix
-    if (whole * ROW_TC < a.M && whole >= c_lo && whole < c_hi && (whole - c_lo) % ROW_NW == wave) {
-        const int end = a.M - whole * ROW_TC;
-        HalfRaw gr[2], xr;
-        HalfParts gp[2], xp[2];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            gr[kk].fetch(G + (size_t)whole * ROW_TC * gs, gs, kk, end, lane);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) gp[kk].split(gr[kk], i);
-        }
-        if (sums) bsum += gr[0].sum() + gr[1].sum();
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                xr.fetch(X + (size_t)whole * ROW_TC * xs + (size_t)cblk[b] * 128, xs, kk, end, lane);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xp[kk].split(xr, i);
-#pragma unroll
-                for (int m = 0; m < 5; ++m) small_mma(part[0], gp[kk], xp[kk], m, kk == 0);
-            }
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) mma_parts(part[0], gp[kk].part(0), xp[kk].part(0));
-            total[b] += part[0];
-        }
-    }
 
     // ---- the waves' sums meet in LDS, two blocks at a time: wave 2 k + jj stores columns 16 jj .. + 15 of block k ----
     f32x4* red = reinterpret_cast<f32x4*>(smem);
@@ -344,7 +307,7 @@ __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<float>::WPE) void sdd_split_
         case 2: sdd_split_body<2>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         case 1: sdd_split_body<1>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         default:
-            if (a.bias_out) sdd_row_body<float, 0>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave);
+            if (a.bias_out) sdd_row_body<float, 0, false>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave);
             break;
     }
 }

@@ -45,6 +45,55 @@ def test_row_kernel(cuda, dtype, tokens, out_f, in_f, counts, slices):
     assert_close(bias.grad, to64(dy).sum(0), dtype, "bias gradient")
 
 
+def _followed_by_nan(shape, dtype, device, seed):
+    """A tensor whose memory goes on with NaN behind its last row."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    whole = torch.full((shape[0] + 64, shape[1]), float("nan"), dtype=dtype, device=device)
+    whole[:shape[0]] = torch.randn(shape, generator=g, device=device).to(dtype)
+    return whole[:shape[0]]
+
+
+@pytest.mark.parametrize("dtype, out_f, in_f, counts, kernel", [
+    (torch.float32, 384, 416, ROWS, "sdd_row_kernel"), (torch.bfloat16, 384, 416, ROWS, "sdd_row_kernel"),
+    (torch.float32, 4096, 4096, [120, 1, 2, 3], "sdd_split_kernel"),
+])
+@pytest.mark.parametrize("past", [1, 7, 8, 9, 15, 16, 17, 24, 31])
+def test_last_chunk_ends_with_the_matrix(cuda, dtype, out_f, in_f, counts, kernel, past):
+    """Tokens behind the last one count as zeros, whatever the memory there holds; a copy instruction covers 8 (fp32) or 16 (bf16) of a chunk's 32."""
+    tokens = (1184 if kernel == "sdd_split_kernel" else 96) + past
+    m = _layer(out_f, in_f, counts, dtype, cuda, past)
+    name = native.matmul_back_kernel_name(tokens, out_f, in_f, m.cols_a.shape[0], dtype)
+    print(name, tokens, out_f, in_f, dtype, flush=True)
+    assert name.startswith(kernel)
+    x, dy = _followed_by_nan((tokens, in_f), dtype, cuda, 1), _followed_by_nan((tokens, out_f), dtype, cuda, 2)
+    data, bias = m.data.detach().clone().requires_grad_(), torch.zeros(out_f, dtype=dtype, device=cuda, requires_grad=True)
+    native.torch_path().linear(x, data, bias, m._buffers, m.schedule()).backward(dy)
+    at = m.build_coo_block_index().long()
+    dense = dy.double().t().contiguous() @ x.double()
+    want = dense.reshape(out_f // 32, 32, in_f // 32, 32).permute(0, 2, 3, 1)[at[0], at[1]].reshape(-1, 32)
+    # (rtol of the oracle comparisons above; bf16: half a unit of the result)
+    limit = 1e-6 if dtype == torch.float32 else 2.0 ** -8
+    assert (data.grad.double() - want).norm() <= limit * want.norm()
+    assert (bias.grad.double() - dy.double().sum(0)).norm() <= limit * dy.double().sum(0).norm()
+
+
+@pytest.mark.parametrize("dtype, out_f", [(torch.float32, 1 << 25), (torch.bfloat16, 1 << 26)])
+def test_chunks_of_four_gigabytes(cuda, dtype, out_f):
+    """A chunk of 32 tokens that is too large to be addressed as one buffer."""
+    rows, tokens = [0, 5, out_f // 64, out_f // 32 - 1], 45
+    m = BlockSparseMatrix.zeros((out_f, 64), blocks=[(r, r % 2) for r in rows], device=cuda, dtype=dtype)
+    dy = torch.zeros(tokens, out_f, dtype=dtype, device=cuda)
+    torch.manual_seed(2)
+    x = torch.randn(tokens, 64, device=cuda).to(dtype)
+    for r in rows:
+        dy[:, 32 * r:32 * r + 32] = torch.randn(tokens, 32, device=cuda).to(dtype)
+    print(dtype, out_f, flush=True)
+    got = m.matmul_with_output_sparse_support(dy, x).double()
+    at = m.build_coo_block_index().tolist()
+    want = torch.cat([x[:, 32 * c:32 * c + 32].double().t().contiguous() @ dy[:, 32 * r:32 * r + 32].double() for r, c in zip(*at)])
+    assert (got - want).norm() <= (1e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
 @pytest.mark.parametrize("tokens,out_f,in_f,counts", [
     (16391, 1600, 512, [7, 0, 3, 16]),     # one rectangle per band sums all 16 rows; the last band has two
     (17000, 1024, 544, [9, 1]),            # two rectangles share the rows, the second with a single column
