@@ -21,7 +21,7 @@
 //   fp32 768 -> 3072 density 0.5, 4096 tokens 123 -> 96, 1024 tokens 56 -> 33;  3072 -> 768 density 0.25 with uneven rows, 4096 tokens
 //   78 -> 50;  768 -> 768 density 0.5, 16384 tokens 122 -> 98;  4096 -> 4096 density 0.25, 16384 tokens 1250 -> 1129 (122 of
 //   155 TFLOP/s);  3072 -> 768 density 0.5, 101 tokens 23 -> 8.7.
-//   bf16 768 -> 3072 density 0.5, 2317 tokens 48 -> 34;  4096 -> 4096 density 0.25, 509 tokens 38 -> 29, 64 tokens 21 -> 8.3.
+//   bf16 768 -> 3072 density 0.5, 2317 tokens 48 -> 28;  4096 -> 4096 density 0.25, 509 tokens 38 -> 29, 64 tokens 21 -> 8.3.
 #pragma once
 #include <type_traits>
 
@@ -239,7 +239,9 @@ struct SddRowCfg {
 };
 
 // The pieces of a matrix of M rows: D DMA instructions of ROWS rows each, zeros for rows behind the last one, so that a matrix's last chunk is one like
-// the others.  FAR: chunks of 4 GB and more, each instruction then has a buffer of its own.
+// the others.  (Loaded by itself behind the loop, one piece after the other and in bf16 two bytes at a time, it cost a workgroup 1 to 6 us: bf16 768 -> 3072
+// density 0.5, 2317 tokens 32.7 -> 28.2, 140 tokens 9.3 -> 5.8; 768 -> 768, 1037 tokens 14.95 -> 9.35, fp32 14.9 -> 13.7; 448 -> 2080 density 0.62, 9336 tokens, in
+// sdd_split_kernel 104 -> 98.  Whole token counts the same to within 1 %.)  FAR: chunks of 4 GB and more, each instruction then has a buffer of its own.
 template <bool FAR, int D, int ROWS>
 struct RowSource {
     const unsigned char* base;
