@@ -623,30 +623,41 @@ static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
     p.tokens_per_split = (int)(chunks_per * TC);
     return p;
 }
-// Estimated time in us, fitted to problems of 256 .. 4096 features, 64 .. 16384 tokens, densities 0.05 .. 0.75 at ten slice counts (fp32 80 below 2^22 tokens x
-// blocks, its choices 2.4 % slower than the best on average, 8.9 % by constants from before the tasks were dealt as they are; bf16 85, 2.0 %): launch, reduction of the slices,
-// chunks x blocks of a wave of the slowest workgroup, at the rate of a full chip or, below 32 workgroups per XCD, of
-// a wave alone, and what each round of workgroups on the chip costs besides.
+// Estimated time in us of units of at most per_unit blocks, in so many slices: launch, reduction of the slices, chunks of a wave of the slowest workgroup, at
+// the rate of a wave alone or of a chip that is full in rounds of 256 workgroups.  Fitted to problems of 256 .. 4096 features, 64 .. 16384 tokens, densities
+// 0.05 .. 0.75 at six sizes of units and eight numbers of slices (fp32: 80 below 2^22 tokens x blocks, within 9 %; bf16: 80 whose operands have less than 52 MB, within 7 %).  The
+// choices it makes are 3 and 1.3 % slower than the best on average, and 1.28 and 1.14 times as fast as units of four in the best number of slices that
+// an estimate of those alone made; two of each 80 are slower by more than 2 %, an fp32 one with very uneven rows by 20 %.
+// (The number of units follows from the average row, so what looks like a full chip may be one workgroup more than that: for fp32, whose rounds are long, the mean
+// of the estimated number and of 4 % more.  The reduction is a launch and an allocation more for the host: 2 (bf16 0.75) us more than the fit has for it.)
 enum RowKernel { ROW_F32, ROW_SPLIT, ROW_BF16 };   // sdd_row_kernel<float>, sdd_split_kernel, sdd_row_kernel<bf16_t>
-static double row_us(RowKernel kernel, long long M, int N, int nnz, int slices, int passes) {
+// workgroups of the fullest XCD
+static double row_tasks(double units, int slices) { return units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices; }
+static double row_us(RowKernel kernel, long long M, int N, int K, int nnz, int per_unit, int slices, int passes) {
+    const double chunks = (double)((M + ROW_TC - 1) / ROW_TC), wave = std::ceil(chunks / (ROW_NW * slices * (double)passes));
+    if (kernel == ROW_SPLIT) {
+        // (units of ROW_NB: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted
+        // without a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
+        const double rows = N / 32;
+        const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
+        const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
+        const double tasks = units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices;
+        const double busy = std::ceil(tasks / 32) * wave * blocks * 0.454, alone = wave * blocks * 0.540;
+        return (slices > 1 ? 3.02 : 0.0) + passes * (7.03 + (busy > alone ? busy : alone) + std::ceil(tasks / 64) * 4.5);
+    }
     struct Model {
-        double launch, reduce, per_slice, busy, alone, round;
-        int resident;   // workgroups per XCD
+        double more, launch, reduce, per_slice, alone, alone_row, busy, busy_row, most, whole, start;   // .._row: of a unit, besides its blocks
     };
-    // (ROW_F32: the fit of the kernels alone has 3.75 for the reduction.  It is a launch and an allocation more for the host as well, and the steps it decides are
-    // mostly the host's: of 991 drawn layers and 64 to 16384 tokens it decides 70, whose training steps take 36 or 62 us (the host's) and 3.6 us more with
-    // 3.75 at the median; 61 are more than 2 % slower with it, 2 faster, by 2 and 6 %.)
-    // (ROW_SPLIT: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted without
-    // a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
-    const Model m = kernel == ROW_F32 ? Model{2.22, 6.3, 0.033, 0.577, 0.608, 2.67, 64}
-                  : kernel == ROW_SPLIT ? Model{7.03, 3.02, 0.0, 0.454, 0.540, 4.5, 64} : Model{5.13, 4.32, 1.0, 0.2025, 0.237, 0.83, 96};
-    const double rows = N / 32, chunks = (double)((M + ROW_TC - 1) / ROW_TC);
-    const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
-    const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
-    const double tasks = units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices, wave = std::ceil(chunks / (ROW_NW * slices * (double)passes)) * blocks;
-    const double busy = std::ceil(tasks / 32) * wave * m.busy, alone = wave * m.alone;
-    return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) +
-           passes * (m.launch + (busy > alone ? busy : alone) + std::ceil(tasks / m.resident) * m.round);
+    const Model m = kernel == ROW_F32 ? Model{1.04, 3.43, 4.82, 0.973, 0.581, 0.113, 0.549, 0.124, 0.340, 0.880, 0.0191}
+                                      : Model{1.0, 3.12, 3.5, 1.31, 0.171, 0.179, 0.140, 0.184, 0.272, 1.0, 0.0128};
+    const double rows = N / 32, row = nnz / rows, columns = K / 32;
+    const double full = nnz / (double)per_unit + rows * (per_unit - 1) / (2.0 * per_unit) * (1.0 - std::exp(-2.0 * row)), units = full + rows * std::exp(-row);
+    const double mean = nnz / full, most = per_unit < columns ? per_unit : columns;   // blocks of a unit
+    const double tasks = row_tasks(units, slices), tasks_more = m.more > 1.0 ? row_tasks(m.more * units, slices) : tasks;
+    const double alone = wave * (m.alone * (mean + m.most * (most - mean)) + m.alone_row);
+    const double rounds = 0.5 * (m.whole * (std::ceil(tasks / 32) + std::ceil(tasks_more / 32)) + (1.0 - m.whole) * (tasks + tasks_more) / 32);
+    const double busy = rounds * wave * (m.busy * mean + m.busy_row);
+    return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) + passes * (m.launch + (busy > alone ? busy : alone) + 0.5 * (tasks + tasks_more) * m.start);
 }
 // Launch; per round of workgroups and chunk what a pass costs and what the blocks of a wave cost; reduction of the slices (75 problems, 256 .. 16384
 // tokens, 256 .. 4096 features, densities 0.05 .. 0.95, one in seven with uneven rows: within 11 % for 16 rows and 9 % for 8).
@@ -683,32 +694,37 @@ constexpr long long SPLIT_BACK_WORK = 1ll << 22;
 // a chunk of 32 tokens that has 4 GB or more: it is not addressed as one buffer
 static bool row_far(int esz, int N, int K) { return (long long)(N > K ? N : K) * esz * ROW_TC >= (1ll << 32); }
 struct RowChoice {
-    int slices, passes;
+    int slices, passes, per_unit;
     bool split;
 };
-static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
+static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool lists, size_t workspace_limit) {
     constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
     const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
     // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 198.
     // (rectangles count the bytes of a chunk in 31 bits)
     const bool rectangles = dtype == PBS_DTYPE_BF16 && N < (1 << 25) && K < (1 << 25);
-    if (rectangles && bytes > 52e6) return {0, 1, false};
+    if (rectangles && bytes > 52e6) return {0, 1, ROW_NB, false};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
-    RowChoice best{1, 1, false};
+    RowChoice best{1, 1, ROW_NB, false};
     double best_us = -1.0;
+    const bool far = row_far(dtype == PBS_DTYPE_F32 ? 4 : 2, N, K), one_list = far || unit_lists_only(N / 32);
     for (const int s : CANDIDATES) {
         if (s > 1 && (s > chunks / 4 || (size_t)nnz * 4096 * s > workspace_limit)) break;
         const int passes = at_least > s ? (int)std::ceil(at_least / s) : 1;
-        auto consider = [&](RowKernel kernel) {
-            const double us = row_us(kernel, M, N, nnz, s, passes);
+        auto consider = [&](RowKernel kernel, int per_unit) {
+            // (a table of larger lists, made in the workspace, takes of the memory of the partial sums: what they and the list of ROW_NB may have stays the bound)
+            if (!lists && per_unit != ROW_NB && (s > 1 ? (size_t)nnz * 4096 * s : 0) + unit_table_bytes(N, nnz, per_unit) > workspace_limit + unit_table_bytes(N, nnz, ROW_NB)) return;
+            // (fp32: sums of longer shares would be less exact than those of units of four in several slices)
+            if (kernel == ROW_F32 && per_unit != ROW_NB && chunks > (long long)(per_unit > ROW_NB ? ROW_LONG : ROW_LONG_GROUPS) * ROW_NW * s * passes) return;
+            const double us = row_us(kernel, M, N, K, nnz, per_unit, s, passes);
             if (best_us < 0.0 || us < best_us) {
-                best = {s, passes, kernel == ROW_SPLIT};
+                best = {s, passes, per_unit, kernel == ROW_SPLIT};
                 best_us = us;
             }
         };
-        consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16);
-        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK && !row_far(4, N, K)) consider(ROW_SPLIT);
+        for (int p = one_list ? ROW_NB : 1; p <= (one_list ? ROW_NB : ROW_SIZES); ++p) consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16, p);
+        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK && !far) consider(ROW_SPLIT, ROW_NB);
     }
     const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
     if (rectangles && fits && rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
@@ -716,16 +732,18 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, size_
 }
 struct BackPlan {
     int slices;   // row kernel; 0: rectangles
+    int per_unit; // blocks of a unit, at most
     bool split;   // fp32 in parts
     int passes, chunks_per_slice;
     SddPlan rect;
     int partials;            // sums of this many slices in the workspace, or none
     size_t partial_bytes;
 };
-static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, size_t workspace_limit) {
+static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, bool lists, size_t workspace_limit) {
     BackPlan p;
-    const RowChoice row = choose_row(dtype, M, N, K, nnz, workspace_limit);
+    const RowChoice row = choose_row(dtype, M, N, K, nnz, lists, workspace_limit);
     p.slices = row.slices;
+    p.per_unit = row.per_unit;
     p.split = row.split;
     p.rect = plan_sdd(M, N, K, nnz);
     // (the workspace of sixteen rows also where eight need less: what an entry point without one refuses does not follow the estimates)
@@ -741,19 +759,22 @@ static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, si
     p.partials = n > 1 ? n : 0;
     return p;
 }
-static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
-    // (a gradient asks three times, for the unit table, for the size of its workspace and when it is launched: the last answer of a thread, by the
-    // sizes it follows from)
+// `lists`: the caller brings a table with all lists of units
+static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, bool lists, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
+    // (a gradient asks three times, for the unit table, for the size of its workspace and when it is launched: the last answers of a thread, by the
+    // sizes they follow from)
     struct Answer {
         int dtype;
         long long M;
         int N, K, nnz;
+        bool lists;
         size_t workspace_limit;
         BackPlan plan;
     };
-    static thread_local Answer last{-1, 0, 0, 0, 0, 0, {}};
-    if (last.dtype != dtype || last.M != M || last.N != N || last.K != K || last.nnz != nnz || last.workspace_limit != workspace_limit)
-        last = Answer{dtype, M, N, K, nnz, workspace_limit, plan_back_anew(dtype, M, N, K, nnz, workspace_limit)};
+    static thread_local Answer kept[16] = {};   // (a model's layers in turn; tokens is never 0 here)
+    Answer& last = kept[(unsigned)((((unsigned)M * 31u + N) * 31u + K) * 31u + nnz + dtype) * 2654435761u >> 28];
+    if (last.dtype != dtype || last.M != M || last.N != N || last.K != K || last.nnz != nnz || last.lists != lists || last.workspace_limit != workspace_limit)
+        last = Answer{dtype, M, N, K, nnz, lists, workspace_limit, plan_back_anew(dtype, M, N, K, nnz, lists, workspace_limit)};
     BackPlan p = last.plan;
     p.partial_bytes = ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * p.partials;   // fp32 sums of each slice: blocks, bias columns
     return p;
@@ -762,22 +783,22 @@ static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bi
 struct BackArgs {
     const void *g, *x;       // [M, N] grad_output, [M, K] input
     const int32_t *ptr, *idx;
-    const void* units;       // nullptr: built in the workspace
+    const void* units;       // nullptr: built in the workspace, if it is needed
+    bool lists;              // it would have all lists
     void* out;               // [nnz*32, 32]
     void* bias_out;          // nullptr or [N]
     int M, N, K, nnz;
 };
 
-static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int nnz, void* table, hipStream_t stream) {
-    const long long units = unit_bound(N, nnz);
+static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int nnz, int only, void* table, hipStream_t stream) {
     int* t = static_cast<int*>(table);
     int* before = nullptr;
     if (unit_prefix_bytes(N)) {
-        before = t + 16 + units * UNIT_INTS;
-        if (int rc = launch(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, before)) return rc;
+        before = t + unit_lists_ints(N, nnz, only);
+        if (int rc = launch(unit_prefix_kernel, dim3(1), dim3(1024), 0, stream, ptr, nnz, N / 32, only, before)) return rc;
     }
-    const UnitArgs a{ptr, idx, nnz, N / 32, K / 32, before, (int)units, t};
-    return launch(unit_table_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, a);
+    const UnitArgs a{ptr, idx, nnz, N / 32, K / 32, before, only, t};
+    return launch(unit_table_kernel, dim3(unit_table_grid(N / 32, nnz, only)), dim3(256), 0, stream, a);
 }
 
 template <typename T>
@@ -789,19 +810,22 @@ static int launch_reduce(const float* partial, const BackArgs& a, int nsplit, hi
 
 template <typename T>
 static int launch_row(const BackArgs& a, const BackPlan& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    const size_t need = p.partial_bytes + (a.units ? 0 : unit_table_bytes(a.N, a.nnz));
+    const int only = a.units ? unit_lists_only(a.N / 32) : p.per_unit;
+    const size_t need = p.partial_bytes + (a.units ? 0 : unit_table_bytes(a.N, a.nnz, only));
     if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
-    const long long grid = NUM_XCD * (long long)p.slices * ((unit_bound(a.N, a.nnz) + NUM_XCD - 1) / NUM_XCD);
+    const long long grid = NUM_XCD * (long long)p.slices * ((unit_bound(a.N / 32, a.nnz, p.per_unit) + NUM_XCD - 1) / NUM_XCD);
     if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
     SddRowArgs r;
     r.g = a.g;
     r.x = a.x;
-    r.table = static_cast<const int*>(a.units);
+    const int* table = static_cast<const int*>(a.units);
     if (!a.units) {
-        void* table = static_cast<unsigned char*>(workspace) + p.partial_bytes;
-        if (int rc = build_units(a.ptr, a.idx, a.N, a.K, a.nnz, table, stream)) return rc;
-        r.table = static_cast<const int*>(table);
+        void* t = static_cast<unsigned char*>(workspace) + p.partial_bytes;
+        if (int rc = build_units(a.ptr, a.idx, a.N, a.K, a.nnz, only, t, stream)) return rc;
+        table = static_cast<const int*>(t);
     }
+    r.count = table + p.per_unit - 1;
+    r.units = table + 16 + units_before(a.N / 32, a.nnz, p.per_unit, only) * UNIT_INTS;
     r.out = a.out;
     r.bias_out = a.bias_out;
     r.partial = p.partial_bytes ? static_cast<float*>(workspace) : nullptr;
@@ -1070,7 +1094,7 @@ static bool back_sizes_ok(int64_t tokens, int out_features, int in_features, int
 
 size_t pbs_blocksparse_matmul_back_units_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
-    return plan_back(dtype, tokens, out_features, in_features, nnz, false).slices > 0 ? unit_table_bytes(out_features, nnz) : 0;
+    return plan_back(dtype, tokens, out_features, in_features, nnz, false, true).slices > 0 ? unit_table_bytes(out_features, nnz, unit_lists_only(out_features / 32)) : 0;
 }
 
 int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int32_t* cols_a, int out_features, int in_features,
@@ -1079,20 +1103,21 @@ int pbs_blocksparse_matmul_back_units(const int32_t* row_start_ends_a, const int
     if ((long long)nnz > (long long)(out_features / 32) * (in_features / 32)) return PBS_ERR_TOO_LARGE;
     if (!row_start_ends_a || (nnz > 0 && !cols_a) || !units) return PBS_ERR_NULL_POINTER;
     if (!aligned16(units)) return PBS_ERR_MISALIGNED;
-    if (units_bytes < unit_table_bytes(out_features, nnz)) return PBS_ERR_WORKSPACE;
-    return build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, units, static_cast<hipStream_t>(stream));
+    const int only = unit_lists_only(out_features / 32);
+    if (units_bytes < unit_table_bytes(out_features, nnz, only)) return PBS_ERR_WORKSPACE;
+    return build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, only, units, static_cast<hipStream_t>(stream));
 }
 
 size_t pbs_blocksparse_matmul_back_bias_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype)) return 0;
-    return plan_back(dtype, tokens, out_features, in_features, nnz, true).partial_bytes;
+    return plan_back(dtype, tokens, out_features, in_features, nnz, true, true).partial_bytes;
 }
 
 size_t pbs_blocksparse_matmul_back_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz,
                                                    int dtype) {
     if (!back_sizes_ok(tokens, out_features, in_features, nnz, dtype) || nnz == 0) return 0;
-    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
-    return p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz) : 0);
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, false);
+    return p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz, p.per_unit) : 0);
 }
 
 int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_a, const int32_t* col_start_ends_b, const int32_t* rows_b,
@@ -1101,7 +1126,7 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
     if (int rc = plan_checks(row_start_ends_a, cols_a, out_features, in_features, nnz, plan_forward, plan_forward_bytes)) return rc;
     if (int rc = plan_checks(col_start_ends_b, rows_b, in_features, out_features, nnz, plan_input, plan_input_bytes)) return rc;
     if (units && !aligned16(units)) return PBS_ERR_MISALIGNED;
-    if (units && units_bytes < unit_table_bytes(out_features, nnz)) return PBS_ERR_WORKSPACE;
+    if (units && units_bytes < unit_table_bytes(out_features, nnz, unit_lists_only(out_features / 32))) return PBS_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int N = out_features / 32, K = in_features / 32;
     const bool with_units = units && !unit_prefix_bytes(out_features);   // (very tall matrices need a launch before that one)
@@ -1110,11 +1135,10 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
     a.list[1] = ListArgs{col_start_ends_b, rows_b, K, N, nnz, static_cast<int*>(plan_input)};
     a.grid[0] = (int)list_plan_grid(N);
     a.grid[1] = (int)list_plan_grid(K);
-    const long long bound = unit_bound(out_features, nnz);
-    a.units = UnitArgs{row_start_ends_a, cols_a, nnz, N, K, nullptr, (int)bound, with_units ? static_cast<int*>(units) : nullptr};
-    const long long grid = a.grid[0] + a.grid[1] + (with_units ? (bound + 255) / 256 : 0);
+    a.units = UnitArgs{row_start_ends_a, cols_a, nnz, N, K, nullptr, 0, with_units ? static_cast<int*>(units) : nullptr};
+    const long long grid = (long long)a.grid[0] + a.grid[1] + (with_units ? unit_table_grid(N, nnz, 0) : 0);
     if (int rc = launch(derive_kernel, dim3((unsigned)grid), dim3(256), 0, s, a)) return rc;
-    return units && !with_units ? build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, units, s) : PBS_OK;
+    return units && !with_units ? build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, unit_lists_only(N), units, s) : PBS_OK;
 }
 
 static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,
@@ -1137,7 +1161,7 @@ static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, s
             if (int rc = zero(a.out, (size_t)a.nnz * 1024)) return rc;
         return a.bias_out ? zero(a.bias_out, a.N) : PBS_OK;
     }
-    const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, a.bias_out != nullptr, workspace_limit);
+    const BackPlan p = plan_back(dtype, tokens, a.N, a.K, a.nnz, a.bias_out != nullptr, a.lists, workspace_limit);
     if (p.slices == 0) return a.bias_out ? launch_rectangles<true>(a, p, workspace, workspace_bytes, s) : launch_rectangles<false>(a, p, workspace, workspace_bytes, s);
     return dtype == PBS_DTYPE_F32 ? launch_row<float>(a, p, workspace, workspace_bytes, s) : launch_row<bf16_t>(a, p, workspace, workspace_bytes, s);
 }
@@ -1146,7 +1170,7 @@ int pbs_blocksparse_matmul_back(const void* dense_a, const void* dense_b, const 
                                 const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                 int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
                                 void* stream) {
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
     return back(a, tokens, dtype, workspace, workspace_bytes, stream);
 }
 
@@ -1155,7 +1179,7 @@ int pbs_blocksparse_matmul_back_bias(const void* dense_a, const void* dense_b, c
                                      int out_features, int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
                                      void* stream) {
     if (!units && pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, dtype) > 0) return PBS_ERR_NULL_POINTER;
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, units, data_out, bias_out, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, units, true, data_out, bias_out, (int)tokens, out_features, in_features, nnz};
     return back(a, tokens, dtype, workspace, workspace_bytes, stream);
 }
 
@@ -1252,13 +1276,13 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
                                         const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                         int in_features, int nnz, int dtype, void* stream) {
     // the array limits the number of slices of the row kernel; the rectangles' is fixed
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
     size_t need = 0, limit = 0;
     if (back_sizes_ok(tokens, out_features, in_features, nnz, dtype) && nnz > 0) {
-        const size_t table = unit_table_bytes(out_features, nnz);
+        const size_t table = unit_table_bytes(out_features, nnz, ROW_NB);
         limit = (size_t)PBS_NOALLOC_SCRATCH_BYTES > table ? (size_t)PBS_NOALLOC_SCRATCH_BYTES - table : 0;
-        const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, limit);
-        need = p.partial_bytes + (p.slices > 0 ? table : 0);
+        const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, false, limit);
+        need = p.partial_bytes + (p.slices > 0 ? unit_table_bytes(out_features, nnz, p.per_unit) : 0);
     }
     if (need > (size_t)PBS_NOALLOC_SCRATCH_BYTES) return PBS_ERR_SCRATCH;
     void* ws = nullptr;
@@ -1285,7 +1309,7 @@ const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_feat
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || out_features <= 0 || in_features <= 0 ||
         nnz <= 0 || (out_features % 32) || (in_features % 32))
         return "";
-    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false);
+    const BackPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, true);
     if (p.slices > 0 && p.split) return p.slices > 1 ? "sdd_split_kernel + sdd_reduce_kernel" : "sdd_split_kernel";
     if (p.slices > 0) return p.slices > 1 ? "sdd_row_kernel + sdd_reduce_kernel" : "sdd_row_kernel";
     return p.rect.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";

@@ -1,11 +1,11 @@
 // dense^T x dense -> block-sparse (weight gradient on the sparse support), and with it the bias gradient:
 //   out[32b + j][i] = sum_t G[t][32r + i] * X[t][32c + j]   for every data block b at (r, c),   bias[n] = sum_t G[t][n].
 //
-// A workgroup takes a unit, up to four blocks of one block row of W, over one slice of the tokens (in fp32, where the slices do not
+// A workgroup takes a unit, up to six blocks of one block row of W, over one slice of the tokens (in fp32, where the slices do not
 // fit the workspace, of a launch's range of them: a later launch adds to what it finds); each of its four waves
-// every fourth chunk of 32 tokens, with all accumulators of the unit (64 registers), so that nothing is shared until the
+// every fourth chunk of 32 tokens, with all accumulators of the unit (16 registers a block), so that nothing is shared until the
 // waves' sums meet in LDS at the end: no barrier and no wait for another wave in the loop, any shape of pattern makes
-// units of one size, and small problems have many workgroups.  A G fragment is read once for four products.
+// units of one size, and small problems have many workgroups.  A G fragment is read once for all products of a unit.
 //
 // What bounds it: the texture path that copies memory to LDS (a KB costs it 23 cycles in 128-byte rows, 35 in 64-byte ones)
 // and the matrix pipe.  fp32: 256 cycles of products per block and chunk against 4 + 4 / NB copies of 23 each: near the matrix rate
@@ -18,10 +18,10 @@
 // 8-byte read serves both); bf16 through transposing reads, the halves chosen so that eight result columns meet in a lane.
 //
 // Measured, us, against the kernels it replaced (fp32: equal shares of bands of 16 rows, barriers; bf16: rectangles):
-//   fp32 768 -> 3072 density 0.5, 4096 tokens 123 -> 96, 1024 tokens 56 -> 33;  3072 -> 768 density 0.25 with uneven rows, 4096 tokens
+//   fp32 768 -> 3072 density 0.5, 4096 tokens 123 -> 96, 1024 tokens 56 -> 30;  3072 -> 768 density 0.25 with uneven rows, 4096 tokens
 //   78 -> 50;  768 -> 768 density 0.5, 16384 tokens 122 -> 98;  4096 -> 4096 density 0.25, 16384 tokens 1250 -> 1129 (122 of
 //   155 TFLOP/s);  3072 -> 768 density 0.5, 101 tokens 23 -> 8.7.
-//   bf16 768 -> 3072 density 0.5, 2317 tokens 48 -> 28;  4096 -> 4096 density 0.25, 509 tokens 38 -> 29, 64 tokens 21 -> 8.3.
+//   bf16 768 -> 3072 density 0.5, 2317 tokens 48 -> 22;  4096 -> 4096 density 0.25, 509 tokens 38 -> 29, 64 tokens 21 -> 8.3.
 #pragma once
 #include <type_traits>
 
@@ -30,42 +30,69 @@
 
 namespace pbs {
 
-constexpr int ROW_NB = 4;       // blocks of a unit, at most
+constexpr int ROW_SIZES = 6;    // lists of units: of at most 1, 2, ... 6 blocks
+constexpr int ROW_NB = 4;       // sdd_split_kernel has registers for this many, and chunks of 4 GB take this list
 constexpr int ROW_NW = 4;       // waves of a workgroup: every ROW_NW-th chunk of tokens each
 constexpr int ROW_TC = 32;      // tokens per chunk
+constexpr int ROW_GROUP = 8;    // fp32, longer shares: chunks of a wave that are summed before they join its total
+constexpr int ROW_LONG = 12, ROW_LONG_GROUPS = 48;   // fp32: chunks of a wave, at most, in units without and with registers for that, other than those of ROW_NB
 constexpr int ROW_PARTS = 4;
 constexpr int ROW_PIECES = 5;   // LDS of a wave, in pieces of 32 tokens x 32 features
 
 // ---- unit table: what the workgroups of a pattern do ----
-// A unit is up to ROW_NB blocks of one block row: {row, blocks, number within the row, 0, columns [4], data blocks [4]} in 16
-// ints.  A row of n blocks has ceil(n / ROW_NB) units of equal size (+- 1), an empty row one without blocks (for the bias
+// A unit is up to P blocks of one block row: {row, blocks, number within the row, 0, columns [6], data blocks [6]} in 16
+// ints.  A row of n blocks has ceil(n / P) units of equal size (+- 1), an empty row one without blocks (for the bias
 // gradient).  Order: (quarter of the row's units, row, unit): units that run at the same time then read neighbouring columns of
-// X from a common L2.  The table starts with the number of units, padded to 16 ints.
+// X from a common L2.  The table starts with the numbers of units of the lists P = 1 .. ROW_SIZES, padded to 16 ints; then the lists, each in
+// room for unit_bound units.
+//
+// Why several lists: one workgroup per CU takes as long as its unit, one more than there are CUs takes twice as long, and small patterns of large
+// units leave most of the chip idle or need several slices of the tokens and their reduction.  The best list and number of slices of 80 problems each are,
+// on average, 1.28 (fp32) and 1.14 (bf16) times as fast as units of four in as many slices as is best for those.
 constexpr int UNIT_INTS = 16;
 constexpr int UNIT_LDS_ROWS = 1024;
 constexpr int ROW_FEW_UNITS = 128;
-static inline long long unit_bound(int N, int nnz) { return (long long)nnz / ROW_NB + N / 32; }   // ceil(n / 4) <= n / 4 + 3 / 4
+static __host__ __device__ __forceinline__ long long unit_bound(int rows, int nnz, int P) { return (long long)nnz / P + rows; }   // ceil(n / P) <= n / P + 1 - 1 / P
+// A table has all lists (only = 0) or one: of more rows than UNIT_LDS_ROWS that of ROW_NB (they fill the chip with any, and tables are mostly rows
+// without blocks), and where a call builds the table in its workspace the one that it takes.
+static __host__ __device__ __forceinline__ int unit_lists_only(int rows) { return rows <= UNIT_LDS_ROWS ? 0 : ROW_NB; }
+static __host__ __device__ __forceinline__ long long units_before(int rows, int nnz, int P, int only) {   // places of the lists before P's
+    long long n = 0;
+    for (int p = 1; p < P && !only; ++p) n += unit_bound(rows, nnz, p);
+    return n;
+}
+static __host__ __device__ __forceinline__ unsigned unit_grid(int rows, int nnz, int P) { return (unsigned)((unit_bound(rows, nnz, P) + 255) / 256); }
+static inline unsigned unit_table_grid(int rows, int nnz, int only) {
+    if (only) return unit_grid(rows, nnz, only);
+    unsigned n = 0;
+    for (int p = 1; p <= ROW_SIZES; ++p) n += unit_grid(rows, nnz, p);
+    return n;
+}
 static inline size_t unit_prefix_bytes(int N) { return N / 32 > UNIT_LDS_ROWS ? ((size_t)ROW_PARTS * (N / 32) + 1) * sizeof(int) : 0; }
-static inline size_t unit_table_bytes(int N, int nnz) { return 64 + (size_t)unit_bound(N, nnz) * UNIT_INTS * sizeof(int) + unit_prefix_bytes(N); }
+static inline size_t unit_lists_ints(int N, int nnz, int only) {
+    const int rows = N / 32;
+    return 16 + (size_t)(only ? unit_bound(rows, nnz, only) : units_before(rows, nnz, ROW_SIZES + 1, 0)) * UNIT_INTS;
+}
+static inline size_t unit_table_bytes(int N, int nnz, int only) { return unit_lists_ints(N, nnz, only) * sizeof(int) + unit_prefix_bytes(N); }
 static __device__ __forceinline__ int row_entries(const int32_t* __restrict__ ptr, int nnz, int r, int* lo) {
     const int a = clamp_entry(ptr[r], nnz), b = clamp_entry(ptr[r + 1], nnz);
     *lo = a;
     return b > a ? b - a : 0;
 }
-static __device__ __forceinline__ int row_units(int n) { return n > 0 ? (n + ROW_NB - 1) / ROW_NB : 1; }
+static __device__ __forceinline__ int row_units(int n, int P) { return n > 0 ? (n + P - 1) / P : 1; }
 static __device__ __forceinline__ int part_lo(int nu, int h) { return (h * nu + ROW_PARTS - 1) / ROW_PARTS; }   // first unit of quarter h
 static __device__ __forceinline__ int unit_entry(int n, int nu, int j) { return (int)((long long)n * j / nu); }
 
-// units before (quarter, row), into before [ROW_PARTS * rows + 1]; all threads of the workgroup
+// units of list P before (quarter, row), into before [ROW_PARTS * rows + 1]; all threads of the workgroup
 template <int NT>
-static __device__ void unit_prefix(const int32_t* __restrict__ ptr, int nnz, int rows, int* before, int* s_wave) {
+static __device__ void unit_prefix(const int32_t* __restrict__ ptr, int nnz, int rows, int P, int* before, int* s_wave) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int carry = 0;
     for (int base = 0; base < ROW_PARTS * rows; base += NT) {
         const int i = base + tid;
         int v = 0, lo;
         if (i < ROW_PARTS * rows) {
-            const int h = i / rows, nu = row_units(row_entries(ptr, nnz, i - h * rows, &lo));
+            const int h = i / rows, nu = row_units(row_entries(ptr, nnz, i - h * rows, &lo), P);
             v = part_lo(nu, h + 1) - part_lo(nu, h);
         }
         int incl = v;
@@ -89,31 +116,34 @@ static __device__ void unit_prefix(const int32_t* __restrict__ ptr, int nnz, int
     __threadfence_block();
     __syncthreads();
 }
-__global__ __launch_bounds__(1024) void unit_prefix_kernel(const int32_t* __restrict__ ptr, int nnz, int rows, int* before) {
+__global__ __launch_bounds__(1024) void unit_prefix_kernel(const int32_t* __restrict__ ptr, int nnz, int rows, int P, int* before) {
     __shared__ int s_wave[16];
-    unit_prefix<1024>(ptr, nnz, rows, before, s_wave);
+    unit_prefix<1024>(ptr, nnz, rows, P, before, s_wave);
 }
 struct UnitArgs {
     const int32_t *ptr, *idx;
     int nnz, rows, cols;
     const int* global_before;   // of unit_prefix_kernel, for patterns whose prefix does not fit LDS
-    int bound;
+    int only;                   // 0: all lists
     int* table;
 };
 // one unit per thread; workgroup `block` (256 threads)
 static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) {
     const int32_t* __restrict__ ptr = a.ptr;
     const int32_t* __restrict__ idx = a.idx;
-    const int nnz = a.nnz, rows = a.rows, cols = a.cols, bound = a.bound;
+    const int nnz = a.nnz, rows = a.rows, cols = a.cols;
     const int* global_before = a.global_before;
-    int* table = a.table;
+    int P = a.only ? a.only : 1;
+    while (!a.only && P < ROW_SIZES && block >= (int)unit_grid(rows, nnz, P)) block -= (int)unit_grid(rows, nnz, P++);
+    const int bound = (int)unit_bound(rows, nnz, P);
+    int* table = a.table + (size_t)units_before(rows, nnz, P, a.only) * UNIT_INTS;
     __shared__ int s_before[ROW_PARTS * UNIT_LDS_ROWS + 1];
     __shared__ int s_wave[4];
-    if (!global_before) unit_prefix<256>(ptr, nnz, rows, s_before, s_wave);
+    if (!global_before) unit_prefix<256>(ptr, nnz, rows, P, s_before, s_wave);
     const int* before = global_before ? global_before : s_before;
     const int total = before[ROW_PARTS * rows] < bound ? before[ROW_PARTS * rows] : bound;   // (a corrupt pointer array may ask for more)
     const int u = block * 256 + threadIdx.x;
-    if (u == 0) table[0] = total;
+    if (u == 0) a.table[P - 1] = total;
     if (u >= total) return;
     int lo = 0, hi = ROW_PARTS * rows - 1;   // the place that holds unit u
     while (lo < hi) {
@@ -122,7 +152,7 @@ static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) 
     }
     const int h = lo / rows, row = lo - h * rows;
     int first;
-    const int n = row_entries(ptr, nnz, row, &first), nu = row_units(n);
+    const int n = row_entries(ptr, nnz, row, &first), nu = row_units(n, P);
     const int j0 = part_lo(nu, h), j = j0 + u - before[lo];
     const int e0 = unit_entry(n, nu, j), e1 = unit_entry(n, nu, j + 1);
     int* o = table + 16 + (size_t)u * UNIT_INTS;
@@ -131,7 +161,7 @@ static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) 
     o[2] = j;
     o[3] = 0;
 #pragma unroll
-    for (int b = 0; b < ROW_NB; ++b) {
+    for (int b = 0; b < ROW_SIZES; ++b) {
         int c = 0, d = -1;
         if (b < e1 - e0) {
             c = idx[2 * (size_t)(first + e0 + b)];
@@ -140,8 +170,7 @@ static __device__ __forceinline__ void unit_table(const UnitArgs& a, int block) 
             d = d < 0 || d >= nnz ? -1 : d;
         }
         o[4 + b] = c;
-        o[8 + b] = d;
-        o[12 + b] = 0;
+        o[4 + ROW_SIZES + b] = d;
     }
 }
 __global__ __launch_bounds__(256) void unit_table_kernel(UnitArgs a) { unit_table(a, blockIdx.x); }
@@ -164,7 +193,8 @@ __global__ __launch_bounds__(256) void derive_kernel(DeriveArgs a) {
 struct SddRowArgs {
     const void* g;           // [M, N] grad_output
     const void* x;           // [M, K] input
-    const int* table;        // unit_table_kernel
+    const int* units;        // a list of unit_table_kernel's
+    const int* count;        // how many it holds
     void* out;               // [nnz*32, 32]
     void* bias_out;          // nullptr or [N]
     float* partial;
@@ -275,7 +305,7 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         cblk[b] = unit[4 + b];
-        bblk[b] = unit[8 + b];
+        bblk[b] = unit[4 + ROW_SIZES + b];
     }
     const bool sums = a.bias_out && unit[2] == 0;
 
@@ -307,6 +337,13 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     // each block's addition runs under the products of the next one
     constexpr bool TOTALS = ESZ == 4 && NB > 0;
     f32x4 total[TOTALS ? NBX : 1][2][2];
+    // and the totals of ROW_GROUP chunks to those of the wave's share: the roundings of a chain of n additions grow with n, those of both levels with
+    // ROW_GROUP + n / ROW_GROUP.  (So that units in few slices have no larger error than those in many: 6984 tokens 704 -> 2720 density 0.106, 55 chunks a wave in
+    // place of 19, 1.35e-7 -> 1.76e-7 without, 1.34e-7 with; 1 to 2 % of the time.)  Not in shares of at most ROW_LONG chunks, and units of five and six blocks, which
+    // have no registers for it, have no longer ones.
+    constexpr bool GROUPS = TOTALS && NB <= ROW_NB;
+    f32x4 grand[GROUPS ? NBX : 1][2][2];
+    float bleft[2] = {0.f, 0.f};   // (the bias sums, two values a lane, carry what each addition has cut off)
     auto fold = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -322,8 +359,38 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) total[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < 2; ++j) {
+                    total[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (GROUPS) grand[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
     }
+    auto next_group = [&]() __attribute__((always_inline)) {
+        if constexpr (GROUPS) {
+#pragma unroll
+            for (int b = 0; b < NBX; ++b)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        grand[b][i][j] += total[b][i][j];
+                        total[b][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+        }
+    };
+    auto add_bias = [&](const F& g) __attribute__((always_inline)) {
+        if constexpr (ESZ == 4) {
+            float of_chunk[2] = {0.f, 0.f};
+            g.sum(of_chunk);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float add = of_chunk[i] - bleft[i], now = bsum[i] + add;
+                bleft[i] = (now - bsum[i]) - add;
+                bsum[i] = now;
+            }
+        } else {
+            g.sum(bsum);
+        }
+    };
 
     int chunk = c_lo + wave;
     if (chunk < c_hi) {
@@ -348,8 +415,13 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
             if constexpr (NB > 0) xf.read(mem + GS * PIECE, s, lane);
         }
         int xat = 0, gat = 0;   // slots of the pieces in xf and gf
+        int group_end = c_hi - c_lo > ROW_LONG * ROW_NW ? chunk + ROW_GROUP * ROW_NW : c_hi;
         for (;; chunk += ROW_NW) {
-            if (sums) gf.sum(bsum);
+            if (GROUPS && chunk >= group_end) {
+                next_group();
+                group_end += ROW_GROUP * ROW_NW;
+            }
+            if (sums) add_bias(gf);
             if constexpr (NB == 0) {
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -362,8 +434,9 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
             for (int b = 0; b < NB; ++b) {
                 // Read below: the next block's piece, asked for XS - 1 blocks ago, and in the chunk's last block the next chunk's
                 // G piece.  The tables have the number of younger DMA instructions, for the orders of issue below.
-                constexpr int YOUNGER4[5][4] = {{0, 0, 0, 0}, {1, 0, 0, 0}, {4, 8, 0, 0}, {8, 12, 5, 0}, {8, 12, 12, 8}};
-                constexpr int YOUNGER2[5][4] = {{0, 0, 0, 0}, {2, 0, 0, 0}, {2, 4, 0, 0}, {4, 6, 4, 0}, {4, 6, 6, 4}};
+                // (From four blocks on it is the two blocks' before, with the G piece if a chunk began in between.)
+                constexpr int YOUNGER4[ROW_SIZES + 1][ROW_SIZES] = {{}, {1}, {4, 8}, {8, 12, 5}, {8, 12, 12, 8}, {8, 12, 12, 8, 8}, {8, 12, 12, 8, 8, 8}};
+                constexpr int YOUNGER2[ROW_SIZES + 1][ROW_SIZES] = {{}, {2}, {2, 4}, {4, 6, 4}, {4, 6, 6, 4}, {4, 6, 6, 4, 4}, {4, 6, 6, 4, 4, 4}};
                 wait_dma(D == 4 ? YOUNGER4[NB][b] : YOUNGER2[NB][b]);
                 const int xnext = xat + 1 == XS ? 0 : xat + 1;
                 const int kb = (b + XS) % NBX;       // the piece that takes this block's slot
@@ -409,7 +482,10 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[b][i][j] += total[b][i][j];
+                for (int j = 0; j < 2; ++j) {
+                    acc[b][i][j] += total[b][i][j];
+                    if constexpr (GROUPS) acc[b][i][j] += grand[b][i][j];
+                }
     }
     // ---- the waves' sums meet in LDS, two blocks at a time: wave 2 k + jj stores rows FEAT(r, jj) of block k ----
     f32x4* red = reinterpret_cast<f32x4*>(smem);
@@ -488,7 +564,7 @@ static __device__ __forceinline__ bool row_task(const SddRowArgs& a, RowTask& t)
     // An XCD takes a run of units and goes through them for one token slice after the other.  Few units do not divide by eight well enough:
     // then it takes an eighth of the tasks, ordered by slice (768 x 768 density 0.5, 16384 tokens fp32, 81 units: 93 us in five slices, of 11 units for
     // most XCDs and so 55 tasks for 64 places, 84 in six with 61 tasks; 141 units 77 against 78).
-    const int units = a.table[0], xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD;
+    const int units = *a.count, xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD;
     int slice, u;
     if (units < ROW_FEW_UNITS) {
         const int tasks = units * a.slices, id = tasks * xcd / NUM_XCD + local;
@@ -501,7 +577,7 @@ static __device__ __forceinline__ bool row_task(const SddRowArgs& a, RowTask& t)
         slice = local / n_u;
         u = u_lo + local - slice * n_u;
     }
-    t.unit = a.table + 16 + (size_t)u * UNIT_INTS;
+    t.unit = a.units + (size_t)u * UNIT_INTS;
     const int chunks = (a.M + ROW_TC - 1) / ROW_TC;
     t.c_lo = a.chunk0 + slice * a.chunks_per_slice;
     t.c_hi = t.c_lo + a.chunks_per_slice < chunks ? t.c_lo + a.chunks_per_slice : chunks;
@@ -517,6 +593,8 @@ __global__ __launch_bounds__(ROW_NW * 64, SddRowCfg<T>::WPE) void sdd_row_kernel
     RowTask t;
     if (!row_task(a, t)) return;
     switch (t.unit[1]) {
+        case 6: if constexpr (!FAR) sdd_row_body<T, 6, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
+        case 5: if constexpr (!FAR) sdd_row_body<T, 5, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         case 4: sdd_row_body<T, 4, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         case 3: sdd_row_body<T, 3, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;
         case 2: sdd_row_body<T, 2, FAR>(a, t.unit, t.c_lo, t.c_hi, t.partial, smem, lane, wave); break;

@@ -63,7 +63,7 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         cblk[b] = unit[4 + b];
-        bblk[b] = unit[8 + b];
+        bblk[b] = unit[4 + ROW_SIZES + b];
     }
     const bool sums = a.bias_out && unit[2] == 0;
 

@@ -55,12 +55,12 @@ def _followed_by_nan(shape, dtype, device, seed):
 
 @pytest.mark.parametrize("dtype, out_f, in_f, counts, kernel", [
     (torch.float32, 384, 416, ROWS, "sdd_row_kernel"), (torch.bfloat16, 384, 416, ROWS, "sdd_row_kernel"),
-    (torch.float32, 4096, 4096, [120, 1, 2, 3], "sdd_split_kernel"),
+    (torch.float32, 4096, 4096, [60, 61, 62, 63], "sdd_split_kernel"),
 ])
 @pytest.mark.parametrize("past", [1, 7, 8, 9, 15, 16, 17, 24, 31])
 def test_last_chunk_ends_with_the_matrix(cuda, dtype, out_f, in_f, counts, kernel, past):
     """Tokens behind the last one count as zeros, whatever the memory there holds; a copy instruction covers 8 (fp32) or 16 (bf16) of a chunk's 32."""
-    tokens = (1184 if kernel == "sdd_split_kernel" else 96) + past
+    tokens = (4096 if kernel == "sdd_split_kernel" else 96) + past
     m = _layer(out_f, in_f, counts, dtype, cuda, past)
     name = native.matmul_back_kernel_name(tokens, out_f, in_f, m.cols_a.shape[0], dtype)
     print(name, tokens, out_f, in_f, dtype, flush=True)
