@@ -174,7 +174,7 @@ class BlockSparseMatrixBase(torch.nn.Module):
     def _block_replace_on_gpu(self, block_replacements, X, Y):
         """The same in one kernel, which writes arrays that are consistent by construction or reports why it cannot."""
         rep = block_replacements.to(dtype=torch.long, device=self.blocks.device).reshape(-1, 3)
-        status, arrays = native.torch_path().replace_blocks(self.blocks, rep, X, Y)
+        status, arrays, schedule = native.torch_path().replace_blocks(self.blocks, rep, X, Y, self.__dict__.get("_schedule"))
         if status & 1:
             raise Exception("block_replacements names a data block outside [0, %d)" % (self.data.shape[0] // self.block_shape[0]))
         if status & 2:
@@ -183,7 +183,7 @@ class BlockSparseMatrixBase(torch.nn.Module):
             raise RuntimeError("block_replacements leaves two blocks at one position")
         for name, array in zip(("blocks", "cols_a", "row_start_ends_a", "rows_b", "col_start_ends_b"), arrays):
             self._buffers[name] = array
-        self._schedule = None
+        self._schedule = schedule
         self.updated_data()
 
     # ------------------------------------------------------------------ constructors

@@ -210,8 +210,14 @@ __global__ __launch_bounds__(INDEX_THREADS) void replace_blocks_kernel(
     }
     __threadfence_block();
     __syncthreads();
+    // (the host may be waiting for the word and not for the kernel: it comes behind all that it stands for, in every cache)
+    auto report = [&](int value) {
+        __threadfence();
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(status, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    };
     if (s_err) {   // the same for every thread
-        if (tid == 0) *status = s_err;
+        report(s_err);
         return;
     }
     auto starts = [&](const unsigned* line, int n, int w, int32_t* ptr) {
@@ -244,7 +250,7 @@ __global__ __launch_bounds__(INDEX_THREADS) void replace_blocks_kernel(
         reinterpret_cast<int2*>(rows_b)[j] = make_int2(r, b);
         reinterpret_cast<int2*>(blocks)[b] = make_int2(c, r);
     }
-    if (tid == 0) *status = 0;
+    report(0);
 }
 
 // ---- consistency of the five arrays, one bit of *status per broken condition (PBS_BAD_* in pbs_hip.h) ----
@@ -308,7 +314,7 @@ __global__ __launch_bounds__(INDEX_THREADS) void validate_indices_kernel(
     }
     if (bad) atomicOr(&s_bad, bad);
     __syncthreads();
-    if (tid == 0) *status = s_bad;
+    if (tid == 0) __hip_atomic_store(status, s_bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // out[c][r] = in[r][c] for a rows x cols matrix of 2- or 4-byte elements (tiles of 32 x 32 through LDS)

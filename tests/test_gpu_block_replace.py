@@ -1,10 +1,12 @@
 """block_replace and validate_indices of a matrix on the GPU (one kernel each) against the host versions, bit for bit and
 message for message: grids whose bitmaps fit LDS and one whose do not, line lengths around multiples of 32."""
+import copy
+
 import numpy as np
 import pytest
 import torch
 
-from pytorch_block_sparse_amd import BlockSparseMatrix
+from pytorch_block_sparse_amd import BlockSparseLinear, BlockSparseMatrix
 
 pytestmark = pytest.mark.gpu
 NAMES = ("blocks", "cols_a", "row_start_ends_a", "rows_b", "col_start_ends_b")
@@ -63,3 +65,54 @@ def test_broken_buffers_give_the_message_of_the_host(cuda):
             t[at] = keep
             m.validate_indices()
         assert messages[0] == messages[1], (name, at, value)
+
+
+def _step(layer, x, dy):
+    y = layer(x)
+    return [y, *torch.autograd.grad(y, (x, layer.weight.get_differentiable_data(), layer.bias), dy)]
+
+
+def _moves(m, count, seed):
+    g = torch.Generator(device=m.blocks.device).manual_seed(seed)
+    free = (~m.block_mask_build(None)).nonzero()
+    to = free[torch.randperm(free.shape[0], generator=g, device=free.device)[:count]]
+    return torch.cat([to, torch.randperm(m.blocks.numel() // 2, generator=g, device=free.device)[:count, None]], 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("other_stream", [False, True])
+def test_steps_between_moves_are_those_of_a_fresh_matrix(cuda, dtype, other_stream):
+    """A trained matrix has the plans of its new pattern made with the arrays: the same steps as of a copy, which derives its own."""
+    np.random.seed(3)
+    layer = BlockSparseLinear(416, 1056, density=0.4, device=cuda, dtype=dtype)
+    with torch.no_grad():
+        layer.weight.data.normal_()
+        layer.bias.normal_()
+    torch.manual_seed(4)
+    x, dy = torch.randn(301, 416, device=cuda).to(dtype).requires_grad_(), torch.randn(301, 1056, device=cuda).to(dtype)
+    stream = torch.cuda.Stream() if other_stream else torch.cuda.current_stream()
+    for turn in range(4):
+        if turn != 1:   # (moves twice without a step between them)
+            _step(layer, x, dy)
+        moves = _moves(layer.weight, 30 + turn, turn)
+        torch.cuda.current_stream().synchronize()
+        layer.weight.block_replace(moves)
+        with torch.cuda.stream(stream):   # (what block_replace returns is complete for every stream)
+            got = _step(layer, x, dy)
+            stream.synchronize()
+        fresh = copy.deepcopy(layer)
+        fresh.weight.validate_indices()
+        for a, b in zip(got, _step(fresh, x, dy)):
+            assert torch.equal(a, b)
+
+
+def test_rejected_moves_of_a_trained_matrix(cuda):
+    np.random.seed(5)
+    layer = BlockSparseLinear(512, 768, density=0.5, device=cuda)
+    torch.manual_seed(5)
+    x, dy = torch.randn(129, 512, device=cuda, requires_grad=True), torch.randn(129, 768, device=cuda)
+    want = _step(layer, x, dy)
+    for _ in range(3):
+        with pytest.raises(Exception, match="block_replacements"):
+            layer.weight.block_replace(torch.tensor([[0, 0, 10 ** 6]], device=cuda))
+        assert all(torch.equal(a, b) for a, b in zip(want, _step(layer, x, dy)))
