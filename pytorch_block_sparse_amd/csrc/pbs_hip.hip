@@ -625,9 +625,9 @@ static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
 }
 // Estimated time in us of units of at most per_unit blocks, in so many slices: launch, reduction of the slices, chunks of a wave of the slowest workgroup, at
 // the rate of a wave alone or of a chip that is full in rounds of 256 workgroups.  Fitted to problems of 256 .. 4096 features, 64 .. 16384 tokens, densities
-// 0.05 .. 0.75 at six sizes of units and eight numbers of slices (fp32: 80 below 2^22 tokens x blocks, within 9 %; bf16: 80 whose operands have less than 52 MB, within 7 %).  The
-// choices it makes are 3 and 1.3 % slower than the best on average, and 1.28 and 1.14 times as fast as units of four in the best number of slices that
-// an estimate of those alone made; two of each 80 are slower by more than 2 %, an fp32 one with very uneven rows by 20 %.
+// 0.05 .. 0.75 at six sizes of units and eight numbers of slices (fp32: 80 below 2^22 tokens x blocks, within 9 %; bf16: 80 whose operands have less than 52 MB,
+// within 7 %, and 70 with 40 to 260 MB, within 10 %).  The choices it makes are 3 and 1.5 % slower than the best on average, and 1.28 and 1.14 times as fast as units of
+// four in the best number of slices that an estimate of those alone made; 4 fp32 ones of the 160 are slower by more than 2 %, one by 13 %.
 // (The number of units follows from the average row, so what looks like a full chip may be one workgroup more than that: for fp32, whose rounds are long, the mean
 // of the estimated number and of 4 % more.  The reduction is a launch and an allocation more for the host: 2 (bf16 0.75) us more than the fit has for it.)
 enum RowKernel { ROW_F32, ROW_SPLIT, ROW_BF16 };   // sdd_row_kernel<float>, sdd_split_kernel, sdd_row_kernel<bf16_t>
@@ -647,17 +647,20 @@ static double row_us(RowKernel kernel, long long M, int N, int K, int nnz, int p
     }
     struct Model {
         double more, launch, reduce, per_slice, alone, alone_row, busy, busy_row, most, whole, start;   // .._row: of a unit, besides its blocks
+        double cached, far, per_mb;   // from so many MB of operands on: how much longer the copies of a full chip take per 100 MB, and what a MB takes at least
     };
-    const Model m = kernel == ROW_F32 ? Model{1.04, 3.43, 4.82, 0.973, 0.581, 0.113, 0.549, 0.124, 0.340, 0.880, 0.0191}
-                                      : Model{1.0, 3.12, 3.5, 1.31, 0.171, 0.179, 0.140, 0.184, 0.272, 1.0, 0.0128};
+    const Model m = kernel == ROW_F32 ? Model{1.04, 3.43, 4.82, 0.973, 0.581, 0.113, 0.549, 0.124, 0.340, 0.880, 0.0191, 0.0, 0.0, 0.0}
+                                      : Model{1.0, 3.12, 3.5, 1.31, 0.171, 0.179, 0.140, 0.184, 0.272, 1.0, 0.0128, 52.0, 0.473, 0.2335};
     const double rows = N / 32, row = nnz / rows, columns = K / 32;
     const double full = nnz / (double)per_unit + rows * (per_unit - 1) / (2.0 * per_unit) * (1.0 - std::exp(-2.0 * row)), units = full + rows * std::exp(-row);
     const double mean = nnz / full, most = per_unit < columns ? per_unit : columns;   // blocks of a unit
     const double tasks = row_tasks(units, slices), tasks_more = m.more > 1.0 ? row_tasks(m.more * units, slices) : tasks;
     const double alone = wave * (m.alone * (mean + m.most * (most - mean)) + m.alone_row);
     const double rounds = 0.5 * (m.whole * (std::ceil(tasks / 32) + std::ceil(tasks_more / 32)) + (1.0 - m.whole) * (tasks + tasks_more) / 32);
-    const double busy = rounds * wave * (m.busy * mean + m.busy_row);
-    return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) + passes * (m.launch + (busy > alone ? busy : alone) + 0.5 * (tasks + tasks_more) * m.start);
+    const double mb = 1e-6 * M * ((double)N + K) * (kernel == ROW_BF16 ? 2 : 4), far = mb > m.cached ? 1.0 + m.far * 0.01 * (mb - m.cached) : 1.0, least = mb > m.cached ? m.per_mb * mb : 0.0;
+    const double busy = rounds * wave * (m.busy * mean + m.busy_row) * far;
+    const double us = busy > alone ? (busy > least ? busy : least) : (alone > least ? alone : least);
+    return (slices > 1 ? m.reduce + m.per_slice * slices * nnz / 1000.0 : 0.0) + passes * (m.launch + us + 0.5 * (tasks + tasks_more) * m.start);
 }
 // Launch; per round of workgroups and chunk what a pass costs and what the blocks of a wave cost; reduction of the slices (75 problems, 256 .. 16384
 // tokens, 256 .. 4096 features, densities 0.05 .. 0.95, one in seven with uneven rows: within 11 % for 16 rows and 9 % for 8).
@@ -700,10 +703,16 @@ struct RowChoice {
 static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool lists, size_t workspace_limit) {
     constexpr int CANDIDATES[] = {1, 2, 3, 4, 5, 6, 8, 11, 16, 24};
     const double bytes = (double)M * ((double)N + K) * (dtype == PBS_DTYPE_F32 ? 4 : 2);
-    // bf16 beyond the size of the L2s: 250 us where the rectangles, which read every panel once per 16 rows, take 198.
     // (rectangles count the bytes of a chunk in 31 bits)
     const bool rectangles = dtype == PBS_DTYPE_BF16 && N < (1 << 25) && K < (1 << 25);
-    if (rectangles && bytes > 52e6) return {0, 1, ROW_NB, false};
+    // bf16 operands beyond the size of the L2s (52 MB): the rectangles read every panel once per 16 or 8 rows of blocks, the units once per block, but only what
+    // they need, so below a density of 0.1 (rectangles with less than 26 of 256 places taken) the units are given what their estimate has at least a tenth faster
+    // (4 of 9 such problems of 52 to 220 MB, in which they are 0.95, with very uneven rows, and 1.39 to 1.56 times as fast: 1152 -> 3360 density 0.086, 5802 tokens 38 -> 24 us).  Above it they are 0.55 to 1.5 times
+    // as fast (4096 -> 4096 density 0.25, 16384 tokens 250 us and 198), where the estimates are not good enough to choose; and where most rows
+    // are empty, units cost what no estimate counts.  What the workspace does not allow the rectangles is refused and not served another way.
+    const bool large = rectangles && bytes > 52e6;
+    const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
+    if (large && (10ll * nnz >= (long long)(N / 32) * (K / 32) || nnz < N / 32 || !fits)) return {0, 1, ROW_NB, false};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
     RowChoice best{1, 1, ROW_NB, false};
@@ -726,8 +735,7 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
         for (int p = one_list ? ROW_NB : 1; p <= (one_list ? ROW_NB : ROW_SIZES); ++p) consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16, p);
         if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK && !far) consider(ROW_SPLIT, ROW_NB);
     }
-    const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
-    if (rectangles && fits && rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
+    if (rectangles && fits && (large ? 0.9 : 1.0) * rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
     return best;
 }
 struct BackPlan {
