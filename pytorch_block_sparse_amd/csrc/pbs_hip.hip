@@ -38,6 +38,27 @@ static int launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipSt
     return (int)e;
 }
 
+// What a call's sizes lead to is worked out once for the sizes that a thread has had last: a call asks for the part of the plan, for its workspace and when it is
+// launched, and a model's layers come in turn.  (The choice for 1 token 4096 -> 4096 in bf16, made twice a call of 6.5 us, 220 -> 49 ns, most of that reading the
+// environment; the weight gradient's for four layers in turn, three times a gradient, 170 -> 12 ns, where one answer was kept.)
+struct Sizes {
+    long long M;
+    int n, k, nnz, what;   // what: all else that the answer follows from
+    bool operator==(const Sizes& o) const { return M == o.M && n == o.n && k == o.k && nnz == o.nnz && what == o.what; }
+};
+template <typename Answer, typename Ask>
+static const Answer& answer(const Sizes& s, const Ask& ask) {   // (the type of `ask` tells the questions apart)
+    struct Kept {
+        bool there = false;
+        Sizes sizes;
+        Answer answer;
+    };
+    static thread_local Kept kept[16];
+    Kept& at = kept[(unsigned)((((unsigned)s.M * 31u + s.n) * 31u + s.k) * 31u + s.nnz + s.what) * 2654435761u >> 28];
+    if (!at.there || !(at.sizes == s)) at = Kept{true, s, ask()};
+    return at.answer;
+}
+
 // Zero fill as a kernel (callers may capture the stream into a graph).
 __global__ __launch_bounds__(256) void fill_zero_kernel(uint32_t* p, size_t nwords) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -194,12 +215,11 @@ static inline ColumnLaunch column_launch(long long M, int n) {
 // faster one for sparse patterns (4096 x 4096: 6 to 30 % at 1 to 24 blocks per column; 2048 x 2048: level at 2 to 4
 // blocks per column, 5 to 13 % from 8), while results of 512 to 1024 columns stay 10 to 30 % faster in the other
 // kernels until their columns hold 32 blocks.
-static bool column_kernel_fits(long long M, int n, int k, int nnz) {
+static bool column_kernel_fits(long long M, int n, int k, int nnz, int wish) {
     if (!column_plan_bytes(n, k) || nnz < 1 || nnz > DC_MAX_BLOCKS || M < 1) return false;
     const ColumnLaunch c = column_launch(M, n);
     const long long tiles_per_wg = (c.m_tiles + c.wg_per_group - 1) / c.wg_per_group;
     if (tiles_per_wg * (k / 64) >= DC_SEQ_INTS) return false;   // a workgroup's steps are numbered through the table
-    const int wish = column_kernel_wish();
     if (wish >= 0) return wish == 1;
     if ((long long)c.m_tiles * c.n_groups < 256) return false;
     const double per_column = (double)nnz / (n / 32);
@@ -272,7 +292,7 @@ struct StreamChoice {
     StreamShape shape;
     double us;
 };
-static StreamChoice choose_stream(int esz, long long M, int n, int k, int nnz) {
+static StreamChoice choose_stream_anew(int esz, long long M, int n, int k, int nnz) {
     StreamChoice best{{0, 0}, -1.0};
     auto consider = [&](StreamShape s) {
         // a lane's offset into its token tile is a 32-bit number
@@ -288,6 +308,47 @@ static StreamChoice choose_stream(int esz, long long M, int n, int k, int nnz) {
         for (const StreamShape& s : STREAM_BF16) consider(s);
     return best;
 }
+static StreamChoice choose_stream(int esz, long long M, int n, int k, int nnz) {
+    return answer<StreamChoice>(Sizes{M, n, k, nnz, esz}, [&] { return choose_stream_anew(esz, M, n, k, nnz); });
+}
+
+// How a launch goes over the chip.  The 8 XCDs as xcd_t ranges of token tiles x 8 / xcd_t sets of columns (every 8 / xcd_t-th of the ranking, so the sets
+// are equally heavy): the split that gives the fullest XCD the fewest workgroups, and of those within 3 % of it the one
+// with the least to read per XCD.
+struct StreamGrid {
+    int m_tiles, xcd_t, group;
+    long long grid;
+};
+static StreamGrid stream_grid(int esz, int tt, long long M, int n, int k, int nnz) {
+    return answer<StreamGrid>(Sizes{M, n, k, nnz, esz * 16 + tt}, [&] {
+        StreamGrid a;
+        a.m_tiles = (int)((M + 16 * tt - 1) / (16 * tt));
+        const int cols = n / 32;
+        const double tile_bytes = 16.0 * tt * k * esz, col_bytes = 1024.0 * esz * nnz / cols;
+        long long fewest = 1ll << 62;
+        double least = 0.0;
+        a.xcd_t = 1;
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int t = 1; t <= NUM_XCD; t *= 2) {
+                const long long tiles = (a.m_tiles + t - 1) / t, sets = (cols + NUM_XCD / t - 1) / (NUM_XCD / t);
+                if (pass == 0) {
+                    if (tiles * sets < fewest) fewest = tiles * sets;
+                } else if (tiles * sets <= fewest + fewest / 32) {
+                    const double bytes = tiles * tile_bytes + sets * col_bytes;
+                    if (least == 0.0 || bytes < least) {
+                        least = bytes;
+                        a.xcd_t = t;
+                    }
+                }
+            }
+        }
+        // as many token tiles to a pass over the columns as an XCD's L2 (4 MB) holds, at least one
+        const double fit = 4e6 / tile_bytes;
+        a.group = fit < 1.0 ? 1 : (fit > a.m_tiles ? a.m_tiles : (int)fit);
+        a.grid = NUM_XCD * (((long long)a.m_tiles + a.xcd_t - 1) / a.xcd_t) * ((cols + NUM_XCD / a.xcd_t - 1) / (NUM_XCD / a.xcd_t));
+        return a;
+    });
+}
 
 template <typename T, int TRANS, int TT, int KS>
 static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
@@ -301,35 +362,12 @@ static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
     a.M = g.M;
     a.N = g.N;
     a.K = g.K;
-    a.m_tiles = (g.M + 16 * TT - 1) / (16 * TT);
-    // The 8 XCDs as xcd_t ranges of token tiles x 8 / xcd_t sets of columns (every 8 / xcd_t-th of the ranking, so the sets
-    // are equally heavy): the split that gives the fullest XCD the fewest workgroups, and of those within 3 % of it the one
-    // with the least to read per XCD.
-    const int cols = g.N / 32;
-    const double tile_bytes = 16.0 * TT * g.K * sizeof(T), col_bytes = 1024.0 * sizeof(T) * g.nnz / cols;
-    long long fewest = 1ll << 62;
-    double least = 0.0;
-    a.xcd_t = 1;
-    for (int pass = 0; pass < 2; ++pass) {
-        for (int t = 1; t <= NUM_XCD; t *= 2) {
-            const long long tiles = (a.m_tiles + t - 1) / t, sets = (cols + NUM_XCD / t - 1) / (NUM_XCD / t);
-            if (pass == 0) {
-                if (tiles * sets < fewest) fewest = tiles * sets;
-            } else if (tiles * sets <= fewest + fewest / 32) {
-                const double bytes = tiles * tile_bytes + sets * col_bytes;
-                if (least == 0.0 || bytes < least) {
-                    least = bytes;
-                    a.xcd_t = t;
-                }
-            }
-        }
-    }
-    // as many token tiles to a pass over the columns as an XCD's L2 (4 MB) holds, at least one
-    const double fit = 4e6 / tile_bytes;
-    a.group = fit < 1.0 ? 1 : (fit > a.m_tiles ? a.m_tiles : (int)fit);
-    const long long grid = NUM_XCD * (((long long)a.m_tiles + a.xcd_t - 1) / a.xcd_t) * ((cols + NUM_XCD / a.xcd_t - 1) / (NUM_XCD / a.xcd_t));
-    if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)grid), dim3(KS * 64), 0, stream, a);
+    const StreamGrid at = stream_grid(sizeof(T), TT, g.M, g.N, g.K, g.nnz);
+    a.m_tiles = at.m_tiles;
+    a.xcd_t = at.xcd_t;
+    a.group = at.group;
+    if (at.grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
+    return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)at.grid), dim3(KS * 64), 0, stream, a);
 }
 
 template <typename T, int TRANS>
@@ -465,16 +503,7 @@ static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
     // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
     if (k > (1 << 16) || (M + 31) / 32 * groups >= (1 << 28)) return false;
-    // (a product asks twice, for the size of its workspace and when it is launched: the last answer of a thread, by the sizes it follows from)
-    struct Answer {
-        long long M;
-        int n, k, nnz;
-        bool fits;
-    };
-    static thread_local Answer last{-1, 0, 0, 0, false};
-    if (last.M != M || last.n != n || last.k != k || last.nnz != nnz)
-        last = Answer{M, n, k, nnz, SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us};
-    return last.fits;
+    return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] { return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us; });
 }
 
 template <int TRANS>
@@ -543,11 +572,10 @@ struct ProductChoice {
     PanelChoice panel;   // splits > 0: panel_kernel or panel_chunk_kernel, which read the list plan like stream_kernel
 };
 constexpr PanelChoice NO_PANEL{0, 0.0, 0, 0};
-static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
-    if (esz == 4) return {PART_LIST, NO_PANEL};
-    const int wish = column_kernel_wish();
+static ProductChoice choose_product_anew(long long M, int n, int k, int nnz, int transpose, bool with_copy, int wish) {
+    constexpr int esz = 2;
     const bool wide = wide_kernel_fits(M, n, k);
-    const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz);
+    const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz, wish);
     if (wish == 1 && column) return {PART_COLUMN, NO_PANEL};
     if (wish == 0 && wide) return {PART_WIDE, NO_PANEL};
     const PanelChoice panel = choose_panel(M, n, k, nnz);
@@ -564,6 +592,12 @@ static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz,
     if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel};
     if (tc < ts && tc < tw) return {PART_COLUMN, NO_PANEL};
     return {tw < ts ? PART_WIDE : PART_LIST, NO_PANEL};
+}
+static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz, int transpose, bool with_copy) {
+    if (esz == 4) return {PART_LIST, NO_PANEL};
+    const int wish = column_kernel_wish();
+    return answer<ProductChoice>(Sizes{M, n, k, nnz, (transpose ? 1 : 0) | (with_copy ? 2 : 0) | (wish + 1) << 2},
+                                 [&] { return choose_product_anew(M, n, k, nnz, transpose, with_copy, wish); });
 }
 
 template <typename T, int TRANS>
@@ -769,21 +803,8 @@ static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, bo
 }
 // `lists`: the caller brings a table with all lists of units
 static BackPlan plan_back(int dtype, long long M, int N, int K, int nnz, bool bias, bool lists, size_t workspace_limit = ROW_WORKSPACE_BYTES) {
-    // (a gradient asks three times, for the unit table, for the size of its workspace and when it is launched: the last answers of a thread, by the
-    // sizes they follow from)
-    struct Answer {
-        int dtype;
-        long long M;
-        int N, K, nnz;
-        bool lists;
-        size_t workspace_limit;
-        BackPlan plan;
-    };
-    static thread_local Answer kept[16] = {};   // (a model's layers in turn; tokens is never 0 here)
-    Answer& last = kept[(unsigned)((((unsigned)M * 31u + N) * 31u + K) * 31u + nnz + dtype) * 2654435761u >> 28];
-    if (last.dtype != dtype || last.M != M || last.N != N || last.K != K || last.nnz != nnz || last.lists != lists || last.workspace_limit != workspace_limit)
-        last = Answer{dtype, M, N, K, nnz, lists, workspace_limit, plan_back_anew(dtype, M, N, K, nnz, lists, workspace_limit)};
-    BackPlan p = last.plan;
+    BackPlan p = answer<BackPlan>(Sizes{M, N, K, nnz, dtype | (lists ? 2 : 0) | (int)((ROW_WORKSPACE_BYTES - workspace_limit) / 16) << 2},
+                                  [&] { return plan_back_anew(dtype, M, N, K, nnz, lists, workspace_limit); });
     p.partial_bytes = ((size_t)nnz * 1024 + (bias ? N : 0)) * sizeof(float) * p.partials;   // fp32 sums of each slice: blocks, bias columns
     return p;
 }
