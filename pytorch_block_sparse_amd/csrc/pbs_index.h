@@ -210,11 +210,15 @@ __global__ __launch_bounds__(INDEX_THREADS) void replace_blocks_kernel(
     }
     __threadfence_block();
     __syncthreads();
-    // (the host may be waiting for the word and not for the kernel: it comes behind all that it stands for, in every cache)
+    // (the host may be waiting for the word and not for the kernel: it comes behind all that it stands for.  Every wave waits until its stores are in the L2 of
+    // their common XCD, one thread writes that back for the others; a fence of all threads takes the kernel from 7 to 12 us)
     auto report = [&](int value) {
-        __threadfence();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (tid == 0) __hip_atomic_store(status, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (tid == 0) {
+            __threadfence();
+            __hip_atomic_store(status, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     };
     if (s_err) {   // the same for every thread
         report(s_err);
