@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 8
+#define PBS_ABI_VERSION 9
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -258,6 +258,22 @@ int pbs_blocksparse_matmul_back_bias(const void* dense_a, const void* dense_b,
                                      void* data_out, void* bias_out,
                                      int64_t tokens, int out_features, int in_features, int nnz,
                                      int dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * The gradients of a linear layer's input, blocks and bias (bias_out may be NULL) in one call: pbs_blocksparse_matmul_ws with
+ * transpose = 0 of grad_output and pbs_blocksparse_matmul_back_bias of grad_output and input, the same results bit for bit, with the
+ * work in front of one product done by a launch of the other where both have any.
+ *
+ *   plan_input  the plan of (col_start_ends_b, rows_b), as for transpose = 0
+ *   units, data_out, bias_out as above; grad_input [tokens, in_features]
+ *   workspace   pbs_blocksparse_linear_back_workspace_bytes() bytes, 16-byte aligned, may be NULL when that is 0
+ */
+size_t pbs_blocksparse_linear_back_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype);
+int pbs_blocksparse_linear_back(const void* grad_output, const void* input, const void* data, const void* plan_input,
+                                const int32_t* row_start_ends_a, const int32_t* cols_a, const void* units,
+                                void* grad_input, void* data_out, void* bias_out,
+                                int64_t tokens, int out_features, int in_features, int nnz,
+                                int dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * The same product with the arguments of the reference's entry point blocksparse_matmul_back_cutlass

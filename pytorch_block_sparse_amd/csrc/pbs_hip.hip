@@ -506,13 +506,15 @@ static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] { return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us; });
 }
 
+// `parts_ready`: the workspace holds the blocks in parts already
 template <int TRANS>
-static int launch_split(const DdsArgs& g, void* workspace, hipStream_t stream) {
+static int launch_split(const DdsArgs& g, void* workspace, bool parts_ready, hipStream_t stream) {
     static std::atomic<uint64_t> done{0};
     auto kernel = split_kernel<TRANS>;
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    if (int rc = launch(split_blocks_kernel<TRANS>, dim3((unsigned)((g.nnz + 3) / 4)), dim3(256), 0, stream, static_cast<const float*>(g.data),
-                        static_cast<unsigned char*>(workspace), g.nnz)) return rc;
+    if (!parts_ready)
+        if (int rc = launch(split_blocks_kernel<TRANS>, dim3(split_blocks_grid(g.nnz)), dim3(256), 0, stream, static_cast<const float*>(g.data),
+                            static_cast<unsigned char*>(workspace), g.nnz)) return rc;
     SplitArgs a;
     a.a = static_cast<const float*>(g.a);
     a.data = static_cast<const float*>(g.data);
@@ -601,7 +603,7 @@ static ProductChoice choose_product(int esz, long long M, int n, int k, int nnz,
 }
 
 template <typename T, int TRANS>
-static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_bytes, hipStream_t stream, bool parts_ready = false) {
     if constexpr (sizeof(T) == 2) {
         const bool copy = workspace && workspace_bytes >= (size_t)g.nnz * 2048 && aligned16(workspace);
         const ProductChoice choice = choose_product(2, g.M, g.N, g.K, g.nnz, !TRANS, copy);
@@ -624,7 +626,7 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
     }
     if constexpr (sizeof(T) == 4) {
         if (workspace && workspace_bytes >= split_workspace_bytes(g.nnz) && aligned16(workspace) && split_kernel_fits(g.M, g.N, g.K, g.nnz))
-            return launch_split<TRANS>(g, workspace, stream);
+            return launch_split<TRANS>(g, workspace, parts_ready, stream);
     }
     return launch_stream<T, TRANS>(g, stream);
 }
@@ -817,6 +819,8 @@ struct BackArgs {
     void* out;               // [nnz*32, 32]
     void* bias_out;          // nullptr or [N]
     int M, N, K, nnz;
+    const void* data;        // nullptr, or blocks that the launch which adds the slices (there has to be one; fp32) writes to `parts` for an input gradient
+    void* parts;
 };
 
 static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int nnz, int only, void* table, hipStream_t stream) {
@@ -833,8 +837,14 @@ static int build_units(const int32_t* ptr, const int32_t* idx, int N, int K, int
 template <typename T>
 static int launch_reduce(const float* partial, const BackArgs& a, int nsplit, hipStream_t stream) {
     const size_t n = (size_t)a.nnz * 1024, total = n + (a.bias_out ? a.N : 0);
-    return launch(sdd_reduce_kernel<T>, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, partial, static_cast<T*>(a.out), n,
-                  static_cast<T*>(a.bias_out), total, nsplit);
+    const unsigned reducing = (unsigned)((total / 4 + 255) / 256);
+    if constexpr (sizeof(T) == 4) {
+        if (a.data)
+            return launch(sdd_reduce_split_kernel, dim3(reducing + split_blocks_grid(a.nnz)), dim3(256), 0, stream, partial, static_cast<float*>(a.out), n,
+                          static_cast<float*>(a.bias_out), total, nsplit, reducing, static_cast<const float*>(a.data), static_cast<unsigned char*>(a.parts),
+                          a.nnz);
+    }
+    return launch(sdd_reduce_kernel<T>, dim3(reducing), dim3(256), 0, stream, partial, static_cast<T*>(a.out), n, static_cast<T*>(a.bias_out), total, nsplit);
 }
 
 template <typename T>
@@ -1088,9 +1098,7 @@ int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* pl
                                      stream);
 }
 
-int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void* plan, const void* bias, void* dense_out,
-                              int64_t tokens, int n, int k, int nnz, int transpose, int dtype, void* workspace,
-                              size_t workspace_bytes, void* stream) {
+static int matmul_checks(const void* dense_a, const void* data, const void* plan, const void* dense_out, int64_t tokens, int n, int k, int nnz, int dtype) {
     if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return PBS_ERR_BAD_DTYPE;
     if (tokens < 0 || n <= 0 || k <= 0 || nnz < 0 || (n % 32) || (k % 32)) return PBS_ERR_BAD_SHAPE;
     if (tokens > (1ll << 30) || (long long)nnz > (long long)(n / 32) * (k / 32) || k > (1 << 24)) return PBS_ERR_TOO_LARGE;
@@ -1098,6 +1106,14 @@ int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void*
     if (!dense_a || !plan || !dense_out) return PBS_ERR_NULL_POINTER;
     if (nnz > 0 && !data) return PBS_ERR_NULL_POINTER;
     if (!aligned16(dense_a) || !aligned16(data) || !aligned16(dense_out) || !aligned16(plan)) return PBS_ERR_MISALIGNED;
+    return PBS_OK;
+}
+
+int pbs_blocksparse_matmul_ws(const void* dense_a, const void* data, const void* plan, const void* bias, void* dense_out,
+                              int64_t tokens, int n, int k, int nnz, int transpose, int dtype, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+    if (int rc = matmul_checks(dense_a, data, plan, dense_out, tokens, n, k, nnz, dtype)) return rc;
+    if (tokens == 0) return PBS_OK;
     DdsArgs g;
     g.a = dense_a;
     g.data = data;
@@ -1199,7 +1215,7 @@ int pbs_blocksparse_matmul_back(const void* dense_a, const void* dense_b, const 
                                 const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                 int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
                                 void* stream) {
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz, nullptr, nullptr};
     return back(a, tokens, dtype, workspace, workspace_bytes, stream);
 }
 
@@ -1208,8 +1224,45 @@ int pbs_blocksparse_matmul_back_bias(const void* dense_a, const void* dense_b, c
                                      int out_features, int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes,
                                      void* stream) {
     if (!units && pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, dtype) > 0) return PBS_ERR_NULL_POINTER;
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, units, true, data_out, bias_out, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, units, true, data_out, bias_out, (int)tokens, out_features, in_features, nnz, nullptr, nullptr};
     return back(a, tokens, dtype, workspace, workspace_bytes, stream);
+}
+
+// A workspace of both products: the slices of the weight gradient, and behind them the blocks in parts.
+static size_t slices_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    return (pbs_blocksparse_matmul_back_bias_workspace_bytes(tokens, out_features, in_features, nnz, dtype) + 255) / 256 * 256;
+}
+size_t pbs_blocksparse_linear_back_workspace_bytes(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    return slices_bytes(tokens, out_features, in_features, nnz, dtype) +
+           pbs_blocksparse_matmul_parts_bytes(tokens, in_features, out_features, nnz, 0, dtype);
+}
+
+int pbs_blocksparse_linear_back(const void* grad_output, const void* input, const void* data, const void* plan_input, const int32_t* row_start_ends_a,
+                                const int32_t* cols_a, const void* units, void* grad_input, void* data_out, void* bias_out, int64_t tokens,
+                                int out_features, int in_features, int nnz, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    if (int rc = matmul_checks(grad_output, data, plan_input, grad_input, tokens, in_features, out_features, nnz, dtype)) return rc;
+    const size_t slices = slices_bytes(tokens, out_features, in_features, nnz, dtype),
+                 parts = pbs_blocksparse_matmul_parts_bytes(tokens, in_features, out_features, nnz, 0, dtype);
+    if (slices + parts > 0 && (!workspace || workspace_bytes < slices + parts || !aligned16(workspace))) return PBS_ERR_WORKSPACE;
+    if (!units && pbs_blocksparse_matmul_back_units_bytes(tokens, out_features, in_features, nnz, dtype) > 0) return PBS_ERR_NULL_POINTER;
+    void* const behind = parts ? static_cast<unsigned char*>(workspace) + slices : nullptr;
+    const DdsArgs g{grad_output, data, static_cast<const int*>(plan_input), nullptr, grad_input, (int)tokens, in_features, out_features, nnz};
+    BackArgs a{grad_output, input, row_start_ends_a, cols_a, units, true, data_out, bias_out, (int)tokens, out_features, in_features, nnz, nullptr, nullptr};
+    auto input_gradient = [&](bool parts_ready) {
+        if (tokens == 0) return (int)PBS_OK;
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        return dtype == PBS_DTYPE_F32 ? dispatch_dds<float, 1>(g, behind, parts, s, parts_ready) : dispatch_dds<bf16_t, 1>(g, nullptr, 0, s);
+    };
+    // with a launch that adds the slices, the blocks are split by that one too, and the input gradient comes last
+    const bool together = parts > 0 && plan_back(dtype, tokens, out_features, in_features, nnz, bias_out != nullptr, true).partials > 0;
+    if (together) {
+        a.data = data;
+        a.parts = behind;
+        if (int rc = back(a, tokens, dtype, workspace, slices, stream)) return rc;
+        return input_gradient(true);
+    }
+    if (int rc = input_gradient(false)) return rc;
+    return back(a, tokens, dtype, workspace, slices, stream);
 }
 
 // ---- the reference's own signature of the sparse-output product ----
@@ -1305,7 +1358,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
                                         const int32_t* cols_a, void* data_out, int64_t tokens, int out_features,
                                         int in_features, int nnz, int dtype, void* stream) {
     // the array limits the number of slices of the row kernel; the rectangles' is fixed
-    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz};
+    const BackArgs a{dense_a, dense_b, row_start_ends_a, cols_a, nullptr, false, data_out, nullptr, (int)tokens, out_features, in_features, nnz, nullptr, nullptr};
     size_t need = 0, limit = 0;
     if (back_sizes_ok(tokens, out_features, in_features, nnz, dtype) && nnz > 0) {
         const size_t table = unit_table_bytes(out_features, nnz, ROW_NB);

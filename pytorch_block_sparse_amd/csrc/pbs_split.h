@@ -45,6 +45,7 @@
 // another round of units (up to 1.38 times faster there, but short columns pay for the choice: 1 % slower on average, uneven patterns too).
 #pragma once
 #include "pbs_common.h"
+#include "pbs_sdd.h"
 #include "pbs_stream.h"
 
 namespace pbs {
@@ -92,9 +93,9 @@ static __device__ __forceinline__ float with_sign(float v, int sign_uniform) {
 // The blocks in parts, as fragments: block b = [half q of k][part][lane = 32 h + n][8 k values], k = 16 q + 8 h + e, 6 KB.  One wave
 // per block.  TRANS as in stream_kernel: 0: stored [k][n], 1: stored [n][k].
 template <int TRANS>
-__global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restrict__ data, unsigned char* __restrict__ parts, int nnz) {
+static __device__ __forceinline__ void split_blocks(const float* __restrict__ data, unsigned char* __restrict__ parts, int nnz, int block) {
     const int lane = threadIdx.x & 63;
-    const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int b = block * 4 + (threadIdx.x >> 6);
     if (b >= nnz) return;
     const float* src = data + (size_t)b * 1024;
     unsigned char* dst = parts + (size_t)b * SP_BLOCK_BYTES + lane * 16;
@@ -117,6 +118,20 @@ __global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restri
 #pragma unroll
         for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4*>(dst + (q * 3 + i) * 1024) = make_uint4(p[i][0], p[i][1], p[i][2], p[i][3]);
     }
+}
+static inline unsigned split_blocks_grid(int nnz) { return (unsigned)((nnz + 3) / 4); }
+template <int TRANS>
+__global__ __launch_bounds__(256) void split_blocks_kernel(const float* __restrict__ data, unsigned char* __restrict__ parts, int nnz) {
+    split_blocks<TRANS>(data, parts, nnz, blockIdx.x);
+}
+// The sums of the slices of a weight gradient, and behind them the blocks of the input gradient that follows: behind a large kernel either takes 5.3 us
+// as a launch of its own, whatever its size.  Training steps, us, with two launches and with this one: 3072 -> 768 density 0.25 in Zipf rows, 4096 tokens
+// 164.1 and 155.5; 768 -> 768 density 0.5, 16384 tokens 229.3 and 224.7; 768 -> 3072 density 0.5, 4096 tokens 230.4 and 230.9 (the card's power: what the pause
+// took, the kernel behind it took less).
+__global__ __launch_bounds__(256) void sdd_reduce_split_kernel(const float* partial, float* out, size_t n, float* bias_out, size_t total, int nsplit,
+                                                               unsigned reducing, const float* __restrict__ data, unsigned char* __restrict__ parts, int nnz) {
+    if (blockIdx.x < reducing) sdd_reduce(partial, out, n, bias_out, total, nsplit, blockIdx.x);
+    else split_blocks<1>(data, parts, nnz, (int)(blockIdx.x - reducing));
 }
 
 struct SplitArgs {

@@ -218,12 +218,12 @@ using PatternPtr = std::shared_ptr<Pattern>;
 
 const void* data_or_null(const Tensor& t) { return t.defined() && t.numel() ? t.const_data_ptr() : nullptr; }
 
-// a [..., k] -> [..., n]; `training`: the products of a backward pass will follow
-Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose, bool training = false) {
+// what matmul asks of its operands; the sizes (n, k) of the product
+std::pair<int, int> check_matmul(const Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose) {
     check_gpu(a_any);
     check_gpu(data);
     check_gpu(bias);
-    const int code = dtype_code(a_any);
+    dtype_code(a_any);
     TORCH_CHECK(data.scalar_type() == a_any.scalar_type(), "dense operand is ", a_any.dtype(), " but the block data is ", data.dtype());
     TORCH_CHECK(!bias.defined() || bias.scalar_type() == a_any.scalar_type(), "bias is ", bias.dtype(), ", expected ", a_any.dtype());
     TORCH_CHECK(data.is_contiguous(), "block data must be contiguous");
@@ -234,6 +234,13 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     TORCH_CHECK(a_any.size(-1) == k, "Invalid matrices sizes ", a_any.sizes(), " x (", k, ", ", n, ")");
     TORCH_CHECK(data.numel() == (int64_t)p.nnz * 1024, "the block data does not match the index buffers");
     TORCH_CHECK(!bias.defined() || (bias.numel() == n && bias.is_contiguous()), "bias should be contiguous and hold ", n, " values");
+    return {n, k};
+}
+
+// a [..., k] -> [..., n]; `training`: the products of a backward pass will follow
+Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor& bias, bool transpose, bool training = false) {
+    const auto [n, k] = check_matmul(p, a_any, data, bias, transpose);
+    const int code = dtype_code(a_any);
     const Tensor a = a_any.is_contiguous() ? a_any : a_any.contiguous();
     const int64_t tokens = a.numel() / k;
     c10::DeviceGuard guard(a.device());
@@ -258,21 +265,26 @@ Tensor matmul(Pattern& p, const Tensor& a_any, const Tensor& data, const Tensor&
     return out;
 }
 
-// packed blocks of a^T b on the pattern, into `out`, and the sums of a's columns, into `sums` (if defined)
-void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out, const Tensor& sums = Tensor()) {
+void check_matmul_back(const Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out) {
     check_gpu(a_any);
     check_gpu(b_any);
     check_gpu(out);
-    const int code = dtype_code(a_any);
+    dtype_code(a_any);
     TORCH_CHECK(b_any.scalar_type() == a_any.scalar_type() && out.scalar_type() == a_any.scalar_type(), "operands and result must share one dtype");
     TORCH_CHECK(b_any.device() == a_any.device() && out.device() == a_any.device() && p.cols.t.device() == a_any.device(),
                 "the operands are on different devices");
     TORCH_CHECK(a_any.size(-1) == p.out_features && b_any.size(-1) == p.in_features && out.numel() == (int64_t)p.nnz * 1024 && out.is_contiguous(),
                 "Invalid matrices sizes ", a_any.sizes(), "^T x ", b_any.sizes());
+    TORCH_CHECK(b_any.numel() / p.in_features == a_any.numel() / p.out_features, "Invalid matrices sizes ", a_any.sizes(), "^T x ", b_any.sizes());
+}
+
+// packed blocks of a^T b on the pattern, into `out`, and the sums of a's columns, into `sums` (if defined)
+void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Tensor& out, const Tensor& sums = Tensor()) {
+    check_matmul_back(p, a_any, b_any, out);
+    const int code = dtype_code(a_any);
     const Tensor a = a_any.is_contiguous() ? a_any : a_any.contiguous();
     const Tensor b = b_any.is_contiguous() ? b_any : b_any.contiguous();
     const int64_t tokens = a.numel() / p.out_features;
-    TORCH_CHECK(b.numel() / p.in_features == tokens, "Invalid matrices sizes ", a.sizes(), "^T x ", b.sizes());
     c10::DeviceGuard guard(a.device());
     void* stream = current_stream(a);
     const Tensor units = p.units_for(tokens, code, stream);
@@ -286,16 +298,47 @@ void matmul_back(Pattern& p, const Tensor& a_any, const Tensor& b_any, const Ten
           "pbs_blocksparse_matmul_back_bias");
 }
 
+// both, of a contiguous dy: dx = dy W, and the blocks of dy^T x with the sums of dy's columns (if defined)
+Tensor both_gradients(Pattern& p, const Tensor& dy, const Tensor& x_any, const Tensor& data, const Tensor& out, const Tensor& sums) {
+    const auto [n, k] = check_matmul(p, dy, data, Tensor(), false);
+    check_matmul_back(p, dy, x_any, out);
+    const int code = dtype_code(dy);
+    const int64_t tokens = dy.numel() / k;
+    if (tokens == 0) {
+        matmul_back(p, dy, x_any, out, sums);
+        return matmul(p, dy, data, Tensor(), false);
+    }
+    const Tensor x = x_any.is_contiguous() ? x_any : x_any.contiguous();
+    c10::DeviceGuard guard(dy.device());
+    void* stream = current_stream(dy);
+    c10::SmallVector<int64_t, 6> sizes(dy.sizes().begin(), dy.sizes().end());
+    sizes.back() = n;
+    Tensor dx = at::empty(sizes, dy.options());
+    const Tensor plan = p.plan_for(false, n, k, pbs_blocksparse_matmul_part(tokens, n, k, p.nnz, 0, code, 1), stream);
+    const Tensor units = p.units_for(tokens, code, stream);
+    const size_t ws_bytes = pbs_blocksparse_linear_back_workspace_bytes(tokens, p.out_features, p.in_features, p.nnz, code);
+    Tensor ws;
+    if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, dy.options().dtype(at::kByte));
+    check(pbs_blocksparse_linear_back(data_or_null(dy), data_or_null(x), data_or_null(data), plan.const_data_ptr(), p.row_ptr.t.const_data_ptr<int>(),
+                                      static_cast<const int*>(data_or_null(p.cols.t)), data_or_null(units), dx.mutable_data_ptr(),
+                                      out.numel() ? out.mutable_data_ptr() : nullptr, sums.defined() ? sums.mutable_data_ptr() : nullptr, tokens,
+                                      p.out_features, p.in_features, p.nnz, code, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream),
+          "pbs_blocksparse_linear_back");
+    check_protocol("pbs_blocksparse_linear_back", dy.device().index());
+    return dx;
+}
+
 // The gradients of x (dx = dy W), of the blocks and of the bias (the sum of dy over the tokens) that are wanted, others undefined.
 std::array<Tensor, 3> linear_backward(Pattern& p, const Tensor& dy_any, const Tensor& x, const Tensor& data, std::array<bool, 3> wanted) {
     at::NoGradGuard no_grad;
     std::array<Tensor, 3> out;
     const Tensor dy = dy_any.is_contiguous() ? dy_any : dy_any.contiguous();
-    if (wanted[0]) out[0] = matmul(p, dy, data, Tensor(), false);
+    if (wanted[0] && !wanted[1]) out[0] = matmul(p, dy, data, Tensor(), false);
     if (wanted[1]) {
         out[1] = at::empty({(int64_t)p.nnz * 32, 32}, x.options());
         if (wanted[2]) out[2] = at::empty({p.out_features}, x.options());
-        matmul_back(p, dy, x, out[1], out[2]);
+        if (wanted[0]) out[0] = both_gradients(p, dy, x, data, out[1], out[2]);
+        else matmul_back(p, dy, x, out[1], out[2]);
     } else if (wanted[2]) {
         out[2] = dy.reshape({-1, dy.size(-1)}).sum(0);
     }

@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libpbs_hip.so")
 
-ABI_VERSION = 8   # PBS_ABI_VERSION of the header that the prototypes below restate
+ABI_VERSION = 9   # PBS_ABI_VERSION of the header that the prototypes below restate
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
 SUPPORTED_DTYPES = tuple(DTYPE_CODES)
@@ -62,6 +62,11 @@ _PROTOTYPES = {
     "pbs_blocksparse_matmul_back_bias": (
         _i32,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp],
+    ),
+    "pbs_blocksparse_linear_back_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_linear_back": (
+        _i32,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp],
     ),
     "pbs_blocksparse_matmul_back_blocks_workspace_bytes": (ctypes.c_size_t, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul_back_blocks": (

@@ -1,0 +1,49 @@
+"""All gradients of a layer in one call: bit for bit those of the separate products, whether or not the launch that adds the weight gradient's slices
+also splits the blocks of the input gradient."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from pytorch_block_sparse_amd import BlockSparseLinear, BlockSparseMatrix, native
+
+pytestmark = pytest.mark.gpu
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+@pytest.mark.parametrize("dtype, tokens, in_f, out_f, nnz, bias", [
+    # slices, and blocks in parts
+    (F32, 4096, 768, 3072, 1152, True), (F32, 3072, 3072, 768, 1151, True), (F32, 4097, 1024, 1024, 1021, False), (F32, 16384, 2048, 2048, 4095, True),
+    (F32, 4099, 768, 768, 286, True),   # slices alone
+    (F32, 130, 768, 3072, 1152, True),  # neither
+    (F32, 1, 32, 32, 1, True), (F32, 64, 416, 160, 0, True), (F32, 0, 768, 3072, 700, True),
+    (BF16, 2317, 768, 3072, 1152, True), (BF16, 8192, 2048, 2048, 2000, True),
+])
+def test_together_like_apart(cuda, dtype, tokens, in_f, out_f, nnz, bias):
+    np.random.seed(nnz)
+    layer = BlockSparseLinear(in_f, out_f, bias=bias, density=0.5, device=cuda, dtype=dtype)
+    layer.weight = BlockSparseMatrix.randn((out_f, in_f), nnz, device=cuda, dtype=dtype)
+    g = torch.Generator(device="cuda").manual_seed(nnz)
+    x = torch.randn((tokens, in_f), generator=g, device=cuda, dtype=dtype).requires_grad_(True)
+    dy = torch.randn((tokens, out_f), generator=g, device=cuda, dtype=dtype)
+    weights = [layer.weight.get_differentiable_data()] + ([layer.bias] if bias else [])
+    y = layer(x)
+    apart = torch.autograd.grad(y, [x], dy, retain_graph=True) + torch.autograd.grad(y, weights, dy, retain_graph=True)
+    together = torch.autograd.grad(y, [x] + weights, dy)
+    for a, b in zip(apart, together):
+        assert torch.equal(a, b)
+
+
+def test_workspace_and_arguments(cuda):
+    """(Refused before anything is launched: none of these pointers is read.)"""
+    lib, p, null = native.load(), ctypes.c_void_p(0x1000), ctypes.c_void_p(0)
+    need = lib.pbs_blocksparse_linear_back_workspace_bytes(4096, 3072, 768, 1152, 0)
+    assert need >= lib.pbs_blocksparse_matmul_back_bias_workspace_bytes(4096, 3072, 768, 1152, 0) + 1152 * 6144
+
+    def call(dy=p, x=p, data=p, dx=p, units=p, tokens=4096, dtype=0, ws=p, size=need):
+        return lib.pbs_blocksparse_linear_back(dy, x, data, p, p, p, units, dx, p, p, tokens, 3072, 768, 1152, dtype, ws, size, null)
+    assert call(size=need - 1) == -5 and call(ws=null) == -5 and call(ws=ctypes.c_void_p(0x1008)) == -5
+    assert call(dy=null) == -1 and call(x=null) == -1 and call(data=null) == -1 and call(dx=null) == -1 and call(units=null) == -1
+    assert call(dx=ctypes.c_void_p(0x1004)) == -4 and call(x=ctypes.c_void_p(0x1004)) == -4
+    assert call(tokens=-1) == -2 and call(dtype=7) == -3
