@@ -332,20 +332,28 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         return Head{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y), __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w)};
     };
 
-    f32x16 total[2], part[2];   // of 32 tokens each: the column so far, and a block
-    int sign = 0;               // of the block in part[1]
-    auto join = [&](int t) __attribute__((always_inline)) {
-        const float one = with_sign(1.f, sign);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) total[t][v] = __builtin_fmaf(part[t][v], one, total[t][v]);
+    // The sums of TH times 32 tokens: the column so far, and a block, which joins it when the next one is under way.
+    struct Whole {
+        f32x16 total[2], part[2];
+        int sign;   // of the block in the last part
     };
-    auto clear = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) total[t][v] = part[t][v] = 0.f;
+    struct Half {
+        f32x16 total[1], part[1];
+        int sign;
     };
-    clear();
+    auto join = [&](auto& sums, int t) __attribute__((always_inline)) {
+        const float one = with_sign(1.f, sums.sign);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sums.total[t][v] = __builtin_fmaf(sums.part[t][v], one, sums.total[t][v]);
+    };
+    auto clear = [&](auto& sums) __attribute__((always_inline)) {
+        sums.sign = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            sums.total[0][v] = sums.part[0][v] = 0.f;
+            if constexpr (sizeof(sums) == sizeof(Whole)) sums.total[1][v] = sums.part[1][v] = 0.f;
+        }
+    };
 
     auto publish = [&](int u) __attribute__((always_inline)) {
         if (lane == 0) lds_poke(s_done + wave, u);
@@ -363,10 +371,12 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         if (!here) give_up();
     };
     // results of a unit, a token's 16 values per lane: columns 8 q + 4 h + e of token 32 t + r
-    auto epilogue = [&](const Head& unit) __attribute__((always_inline)) {
+    auto epilogue = [&](const Head& unit, auto& sums) __attribute__((always_inline)) {
+        constexpr int TH = sizeof(sums) == sizeof(Whole) ? 2 : 1;
+        auto& total = sums.total;
         const int col = unit.col, row0 = unit.row & ~3;
         if (col < 0) return;
-        join(1);   // (of the last block)
+        join(sums, TH - 1);   // (of the last block)
         int at = lane;   // (opaque: the addresses below are made here, not kept in registers while the column is multiplied)
         asm volatile("" : "+v"(at));
         const int r = at & 31, h = at >> 5;
@@ -375,15 +385,14 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
 #pragma unroll
         for (int v = 0; v < 16; ++v) b[v] = g.bias ? g.bias[col * 32 + 8 * (v >> 2) + 4 * h + (v & 3)] : 0.f;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            if (t == 0 && unit.row & 3) continue;
+        for (int t = 0; t < TH; ++t) {
             float off = 0.f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 total[t][v] *= SP_UNSCALE;
                 off = __builtin_fmaf(total[t][v], 0.f, off);
             }
-            const int row = row0 + (t == 1 && !(unit.row & 1) ? 32 : 0) + r;
+            const int row = row0 + (TH == 2 ? t * 32 : (unit.row & 1 ? 0 : 32)) + r;
             if (__any(off != 0.f || off != off)) {
                 // again, with fp32 instructions and operands as they are, each block's products summed by themselves as well: infinities, NaN, results
                 // beyond the scaled range
@@ -442,7 +451,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     };
     auto arrived = [](int2& w) __attribute__((always_inline)) { asm volatile("" : "+v"(w.x), "+v"(w.y)); };
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 fw[2][6];   // [k half][part] of an item's block, and of the next item's
+    u32x4 first[6];   // [k half][part] of the block that a unit starts with
     const unsigned lane16 = lane * 16u;
     auto load_block = [&](u32x4 (&w)[6], int b) __attribute__((always_inline)) {
         const unsigned char* src = g.parts + (size_t)(unsigned)b * SP_BLOCK_BYTES;
@@ -457,117 +466,234 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     int2 ev = window(unit, 0), ev1 = window(head_of(1), 0), ev2 = make_int2(0, 0);
     arrived(ev);
     arrived(ev1);
-    load_block(fw[0], __builtin_amdgcn_readlane(ev.y, 0));
+    load_block(first, __builtin_amdgcn_readlane(ev.y, 0));
     int raw = 0, slot = 0;
     for (int j = 0; j < mine; ++j) {
         const int n = unit.n, u0 = j * KB;
         ev2 = window(head_of(j + 2), 0);
         if (n > 0) {
-            // a wave with 32 tokens of the tile has them in total[1], part[1]: the block before joins its total while the operands come from LDS
-            const bool half = unit.row & 3;
-            const int x_second = unit.row & 1 ? 0 : 2048;
             int kb = __builtin_amdgcn_readlane(ev.x, 0);
             publish(u0 + kb);
             slot = slot_of(u0 + kb);
-            // one item: w = its block, w_next takes the next one's (behind the last one the first of the next unit)
-            auto item = [&](int i, u32x4 (&w)[6], u32x4 (&w_next)[6]) __attribute__((always_inline)) {
-                const int u = u0 + kb;
-                const int this_sign = block_sign(kb);
-                const bool last = i + 1 == n;
-                if (((i + 1) & 63) == 0 && !last) {
-                    ev = window(unit, i + 1);
-                    arrived(ev);
-                }
-                const int kb_in = __builtin_amdgcn_readlane(ev.x, (i + 1) & 63), kb_out = KB + __builtin_amdgcn_readlane(ev1.x, 0);
-                kb = last ? kb_out : kb_in;
-                const int b_in = __builtin_amdgcn_readlane(ev.y, (i + 1) & 63), b_out = __builtin_amdgcn_readlane(ev1.y, 0);
-                load_block(w_next, last ? b_out : b_in);
-                if (__builtin_expect(__builtin_amdgcn_readfirstlane(raw) <= u, 0)) wait_for(u);
-                asm volatile("" ::: "memory");
-                const unsigned char* p0 = smem + (x_at + slot * SLOT);
-                const unsigned char* p1 = smem + ((x_at ^ 32) + slot * SLOT);
-                u32x4 x[2][3];   // [half of k][part] of 32 tokens
-                auto read = [&](int t, int q, int p) __attribute__((always_inline)) {
-                    x[q][p] = *reinterpret_cast<const u32x4*>((q ? p1 : p0) + p * PLANE + (t ? x_second : 0));
+            int i = 0;
+            if (unit.row & 3) {
+                // A wave with 32 tokens of the tile: an item is shorter than a block's way from the L2, and waiting for its operands would be a third of it.  The
+                // registers of the other 32 tokens are free: blocks are asked for two items ahead, and an operand is read for the next item once it is used.  On a
+                // path of its own (the choice cost the whole tiles 1.3 %): 28 products with Zipf rows 1.045 times as fast forward, 1.014 input gradient, up to 1.12
+                // (1824 -> 1472 density 0.667, 2720 tokens 86 -> 77 us).  The same for whole tiles, and filling waves that wait for no LDS access they have just
+                // made, give nothing (0.98 to 1.0): these kernels are bound by power, and the clock gives back what their cycles save.
+                Half sums;
+                clear(sums);
+                u32x4 x[2][3];   // [half of k][part]
+                const unsigned x_half = x_at + (unit.row & 1 ? 0 : 2048);
+                auto read = [&](int q, int p) __attribute__((always_inline)) {
+                    x[q][p] = *reinterpret_cast<const u32x4*>(smem + ((q ? x_half ^ 32 : x_half) + slot * SLOT) + p * PLANE);
                 };
-                if (!half) {
+                auto here = [&]() __attribute__((always_inline)) {
+                    if (__builtin_expect(__builtin_amdgcn_readfirstlane(raw) <= u0 + kb, 0)) wait_for(u0 + kb);
+                    asm volatile("" ::: "memory");
+                };
+                int kb_next = 0;
+                auto entry = [&](int i, int& at, int& b) __attribute__((always_inline)) {   // (behind the last one the first of the next unit)
+                    const bool inside = i < n;
+                    if ((i & 63) == 0 && inside) {
+                        ev = window(unit, i);
+                        arrived(ev);
+                    }
+                    const int kb_in = __builtin_amdgcn_readlane(ev.x, i & 63), kb_out = KB + __builtin_amdgcn_readlane(ev1.x, 0);
+                    const int b_in = __builtin_amdgcn_readlane(ev.y, i & 63), b_out = __builtin_amdgcn_readlane(ev1.y, 0);
+                    at = inside ? kb_in : kb_out;
+                    b = inside ? b_in : b_out;
+                };
+                auto item = [&](int i, const u32x4 (&w)[6], u32x4 (&w_ahead)[6]) __attribute__((always_inline)) {
+                    const bool more = i + 1 < n;
+                    int kb_ahead, b_ahead;
+                    entry(i + 2, kb_ahead, b_ahead);
+                    const int this_sign = block_sign(kb);
+                    load_block(w_ahead, b_ahead);
+                    kb = kb_next;
+                    kb_next = kb_ahead;
+                    slot = slot_of(u0 + kb);
+                    __builtin_amdgcn_sched_barrier(0);
+                    join(sums, 0);   // the block before
+                    sums.sign = this_sign;
+                    asm volatile("" : "+v"(sums.total[0]));
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sums.part[0][v] = 0.f;
+                    auto mma = [&](int q, int pw, int px) __attribute__((always_inline)) {
+                        sums.part[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[q][px]),
+                                                                               sums.part[0], 0, 0, 0);
+                    };
+                    mma(0, 0, 2);
+                    mma(0, 1, 1);
+                    mma(0, 0, 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every read of the slot
+                    publish(u0 + kb);   // (behind the last item this may be less than the next unit needs, never more)
+                    raw = landed(slot);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma(0, 2, 0);
+                    mma(0, 1, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (more) {
+                        here();
+                        read(0, 2);
+                        read(0, 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma(1, 0, 2);
+                    mma(1, 1, 1);
+                    mma(1, 0, 1);
+                    mma(1, 2, 0);
+                    mma(1, 1, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (more) {
+                        read(1, 2);
+                        read(1, 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma(0, 0, 0);
+                    mma(1, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (more) {
+                        read(0, 0);
+                        read(1, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                u32x4 w0[6], w1[6], w2[6];
+                here();
+#pragma unroll
+                for (int k = 0; k < 6; ++k) read(k / 3, 2 - k % 3);
+#pragma unroll
+                for (int k = 0; k < 6; ++k) w0[k] = first[k];
+                int b_next;
+                entry(1, kb_next, b_next);
+                load_block(w1, b_next);
+                while (true) {
+                    item(i, w0, w2);
+                    if (++i == n) {
+#pragma unroll
+                        for (int k = 0; k < 6; ++k) first[k] = w1[k];
+                        break;
+                    }
+                    item(i, w1, w0);
+                    if (++i == n) {
+#pragma unroll
+                        for (int k = 0; k < 6; ++k) first[k] = w2[k];
+                        break;
+                    }
+                    item(i, w2, w1);
+                    if (++i == n) {
+#pragma unroll
+                        for (int k = 0; k < 6; ++k) first[k] = w0[k];
+                        break;
+                    }
+                }
+                epilogue(unit, sums);
+            } else {
+                Whole sums;
+                clear(sums);
+                // one item: w = its block, w_next takes the next one's (behind the last one the first of the next unit)
+                auto item = [&](int i, u32x4 (&w)[6], u32x4 (&w_next)[6]) __attribute__((always_inline)) {
+                    const int u = u0 + kb;
+                    const int this_sign = block_sign(kb);
+                    const bool last = i + 1 == n;
+                    if (((i + 1) & 63) == 0 && !last) {
+                        ev = window(unit, i + 1);
+                        arrived(ev);
+                    }
+                    const int kb_in = __builtin_amdgcn_readlane(ev.x, (i + 1) & 63), kb_out = KB + __builtin_amdgcn_readlane(ev1.x, 0);
+                    kb = last ? kb_out : kb_in;
+                    const int b_in = __builtin_amdgcn_readlane(ev.y, (i + 1) & 63), b_out = __builtin_amdgcn_readlane(ev1.y, 0);
+                    load_block(w_next, last ? b_out : b_in);
+                    if (__builtin_expect(__builtin_amdgcn_readfirstlane(raw) <= u, 0)) wait_for(u);
+                    asm volatile("" ::: "memory");
+                    const unsigned char* p0 = smem + (x_at + slot * SLOT);
+                    const unsigned char* p1 = smem + ((x_at ^ 32) + slot * SLOT);
+                    u32x4 x[2][3];   // [half of k][part] of 32 tokens
+                    auto read = [&](int t, int q, int p) __attribute__((always_inline)) {
+                        x[q][p] = *reinterpret_cast<const u32x4*>((q ? p1 : p0) + p * PLANE + t * 2048);
+                    };
 #pragma unroll
                     for (int k = 0; k < 6; ++k) read(0, k / 3, 2 - k % 3);
-                }
-                slot = slot_of(u0 + kb);
-                auto reads_back = [&]() __attribute__((always_inline)) {   // every read of the slot
-                    raw = landed(slot);
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    publish(u0 + kb);   // (behind the last item this may be less than the next unit needs, never more)
-                };
-                __builtin_amdgcn_sched_barrier(0);
+                    slot = slot_of(u0 + kb);
+                    auto reads_back = [&]() __attribute__((always_inline)) {   // every read of the slot
+                        raw = landed(slot);
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                        publish(u0 + kb);   // (behind the last item this may be less than the next unit needs, never more)
+                    };
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const bool mine = t == 1 || !half;
-                    f32x16& c = part[t];
-                    auto mma = [&](int q, int pw, int px) __attribute__((always_inline)) {
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[q][px]), c, 0, 0, 0);
-                    };
-                    auto small = [&](int q) __attribute__((always_inline)) {   // (first those whose operands are read first)
-                        mma(q, 0, 2);
-                        mma(q, 1, 1);
-                        mma(q, 0, 1);
-                        mma(q, 2, 0);
-                        mma(q, 1, 0);
-                    };
-                    if (mine) {
+                    for (int t = 0; t < 2; ++t) {
+                        f32x16& c = sums.part[t];
+                        auto mma = [&](int q, int pw, int px) __attribute__((always_inline)) {
+                            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[3 * q + pw]), __builtin_bit_cast(bf16x8, x[q][px]), c, 0, 0, 0);
+                        };
+                        auto small = [&](int q) __attribute__((always_inline)) {   // (first those whose operands are read first)
+                            mma(q, 0, 2);
+                            mma(q, 1, 1);
+                            mma(q, 0, 1);
+                            mma(q, 2, 0);
+                            mma(q, 1, 0);
+                        };
 #pragma unroll
                         for (int v = 0; v < 16; ++v) c[v] = 0.f;
                         small(0);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (t == 0) {
-                        read(1, 0, 2);
-                        read(1, 0, 1);
-                    }
-                    if (t == 0 || !half) join(t ^ 1);   // t = 0: of the block before
-                    if (t == 0) sign = this_sign;
-                    asm volatile("" : "+v"(total[t ^ 1]));   // (here, where matrix instructions are under way, and not at the end)
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (mine) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (t == 0) {
+                            read(1, 0, 2);
+                            read(1, 0, 1);
+                        }
+                        join(sums, t ^ 1);   // t = 0: of the block before
+                        if (t == 0) sums.sign = this_sign;
+                        asm volatile("" : "+v"(sums.total[t ^ 1]));   // (here, where matrix instructions are under way, and not at the end)
+                        __builtin_amdgcn_sched_barrier(0);
                         small(1);
                         mma(0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (t == 0) {
+                            read(1, 0, 0);
+                            read(1, 1, 2);
+                            read(1, 1, 1);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        mma(1, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (t == 0) {
+                            read(1, 1, 0);
+                            reads_back();
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (t == 0) {
-                        read(1, 0, 0);
-                        read(1, 1, 2);
-                        read(1, 1, 1);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (mine) mma(1, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (t == 0) {
-                        read(1, 1, 0);
-                        reads_back();
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                };
+                u32x4 w1[6];
+                bool odd;
+                while (true) {
+                    item(i, first, w1);
+                    odd = true;
+                    if (++i == n) break;
+                    item(i, w1, first);
+                    odd = false;
+                    if (++i == n) break;
                 }
-            };
-            int i = 0;
-            bool odd;
-            while (true) {
-                item(i, fw[0], fw[1]);
-                odd = true;
-                if (++i == n) break;
-                item(i, fw[1], fw[0]);
-                odd = false;
-                if (++i == n) break;
-            }
-            epilogue(unit);
-            clear();
-            if (odd) {
+                epilogue(unit, sums);
+                if (odd) {
 #pragma unroll
-                for (int k = 0; k < 6; ++k) fw[0][k] = fw[1][k];
+                    for (int k = 0; k < 6; ++k) first[k] = w1[k];
+                }
             }
         } else {
-            epilogue(unit);   // (the sums are zero)
-            if (j + 1 < mine) load_block(fw[0], __builtin_amdgcn_readlane(ev1.y, 0));
+            if (unit.row & 3) {
+                Half sums;
+                clear(sums);
+                epilogue(unit, sums);
+            } else {
+                Whole sums;
+                clear(sums);
+                epilogue(unit, sums);
+            }
+            if (j + 1 < mine) load_block(first, __builtin_amdgcn_readlane(ev1.y, 0));
         }
         arrived(ev2);
         unit = head_of(j + 1);

@@ -1,0 +1,50 @@
+"""fp32 products on the bf16 cores with columns that two waves share and tiles of 32 tokens: columns of one block to all, next to each other and far apart."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from pytorch_block_sparse_amd import BlockSparseMatrix, native
+
+pytestmark = pytest.mark.gpu
+# blocks per column, of 128: the first ones are heavy (more than twice the average); around the 64 entries that a wave has at hand, and of every length modulo
+# the three blocks in flight
+UNEVEN = [128, 128, 127, 67, 66, 65, 64, 63, 1, 2, 3, 4, 5, 6, 7, 0, 1, 2, 1, 3, 2, 0, 1, 4]
+
+
+@pytest.mark.parametrize("transpose", [True, False])
+@pytest.mark.parametrize("tokens, counts", [
+    (4096, UNEVEN), (4133, UNEVEN), (8191, UNEVEN), (3300, UNEVEN),   # one group of columns more than without heavy ones
+    (4100, [128] * 8 + [9] * 24),                                     # heavy columns alone in their groups
+    (4127, [26] * 24),                                                # none: 32-token tiles of sparse columns
+])
+def test_halves(cuda, tokens, counts, transpose):
+    n, k = 32 * len(counts), 4096
+    rng = np.random.default_rng(tokens)
+    of_column = [np.sort(rng.choice(128, c, replace=False)) if c != 2 else np.array([0, 127]) for c in counts]   # (two: as far apart as can be)
+    cells = [(c, int(i)) if transpose else (int(i), c) for c, rows in enumerate(of_column) for i in rows]
+    rng.shuffle(cells)
+    shape = (n, k) if transpose else (k, n)
+    m = BlockSparseMatrix.zeros(shape, blocks=[tuple(int(v) for v in c) for c in cells], device=cuda, dtype=torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    with torch.no_grad():
+        m.data.normal_(generator=g)
+    a = torch.randn((tokens, k), generator=g, device=cuda)
+    kernel = native.load().pbs_blocksparse_matmul_kernel_name(tokens, n, k, len(cells), int(transpose), 0, 1)
+    assert b"split_kernel" in kernel
+    got = m.reverse_matmul(a, transpose=transpose)
+    failures = ctypes.c_uint()
+    assert native.load().pbs_protocol_failures(ctypes.byref(failures)) == 0 and failures.value == 0
+    dense = m.to_dense().double()
+    dense = dense.t() if transpose else dense
+    rows = torch.cat([torch.arange(0, tokens, 61), torch.arange(tokens - 70, tokens)]).to(cuda)
+    want, most = a[rows].double() @ dense.contiguous(), a[rows].double().abs() @ dense.abs().contiguous()
+    # a block's twelve products of parts and their sums (32 each) in fp32, the products that are left out, one rounding per block, each 2^-24 of at most the sum of
+    # the magnitudes
+    bound = (12 * 32 + 1 + max(counts)) * 2.0 ** -24 * most
+    assert bool(((got[rows].double() - want).abs() <= bound).all())
+    # the bits of a token are the same in any call
+    fewer = m.reverse_matmul(a[:tokens - 37].contiguous(), transpose=transpose)
+    if b"split_kernel" in native.load().pbs_blocksparse_matmul_kernel_name(tokens - 37, n, k, len(cells), int(transpose), 0, 1):
+        assert torch.equal(fewer, got[:tokens - 37])
