@@ -527,8 +527,13 @@ static int launch_split(const DdsArgs& g, void* workspace, bool parts_ready, hip
     a.K = g.K;
     const int groups_even = split_groups(g.N);
     a.heavy = (int)(2ll * g.nnz / (g.N / 32));
-    a.tiles = split_tiles(g.M, groups_even).full;
-    a.low_tiles = g.M > a.tiles * SP_BM ? (g.M - a.tiles * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
+    long long units = 0;   // at most
+    for (int more = 0; more <= SP_MORE; ++more) {
+        a.tiles[more] = split_tiles(g.M, groups_even + more).full;
+        const long long low = g.M > (long long)a.tiles[more] * SP_BM ? (g.M - (long long)a.tiles[more] * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
+        if (a.tiles[more] + low > units) units = a.tiles[more] + low;
+    }
+    units *= groups_even + groups_even / 2 + 1;
     // the 32 workgroups of an XCD work on tile_block token tiles x 32 / tile_block groups: the split with the least to read per k-block
     const double w_bytes = (double)SP_NC * SP_BLOCK_BYTES * g.nnz / ((double)(g.N / 32) * (g.K / 32)), x_bytes = SP_BM * 128.0;
     double least = 0.0;
@@ -542,7 +547,6 @@ static int launch_split(const DdsArgs& g, void* workspace, bool parts_ready, hip
             }
     }
     // one workgroup per CU; more where each would have more units than it keeps the heads of
-    const long long units = (long long)(a.tiles + a.low_tiles) * (groups_even + groups_even / 2 + 1);
     long long per_xcd = (units + NUM_XCD - 1) / NUM_XCD + 1;
     if (per_xcd > 32) per_xcd = per_xcd > 32 * (SP_MAX_UNITS - 1) ? per_xcd / (SP_MAX_UNITS - 1) + 1 : 32;
     return launch(kernel, dim3((unsigned)(NUM_XCD * per_xcd)), dim3((SP_NC + SP_NP) * 64), SP_LDS, stream, a);

@@ -57,6 +57,7 @@ constexpr int SP_SPIN_LIMIT = 1 << 20;
 constexpr int SP_BLOCK_BYTES = 6144;     // a block's three parts
 constexpr float SP_SCALE = 0x1p30f, SP_UNSCALE = 0x1p-60f;
 constexpr int SP_BM = 64;                // tokens of a tile (of a low one 32)
+constexpr int SP_MORE = 3;               // (with more groups than that more, as with that many)
 constexpr int SP_RS = 12;                // ring slots; a multiple of SP_NP: a slot has one writer
 constexpr int SP_PLANE = SP_BM * 64;     // one part of a panel: 64 bytes per token
 constexpr int SP_SLOT = 3 * SP_PLANE;
@@ -142,7 +143,7 @@ struct SplitArgs {
     const float* bias;            // nullptr or [N]
     float* out;                   // [M, N] row-major
     int M, N, K;
-    int tiles, low_tiles;         // of 64 tokens, and behind them of 32
+    int tiles[SP_MORE + 1];       // of 64 tokens, the others of 32 behind them; with so many groups more than without heavy columns
     int heavy;                    // columns of more blocks than this take two waves
     int tile_block;               // units are ordered by blocks of this many token tiles, then groups, then tiles
 };
@@ -163,7 +164,8 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     // A column of many more blocks than the others keeps its wave busy when all others are done.  So the columns of more than twice the average are
     // taken by two waves, 32 tokens of a tile each, in more groups if need be (3072 -> 768 with Zipf rows, 96 blocks of 24 on average, 4096 tokens: 66 -> 54 us
     // with the launch that splits the blocks).  Splitting more of them, or wherever a sum of rounds and longest stays says so, costs even patterns up to
-    // 40 % (another group is another time that the panels are split).
+    // 40 % (another group is another time that the panels are split).  Which tiles are full follows from the groups there are: with those of even columns,
+    // 3072 -> 768 with Zipf rows, 8192 tokens took 129 us (98), 3360 -> 3488 density 0.32, 1688 tokens 158 (117), level where there are no heavy columns.
     // Place v of the dealing: below 2 * heavy half v % 2 of column v / 2 of the ranking, else column v - heavy.
     int heavy = 0;
     {
@@ -177,14 +179,15 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         }
         heavy = __builtin_amdgcn_readfirstlane(heavy < ncols / 2 ? heavy : ncols / 2);   // (more only where a list holds more entries than there are blocks)
     }
-    const int groups = (ncols + heavy + SP_NC - 1) / SP_NC;
+    const int groups = (ncols + heavy + SP_NC - 1) / SP_NC, more_groups = groups - (ncols + SP_NC - 1) / SP_NC;
+    const int tiles = g.tiles[more_groups < SP_MORE ? more_groups : SP_MORE], low_tiles = g.M > tiles * SP_BM ? (g.M - tiles * SP_BM + SP_BM / 2 - 1) / (SP_BM / 2) : 0;
 
     // The units of this XCD: its share of the tiles x groups, then of the low tiles x groups.  Its workgroups take them in turn, every other round
     // from the other end: who has started with one of the first, which hold the longest columns, does not get the odd one at the end as well.
     const int xcd = blockIdx.x % NUM_XCD, local = blockIdx.x / NUM_XCD, peers = gridDim.x / NUM_XCD;
     auto share = [&](int units, int x) __attribute__((always_inline)) { return (int)((long long)units * x / NUM_XCD); };
-    const int full0 = share(g.tiles * groups, xcd), n_full = share(g.tiles * groups, xcd + 1) - full0;
-    const int low0 = share(g.low_tiles * groups, xcd), n_low = share(g.low_tiles * groups, xcd + 1) - low0;
+    const int full0 = share(tiles * groups, xcd), n_full = share(tiles * groups, xcd + 1) - full0;
+    const int low0 = share(low_tiles * groups, xcd), n_low = share(low_tiles * groups, xcd + 1) - low0;
     const int rounds = (n_full + n_low) / peers;
     const int mine = rounds + ((rounds & 1 ? peers - 1 - local : local) < (n_full + n_low) % peers ? 1 : 0);
     if (mine == 0) return;
@@ -192,13 +195,13 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     auto unit_of = [&](int j, int& group, int& row0, bool& low) __attribute__((always_inline)) {
         const int w = j * peers + (j & 1 ? peers - 1 - local : local);
         low = w >= n_full;
-        const int v = low ? low0 + w - n_full : full0 + w, of = low ? g.low_tiles : g.tiles;
+        const int v = low ? low0 + w - n_full : full0 + w, of = low ? low_tiles : tiles;
         const int tb = v / (g.tile_block * groups), rem = v - tb * (g.tile_block * groups);
-        int tiles = of - tb * g.tile_block;
-        tiles = tiles < g.tile_block ? tiles : g.tile_block;
-        group = rem / tiles;
-        const int tile = tb * g.tile_block + rem - group * tiles;
-        row0 = low ? g.tiles * SP_BM + tile * (SP_BM / 2) : tile * SP_BM;
+        int in_block = of - tb * g.tile_block;
+        in_block = in_block < g.tile_block ? in_block : g.tile_block;
+        group = rem / in_block;
+        const int tile = tb * g.tile_block + rem - group * in_block;
+        row0 = low ? tiles * SP_BM + tile * (SP_BM / 2) : tile * SP_BM;
     };
 
     if (tid < RS + SP_NC + 1) s_landed[tid] = 0;
