@@ -60,11 +60,18 @@ typedef int __attribute__((address_space(3))) lds_int;
 static __device__ __forceinline__ int lds_peek(const int* p) { return *(const volatile lds_int*)p; }
 static __device__ __forceinline__ void lds_poke(int* p, int v) { *(volatile lds_int*)p = v; }
 
+// the lane's number, made where it is asked for: it needs no register until then
+static __device__ __forceinline__ int lane_now() {
+    int lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(lane));
+    return lane;
+}
+
 // Waits of the barrier-free kernels that ran into their bound, counted over the life of the process (one word per
 // GPU).  Such a wait means a broken progress protocol; the kernel also turns the affected results into NaN.
 static __device__ unsigned g_protocol_failures;
 static __device__ __forceinline__ void count_protocol_failure() {
-    if ((threadIdx.x & 63) == 0) atomicAdd(&g_protocol_failures, 1u);
+    if (lane_now() == 0) atomicAdd(&g_protocol_failures, 1u);
 }
 
 // a wave-uniform pointer, forced into scalar registers

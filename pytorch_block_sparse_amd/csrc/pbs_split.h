@@ -157,8 +157,8 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     int* const s_done = s_landed + RS;                            // [SP_NC]
     int* const s_fail = s_done + SP_NC;
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = lane_now();   // (what is kept of the thread's number over the multiplying waves' loops would be spilled)
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int KB = g.K >> 5, ncols = g.N >> 5;
 
     // A column of many more blocks than the others keeps its wave busy when all others are done.  So the columns of more than twice the average are
@@ -204,7 +204,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         row0 = low ? tiles * SP_BM + tile * (SP_BM / 2) : tile * SP_BM;
     };
 
-    if (tid < RS + SP_NC + 1) s_landed[tid] = 0;
+    if ((int)threadIdx.x < RS + SP_NC + 1) s_landed[threadIdx.x] = 0;
     __syncthreads();
     bool gave_up = false;
     auto give_up = [&]() __attribute__((always_inline)) {
@@ -380,8 +380,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
         const int col = unit.col, row0 = unit.row & ~3;
         if (col < 0) return;
         join(sums, TH - 1);   // (of the last block)
-        int at = lane;   // (opaque: the addresses below are made here, not kept in registers while the column is multiplied)
-        asm volatile("" : "+v"(at));
+        const int at = lane_now();   // (the addresses below are made here, not kept in registers while the column is multiplied)
         const int r = at & 31, h = at >> 5;
         const bool failed = gave_up || __builtin_amdgcn_readfirstlane(lds_peek(s_fail)) != 0;
         float b[16];   // (word by word: a bias need not be aligned to more)
@@ -447,7 +446,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     auto window = [&](const Head& unit, int i0) __attribute__((always_inline)) {
         int2 e = make_int2(0, 0);
         if (unit.n > 0) {
-            const int l = i0 + lane;
+            const int l = i0 + lane_now();
             e = records[list_record(KB, unit.rank) + LIST_HEAD + (l < unit.n ? l : unit.n - 1)];
         }
         return e;
@@ -473,7 +472,6 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
     int raw = 0, slot = 0;
     for (int j = 0; j < mine; ++j) {
         const int n = unit.n, u0 = j * KB;
-        ev2 = window(head_of(j + 2), 0);
         if (n > 0) {
             int kb = __builtin_amdgcn_readlane(ev.x, 0);
             publish(u0 + kb);
@@ -593,6 +591,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                         break;
                     }
                 }
+                ev2 = window(head_of(j + 2), 0);
                 epilogue(unit, sums);
             } else {
                 Whole sums;
@@ -680,6 +679,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                     odd = false;
                     if (++i == n) break;
                 }
+                ev2 = window(head_of(j + 2), 0);
                 epilogue(unit, sums);
                 if (odd) {
 #pragma unroll
@@ -687,6 +687,7 @@ __global__ __launch_bounds__((SP_NC + SP_NP) * 64, 3) void split_kernel(SplitArg
                 }
             }
         } else {
+            ev2 = window(head_of(j + 2), 0);
             if (unit.row & 3) {
                 Half sums;
                 clear(sums);
