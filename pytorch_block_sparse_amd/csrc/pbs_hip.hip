@@ -670,21 +670,17 @@ static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
 // four in the best number of slices that an estimate of those alone made; 4 fp32 ones of the 160 are slower by more than 2 %, one by 13 %.
 // (The number of units follows from the average row, so what looks like a full chip may be one workgroup more than that: for fp32, whose rounds are long, the mean
 // of the estimated number and of 4 % more.  The reduction is a launch and an allocation more for the host: 2 (bf16 0.75) us more than the fit has for it.)
+// fp32 on the bf16 matrix cores (sdd_split_kernel) where its estimate is the smaller one, from 2^22 tokens x blocks in units of four (2048 -> 2048 density 0.25, 4096 tokens
+// 98 -> 86 us, 4096 -> 4096 density 0.25, 16384 tokens 1267 -> 1091), from 2^20 on, with 256 blocks and more, in units of two to four and at most 8 slices: 50 such problems
+// 1.09 times as fast as the fp32 kernel in what its own estimate picks (3072 -> 768 with Zipf rows, 4096 tokens 58 -> 49; 768 -> 3072 density 0.5, 1024 tokens 30.7 -> 27.5; up to 1.28).  Of
+// fewer blocks the estimates do not tell which is ahead (0.87 to 1.14), nor of more slices; between 2^17 and 2^20 it is 1.5 % the slower one at its best (36 problems, 0.80 to 1.11).
+constexpr long long SPLIT_BACK_WORK = 1ll << 20, SPLIT_BACK_LARGE = 1ll << 22;
+constexpr int SPLIT_BACK_BLOCKS = 256, SPLIT_BACK_SLICES = 8;
 enum RowKernel { ROW_F32, ROW_SPLIT, ROW_BF16 };   // sdd_row_kernel<float>, sdd_split_kernel, sdd_row_kernel<bf16_t>
 // workgroups of the fullest XCD
 static double row_tasks(double units, int slices) { return units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices; }
 static double row_us(RowKernel kernel, long long M, int N, int K, int nnz, int per_unit, int slices, int passes) {
     const double chunks = (double)((M + ROW_TC - 1) / ROW_TC), wave = std::ceil(chunks / (ROW_NW * slices * (double)passes));
-    if (kernel == ROW_SPLIT) {
-        // (units of ROW_NB: 60 problems of 2^22 tokens x blocks and more at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted
-        // without a bound, the cost of a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
-        const double rows = N / 32;
-        const double units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
-        const double blocks = nnz / units > 0.5 ? nnz / units : 0.5;
-        const double tasks = units < ROW_FEW_UNITS ? std::ceil(units * slices / NUM_XCD) : std::ceil(units / NUM_XCD) * slices;
-        const double busy = std::ceil(tasks / 32) * wave * blocks * 0.454, alone = wave * blocks * 0.540;
-        return (slices > 1 ? 3.02 : 0.0) + passes * (7.03 + (busy > alone ? busy : alone) + std::ceil(tasks / 64) * 4.5);
-    }
     struct Model {
         double more, launch, reduce, per_slice, alone, alone_row, busy, busy_row, most, whole, start;   // .._row: of a unit, besides its blocks
         double cached, far, per_mb;   // from so many MB of operands on: how much longer the copies of a full chip take per 100 MB, and what a MB takes at least
@@ -694,6 +690,26 @@ static double row_us(RowKernel kernel, long long M, int N, int K, int nnz, int p
     const double rows = N / 32, row = nnz / rows, columns = K / 32;
     const double full = nnz / (double)per_unit + rows * (per_unit - 1) / (2.0 * per_unit) * (1.0 - std::exp(-2.0 * row)), units = full + rows * std::exp(-row);
     const double mean = nnz / full, most = per_unit < columns ? per_unit : columns;   // blocks of a unit
+    if (kernel == ROW_SPLIT) {
+        if (M * nnz >= SPLIT_BACK_LARGE) {
+            // (units of ROW_NB: 60 such problems at ten slice counts, within 10 %, its choices 1.1 % slower than the best on average.  Fitted without a bound, the cost of
+            // a slice came out below nothing, and large gradients were cut into too many: 2048 -> 2048 density 0.25, 4096 tokens 102 -> 86 us)
+            const double all_units = nnz >= rows ? nnz / (double)ROW_NB + 0.4 * rows : rows * (1.0 - std::exp(-nnz / rows));   // (those with blocks)
+            const double blocks = nnz / all_units > 0.5 ? nnz / all_units : 0.5, tasks = row_tasks(all_units, slices);
+            const double busy = std::ceil(tasks / 32) * wave * blocks * 0.454, alone = wave * blocks * 0.540;
+            return (slices > 1 ? 3.02 : 0.0) + passes * (7.03 + (busy > alone ? busy : alone) + std::ceil(tasks / 64) * 4.5);
+        }
+        // (units of two to four: 105 problems of 2^20 tokens x blocks and more, at up to ten numbers of slices, within 6 %; its choices are 1.8 % slower than the best on
+        // average, in the larger ones 0.1 % more than those above.  A CU has two workgroups at a time: rounds of 64 over an XCD's 32 CUs, of which the last takes less if no CU has two.)
+        const double one = wave * (0.341 * most + 0.591), two = wave * (0.792 * mean + 0.737);
+        auto all = [&](double tasks) {
+            const double whole = std::floor(tasks / 64), rest = tasks - 64 * whole;
+            const double rounds = whole * two + (rest == 0.0 ? 0.0 : rest <= 32 || one > two ? one : two), us = 0.595 * rounds + 0.405 * tasks / 64 * two;
+            return (us > one ? us : one) + 0.889 * tasks / 64;
+        };
+        return (slices > 1 ? 2.0 + 0.4 * slices * nnz / 1000.0 + 0.272 * slices : 0.0) +
+               passes * (4.66 + 0.5 * (all(row_tasks(units, slices)) + all(row_tasks(1.03 * units, slices))));
+    }
     const double tasks = row_tasks(units, slices), tasks_more = m.more > 1.0 ? row_tasks(m.more * units, slices) : tasks;
     const double alone = wave * (m.alone * (mean + m.most * (most - mean)) + m.alone_row);
     const double rounds = 0.5 * (m.whole * (std::ceil(tasks / 32) + std::ceil(tasks_more / 32)) + (1.0 - m.whole) * (tasks + tasks_more) / 32);
@@ -730,10 +746,8 @@ static SddPlan plan_sdd(long long M, int N, int K, int nnz) {
 // 4 x 2 1199 against 1222, 0.5 2 x 4 2258 against 2347, 1 1 x 8 4131 against 4297; 65536 tokens, density 1 1 x 33 16538 against
 // 16998; 8192 -> 8192, 16384 tokens, density 0.25 1 x 16 4805 against 5211, 0.5 9264 against 10299.
 constexpr size_t ROW_WORKSPACE_BYTES = 64u << 20;
-// fp32 on the bf16 matrix cores (sdd_split_kernel) from 2^22 tokens x blocks where its estimate is the smaller one (2048 -> 2048 density 0.25, 4096 tokens
-// 98 -> 86 us, 4096 -> 4096 density 0.25, 16384 tokens 1267 -> 1091).  Between 2^21 and 2^22 its time is 0.7 to 1.24 of the fp32 kernel's and the estimates do not tell which
-// (25 problems, 0.95 on average; 3072 -> 768 with Zipf rows 52 and 48 us, 2016 -> 1408 at 2779 tokens 51 and 63), below 2^21 the same on average.
-constexpr long long SPLIT_BACK_WORK = 1ll << 22;
+// where the input gradient's blocks are split, the launch that adds the slices does it
+constexpr double REDUCE_SAVES = 4.0;
 // a chunk of 32 tokens that has 4 GB or more: it is not addressed as one buffer
 static bool row_far(int esz, int N, int K) { return (long long)(N > K ? N : K) * esz * ROW_TC >= (1ll << 32); }
 struct RowChoice {
@@ -757,6 +771,7 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
     RowChoice best{1, 1, ROW_NB, false};
     double best_us = -1.0;
+    const double saved = dtype == PBS_DTYPE_F32 && split_kernel_fits(M, K, N, nnz) ? REDUCE_SAVES : 0.0;
     const bool far = row_far(dtype == PBS_DTYPE_F32 ? 4 : 2, N, K), one_list = far || unit_lists_only(N / 32);
     for (const int s : CANDIDATES) {
         if (s > 1 && (s > chunks / 4 || (size_t)nnz * 4096 * s > workspace_limit)) break;
@@ -766,14 +781,18 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
             if (!lists && per_unit != ROW_NB && (s > 1 ? (size_t)nnz * 4096 * s : 0) + unit_table_bytes(N, nnz, per_unit) > workspace_limit + unit_table_bytes(N, nnz, ROW_NB)) return;
             // (fp32: sums of longer shares would be less exact than those of units of four in several slices)
             if (kernel == ROW_F32 && per_unit != ROW_NB && chunks > (long long)(per_unit > ROW_NB ? ROW_LONG : ROW_LONG_GROUPS) * ROW_NW * s * passes) return;
-            const double us = row_us(kernel, M, N, K, nnz, per_unit, s, passes);
+            const double us = row_us(kernel, M, N, K, nnz, per_unit, s, passes) - (s > 1 ? saved : 0.0);
             if (best_us < 0.0 || us < best_us) {
                 best = {s, passes, per_unit, kernel == ROW_SPLIT};
                 best_us = us;
             }
         };
         for (int p = one_list ? ROW_NB : 1; p <= (one_list ? ROW_NB : ROW_SIZES); ++p) consider(dtype == PBS_DTYPE_F32 ? ROW_F32 : ROW_BF16, p);
-        if (dtype == PBS_DTYPE_F32 && M * nnz >= SPLIT_BACK_WORK && !far) consider(ROW_SPLIT, ROW_NB);
+        if (dtype == PBS_DTYPE_F32 && !far) {
+            if (M * nnz >= SPLIT_BACK_LARGE) consider(ROW_SPLIT, ROW_NB);
+            else if (M * nnz >= SPLIT_BACK_WORK && nnz >= SPLIT_BACK_BLOCKS && s <= SPLIT_BACK_SLICES)
+                for (int p = one_list ? ROW_NB : 2; p <= ROW_NB; ++p) consider(ROW_SPLIT, p);
+        }
     }
     if (rectangles && fits && (large ? 0.9 : 1.0) * rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
     return best;

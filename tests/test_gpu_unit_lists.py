@@ -52,6 +52,9 @@ def test_every_list_holds_every_block_once(cuda, out_f, in_f, nnz):
     (F32, 5, 1, 33, 3072, 416, 842), (F32, 6, 1, 33, 3072, 768, 1050),
     (F32, 1, 2, 1500, 416, 160, 3), (F32, 2, 2, 2317, 3072, 160, 25), (F32, 3, 2, 3000, 416, 768, 76), (F32, 4, 2, 2317, 416, 416, 62),
     (F32, 5, 2, 3000, 2048, 416, 113), (F32, 6, 2, 2317, 416, 992, 256),
+    # sdd_split_kernel
+    (F32, 2, 1, 1500, 2912, 320, 906), (F32, 2, 2, 4097, 3072, 128, 262), (F32, 3, 1, 1500, 800, 928, 707), (F32, 3, 2, 3000, 160, 2496, 353),
+    (F32, 4, 1, 700, 1248, 1248, 1503), (F32, 4, 2, 1500, 2112, 352, 723),
     (BF16, 1, 1, 33, 416, 160, 3), (BF16, 2, 1, 33, 3072, 160, 197), (BF16, 3, 1, 33, 3072, 768, 464), (BF16, 4, 1, 33, 3072, 416, 673),
     (BF16, 5, 1, 33, 3072, 768, 881), (BF16, 6, 1, 33, 3072, 416, 1092),
     (BF16, 1, 2, 2317, 416, 160, 3), (BF16, 2, 2, 2317, 416, 160, 21), (BF16, 3, 2, 3000, 2048, 160, 17), (BF16, 4, 2, 3000, 1024, 160, 60),
