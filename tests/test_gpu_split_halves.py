@@ -48,3 +48,20 @@ def test_halves(cuda, tokens, counts, transpose):
     fewer = m.reverse_matmul(a[:tokens - 37].contiguous(), transpose=transpose)
     if b"split_kernel" in native.load().pbs_blocksparse_matmul_kernel_name(tokens - 37, n, k, len(cells), int(transpose), 0, 1):
         assert torch.equal(fewer, got[:tokens - 37])
+
+
+@pytest.mark.parametrize("tokens, k, n, nnz, parts", [
+    (9738, 256, 1184, 168, True), (7337, 960, 448, 246, True),   # between 1.5 and 2 2^20 tokens x blocks: by estimate
+    (1024, 3072, 768, 1600, False),
+    (6393, 960, 448, 246, False), (9361, 256, 1184, 168, False),   # the last count below 1.5 2^20
+])
+def test_smaller_products(cuda, tokens, k, n, nnz, parts):
+    np.random.seed(tokens)
+    m = BlockSparseMatrix.randn((n, k), nnz, device=cuda, dtype=torch.float32)
+    assert (native.load().pbs_blocksparse_matmul_parts_bytes(tokens, n, k, nnz, 1, 0) > 0) == parts
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    a = torch.randn((tokens, k), generator=g, device=cuda)
+    got, dense = m.reverse_matmul(a, transpose=True), m.to_dense().double().t().contiguous()
+    want, most = a.double() @ dense, a.double().abs() @ dense.abs()
+    # as above; with fp32 instructions a chain of at most k products
+    assert bool(((got.double() - want).abs() <= max(12 * 32 + 1 + k // 32, k) * 2.0 ** -24 * most).all())
