@@ -399,8 +399,9 @@ struct PanelChoice {
 static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
     PanelChoice best{0, 0.0, 0, 0};
     const int cols = n / 32;
-    // (below 1024 tokens, or with fewer columns than waves, it was the faster one nowhere)
-    if (nnz < 1 || M < 1024 || cols < PANEL_NW) return best;
+    // (with fewer columns than waves it was the faster one nowhere; below 1024 tokens only in chunks, from 768 on where a contraction of 2048 and 48 columns of 16
+    // blocks leave the stream kernel more to copy than two workgroups per CU take: 2720 -> 4064 density 0.5, 1015 tokens 31 -> 23 us, 2784 -> 3808 density 0.29, 954 tokens 22.5 -> 18)
+    if (nnz < 1 || cols < PANEL_NW || (M < 1024 && (M < 768 || k < 2048 || cols < 48 || nnz < 16 * cols))) return best;
     const double tiles = (double)((M + 16 * PANEL_TT - 1) / (16 * PANEL_TT));
     if (k > PANEL_MAX_K) {
         if (nnz < 5 * cols) return best;   // (shorter columns pay for chunks they do not use: 4 to 13 % slower than the stream kernel at 3 to 4 blocks)

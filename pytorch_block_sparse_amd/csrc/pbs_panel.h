@@ -214,7 +214,7 @@ __global__ __launch_bounds__(PANEL_NW * 64, 4) void panel_kernel(PanelArgs g) {
 // What bounds it: a chunk's copy, 64 KB at the texture path's rate (1.5 k cycles) and its latency behind the barrier (0.8 us per chunk in all).
 // Measured, us, against the stream kernel: 3072 -> 768 density 0.5, 2317 tokens 21.8 -> 16.5, 4096 tokens 27.8 -> 22.7; 4096 -> 4096
 // density 0.25, 1024 tokens 30.3 -> 24.1; 4096 -> 1024 density 0.75, 4096 tokens 69.8 -> 36.7; 1536 -> 2976 density 0.4, 2317 tokens
-// 31.8 -> 20.1.  Below 1024 tokens it is the slower one (3072 -> 768, 509 tokens 7.6 against 12.2).
+// 31.8 -> 20.1.  With fewer tokens and columns it is the slower one (3072 -> 768, 509 tokens 7.6 against 12.2).
 constexpr int PANEL_KC = 512;         // features of a chunk: 64 rows of 1 KB
 constexpr int PANEL_CHUNK_LDS = 2 * 16 * PANEL_TT * 1024 + PANEL_NW * 2048;
 template <int TRANS, int S>
