@@ -47,3 +47,37 @@ def test_workspace_and_arguments(cuda):
     assert call(dy=null) == -1 and call(x=null) == -1 and call(data=null) == -1 and call(dx=null) == -1 and call(units=null) == -1
     assert call(dx=ctypes.c_void_p(0x1004)) == -4 and call(x=ctypes.c_void_p(0x1004)) == -4
     assert call(tokens=-1) == -2 and call(dtype=7) == -3
+
+
+def test_graph_replays(cuda):
+    """A captured step: every replay, with eager steps between them, gives what the eager step gives."""
+    np.random.seed(5)
+    layer = BlockSparseLinear(3072, 768, density=0.5, device=cuda, dtype=F32)
+    x = torch.randn((4096, 3072), device=cuda).requires_grad_(True)
+    dy = torch.randn((4096, 768), device=cuda)
+    weights = [layer.weight.get_differentiable_data(), layer.bias]
+
+    def step():
+        return torch.autograd.grad(layer(x), [x] + weights, dy)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for seed in range(4):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        with torch.no_grad():
+            x.normal_(generator=g)
+            dy.normal_(generator=g)
+            layer.weight.data.normal_(generator=g)
+        eager = step()
+        for t in captured:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(captured, eager):
+            assert torch.equal(a, b)

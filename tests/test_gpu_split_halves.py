@@ -50,6 +50,30 @@ def test_halves(cuda, tokens, counts, transpose):
         assert torch.equal(fewer, got[:tokens - 37])
 
 
+def test_values_that_have_no_parts(cuda):
+    """In both halves of a tile that two waves share, and in a tile of 32 tokens at the end."""
+    tokens, k = 8191, 4096
+    rng = np.random.default_rng(7)
+    m = BlockSparseMatrix.zeros((32 * len(UNEVEN), k), blocks=[(c, int(i)) for c, n in enumerate(UNEVEN) for i in rng.choice(128, n, replace=False)],
+                                device=cuda, dtype=torch.float32)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    with torch.no_grad():
+        m.data.normal_(generator=g)
+    x = torch.randn((tokens, k), generator=g, device=cuda)
+    rows, at = [3, 40, 100, 8170, 8190], [5, 1000, 2000, 3000, 4095]
+    x[rows, at] = 0.0
+    x[[7, 50, 8180]] *= 2.0 ** 100   # beyond what is scaled
+    clean, bad = m.reverse_matmul(x, transpose=True), x.clone()
+    bad[rows, at] = torch.tensor([float("inf"), -float("inf"), float("nan"), float("inf"), float("nan")], device=cuda)
+    got, w = m.reverse_matmul(bad, transpose=True), m.to_dense()
+    reached = torch.zeros_like(got, dtype=torch.bool)
+    reached[rows] = (w != 0).t()[at]
+    assert reached.any(1)[rows].all() and torch.equal(torch.isfinite(got), ~reached) and torch.equal(got[~reached], clean[~reached])
+    want, most = x[[7, 50, 8180]].double() @ w.double().t().contiguous(), x[[7, 50, 8180]].double().abs() @ w.double().t().contiguous().abs()
+    # fp32 instructions: a block's chain of 32 products, and one rounding per block
+    assert bool(((got[[7, 50, 8180]].double() - want).abs() <= (32 + 1 + max(UNEVEN)) * 2.0 ** -24 * most).all())
+
+
 @pytest.mark.parametrize("tokens, k, n, nnz, parts", [
     (9738, 256, 1184, 168, True), (7337, 960, 448, 246, True),   # between 1.5 and 2 2^20 tokens x blocks: by estimate
     (1024, 3072, 768, 1600, False),
