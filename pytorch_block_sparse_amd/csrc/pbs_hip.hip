@@ -1213,9 +1213,7 @@ int pbs_blocksparse_derive(const int32_t* row_start_ends_a, const int32_t* cols_
     return units && !with_units ? build_units(row_start_ends_a, cols_a, out_features, in_features, nnz, unit_lists_only(N), units, s) : PBS_OK;
 }
 
-static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,
-                size_t workspace_limit = ROW_WORKSPACE_BYTES) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
+static int back_checks(const BackArgs& a, int64_t tokens, int dtype) {
     if (dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) return PBS_ERR_BAD_DTYPE;
     if (tokens < 0 || a.N <= 0 || a.K <= 0 || a.nnz < 0 || (a.N % 32) || (a.K % 32)) return PBS_ERR_BAD_SHAPE;
     if (tokens > (1ll << 30) || (long long)a.nnz > (long long)(a.N / 32) * (a.K / 32)) return PBS_ERR_TOO_LARGE;
@@ -1223,6 +1221,13 @@ static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, s
     if (!a.ptr || (a.nnz > 0 && (!a.idx || !a.out))) return PBS_ERR_NULL_POINTER;
     if (tokens > 0 && (!a.g || !a.x)) return PBS_ERR_NULL_POINTER;
     if (!aligned16(a.g) || !aligned16(a.x) || !aligned16(a.out) || !aligned16(a.bias_out) || !aligned16(a.units)) return PBS_ERR_MISALIGNED;
+    return PBS_OK;
+}
+static int back(const BackArgs& a, int64_t tokens, int dtype, void* workspace, size_t workspace_bytes, void* stream,
+                size_t workspace_limit = ROW_WORKSPACE_BYTES) {
+    if (int rc = back_checks(a, tokens, dtype)) return rc;
+    if (a.nnz == 0 && !a.bias_out) return PBS_OK;
+    hipStream_t s = static_cast<hipStream_t>(stream);
     if (tokens == 0) {
         const size_t esz = dtype == PBS_DTYPE_F32 ? 4 : 2;
         auto zero = [&](void* p, size_t values) {
@@ -1275,6 +1280,7 @@ int pbs_blocksparse_linear_back(const void* grad_output, const void* input, cons
     void* const behind = parts ? static_cast<unsigned char*>(workspace) + slices : nullptr;
     const DdsArgs g{grad_output, data, static_cast<const int*>(plan_input), nullptr, grad_input, (int)tokens, in_features, out_features, nnz};
     BackArgs a{grad_output, input, row_start_ends_a, cols_a, units, true, data_out, bias_out, (int)tokens, out_features, in_features, nnz, nullptr, nullptr};
+    if (int rc = back_checks(a, tokens, dtype)) return rc;   // (before the input gradient is launched)
     auto input_gradient = [&](bool parts_ready) {
         if (tokens == 0) return (int)PBS_OK;
         hipStream_t s = static_cast<hipStream_t>(stream);

@@ -46,6 +46,7 @@ def test_workspace_and_arguments(cuda):
     assert call(size=need - 1) == -5 and call(ws=null) == -5 and call(ws=ctypes.c_void_p(0x1008)) == -5
     assert call(dy=null) == -1 and call(x=null) == -1 and call(data=null) == -1 and call(dx=null) == -1 and call(units=null) == -1
     assert call(dx=ctypes.c_void_p(0x1004)) == -4 and call(x=ctypes.c_void_p(0x1004)) == -4
+    assert call(x=null, tokens=130) == -1 and call(x=ctypes.c_void_p(0x1004), tokens=130) == -4   # (the input gradient would come first)
     assert call(tokens=-1) == -2 and call(dtype=7) == -3
 
 
