@@ -259,6 +259,14 @@ struct RowFrag<bf16_t> {
     }
 };
 
+// sum += v; what the addition cuts off goes into the next one (Kahan's compensated sum).  Of an infinity, or a sum that has become one, nothing finite is cut
+// off: inf - inf would make the next sum NaN where a plain one stays infinite.
+static __device__ __forceinline__ void add_with_rest(float& sum, float& rest, float v) {
+    const float add = v - rest, now = sum + add, left = (now - sum) - add;
+    rest = left - left == 0.f ? left : 0.f;
+    sum = now;
+}
+
 template <typename T>
 struct SddRowCfg {
     static constexpr int PIECE = 1024 * Elem<T>::ESZ;
@@ -382,11 +390,7 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
             float of_chunk[2] = {0.f, 0.f};
             g.sum(of_chunk);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const float add = of_chunk[i] - bleft[i], now = bsum[i] + add;
-                bleft[i] = (now - bsum[i]) - add;
-                bsum[i] = now;
-            }
+            for (int i = 0; i < 2; ++i) add_with_rest(bsum[i], bleft[i], of_chunk[i]);
         } else {
             g.sum(bsum);
         }

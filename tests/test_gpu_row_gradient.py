@@ -77,6 +77,45 @@ def test_last_chunk_ends_with_the_matrix(cuda, dtype, out_f, in_f, counts, kerne
     assert (bias.grad.double() - dy.double().sum(0)).norm() <= limit * dy.double().sum(0).norm()
 
 
+@pytest.mark.parametrize("tokens, out_f, counts, kernel", [
+    (32, 384, [2], "sdd_row_kernel"), (64, 384, [2], "sdd_row_kernel"),   # one chunk a wave
+    (257, 384, ROWS, "sdd_row_kernel"), (500, 384, [0, 2], "sdd_row_kernel"), (2317, 384, [0, 1], "sdd_row_kernel + sdd_reduce_kernel"),
+    (2200, 1024, [40, 0, 38], "sdd_split_kernel"), (4103, 384, [60, 0, 63], "sdd_split_kernel + sdd_reduce_kernel"),
+])
+def test_bias_gradient_of_infinities(cuda, tokens, out_f, counts, kernel):
+    """An infinity, a sum that overflows and NaN come out as they do of a plain sum, whichever chunk of a wave's share they are in, in rows with and
+    without blocks."""
+    in_f = 2048
+    m = _layer(out_f, in_f, counts, torch.float32, cuda, 5)
+    nnz = m.cols_a.shape[0]
+    print(kernel, tokens, out_f, nnz, flush=True)
+    assert native.matmul_back_kernel_name(tokens, out_f, in_f, nnz, torch.float32) == kernel
+    inf, nan, big = float("inf"), float("nan"), 2.0 ** 127
+    torch.manual_seed(tokens)
+    dy = torch.randn(tokens, out_f, device=cuda)
+    x = torch.randn(tokens, in_f, device=cuda)
+    want = {0: inf, 1: -inf, 2: nan, 3: nan, 4: inf, 5: -inf}
+    for at in (0, tokens // 2, tokens - 1):   # the first chunk, one in between and the last
+        here, other = dy.clone(), (at + 128) % tokens   # (the next chunk of the same wave, if there is one)
+        for row in range(out_f // 32):
+            f = 32 * row
+            here[at, f], here[at, f + 1], here[at, f + 2] = inf, -inf, nan
+            here[at, f + 3], here[other, f + 3] = inf, -inf
+            here[:, f + 4:f + 6] = 0.0
+            here[at, f + 4], here[other, f + 4] = big, big
+            here[at, f + 5], here[other, f + 5] = -big, -big
+        if other == at:
+            here[at, 3::32], here[at, 4::32], here[at, 5::32] = nan, inf, -inf
+        data, bias = m.data.detach().clone().requires_grad_(), torch.zeros(out_f, device=cuda, requires_grad=True)
+        native.torch_path().linear(x, data, bias, m._buffers, m.schedule()).backward(here)
+        got = bias.grad.view(-1, 32)
+        for i, value in want.items():
+            assert torch.equal(got[:, i], torch.full_like(got[:, i], value)) or (value != value and bool(got[:, i].isnan().all())), (at, i, got[:, i].tolist())
+        rest = here.double().sum(0).view(-1, 32)[:, 6:]
+        # (a chunk's sums in three levels, the four waves and the slices: fewer than 16 roundings of 2^-24)
+        assert bool(((got[:, 6:].double() - rest).abs() <= 16 * 2.0 ** -24 * here.double().abs().sum(0).view(-1, 32)[:, 6:]).all())
+
+
 @pytest.mark.parametrize("dtype, out_f", [(torch.float32, 1 << 25), (torch.bfloat16, 1 << 26)])
 def test_chunks_of_four_gigabytes(cuda, dtype, out_f):
     """A chunk of 32 tokens that is too large to be addressed as one buffer."""
