@@ -87,7 +87,7 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
         for (int v = 0; v < 16; ++v) total[b][v] = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) part[0][v] = part[1][v] = 0.f;
-    float bsum = 0.f;
+    float bsum = 0.f, bleft = 0.f;
 
     int chunk = c_lo + wave;
     if (chunk < c_hi) {
@@ -120,7 +120,7 @@ static __device__ __forceinline__ void sdd_split_body(const SddRowArgs& a, const
         int xat = 0, gat = 0;   // slots of the pieces that have been read last
         int early = (XS - 1 + NB - 1) / NB;   // chunks: the pieces asked for above have fewer DMA instructions behind them than the later ones
         for (;; chunk += ROW_NW) {
-            if (sums) bsum += gr[0].sum() + gr[1].sum();
+            if (sums) add_with_rest(bsum, bleft, gr[0].sum() + gr[1].sum());
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const int xnext = xat + 1 == XS ? 0 : xat + 1, gnext = GS == 2 ? gat ^ 1 : 0;

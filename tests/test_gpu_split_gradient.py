@@ -83,3 +83,17 @@ def test_values_that_have_no_parts(cuda):
         distance = ((got - want).norm() / want.norm()).item()
         print(scale_x, scale_dy, distance, flush=True)
         assert distance <= 0.35 * 2.0 ** -24 * np.sqrt(32 + tokens / 128) + 2.0 ** -25, (scale_x, scale_dy)
+
+
+@pytest.mark.parametrize("tokens, counts", [(5797, [26, 27]), (4801, [28])])
+def test_bias_gradient_of_long_shares(cuda, tokens, counts):
+    """Up to 46 and 38 chunks of a wave one behind the other: what the additions cut off is carried along."""
+    m = _layer(cuda, 2048, 2048, counts)
+    print(tokens, _name(m, tokens), flush=True)
+    assert _name(m, tokens) == "sdd_split_kernel"   # one slice
+    torch.manual_seed(tokens)
+    x, dy = torch.randn(tokens, 2048, device=cuda), torch.randn(tokens, 2048, device=cuda)
+    got, want = _gradients(m, dy, x)[1].double(), dy.double().sum(0)
+    # four roundings of a chunk's sum of 16, one of the carried sum, one of two lanes, three of the waves; each at most 2^-24 of what it rounds, a third of that
+    # squared on average, in a random walk
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -24 * np.sqrt((4 + 1 + 1 + 3) / 3)
