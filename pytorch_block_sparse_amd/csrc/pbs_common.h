@@ -93,6 +93,14 @@ static __device__ __forceinline__ void dma16(unsigned lds_base_uniform, const un
                  : "memory");
 }
 
+// the same with an address per lane
+static __device__ __forceinline__ void dma16_lanes(unsigned lds_base_uniform, const unsigned char* at) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+                 :
+                 : "s"(lds_base_uniform), "v"(at)
+                 : "memory");
+}
+
 // 16 bytes per lane from `off` on in a buffer of `bytes` bytes (both below 2^31; base and bytes wave-uniform); zeros, and no memory
 // access, where off lies behind its end
 static __device__ __forceinline__ uint4 buffer16(const unsigned char* base_uniform, unsigned bytes, unsigned off) {

@@ -279,22 +279,35 @@ struct SddRowCfg {
 // The pieces of a matrix of M rows: D DMA instructions of ROWS rows each, zeros for rows behind the last one, so that a matrix's last chunk is one like
 // the others.  (Loaded by itself behind the loop, one piece after the other and in bf16 two bytes at a time, it cost a workgroup 1 to 6 us: bf16 768 -> 3072
 // density 0.5, 2317 tokens 32.7 -> 28.2, 140 tokens 9.3 -> 5.8; 768 -> 768, 1037 tokens 14.95 -> 9.35, fp32 14.9 -> 13.7; 448 -> 2080 density 0.62, 9336 tokens, in
-// sdd_split_kernel 104 -> 98.  Whole token counts the same to within 1 %.)  FAR: chunks of 4 GB and more, each instruction then has a buffer of its own.
+// sdd_split_kernel 104 -> 98.  Whole token counts the same to within 1 %.)
+// A chunk is one buffer, and offsets in it are 32-bit numbers.  FAR: chunks of 4 GB and more; lanes have addresses of their own, those behind the last row that of zeros.
+static __device__ const uint4 g_zeros = {0, 0, 0, 0};
 template <bool FAR, int D, int ROWS>
 struct RowSource {
     const unsigned char* base;
     size_t stride;
     int M;
-    unsigned voff[FAR ? 1 : D];
+    unsigned voff[D];
     __device__ __forceinline__ RowSource(const unsigned char* base, size_t stride, int M, int row, int place) : base(base), stride(stride), M(M) {
 #pragma unroll
-        for (int i = 0; i < (FAR ? 1 : D); ++i) voff[i] = (unsigned)(i * ROWS + row) * (unsigned)stride + place * 16;
+        for (int i = 0; i < D; ++i) voff[i] = (unsigned)(i * ROWS + row) * (unsigned)stride + place * 16;
     }
-    __device__ __forceinline__ void dma(unsigned lds, int chunk, unsigned column_bytes, int i) const {
-        const int t0 = chunk * ROW_TC + (FAR ? i * ROWS : 0), rows = FAR ? ROWS : ROW_TC;
-        const int left = M - t0 < rows ? M - t0 : rows;
-        dma16_bounded(lds, bounded_buffer(base + (size_t)t0 * stride + (FAR ? column_bytes : 0), FAR && left < 0 ? 0u : (unsigned)left * (unsigned)stride),
-                      voff[FAR ? 0 : i] + (FAR ? 0 : column_bytes));
+    __device__ __forceinline__ void dma(unsigned lds, int chunk, size_t column_bytes, int i) const {
+        const int t0 = chunk * ROW_TC, left = M - t0 < ROW_TC ? M - t0 : ROW_TC;
+        dma16_bounded(lds, bounded_buffer(base + (size_t)t0 * stride, (unsigned)left * (unsigned)stride), voff[i] + (unsigned)column_bytes);
+    }
+};
+template <int D, int ROWS>
+struct RowSource<true, D, ROWS> {
+    const unsigned char* base;
+    size_t stride;
+    int M;
+    __device__ __forceinline__ RowSource(const unsigned char* base, size_t stride, int M, int, int) : base(base), stride(stride), M(M) {}
+    __device__ __forceinline__ void dma(unsigned lds, int chunk, size_t column_bytes, int i) const {
+        constexpr int CPR = 64 / ROWS;
+        const int lane = lane_now();   // (addresses kept over the loop would be spilled)
+        const int t = chunk * ROW_TC + i * ROWS + lane / CPR;
+        dma16_lanes(lds, t < M ? base + (size_t)t * stride + column_bytes + lane % CPR * 16 : reinterpret_cast<const unsigned char*>(&g_zeros));
     }
 };
 
@@ -329,7 +342,7 @@ static __device__ __forceinline__ void sdd_row_body(const SddRowArgs& a, const i
     RowSource<FAR, D, RPI> from_g(G, gs, a.M, lane / CPR, lane % CPR), from_x(X, xs, a.M, lane / CPR, lane % CPR);
     auto dma_g = [&](int slot, int chunk, int i) __attribute__((always_inline)) { from_g.dma(lds + slot * PIECE + i * 1024, chunk, 0, i); };
     auto dma_x = [&](int slot, int chunk, int c, int i) __attribute__((always_inline)) {
-        from_x.dma(lds + (GS + slot) * PIECE + i * 1024, chunk, c * (32 * ESZ), i);
+        from_x.dma(lds + (GS + slot) * PIECE + i * 1024, chunk, (size_t)c * (32 * ESZ), i);
     };
 
     f32x4 acc[NBX][2][2];

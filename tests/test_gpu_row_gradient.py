@@ -116,10 +116,8 @@ def test_bias_gradient_of_infinities(cuda, tokens, out_f, counts, kernel):
         assert bool(((got[:, 6:].double() - rest).abs() <= 16 * 2.0 ** -24 * here.double().abs().sum(0).view(-1, 32)[:, 6:]).all())
 
 
-@pytest.mark.parametrize("dtype, out_f", [(torch.float32, 1 << 25), (torch.bfloat16, 1 << 26)])
-def test_chunks_of_four_gigabytes(cuda, dtype, out_f):
-    """A chunk of 32 tokens that is too large to be addressed as one buffer."""
-    rows, tokens = [0, 5, out_f // 64, out_f // 32 - 1], 45
+def _wide_rows(cuda, dtype, out_f, tokens):
+    rows = [0, 5, out_f // 64, out_f // 32 - 1]
     m = BlockSparseMatrix.zeros((out_f, 64), blocks=[(r, r % 2) for r in rows], device=cuda, dtype=dtype)
     dy = torch.zeros(tokens, out_f, dtype=dtype, device=cuda)
     torch.manual_seed(2)
@@ -131,6 +129,18 @@ def test_chunks_of_four_gigabytes(cuda, dtype, out_f):
     at = m.build_coo_block_index().tolist()
     want = torch.cat([x[:, 32 * c:32 * c + 32].double().t().contiguous() @ dy[:, 32 * r:32 * r + 32].double() for r, c in zip(*at)])
     assert (got - want).norm() <= (1e-6 if dtype == torch.float32 else 2.0 ** -8) * want.norm()
+
+
+@pytest.mark.parametrize("dtype, out_f", [(torch.float32, 1 << 25), (torch.bfloat16, 1 << 26)])
+def test_chunks_of_four_gigabytes(cuda, dtype, out_f):
+    """A chunk of 32 tokens that is too large to be addressed as one buffer."""
+    _wide_rows(cuda, dtype, out_f, 45)
+
+
+@pytest.mark.parametrize("dtype, out_f, tokens", [(torch.float32, 1 << 27, 33), (torch.bfloat16, 1 << 27, 45), (torch.bfloat16, 1 << 28, 33), (torch.float32, 1 << 28, 17)])
+def test_rows_of_half_a_gigabyte(cuda, dtype, out_f, tokens):
+    """The rows that one copy instruction reads, 8 (fp32) or 16, have 4 GB and more."""
+    _wide_rows(cuda, dtype, out_f, tokens)
 
 
 @pytest.mark.parametrize("tokens,out_f,in_f,counts", [
