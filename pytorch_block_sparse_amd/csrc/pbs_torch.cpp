@@ -174,9 +174,9 @@ struct Pattern {
     // a training step's plans in one launch, if there is none yet
     void train(int64_t tokens, int code, void* stream) {
         std::lock_guard<std::mutex> hold(lock);
+        derive_all(tokens, code, stream);
         trained_tokens = tokens;
         trained_code = code;
-        derive_all(tokens, code, stream);
     }
     void derive_all(int64_t tokens, int code, void* stream) {
         if (parts[0] || parts[1] || units.t.defined() || !row_ptr.t.is_cuda() || !cols.t.is_cuda() || !col_ptr.t.is_cuda() ||
@@ -672,10 +672,15 @@ PyObject* py_replace_blocks(PyObject*, PyObject* const* args, Py_ssize_t n) {
             code = before->trained_code;
         }
         if (tokens && before->out_features == 32 * X && before->in_features == 32 * Y) {
-            // (arrays of rejected moves hold anything: the kernels that read them clamp what they find)
-            after = pattern_of(made[2], made[1], made[4], made[3]);
-            std::lock_guard<std::mutex> hold(after->lock);
-            after->derive_all(tokens, code, stream);
+            // (arrays of rejected moves hold anything: the kernels that read them clamp what they find.  The moves need no plans: without room for these, the next
+            // product makes its own or says why not.  The status is waited for in any case, as the kernel that writes it is under way.)
+            try {
+                after = pattern_of(made[2], made[1], made[4], made[3]);
+                std::lock_guard<std::mutex> hold(after->lock);
+                after->derive_all(tokens, code, stream);
+            } catch (const std::exception&) {
+                after.reset();
+            }
         }
         status = read_status(word, stream);
     }

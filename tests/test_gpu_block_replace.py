@@ -116,3 +116,35 @@ def test_rejected_moves_of_a_trained_matrix(cuda):
         with pytest.raises(Exception, match="block_replacements"):
             layer.weight.block_replace(torch.tensor([[0, 0, 10 ** 6]], device=cuda))
         assert all(torch.equal(a, b) for a, b in zip(want, _step(layer, x, dy)))
+
+
+def test_moves_without_room_for_plans(cuda):
+    """The moves themselves need a few kilobytes: where the new pattern's plans find no memory, they succeed all the same, and refused ones say why."""
+    np.random.seed(7)
+    layer = BlockSparseLinear(16384, 16384, density=0.004, device=cuda)   # plans of 2 MB each
+    torch.manual_seed(7)
+    x, dy = torch.randn(40, 16384, device=cuda, requires_grad=True), torch.randn(40, 16384, device=cuda)
+    _step(layer, x, dy)
+    layer.weight.block_replace(_moves(layer.weight, 50, 0))
+    _step(layer, x, dy)
+    moves, bad = _moves(layer.weight, 50, 1), torch.tensor([[0, 0, 10 ** 6]], device=cuda)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total, filler = torch.cuda.get_device_properties(cuda).total_memory, []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while len(filler) < 1 << 16:
+                filler.append(torch.empty(3 << 19, dtype=torch.uint8, device=cuda))
+        with pytest.raises(Exception, match="block_replacements"):
+            layer.weight.block_replace(bad)
+        layer.weight.block_replace(moves)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            _step(layer, x, dy)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    filler.clear()
+    layer.weight.validate_indices()
+    fresh = copy.deepcopy(layer)
+    for a, b in zip(_step(layer, x, dy), _step(fresh, x, dy)):
+        assert torch.equal(a, b)
