@@ -148,3 +148,34 @@ def test_larger_fp32_products_of_short_lists(cuda, first, counts):
     # as in tests/test_gpu_split_kernel.py: four roundings per block of the fullest column, and that of the result
     limit = 0.35 * 2.0 ** -24 * (4 * max(counts)) ** 0.5 + 2.0 ** -25
     assert (got.double() - want).norm() <= limit * want.norm()
+
+
+def test_lists_of_anything(cuda):
+    """Every other column has all entries, in any order, many to a k-block: the first good one of each is found in about the time that the entries take to read."""
+    n, k, nnz = 512 * 32, 512 * 32, 100000
+    lib, rng = native.load(), np.random.RandomState(2)
+    ptr = np.array([0, nnz] * 256 + [0])
+    entries = np.stack([rng.randint(-3, 515, nnz), rng.randint(-5, nnz + 5, nnz)], 1)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    dptr, dent = (torch.from_numpy(v.astype(np.int32)).to(cuda) for v in (ptr, entries))
+    plan = torch.full((lib.pbs_blocksparse_matmul_plan_part_bytes(n, k),), 0x7f, dtype=torch.uint8, device=cuda)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    times = []
+    for _ in range(3):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        assert lib.pbs_blocksparse_matmul_plan_part(p(dptr), p(dent), n, k, nnz, 1, p(plan), plan.numel(), stream) == 0
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    print(times, flush=True)
+    first = {}
+    for x, b in entries:
+        if 0 <= x < 512 and 0 <= b < nnz:
+            first.setdefault(int(x), int(b))
+    want = np.array(sorted(first.items()))
+    records = plan.view(torch.int32).cpu().numpy()[:512 * 514 * 2].reshape(512, 514, 2)
+    assert [tuple(r[0]) for r in records] == [(c, len(want)) for c in range(0, 512, 2)] + [(c, 0) for c in range(1, 512, 2)]
+    for r in records[:256]:
+        assert np.array_equal(r[2:2 + len(want)], want)
+    assert min(times) < 5.0   # ms; 100000 entries of a wave are three times 1563 loads
