@@ -190,8 +190,8 @@ int pbs_blocksparse_matmul(const void* dense_a, const void* data, const void* pl
  *
  * Bits.  A token's fp32 result is the same, to the last bit, in all calls of a pattern and direction that take the same of these two ways, whatever other
  * tokens share the call; between the two it differs by rounding.  Which way a call takes follows from its sizes: with the workspace the bf16 cores' from
- * 512 tokens and 2^21 tokens x blocks on at densities of 0.2 and more, apart from token counts for which an estimate sees the fp32 instructions ahead by a tenth,
- * and from three quarters of those tokens x blocks on where it sees them behind by an eighth (pbs_blocksparse_matmul_parts_bytes() > 0 tells).  A caller who needs the same bits for requests batched in any way passes no workspace.  bf16
+ * 512 tokens and 2^21 tokens x blocks on at densities of 0.2 and more, apart from token counts for which an estimate sees the fp32 instructions ahead by a tenth
+ * (pbs_blocksparse_matmul_parts_bytes() > 0 tells).  A caller who needs the same bits for requests batched in any way passes no workspace.  bf16
  * results, and the gradient of the blocks in either dtype, may differ by rounding between calls of different numbers of tokens.
  */
 size_t pbs_blocksparse_matmul_workspace_bytes(int64_t tokens, int n, int k, int nnz, int transpose, int dtype);

@@ -489,7 +489,7 @@ static double split_us(long long M, int n, int k, int nnz) {
     return 6.61 + 0.00319 * nnz + split_tiles(M, groups).rounds * (0.101 * (k / 32) + 1.07 * nnz / (n / 32) * (0.669 + 0.331 * full) + 2.48);
 }
 // Which problems: a density of 0.2 and more, groups of 8 columns that are filled to three quarters, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and not
-// where the estimates see stream_kernel ahead by a tenth; from three quarters of those operations on, what the estimate has an eighth faster.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05:
+// where the estimates see stream_kernel ahead by a tenth.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05:
 // half as fast); with emptier groups waves have no column; with fewer tokens or products the launch that splits and the first panels weigh too much.
 // The tenth is for a result's bits: those of a token are the same, to the last bit, in all calls of a pattern that are served alike, and a line
 // at level estimates would part the calls of a 4096 -> 4096 layer of density 0.25 seven times between 512 and 2177 tokens.  Of the 821 products 802 are taken, 1.28
@@ -498,16 +498,15 @@ static double split_us(long long M, int n, int k, int nnz) {
 // Columns that are more uneven than that are not known here: 311 of 312 such products (Zipf rows) are taken, 1.10 times faster on average, but 80 of them more than
 // 2 % slower, down to 0.57 times as fast where a full column among short ones meets a single round of units (2186 tokens 3104 -> 1472, 1397 blocks
 // 59 -> 105 us).
-// Below 2^21 tokens x blocks: of 130 products between 1.5 and 2 2^20 about half are taken, 49 even ones 1.14 times as fast on average (256 -> 1184 density 0.57, 9738 tokens
-// 44 -> 33 us), 2 of them more than 2 % slower (0.91), 16 with Zipf rows 1.08 (0.81 to 1.40); at level estimates a sixth would be slower, and between 2^20 and 1.5 2^20
-// Zipf rows lose (0.95).
-constexpr double SPLIT_MARGIN = 0.91, SPLIT_SMALL_MARGIN = 1.12;
+// (Between 1.5 and 2 2^20 tokens x blocks, what the estimate has an eighth faster is 1.10 times as fast with even columns, 1 of 13 slower, and 0.99 with Zipf rows, 6 of 13
+// slower, down to 0.79: which of these a pattern is is not known here.)
+constexpr double SPLIT_MARGIN = 0.91;
 static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     const long long cols = n / 32, groups = split_groups(n);
-    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (3 << 19)) return false;
+    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
     // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
     if (k > (1 << 16) || (M + 31) / 32 * groups >= (1 << 28)) return false;
-    return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] { return (M * nnz < (1 << 21) ? SPLIT_SMALL_MARGIN : SPLIT_MARGIN) * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us; });
+    return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] { return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us; });
 }
 
 // `parts_ready`: the workspace holds the blocks in parts already

@@ -75,9 +75,9 @@ def test_values_that_have_no_parts(cuda):
 
 
 @pytest.mark.parametrize("tokens, k, n, nnz, parts", [
-    (9738, 256, 1184, 168, True), (7337, 960, 448, 246, True),   # between 1.5 and 2 2^20 tokens x blocks: by estimate
-    (1024, 3072, 768, 1600, False),
-    (6393, 960, 448, 246, False), (9361, 256, 1184, 168, False),   # the last count below 1.5 2^20
+    (8192, 1024, 768, 256, True), (8191, 1024, 768, 256, False),   # 2^21 tokens x blocks, and fewer
+    (9738, 256, 1184, 168, False), (7337, 960, 448, 246, False), (6317, 640, 2336, 303, False), (1024, 3072, 768, 1600, False),
+    (6393, 960, 448, 246, False), (9361, 256, 1184, 168, False),
 ])
 def test_smaller_products(cuda, tokens, k, n, nnz, parts):
     np.random.seed(tokens)
