@@ -763,13 +763,14 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
     // (rectangles count the bytes of a chunk in 31 bits)
     const bool rectangles = dtype == PBS_DTYPE_BF16 && N < (1 << 25) && K < (1 << 25);
     // bf16 operands beyond the size of the L2s (52 MB): the rectangles read every panel once per 16 or 8 rows of blocks, the units once per block, but only what
-    // they need, so below a density of 0.1 (rectangles with less than 26 of 256 places taken) the units are given what their estimate has at least a tenth faster
-    // (4 of 9 such problems of 52 to 220 MB, in which they are 0.95, with very uneven rows, and 1.39 to 1.56 times as fast: 1152 -> 3360 density 0.086, 5802 tokens 38 -> 24 us).  Above it they are 0.55 to 1.5 times
-    // as fast (4096 -> 4096 density 0.25, 16384 tokens 250 us and 198), where the estimates are not good enough to choose; and where most rows
-    // are empty, units cost what no estimate counts.  What the workspace does not allow the rectangles is refused and not served another way.
+    // they need, so below a density of 0.1 (rectangles with less than 26 of 256 places taken) and 90 MB the units are given what their estimate has at least a tenth faster
+    // (of such problems with 52 to 88 MB they take 19 that were the rectangles', 1.18 times as fast on average, 2 of them slower (0.91 and 0.96): 8690 tokens 1184 -> 1888 density 0.05
+    // 32 -> 24 us.  Of 8 with 97 to 130 MB 3 were slower, 0.96 on average: 12921 tokens 1024 -> 2720 density 0.054 40 -> 55, 10498 tokens 2592 -> 3616 density 0.06 84 -> 109.)
+    // Above that density they are 0.55 to 1.5 times as fast (4096 -> 4096 density 0.25, 16384 tokens 250 us and 198), where the estimates are not good enough to choose; and where
+    // most rows are empty, units cost what no estimate counts.  What the workspace does not allow the rectangles is refused and not served another way.
     const bool large = rectangles && bytes > 52e6;
     const bool fits = workspace_limit >= ROW_WORKSPACE_BYTES || plan_rectangles(M, N, K, 16).nsplit * (size_t)nnz * 4096 <= workspace_limit;
-    if (large && (10ll * nnz >= (long long)(N / 32) * (K / 32) || nnz < N / 32 || !fits)) return {0, 1, ROW_NB, false};
+    if (large && (bytes > 90e6 || 10ll * nnz >= (long long)(N / 32) * (K / 32) || nnz < N / 32 || !fits)) return {0, 1, ROW_NB, false};
     const long long chunks = (M + ROW_TC - 1) / ROW_TC;
     const double at_least = dtype == PBS_DTYPE_F32 ? std::floor(bytes / 64e6) : 1.0;
     RowChoice best{1, 1, ROW_NB, false};

@@ -187,3 +187,12 @@ def test_reference_side_binding_matches_the_header(lib):
     assert b.lib.pbs_abi_version() == lib.pbs_abi_version()
     with pytest.raises(RuntimeError, match="pbs:"):
         b._check(b.lib.pbs_blocksparse_matmul(None, None, None, None, None, 4, 64, 64, 1, 1, 0, None), "matmul")
+
+
+@pytest.mark.parametrize("tokens, in_f, out_f, nnz, kernel", [
+    (8690, 1184, 1888, 114, b"sdd_row_kernel"), (15227, 640, 1888, 98, b"sdd_row_kernel"),        # 53 and 77 MB of operands
+    (12921, 1024, 2720, 146, b"sdd_bf16_kernel"), (10498, 2592, 3616, 572, b"sdd_bf16_kernel"),   # 97 and 130 MB
+    (8424, 2624, 3648, 650, b"sdd_bf16_kernel"), (16384, 4096, 4096, 4096, b"sdd_bf16_kernel"),
+])
+def test_large_sparse_bf16_gradients_are_rectangles_from_90_mb_on(lib, tokens, in_f, out_f, nnz, kernel):
+    assert lib.pbs_blocksparse_matmul_back_kernel_name(tokens, out_f, in_f, nnz, 1).startswith(kernel)
