@@ -12,15 +12,22 @@ pytestmark = pytest.mark.gpu
 F32, BF16 = torch.float32, torch.bfloat16
 
 
-@pytest.mark.parametrize("dtype, tokens, in_f, out_f, nnz, bias", [
-    # slices, and blocks in parts
-    (F32, 4096, 768, 3072, 1152, True), (F32, 3072, 3072, 768, 1151, True), (F32, 4097, 1024, 1024, 1021, False), (F32, 16384, 2048, 2048, 4095, True),
-    (F32, 4099, 768, 768, 286, True),   # slices alone
-    (F32, 130, 768, 3072, 1152, True),  # neither
-    (F32, 1, 32, 32, 1, True), (F32, 64, 416, 160, 0, True), (F32, 0, 768, 3072, 700, True),
-    (BF16, 2317, 768, 3072, 1152, True), (BF16, 8192, 2048, 2048, 2000, True),
+def _shared(tokens, in_f, out_f, nnz, dtype):
+    """(slices that a launch adds, blocks in parts): with both, one launch does both."""
+    lib, code = native.load(), native.DTYPE_CODES[dtype]
+    return (lib.pbs_blocksparse_matmul_back_bias_workspace_bytes(tokens, out_f, in_f, nnz, code) > 0,
+            lib.pbs_blocksparse_matmul_parts_bytes(tokens, in_f, out_f, nnz, 0, code) > 0)
+
+
+@pytest.mark.parametrize("dtype, tokens, in_f, out_f, nnz, bias, slices, parts", [
+    (F32, 4096, 768, 3072, 1152, True, True, True), (F32, 3072, 3072, 768, 1151, True, True, True), (F32, 4097, 1024, 1024, 1021, False, True, True),
+    (F32, 16384, 2048, 2048, 4095, True, True, True),
+    (F32, 5797, 2048, 2048, 1696, True, False, True), (F32, 4099, 768, 768, 286, True, True, False), (F32, 130, 768, 3072, 1152, True, False, False),
+    (F32, 1, 32, 32, 1, True, False, False), (F32, 64, 416, 160, 0, True, False, False), (F32, 0, 768, 3072, 700, True, False, False),
+    (BF16, 2317, 768, 3072, 1152, True, False, False), (BF16, 8192, 2048, 2048, 2000, True, True, False),
 ])
-def test_together_like_apart(cuda, dtype, tokens, in_f, out_f, nnz, bias):
+def test_together_like_apart(cuda, dtype, tokens, in_f, out_f, nnz, bias, slices, parts):
+    assert _shared(tokens, in_f, out_f, nnz, dtype) == (slices, parts)
     np.random.seed(nnz)
     layer = BlockSparseLinear(in_f, out_f, bias=bias, density=0.5, device=cuda, dtype=dtype)
     layer.weight = BlockSparseMatrix.randn((out_f, in_f), nnz, device=cuda, dtype=dtype)
@@ -54,6 +61,7 @@ def test_graph_replays(cuda):
     """A captured step: every replay, with eager steps between them, gives what the eager step gives."""
     np.random.seed(5)
     layer = BlockSparseLinear(3072, 768, density=0.5, device=cuda, dtype=F32)
+    assert _shared(4096, 3072, 768, layer.weight.cols_a.shape[0], F32) == (True, True)
     x = torch.randn((4096, 3072), device=cuda).requires_grad_(True)
     dy = torch.randn((4096, 768), device=cuda)
     weights = [layer.weight.get_differentiable_data(), layer.bias]

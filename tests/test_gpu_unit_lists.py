@@ -52,7 +52,7 @@ def test_every_list_holds_every_block_once(cuda, out_f, in_f, nnz):
     (F32, 5, 1, 33, 3072, 416, 842), (F32, 6, 1, 33, 3072, 768, 1050),
     (F32, 1, 2, 1500, 416, 160, 3), (F32, 2, 2, 2317, 3072, 160, 25), (F32, 3, 2, 3000, 416, 768, 76), (F32, 4, 2, 2317, 416, 416, 62),
     (F32, 5, 2, 3000, 2048, 416, 113), (F32, 6, 2, 2317, 416, 992, 256),
-    # sdd_split_kernel
+    # sdd_split_kernel: 2^20 tokens x blocks and more
     (F32, 2, 1, 1500, 2912, 320, 906), (F32, 2, 2, 4097, 3072, 128, 262), (F32, 3, 1, 1500, 800, 928, 707), (F32, 3, 2, 3000, 160, 2496, 353),
     (F32, 4, 1, 700, 1248, 1248, 1503), (F32, 4, 2, 1500, 2112, 352, 723),
     (BF16, 1, 1, 33, 416, 160, 3), (BF16, 2, 1, 33, 3072, 160, 197), (BF16, 3, 1, 33, 3072, 768, 464), (BF16, 4, 1, 33, 3072, 416, 673),
@@ -63,6 +63,8 @@ def test_every_list_holds_every_block_once(cuda, out_f, in_f, nnz):
 def test_kernels_with_every_list(cuda, dtype, per_unit, slices, tokens, out_f, in_f, nnz):
     """`slices` 2: several."""
     lib, code = native.load(), native.DTYPE_CODES[dtype]
+    kernel = "sdd_split_kernel" if dtype == F32 and tokens * nnz >= 1 << 20 else "sdd_row_kernel"
+    assert native.matmul_back_kernel_name(tokens, out_f, in_f, nnz, dtype) == (kernel if slices == 1 else kernel + " + sdd_reduce_kernel")
     size = lib.pbs_blocksparse_matmul_back_workspace_bytes(tokens, out_f, in_f, nnz, code)
     partial = size - 64 - (nnz // per_unit + out_f // 32) * 64   # what the list of these units leaves
     assert partial % (nnz * 4096) == 0 and (partial > 0) == (slices > 1)
