@@ -132,8 +132,8 @@ static __device__ __forceinline__ void dma4(unsigned lds_base_uniform, const uns
                  : "s"(lds_base_uniform), "v"(voff), "s"(base_uniform)
                  : "memory");
 }
-// wait until at most n (wave-uniform; a constant: the branches of a variable one cost a third of a kernel's time) of this wave's DMA loads are
-// outstanding.  Loads retire in order, so a smaller n than necessary is only slower, never wrong.
+// wait until at most n (wave-uniform) of this wave's DMA loads are outstanding.  Loads retire in order, so a smaller n than necessary is only slower, never wrong.
+// n is a constant, or one of two (one branch): the branches over all counts, with one that a loop works out, cost a third of a kernel's time.
 static __device__ __forceinline__ void wait_dma(int n) {
 #define PBS_W(N) case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
     switch (n) {
