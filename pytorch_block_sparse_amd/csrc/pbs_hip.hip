@@ -670,7 +670,8 @@ static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
 // the rate of a wave alone or of a chip that is full in rounds of 256 workgroups.  Fitted to problems of 256 .. 4096 features, 64 .. 16384 tokens, densities
 // 0.05 .. 0.75 at six sizes of units and eight numbers of slices (fp32: 80 below 2^22 tokens x blocks, within 9 %; bf16: 80 whose operands have less than 52 MB,
 // within 7 %, and 70 with 40 to 260 MB, within 10 %).  The choices it makes are 3 and 1.5 % slower than the best on average, and 1.28 and 1.14 times as fast as units of
-// four in the best number of slices that an estimate of those alone made; 4 fp32 ones of the 160 are slower by more than 2 %, one by 13 %.
+// four in the best number of slices that an estimate of those alone made; 4 fp32 ones of the 160 are slower by more than 2 %, one by 13 %.  Drawn anew, with the
+// split kernel and the rectangles among the choices: 864 fp32 problems 1.20 times as fast (23 slower by more than 5 %, the worst 0.87), 621 bf16 ones 1.21 (11, 0.79).
 // (The number of units follows from the average row, so what looks like a full chip may be one workgroup more than that: for fp32, whose rounds are long, the mean
 // of the estimated number and of 4 % more.  The reduction is a launch and an allocation more for the host: 2 (bf16 0.75) us more than the fit has for it.)
 // fp32 on the bf16 matrix cores (sdd_split_kernel) where its estimate is the smaller one, from 2^22 tokens x blocks in units of four (2048 -> 2048 density 0.25, 4096 tokens

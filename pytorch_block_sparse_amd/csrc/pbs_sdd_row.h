@@ -44,7 +44,8 @@ constexpr int ROW_PIECES = 5;   // LDS of a wave, in pieces of 32 tokens x 32 fe
 // ints.  A row of n blocks has ceil(n / P) units of equal size (+- 1), an empty row one without blocks (for the bias
 // gradient).  Order: (quarter of the row's units, row, unit): units that run at the same time then read neighbouring columns of
 // X from a common L2.  The table starts with the numbers of units of the lists P = 1 .. ROW_SIZES, padded to 16 ints; then the lists, each in
-// room for unit_bound units.
+// room for unit_bound units: some 160 bytes per block of the pattern, where one list of four would take 16.  Derived with the lists of both directions in one
+// launch, six lists take 1.3 to 1.8 us more than one (768 -> 3072 density 0.5 6.2 -> 7.6 us, 4096 -> 4096 density 0.25 6.5 -> 8.3).
 //
 // Why several lists: one workgroup per CU takes as long as its unit, one more than there are CUs takes twice as long, and small patterns of large
 // units leave most of the chip idle or need several slices of the tokens and their reduction.  The best list and number of slices of 80 problems each are,

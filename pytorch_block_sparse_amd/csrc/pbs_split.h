@@ -39,7 +39,7 @@
 // Workgroups are persistent, one per CU: units (token tile, group of columns) are dealt so that an XCD's workgroups share panels
 // and blocks in its L2.  Columns are ranked by their number of blocks in the list plan (pbs_stream.h) and dealt to the groups and SIMDs in turn.
 // A wave goes through its column by k-block whatever the tile, so a token's result has the same bits in any call that this kernel serves.
-// Measured and not kept: blocks two items ahead, or touched three items ahead for the L2 (registers: 7 % and more slower), wave priorities (2 to 6 %
+// Measured and not kept: blocks of whole tiles two items ahead (waves with 32 tokens have the registers, below), or touched three items ahead for the L2 (7 % and more slower), wave priorities (2 to 6 %
 // slower), another order of the six products (nothing), rings of 8 slots (3 % slower); columns of equal length to a group (a group waits for its longest
 // column, but its units then differ: even patterns 3 % slower, uneven ones 0.74 to 1.16 times as fast); fewer columns in halves where their groups take
 // another round of units (up to 1.38 times faster there, but short columns pay for the choice: 1 % slower on average, uneven patterns too).
