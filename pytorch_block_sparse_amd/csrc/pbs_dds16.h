@@ -136,6 +136,7 @@ struct D16Args {
     int M, N, K, nnz;
     int m_tiles, n_groups, group_ints;
     int wg_per_group;      // workgroups that share the token tiles of one column group
+    int stream_step;       // of their numbering (stream_and_group)
 };
 
 template <int TM_, int RS, int RB, int NP>
@@ -189,10 +190,8 @@ __global__ __launch_bounds__((8 + NP) * 64) void dds16_kernel(D16Args g) {
     // Workgroup -> (column group, first token tile).  Workgroups are handed to the 8 XCDs round-robin;
     // the workgroups of one XCD cover all column groups of the same few token tiles, so a panel is
     // fetched into that XCD's L2 once and read there by every group.
-    const int wg = blockIdx.x;
-    const int ng = (wg >> 3) % g.n_groups;
-    const int p = (wg & 7) + 8 * ((wg >> 3) / g.n_groups);
-    if (p >= g.wg_per_group) return;
+    int ng, p;
+    if (!stream_and_group(blockIdx.x, g.wg_per_group, g.stream_step, g.n_groups, 1, p, ng)) return;
     const int ntiles = (g.m_tiles - p + g.wg_per_group - 1) / g.wg_per_group;   // token tiles p, p + P, ...
     const int nb0 = ng * D16_NB;
 

@@ -277,6 +277,7 @@ struct DdscArgs {
     int M, N, K, nnz;
     int m_tiles, n_groups, group_ints;
     int wg_per_group;      // workgroups that share the token tiles of one column group
+    int stream_step;       // of their numbering (stream_and_group)
 };
 
 template <int RS>
@@ -327,21 +328,14 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     // Workgroup -> (column group, first token tile).  The workgroups of one XCD (blockIdx % 8) cover half of the
-    // column groups and every fourth token stream (with an odd number of groups: all groups, every eighth stream),
+    // column groups (with an odd number of groups: all groups) and a quarter (an eighth) of the token streams,
     // so a panel is fetched into two L2s and the blocks an XCD keeps re-reading (once per token tile) are 4 MB
     // at 4096 x 4096, which its L2 holds.  All groups per XCD (a panel in one L2, 8 MB of blocks) is 1.2 % slower
     // at both densities, a quarter of the groups per XCD 6 % slower at density 0.25.
-    const int wg = blockIdx.x;
+    // us, whole streams to an XCD -> here (16384 tokens if no other number): 3584 -> 3584 density 0.25 230 -> 175, 9000 tokens 158 -> 110; 3072 -> 1536 input gradient
+    // 165 -> 110; 2304 -> 2752, 13000 tokens 127 -> 81; 2560 -> 2560 124 -> 109; layers of 512, 1024, 2048 and 4096 features as before.
     int ng, p;
-    if ((g.n_groups & 1) == 0) {
-        const int x = wg & 7, r = wg >> 3, gs = g.n_groups >> 1;
-        ng = (x & 1) * gs + (r % gs);
-        p = (x >> 1) + 4 * (r / gs);
-    } else {
-        ng = (wg >> 3) % g.n_groups;
-        p = (wg & 7) + 8 * ((wg >> 3) / g.n_groups);
-    }
-    if (p >= g.wg_per_group) return;
+    if (!stream_and_group(blockIdx.x, g.wg_per_group, g.stream_step, g.n_groups, g.n_groups & 1 ? 1 : 2, p, ng)) return;
     const int ntiles = (g.m_tiles - p + g.wg_per_group - 1) / g.wg_per_group;   // token tiles p, p + P, ...
 
     const int KB = g.K / 32, KP = KB / 2;

@@ -177,11 +177,10 @@ static int launch_dds16(const DdsArgs& g, hipStream_t stream) {
     if (P < 1) P = 1;
     if (P > a.m_tiles) P = a.m_tiles;
     a.wg_per_group = P;
+    a.stream_step = stream_step(P, a.m_tiles);
     const size_t lds = (size_t)C::WORK_BYTES + (size_t)a.group_ints * sizeof(int);
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    const long long grid = 8ll * a.n_groups * ((P + 7) / 8);
-    if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    return launch(kernel, dim3((unsigned)grid), dim3(C::NT), lds, stream, a);
+    return launch(kernel, dim3(stream_grid_blocks(P, a.n_groups, 1)), dim3(C::NT), lds, stream, a);
 }
 
 // ---- bf16 kernel with one block column per wave ----
@@ -253,10 +252,9 @@ static int launch_ddsc(const DdsArgs& g, const void* data_nk, hipStream_t stream
     a.group_ints = (int)ddsc_plan_group_ints(g.K / 32);
     a.seq = a.plan + (size_t)a.n_groups * a.group_ints;
     a.wg_per_group = c.wg_per_group;
+    a.stream_step = stream_step(c.wg_per_group, c.m_tiles);
     if (int rc = raise_lds_limit(kernel, 160 * 1024, done)) return rc;
-    const long long grid = 8ll * a.n_groups * ((c.wg_per_group + 7) / 8);
-    if (grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    return launch(kernel, dim3((unsigned)grid), dim3(C::NT), C::LDS_BYTES, stream, a);
+    return launch(kernel, dim3(stream_grid_blocks(c.wg_per_group, c.n_groups, c.n_groups & 1 ? 1 : 2)), dim3(C::NT), C::LDS_BYTES, stream, a);
 }
 
 // ---- one block column per workgroup ----
