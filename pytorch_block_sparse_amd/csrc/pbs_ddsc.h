@@ -68,7 +68,7 @@
 //   [64 + s]                          k-pair index of step s
 //   [64 + KP + 2 (c KB + i)]          item i of column c: step | (k & 1) << 9 | (1 << 10 if it is the column's last)
 //   [64 + KP + 2 (c KB + i) + 1]      byte offset in the data of the block of the column's item i + DC_L (cyclically)
-//   (KP = K / 64, KB = K / 32)
+//   (KB = K / 32, KP = KB / 2 rounded up: of an odd number of k-blocks the last one is a pair by itself, whose second half is never an item)
 #pragma once
 #include <type_traits>
 
@@ -90,7 +90,7 @@ constexpr int DC_SEQ_INTS = 16384;      // the table 0, 1, 2, ...: a workgroup's
 #ifndef DC_SLEEP
 #define DC_SLEEP 8
 #endif
-static inline size_t ddsc_plan_group_ints(int KB) { return (size_t)DC_HDR + (KB / 2) + (size_t)DC_NB * 2 * KB; }
+static inline size_t ddsc_plan_group_ints(int KB) { return (size_t)DC_HDR + (KB + 1) / 2 + (size_t)DC_NB * 2 * KB; }
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void ddsc_plan_kernel(const int32_t* __restric
     __shared__ int s_lo[DC_NB], s_hi[DC_NB];
     __shared__ int s_part[256];
     const int tid = threadIdx.x;
-    const int KP = KB / 2;
+    const int KP = (KB + 1) / 2;
     int* out = plan + (size_t)blockIdx.x * group_ints;
     if (tid < DC_NB) {
         const int c = cols[blockIdx.x * DC_NB + tid];
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64) void ddsc_plan_ahead_kernel(int KB, int* plan, 
     const int tid = threadIdx.x;
     if (tid >= DC_NB) return;
     int* out = plan + (size_t)blockIdx.x * group_ints;
-    const int KP = KB / 2;
+    const int KP = (KB + 1) / 2;
     const int n = out[1 + tid];
     if (n <= 0) return;
     int* items = out + DC_HDR + KP + (size_t)tid * 2 * KB;
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     if (!stream_and_group(blockIdx.x, g.wg_per_group, g.stream_step, g.n_groups, g.n_groups & 1 ? 1 : 2, p, ng)) return;
     const int ntiles = (g.m_tiles - p + g.wg_per_group - 1) / g.wg_per_group;   // token tiles p, p + P, ...
 
-    const int KB = g.K / 32, KP = KB / 2;
+    const int KB = g.K / 32, KP = (KB + 1) / 2;
     const int* gplan = g.plan + (size_t)ng * g.group_ints;
     // the header, one int per lane
     const int v_hdr = gplan[lane];
@@ -411,8 +411,9 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
         int lc = lane;
         asm volatile("" : "+v"(lc));
         const unsigned voff_row = (unsigned)(lc >> 3) * a_row_bytes;
-        const unsigned voff_even = voff_row + (unsigned)(((lc & 7) ^ (lc >> 4)) * 16);
-        const unsigned voff_odd = voff_row + (unsigned)(((lc & 7) ^ (lc >> 4) ^ 4) * 16);
+        const int there = 2 * pair + 1 < KB ? 7 : 3;   // (a last pair of one k-block has that in both halves: nothing behind a row is read)
+        const unsigned voff_even = voff_row + (unsigned)((((lc & 7) ^ (lc >> 4)) & there) * 16);
+        const unsigned voff_odd = voff_row + (unsigned)((((lc & 7) ^ (lc >> 4) ^ 4) & there) * 16);
 #pragma unroll 1
         for (int i = 0; i < C::BM / 8; i += 2) {
             if (8 * i + 15 <= a_last_row) {
@@ -427,7 +428,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
                 for (int ii = 0; ii < 2; ++ii) {
                     const int row = 8 * (i + ii) + (l >> 3);
                     const int r = row < a_last_row ? row : a_last_row;   // row of the tile, never negative
-                    const unsigned voff = (unsigned)r * a_row_bytes + (unsigned)(((l & 7) ^ ((row >> 1) & 7)) * 16);
+                    const unsigned voff = (unsigned)r * a_row_bytes + (unsigned)((((l & 7) ^ ((row >> 1) & 7)) & there) * 16);
                     dma16(stage + (i + ii) * 1024, src, voff);
                 }
             }

@@ -111,7 +111,9 @@ static inline int column_groups(int n) { return (n / 32 + DC_NB - 1) / DC_NB; }
 static inline size_t column_table_bytes(int n) { return ((size_t)column_groups(n) * DC_NB * sizeof(int) + 63) / 64 * 64; }
 static inline size_t column_plan_bytes(int n, int k) {
     // k-pairs, and the lists of a group of 16 columns must fit the kernel's LDS area (16 * k / 32 items)
-    if ((k % 64) || DC_NB * (k / 32) > DC_ITEMS_LDS) return 0;
+    // (an odd number of them where no panel kernel holds the whole contraction, and not next to the largest k: the size of the plan of 4064 features stays as it was)
+    if (k % 64 && (k <= PANEL_MAX_K || DC_NB * (k / 32 + 1) >= DC_ITEMS_LDS)) return 0;
+    if (DC_NB * (k / 32) > DC_ITEMS_LDS) return 0;
     return column_table_bytes(n) + ((size_t)column_groups(n) * ddsc_plan_group_ints(k / 32) + DC_SEQ_INTS) * sizeof(int);
 }
 static inline size_t part_plan_bytes(int n, int k) { return column_plan_offset(n, k) + column_plan_bytes(n, k); }
@@ -214,12 +216,15 @@ static inline ColumnLaunch column_launch(long long M, int n) {
 // faster one for sparse patterns (4096 x 4096: 6 to 30 % at 1 to 24 blocks per column; 2048 x 2048: level at 2 to 4
 // blocks per column, 5 to 13 % from 8), while results of 512 to 1024 columns stay 10 to 30 % faster in the other
 // kernels until their columns hold 32 blocks.
-static bool column_kernel_fits(long long M, int n, int k, int nnz, int wish) {
+static bool column_kernel_runs(long long M, int n, int k, int nnz) {
     if (!column_plan_bytes(n, k) || nnz < 1 || nnz > DC_MAX_BLOCKS || M < 1) return false;
     const ColumnLaunch c = column_launch(M, n);
     const long long tiles_per_wg = (c.m_tiles + c.wg_per_group - 1) / c.wg_per_group;
-    if (tiles_per_wg * (k / 64) >= DC_SEQ_INTS) return false;   // a workgroup's steps are numbered through the table
-    if (wish >= 0) return wish == 1;
+    return tiles_per_wg * ((k + 32) / 64) < DC_SEQ_INTS;   // (a workgroup's steps are numbered through the table)
+}
+static bool column_kernel_fits(long long M, int n, int k, int nnz) {
+    if (k % 64 || !column_kernel_runs(M, n, k, nnz)) return false;
+    const ColumnLaunch c = column_launch(M, n);
     if ((long long)c.m_tiles * c.n_groups < 256) return false;
     const double per_column = (double)nnz / (n / 32);
     if (per_column >= DDSC_MIN_BLOCKS_PER_COLUMN) return true;
@@ -568,6 +573,14 @@ static double column_us(long long M, int n, int k, int nnz, bool copy) {
     const ColumnLaunch c = column_launch(M, n);
     return (double)((c.m_tiles + c.wg_per_group - 1) / c.wg_per_group) * (0.262 * (k / 64) + 0.429 * nnz / (n / 32) + 12.2) + (copy ? 0.0031 * nnz : 0.0);
 }
+// The column kernel's time outside column_kernel_fits, where its workgroups may be few and its k-blocks odd in number: 274 products (448 to 4096 features, 1200 to 16384
+// tokens, densities 0.05 to 0.75, both directions) within 6 % on average.
+static double column_anywhere_us(long long M, int n, int k, int nnz, bool copy) {
+    const ColumnLaunch c = column_launch(M, n);
+    const double tiles = (double)c.m_tiles / c.wg_per_group, rounds = 0.72 * std::ceil(tiles) + 0.28 * tiles, full = c.n_groups * c.wg_per_group / 256.0;
+    return 10.4 + rounds * ((k + 32) / 64 * (0.214 + 0.0492 * full) + (double)nnz / (n / 32) * (0.341 + 0.318 * full)) + 1e-6 * 0.131 * M * (n + k) +
+           (copy ? 4.2 + 0.00054 * nnz : 0.0);
+}
 // The column kernel where column_kernel_fits: from 8192 tokens against the stream and the wide kernel without further question
 // (it is the faster one in nearly all of that range and within a few us in the rest), otherwise the smallest estimate.
 // The panel kernel against it: its estimate is up to 25 % short where a wave takes many full columns (the matrix cores, and
@@ -582,20 +595,26 @@ constexpr PanelChoice NO_PANEL{0, 0.0, 0, 0};
 static ProductChoice choose_product_anew(long long M, int n, int k, int nnz, int transpose, bool with_copy, int wish) {
     constexpr int esz = 2;
     const bool wide = wide_kernel_fits(M, n, k);
-    const bool column = (!transpose || with_copy) && column_kernel_fits(M, n, k, nnz, wish);
-    if (wish == 1 && column) return {PART_COLUMN, NO_PANEL};
+    const bool runs = (!transpose || with_copy) && wish != 0 && column_kernel_runs(M, n, k, nnz), column = runs && column_kernel_fits(M, n, k, nnz);
+    if (wish == 1 && runs) return {PART_COLUMN, NO_PANEL};
     if (wish == 0 && wide) return {PART_WIDE, NO_PANEL};
     const PanelChoice panel = choose_panel(M, n, k, nnz);
     const double tc = column ? column_us(M, n, k, nnz, transpose != 0) : 1e300;
-    if (column && M >= 8192) {
-        const bool panel_first = panel.splits && !panel.ways && (1.0 + 0.03 * panel.turns) * panel.us < 4.0 + 0.88 * tc;
-        return panel_first ? ProductChoice{PART_LIST, panel} : ProductChoice{PART_COLUMN, NO_PANEL};
-    }
+    const bool panel_first = panel.splits && !panel.ways && (1.0 + 0.03 * panel.turns) * panel.us < 4.0 + 0.88 * tc;
+    if (column && M >= 8192 && !panel_first) return {PART_COLUMN, NO_PANEL};
     // (where the estimates are within 6 % of each other panel_kernel was up to 5 % the slower one as often as the faster: 70 drawn
     // problems, of which it takes 20 and is 1.02 to 1.8 times faster in them; panel_chunk_kernel's is up to 15 % short)
     const double tp = panel.splits ? (panel.ways ? 1.1 : 1.06) * panel.us : 1e300;
     const double ts = choose_stream(esz, M, n, k, nnz).us;
     const double tw = wide ? wide_us(M, n, k, nnz) : 1e300;
+    // Elsewhere, from 2048 tokens and 1024 features on, where its estimate is a fourteenth below all others: of the 274 products 24 more, 1.22 times as fast on average, one
+    // 5 % slower (13394 tokens 2720 -> 1728 density 0.32 118 -> 69 us, 5332 tokens 3616 -> 1888 density 0.32 77 -> 49, 3983 tokens 3648 -> 1568 density 0.33 35 -> 29).
+    // At level estimates five would be slower, down to 0.93.
+    if (runs && M >= 2048 && k >= 1024) {
+        const double least = tp < ts ? (tp < tw ? tp : tw) : (ts < tw ? ts : tw);
+        if (column_anywhere_us(M, n, k, nnz, transpose != 0) < 0.93 * least) return {PART_COLUMN, NO_PANEL};
+    }
+    if (column && M >= 8192) return {PART_LIST, panel};
     if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel};
     if (tc < ts && tc < tw) return {PART_COLUMN, NO_PANEL};
     return {tw < ts ? PART_WIDE : PART_LIST, NO_PANEL};

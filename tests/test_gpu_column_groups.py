@@ -37,3 +37,25 @@ def test_every_tile_of_every_group(cuda, monkeypatch, kernel, out_f, in_f, token
     w = O.to_dense(to64(m.data), m.build_coo_block_index().cpu().numpy(), (out_f, in_f))
     print(kernel, out_f, in_f, tokens, flush=True)
     assert_close(m.reverse_matmul(x.to(cuda), transpose=True), to64(x) @ w.T, BF16, "forward")
+
+
+@pytest.mark.parametrize("out_f, in_f, tokens, nnz", [
+    (1056, 1120, 1, 400),
+    (1056, 1120, 300, 35 * 33),      # every block
+    (1120, 1056, 128 * 129 + 77, 60),
+    (2080, 4000, 128 * 70, 2500),    # lists of more than 64 items
+])
+def test_odd_numbers_of_k_blocks(cuda, monkeypatch, out_f, in_f, tokens, nnz):
+    """The last pair of k-blocks is one k-block: its second half is never multiplied, whatever lies behind the row (here NaN: the next row's start)."""
+    monkeypatch.setenv("PBS_COLUMN_KERNEL", "1")
+    np.random.seed(nnz)
+    torch.manual_seed(nnz)
+    m = BlockSparseMatrix.randn((out_f, in_f), nnz, device="cpu", dtype=BF16).to(cuda)
+    w = O.to_dense(to64(m.data), m.build_coo_block_index().cpu().numpy(), (out_f, in_f))
+    for transpose, n, k, wt in ((True, out_f, in_f, w.T), (False, in_f, out_f, w)):
+        assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16, True) == "ddsc_kernel"
+        a = torch.randn(tokens, k).to(BF16)
+        a[1::2] = float("nan")
+        print(n, k, tokens, nnz, transpose, flush=True)
+        got = m.reverse_matmul(a.to(cuda), transpose=transpose)
+        assert_close(got[0::2], to64(a[0::2]) @ wt, BF16, "transpose %d" % transpose)
