@@ -86,6 +86,7 @@ constexpr int DC_MAX_KP = 512;          // k-pairs (K <= 32768): 9 bits of an it
 constexpr int DC_ITEM_LAST = 1 << 10;
 constexpr int DC_MAX_BLOCKS = 1 << 21;  // byte offsets of blocks stay below 2^32
 constexpr int DC_ITEMS_LDS = 2048;      // items of a group kept in LDS (every pattern up to K = 4096)
+constexpr int DC_AHEAD = 8;             // steps between a copy and the touch of a later step's lines
 constexpr int DC_SEQ_INTS = 16384;      // the table 0, 1, 2, ...: a workgroup's steps are numbered below this (a power of two)
 #ifndef DC_SLEEP
 #define DC_SLEEP 8
@@ -277,6 +278,7 @@ struct DdscArgs {
     int M, N, K, nnz;
     int m_tiles, n_groups, group_ints;
     int wg_per_group;      // workgroups that share the token tiles of one column group
+    int touch;             // whether lines are asked for DC_AHEAD steps ahead
     int stream_step;       // of their numbering (stream_and_group)
 };
 
@@ -291,7 +293,8 @@ struct DdscCfg {
     static constexpr int DONE_OFF = STEPS_OFF + DC_MAX_KP * 4;           // done[16][64]
     static constexpr int LANDED_OFF = DONE_OFF + NW * 256;               // landed[8], failure word
     static constexpr int BIAS_OFF = LANDED_OFF + 256;                    // bias[16][32], 2 bytes each
-    static constexpr int LDS_BYTES = BIAS_OFF + NW * 64;
+    static constexpr int DUMP_OFF = BIAS_OFF + NW * 64;                  // what a touch loads, never read
+    static constexpr int LDS_BYTES = DUMP_OFF + 256;
     static constexpr int SPIN_LIMIT = 1 << 18;
     static_assert(RS >= 4 && RS <= 8, "ring depth");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS");
@@ -390,6 +393,31 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     bool gave_up = false;
     int md = 0;            // last minimum of done[] seen (it only grows)
 
+    // One word of each of the 128 lines of a step.  A dense operand that is not in the last-level cache (256 MB, for all operands and results) arrives a memory
+    // access later than the ring is deep for: 4096 -> 4096 density 0.25, 16384 tokens take 168 us with the same operand in every call and 196 with three in turn.
+    // So who copies a step then asks for the lines of the step a ring further on, one workgroup of those that share them in an XCD's L2 for all: 183 us (the
+    // input gradient in a training step 198 -> 190; at density 0.07 138 -> 125 and 140 -> 131).  For operands that are there it costs 2 to 5 %, with
+    // few workgroups to share it up to 13 %, and dense patterns, which wait for their products, gain nothing: the host decides (touches).  12, 16 and 64 steps
+    // ahead are level or 1 % slower, 4 half as good; the first steps touched before the loop, 2 us for every call.
+    const unsigned lds_dump = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(smem + C::DUMP_OFF));
+    const int touch_of = g.n_groups & 1 ? g.n_groups : g.n_groups >> 1, touch_at = ng % touch_of;
+    auto touch_step = [&](int t) __attribute__((always_inline)) {
+        int tile = ns > 1 ? (int)__builtin_amdgcn_readfirstlane((int)__umulhi((unsigned)t, magic_ns)) : t;
+        tile = tile < ntiles ? tile : ntiles - 1;
+        int step = t - tile * ns;
+        step = step < 0 ? 0 : (step >= ns ? ns - 1 : step);
+        const int m0 = (p + tile * g.wg_per_group) * C::BM;
+        const int a_last_row = g.M - 1 - m0;
+        int pair = __builtin_amdgcn_readfirstlane(s_steps[step]);
+        pair = pair < 0 ? 0 : (pair >= KP ? KP - 1 : pair);
+        const unsigned char* src = uniform_ptr(A + (size_t)m0 * a_row_bytes + (size_t)pair * C::ROWB);
+        int lc = lane;
+        asm volatile("" : "+v"(lc));
+        const int r0 = lc < a_last_row ? lc : a_last_row, r1 = 64 + lc < a_last_row ? 64 + lc : a_last_row;
+        dma4(lds_dump, src, (unsigned)r0 * a_row_bytes);
+        dma4(lds_dump, src, (unsigned)r1 * a_row_bytes);
+    };
+
     // Lane l of DMA instruction i of a step: row 8 i + l / 8, physical chunk l % 8 = logical chunk (l % 8) ^ ((row / 2) % 8):
     // the swizzle term is (l / 16) for even i and (l / 16) ^ 4 for odd i, so two per-lane offsets serve all rows (the row
     // advances in the scalar base address).
@@ -441,6 +469,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
         dma4_lane0((unsigned)(uintptr_t)(s_landed + (t & (RS - 1))),
                    uniform_ptr(reinterpret_cast<const unsigned char*>(g.seq + ((t + 1) & (DC_SEQ_INTS - 1)))));
 #endif
+        if (g.touch && t + DC_AHEAD < nsteps && (unsigned)(t + DC_AHEAD) % (unsigned)touch_of == (unsigned)touch_at) touch_step(t + DC_AHEAD);
     };
 
     // ---------------- progress words ----------------

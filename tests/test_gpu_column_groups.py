@@ -23,6 +23,7 @@ BF16 = torch.bfloat16
     ("column", 3584, 64, 1),                   # one tile: one stream
     ("column", 4096, 128, 128 * 33),
     ("column", 4608, 64, 128 * 30),
+    ("column", 2048, 4096, 12300),             # an operand of 100 MB: lines asked for ahead
     ("wide", 1536, 128, 128 * 86 + 5),
     ("wide", 3584, 64, 128 * 37),
 ])
