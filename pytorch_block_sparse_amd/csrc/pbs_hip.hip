@@ -15,6 +15,7 @@
 #include "pbs_panel.h"
 #include "pbs_split.h"
 #include "pbs_stream.h"
+#include "pbs_walk.h"
 #include "pbs_index.h"
 #include "pbs_sdd.h"
 #include "pbs_sdd_bf16.h"
@@ -381,8 +382,62 @@ static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
     return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)at.grid), dim3(KS * 64), 0, stream, a);
 }
 
+// fp32 with enough token tiles: the number of tiles that a wave of walk_kernel takes, or 0 for stream_kernel.  The estimate: launch, the blocks of the fullest CU, a wave's own
+// chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75, runs of 1 to 3) within 8 % on average.  It has to be a fourteenth below
+// stream_kernel's, from 10 us on.  How uneven columns are is not known here, and a wave multiplies a column alone: so a full column may take as long as the launch
+// at most (half a microsecond per block).  Of 260 products that stream_kernel served 89 are taken, 1.105 times as fast on average, two of them, with Zipf rows, slower (0.91 and 0.95); without
+// the bound on full columns one of 9 Zipf products was at 0.57, without the 10 us three small ones between 0.83 and 0.91.
+constexpr double WALK_MARGIN = 0.93, WALK_LEAST = 10.0, WALK_BLOCK = 0.5;
+constexpr int WALK_RUNS = 3;
+static long long walk_grid(int m_tiles, int xcd_t, int n, int run) {
+    const long long tiles = (m_tiles + xcd_t - 1) / xcd_t, sets = NUM_XCD / xcd_t;
+    return NUM_XCD * ((tiles + run - 1) / run) * ((n / 32 + sets - 1) / sets);
+}
+static int choose_walk(long long M, int n, int k, int nnz) {
+    return answer<int>(Sizes{M, n, k, nnz, 0}, [&] {
+        const double us = choose_stream(4, M, n, k, nnz).us;
+        // (a lane's offset into its token tile is a 32-bit number)
+        if (us < WALK_LEAST || 16ll * WALK_TT * k * 4 > 0xffffffffll) return 0;
+        const StreamGrid at = stream_grid(4, WALK_TT, M, n, k, nnz);
+        const double blocks = (double)nnz / (n / 32);
+        int best = 0;
+        double least = WALK_MARGIN * us;
+        for (int run = 1; run <= WALK_RUNS; ++run) {
+            const double per_cu = std::ceil((double)((at.m_tiles + run - 1) / run) * (n / 32) / 256.0);
+            const double t = 3.6 + per_cu * run * (0.122 * blocks + 0.136) + run * 0.493 * (std::ceil(blocks) + 1.0) + 0.0712e-6 * (double)M * ((double)n + k);
+            if (t >= least || WALK_BLOCK * run * (k / 32) > t || walk_grid(at.m_tiles, at.xcd_t, n, run) > (1ll << 30)) continue;
+            least = t;
+            best = run;
+        }
+        return best;
+    });
+}
+template <int TRANS>
+static int launch_walk(const DdsArgs& g, int run, hipStream_t stream) {
+    WalkArgs w;
+    StreamArgs& a = w.s;
+    a.a = g.a;
+    a.data = g.data;
+    a.plan = g.plan;
+    a.bias = g.bias;
+    a.out = g.out;
+    a.M = g.M;
+    a.N = g.N;
+    a.K = g.K;
+    const StreamGrid at = stream_grid(4, WALK_TT, g.M, g.N, g.K, g.nnz);
+    a.m_tiles = at.m_tiles;
+    a.xcd_t = at.xcd_t;
+    a.group = at.group / run < 1 ? 1 : at.group / run;   // (in runs)
+    w.run = run;
+    const dim3 grid((unsigned)walk_grid(at.m_tiles, at.xcd_t, g.N, run));
+    return stream_waves_f32(g.N, g.nnz) == 4 ? launch(walk_kernel<TRANS, 4>, grid, dim3(64), 0, stream, w) : launch(walk_kernel<TRANS, 2>, grid, dim3(64), 0, stream, w);
+}
+
 template <typename T, int TRANS>
 static int launch_stream(const DdsArgs& g, hipStream_t stream) {
+    if constexpr (sizeof(T) == 4) {
+        if (const int run = choose_walk(g.M, g.N, g.K, g.nnz)) return launch_walk<TRANS>(g, run, stream);
+    }
     const StreamShape s = choose_stream(sizeof(T), g.M, g.N, g.K, g.nnz).shape;
 #define PBS_STREAM(TT, KS) \
     if (s.tt == TT && s.ks == KS) return launch_stream_shape<T, TRANS, TT, KS>(g, stream);
@@ -1443,6 +1498,7 @@ const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || n <= 0 || k <= 0 || (n % 32) || (k % 32)) return "";
     const ProductChoice c = choose_product(dtype == PBS_DTYPE_F32 ? 4 : 2, tokens, n, k, nnz, transpose, with_workspace != 0);
     if (dtype == PBS_DTYPE_F32 && with_workspace && nnz > 0 && split_kernel_fits(tokens, n, k, nnz)) return "split_kernel";
+    if (dtype == PBS_DTYPE_F32 && choose_walk(tokens, n, k, nnz)) return "walk_kernel";
     return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (!c.panel.splits ? "stream_kernel" : (c.panel.ways ? "panel_chunk_kernel" : "panel_kernel")));
 }
 
