@@ -725,14 +725,16 @@ static int dispatch_dds(const DdsArgs& g, void* workspace, size_t workspace_byte
 // bf16 while the operands are small enough, and for large bf16 problems rectangles of 16 x 16 or 8 x 16 block positions
 // (pbs_sdd_bf16.h).
 struct SddPlan {
-    int rows, tiles_r, tiles_c, nsplit, tokens_per_split;   // rows: block rows of a rectangle, 16 or 8
+    int rows, tiles_r, tiles_c, nsplit, tokens_per_split;   // rows: block rows of a rectangle, 16 or 8 at most
+    bool even;                                              // the same number in all bands
 };
-static SddPlan plan_rectangles(long long M, int N, int K, int rows) {
+static SddPlan plan_rectangles(long long M, int N, int K, int rows, int more_r = 0, int more_c = 0) {   // more bands, and rectangles of a band, than there have to be
     constexpr int SC = SddBf16Cfg<16>::SC, TC = SddBf16Cfg<16>::TC;
     SddPlan p;
     p.rows = rows;
-    p.tiles_r = (N / 32 + rows - 1) / rows;
-    p.tiles_c = (K / 32 + SC - 1) / SC;
+    p.even = false;
+    p.tiles_r = (N / 32 + rows - 1) / rows + more_r;
+    p.tiles_c = (K / 32 + SC - 1) / SC + more_c;
     const long long tiles = (long long)p.tiles_r * p.tiles_c;
     const long long chunks = (M + TC - 1) / TC;
     // Aim at one workgroup per CU and never slightly more (the kernel's registers and LDS allow one
@@ -817,9 +819,45 @@ static double rectangle_us(const SddPlan& p, int nnz) {
 // Rectangles of eight block rows read X once per eight rows but need one pass where sixteen rows hold more blocks than the accumulators, and half the
 // slices: 4096 -> 4096, 16384 tokens, density 0.25 198 us with sixteen rows and 265 with eight, 0.5 383 and 339; 768 -> 3072 density 0.5 103 and 77.
 // Of the 75 problems the estimates pick the faster one or one within 2 %.
-static SddPlan plan_sdd(long long M, int N, int K, int nnz) {
+static SddPlan plan_small(long long M, int N, int K, int nnz) {
     const SddPlan tall = plan_rectangles(M, N, K, 16), flat = plan_rectangles(M, N, K, 8);
     return rectangle_us(flat, nnz) < rectangle_us(tall, nnz) ? flat : tall;
+}
+// Operands beyond 52 MB: more rectangles than there have to be where the fullest would hold more blocks than the accumulators.  It takes two passes over its tokens then, and the
+// launch waits for it: 77 blocks take 1.4 times as long as 66.  The fullest one: the rows of the largest band, the columns (dealt in pairs by their blocks)
+// of the largest rectangle, and 1.6 times the deviation of a band's blocks.  Fitted to 34 problems of 90 MB and more in 16 partitions each, within 6 % on average.
+// Of 50 others 11 are partitioned in another way than by rectangle_us, 1.20 to 1.42 times as fast, one with Zipf rows 5 % slower.
+// us: 15343 tokens 1760 -> 2784 density 0.71 249 -> 166, 13000 tokens 2304 -> 2752 density 0.3 140 -> 96, 12000 tokens 3072 -> 3072 density 0.3 153 -> 119,
+// 16384 tokens 2048 -> 2048 density 0.6 171 -> 127; 4096 -> 4096 at density 0.25 and 0.5 as before.
+static double partition_us(const SddPlan& p, int N, int K, int nnz) {
+    using C = SddBf16Cfg<16>;
+    const double rows = N / 32, columns = K / 32, row = nnz / rows, density = row / columns;
+    const int row_pairs = (N / 32 + 1) / 2, column_pairs = (K / 32 + 1) / 2;
+    int band = 2 * ((row_pairs + p.tiles_r - 1) / p.tiles_r);
+    if (!p.even || band > p.rows) band = p.rows;
+    double share = 2.0 * ((column_pairs + p.tiles_c - 1) / p.tiles_c) / columns;
+    if (share > 1.0) share = 1.0;
+    const double most = row * band * share + 1.6 * std::sqrt(band * columns * density * (density < 1.0 ? 1.0 - density : 0.0)) / p.tiles_c + 1.0;
+    const double passes = std::ceil(most / C::QMAX), rounds = std::ceil((double)p.tiles_r * p.tiles_c * p.nsplit / 256), chunks = p.tokens_per_split / C::TC;
+    const double us = p.rows == 16 ? 15.2 + rounds * (8.6 + chunks * (0.806 * passes + 0.053 * most / 8)) : 14.9 + rounds * (8.3 + chunks * (0.77 * passes + 0.027 * most / 8));
+    return us + (p.nsplit > 1 ? 2.5 + 0.68 * p.nsplit * (nnz / 1000.0) : 0.0);
+}
+static SddPlan plan_sdd(long long M, int N, int K, int nnz) {
+    SddPlan best = plan_small(M, N, K, nnz);
+    if (2.0 * (double)M * ((double)N + K) <= 52e6) return best;
+    double least = 0.93 * partition_us(best, N, K, nnz);   // (differences below that are within the estimate)
+    for (int rows = 16; rows >= 8; rows -= 8)
+        for (int more_r = 0; more_r <= 4; ++more_r)
+            for (int more_c = 0; more_c <= 2; ++more_c) {
+                SddPlan p = plan_rectangles(M, N, K, rows, more_r, more_c);
+                p.even = true;
+                const double us = partition_us(p, N, K, nnz);
+                if (us < least) {
+                    best = p;
+                    least = us;
+                }
+            }
+    return best;
 }
 // The kernel and, for the row kernel, the number of token slices of a launch (0: rectangles) and of launches, one behind the
 // other over consecutive ranges of the tokens.
@@ -881,7 +919,7 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
                 for (int p = one_list ? ROW_NB : 2; p <= ROW_NB; ++p) consider(ROW_SPLIT, p);
         }
     }
-    if (rectangles && fits && (large ? 0.9 : 1.0) * rectangle_us(plan_sdd(M, N, K, nnz), nnz) < best_us) best.slices = 0;
+    if (rectangles && fits && (large ? 0.9 : 1.0) * rectangle_us(plan_small(M, N, K, nnz), nnz) < best_us) best.slices = 0;
     return best;
 }
 struct BackPlan {
@@ -1009,6 +1047,7 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     a.K = b.K;
     a.nnz = b.nnz;
     a.rows = p.rows;
+    a.even = p.even;
     a.tiles_r = p.tiles_r;
     a.tiles_c = p.tiles_c;
     a.nsplit = p.nsplit;

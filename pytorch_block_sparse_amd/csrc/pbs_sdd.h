@@ -17,12 +17,13 @@ struct SddArgs {
     float* partial;          // [nsplit][nnz*1024, then N] fp32 when nsplit > 1
     int M, N, K, nnz;
     int rows;                // block rows of a rectangle, 16 or 8
+    int even;                // whether the rows are spread evenly over the bands
     int tiles_r, tiles_c, nsplit;
     int tokens_per_split;    // multiple of TC
 };
 
 // Which block rows of W form row band `band` of rectangles (SR places; -1 = no row).  Normally they are
-// rows SR*band .. SR*band + SR - 1.  When the per-row block counts are very uneven (largest > 2x the
+// rows SR*band .. SR*band + SR - 1, or (`even`) as many consecutive ones as in the other bands.  When the per-row block counts are very uneven (largest > 2x the
 // mean) the rows are ranked by count and dealt to the bands in serpentine order, so that all
 // rectangles hold about the same number of blocks.  Every workgroup derives its own band from the
 // row pointer array (a few microseconds at most; above SDD_BALANCE_MAX_ROWS rows the natural order
@@ -30,7 +31,7 @@ struct SddArgs {
 // whether the row pointers were scanned; then s_ptr_copy (nblk_r + 1 ints of LDS) holds them.
 constexpr int SDD_BALANCE_MAX_ROWS = 1024;
 static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__ ptr, int nnz, int nblk_r, int tiles_r, int band,
-                                                     int SR, int* s_rowid, int* scratch, int tid, int nthreads,
+                                                     int SR, bool even, int* s_rowid, int* scratch, int tid, int nthreads,
                                                      int* s_ptr_copy) {
     bool skewed = false;
     const bool scanned = nblk_r <= SDD_BALANCE_MAX_ROWS && tiles_r >= 2;
@@ -58,8 +59,10 @@ static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__
         skewed = (long long)most * nblk_r > 2ll * sum;
     }
     if (tid < SR) {
-        const int r = band * SR + tid;
-        s_rowid[tid] = (!skewed && r < nblk_r) ? r : -1;
+        // (even bands in whole pairs of rows: 128 bytes of G)
+        const int pairs = (nblk_r + 1) / 2, lo = even ? 2 * (int)((long long)pairs * band / tiles_r) : band * SR;
+        const int hi = even ? 2 * (int)((long long)pairs * (band + 1) / tiles_r) : lo + SR, r = lo + tid;
+        s_rowid[tid] = (!skewed && r < hi && r < nblk_r) ? r : -1;
     }
     __syncthreads();
     if (skewed) {
