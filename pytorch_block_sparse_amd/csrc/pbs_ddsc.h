@@ -395,12 +395,12 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
 
     // One word of each of the 128 lines of a step.  A dense operand that is not in the last-level cache (256 MB, for all operands and results) arrives a memory
     // access later than the ring is deep for: 4096 -> 4096 density 0.25, 16384 tokens take 168 us with the same operand in every call and 196 with three in turn.
-    // So who copies a step then asks for the lines of the step a ring further on, one workgroup of those that share them in an XCD's L2 for all: 183 us (the
-    // input gradient in a training step 198 -> 190; at density 0.07 138 -> 125 and 140 -> 131).  For operands that are there it costs 2 to 5 %, with
-    // few workgroups to share it up to 13 %, and dense patterns, which wait for their products, gain nothing: the host decides (touches).  12, 16 and 64 steps
-    // ahead are level or 1 % slower, 4 half as good; the first steps touched before the loop, 2 us for every call.
+    // So who copies a step then asks for the lines of the step a ring further on, one workgroup of all that read them for the chip: 183 us.  What has to arrive early is
+    // the line in the last-level cache; a touch fills 16 KB of L1 like a copy, so one in each of the two L2s that a panel is read through took 186 us, and 171 for 169 where the
+    // operand is there (the training step 584 us and 553 with the same tensors every time, now 574 and 542; without touches 598 and 551).  With few groups to share it
+    // it costs up to 13 %, and dense patterns, which wait for their products, gain nothing: the host decides (touches).  5 to 16 steps
+    // ahead are level, 24 and 40 1 to 2 % slower; the first steps touched before the loop, 2 us for every call.  Non-temporal touches are 10 % slower, past the L1 (sc0, sc1) level.
     const unsigned lds_dump = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(smem + C::DUMP_OFF));
-    const int touch_of = g.n_groups & 1 ? g.n_groups : g.n_groups >> 1, touch_at = ng % touch_of;
     auto touch_step = [&](int t) __attribute__((always_inline)) {
         int tile = ns > 1 ? (int)__builtin_amdgcn_readfirstlane((int)__umulhi((unsigned)t, magic_ns)) : t;
         tile = tile < ntiles ? tile : ntiles - 1;
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
         dma4_lane0((unsigned)(uintptr_t)(s_landed + (t & (RS - 1))),
                    uniform_ptr(reinterpret_cast<const unsigned char*>(g.seq + ((t + 1) & (DC_SEQ_INTS - 1)))));
 #endif
-        if (g.touch && t + DC_AHEAD < nsteps && (unsigned)(t + DC_AHEAD) % (unsigned)touch_of == (unsigned)touch_at) touch_step(t + DC_AHEAD);
+        if (g.touch && t + DC_AHEAD < nsteps && (unsigned)(t + DC_AHEAD) % (unsigned)g.n_groups == (unsigned)ng) touch_step(t + DC_AHEAD);
     };
 
     // ---------------- progress words ----------------

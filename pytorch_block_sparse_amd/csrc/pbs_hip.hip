@@ -236,8 +236,8 @@ static bool column_kernel_fits(long long M, int n, int k, int nnz) {
 }
 
 // Whether its copies ask for lines ahead (pbs_ddsc.h): a dense operand of 100 MB and more is taken to be in memory.  Of 60 products with operands of 12 to 98 MB, three in
-// turn, it makes 6 one to two hundredths faster and the others up to 7 slower (with one group in a set up to 13); of 11 with 98 to 134 MB and columns of up to 48 blocks 10 faster,
-// 1.01 to 1.10 times, one level; with 64 blocks to a column forward is 1 % faster and the weight gradient behind it 2 % slower (the card's power).
+// turn, it makes 6 to 9 one to seven hundredths faster and the others up to 9 slower (with one group in a set up to 13); of 16 with 98 to 134 MB and columns of up to 48 blocks
+// 14 faster, 1.01 to 1.10 times, two level.  With 62 to 64 blocks to a column training steps are 1 % faster (4096 -> 4096) or 2 % slower (3328 -> 3264), with 96 level.
 static bool touches(long long M, int n, int k, int nnz) {
     const int groups = column_groups(n);
     return 2.0 * (double)M * k >= 100e6 && (groups & 1 ? groups : groups / 2) >= 2 && nnz <= 48ll * (n / 32);
@@ -465,7 +465,7 @@ struct PanelChoice {
 static PanelChoice choose_panel(long long M, int n, int k, int nnz) {
     PanelChoice best{0, 0.0, 0, 0};
     const int cols = n / 32;
-    // (with fewer columns than waves it was the faster one nowhere; below 1024 tokens only in chunks, from 768 on where a contraction of 2048 and 48 columns of 16
+    // (with fewer columns than waves the estimates would take 17 of 108 products, 0.75 to 1.3 times as fast, 0.97 on average; below 1024 tokens only in chunks, from 768 on where a contraction of 2048 and 48 columns of 16
     // blocks leave the stream kernel more to copy than two workgroups per CU take: 2720 -> 4064 density 0.5, 1015 tokens 31 -> 23 us, 2784 -> 3808 density 0.29, 954 tokens 22.5 -> 18)
     if (nnz < 1 || cols < PANEL_NW || (M < 1024 && (M < 768 || k < 2048 || cols < 48 || nnz < 16 * cols))) return best;
     const double tiles = (double)((M + 16 * PANEL_TT - 1) / (16 * PANEL_TT));
