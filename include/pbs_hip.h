@@ -347,7 +347,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
  * the device.  The Python layer checks it after every product when PBS_DEBUG is set and raises.
  *
  * pbs_blocksparse_matmul_kernel_name / ..._back_kernel_name: which kernel(s) a call with these sizes runs
- * ("stream_kernel", "split_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel", "sdd_split_kernel",
+ * ("stream_kernel", "walk_kernel", "split_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel", "sdd_split_kernel",
  * "sdd_bf16_kernel", with " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
  */

@@ -567,7 +567,7 @@ static double split_us(long long M, int n, int k, int nnz) {
 // (Between 1.5 and 2 2^20 tokens x blocks, what the estimate has an eighth faster is 1.10 times as fast with even columns, 1 of 13 slower, and 0.99 with Zipf rows, 6 of 13
 // slower, down to 0.79: which of these a pattern is is not known here.)
 // Groups that are less than three quarters full (9, 10, 11 and 17 columns) take what the estimate, 9 % long for them, leaves: of 56 products 22, 1.14 times as fast, one 3 % slower
-// (14922 tokens 3744 -> 288 density 0.65 232 -> 181 us; 35 with an estimate 7 % shorter, four slower, down to 0.93).
+// (15776 tokens 1472 -> 288 density 0.73 97 -> 75 us, 12170 tokens 2368 -> 544 density 0.41 133 -> 110; 35 with an estimate 7 % shorter, four slower, down to 0.93).
 constexpr double SPLIT_MARGIN = 0.91;
 static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     const long long cols = n / 32, groups = split_groups(n);

@@ -1,5 +1,5 @@
 // dense x block-sparse -> dense (forward Y = X.W^T and input gradient dX = dY.W), one block column of the result per
-// workgroup.  The smaller and sparser fp32 products (the others: pbs_split.h), and the bf16 ones whose token count or pattern gives the kernels with shared operand
+// workgroup.  The smaller and sparser fp32 products (the others: pbs_split.h; of many token tiles and short columns: pbs_walk.h), and the bf16 ones whose token count or pattern gives the kernels with shared operand
 // panels (pbs_dds16.h, pbs_ddsc.h) too little to share.
 //
 // Work decomposition.  A workgroup owns 16 TT tokens x one block column (32 columns) of the result; its KS waves take the
