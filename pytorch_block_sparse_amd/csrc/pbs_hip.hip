@@ -676,7 +676,12 @@ static ProductChoice choose_product_anew(long long M, int n, int k, int nnz, int
     // 5 % slower (13394 tokens 2720 -> 1728 density 0.32 118 -> 69 us, 5332 tokens 3616 -> 1888 density 0.32 77 -> 49, 3983 tokens 3648 -> 1568 density 0.33 35 -> 29).
     // At level estimates five would be slower, down to 0.93.
     if (runs && M >= 2048 && k >= 1024) {
-        const double least = tp < ts ? (tp < tw ? tp : tw) : (ts < tw ? ts : tw);
+        // (an operand of more than 40 MB goes through memory again for the sets of columns that an XCD has of stream_kernel's, which its estimate does not count: 11386 tokens 3808 -> 2720
+        // with 7 blocks a column 68 us where it has 48.  So up to 16 % are added to it here: of 90 drawn layers 13 products more are the column kernel's, 1.23 times as fast, none slower: 15003
+        // tokens 2016 -> 3936 density 0.09 100 -> 68, 10288 tokens 3808 -> 2944 density 0.09 87 -> 60.  Without a bound 6 of 17 were slower, down to 0.90; panel and wide kernel chosen for it are 0.81 to
+        // 1.13 times as fast.)
+        const double mb = 2e-6 * (double)M * k, far = ts + (mb > 40.0 ? std::fmin(2.5e-4 * (mb - 40.0) * n, 0.16 * ts) : 0.0);
+        const double least = tp < far ? (tp < tw ? tp : tw) : (far < tw ? far : tw);
         if (column_anywhere_us(M, n, k, nnz, transpose != 0) < 0.93 * least) return {PART_COLUMN, NO_PANEL};
     }
     if (column && M >= 8192) return {PART_LIST, panel};

@@ -60,3 +60,25 @@ def test_odd_numbers_of_k_blocks(cuda, monkeypatch, out_f, in_f, tokens, nnz):
         print(n, k, tokens, nnz, transpose, flush=True)
         got = m.reverse_matmul(a.to(cuda), transpose=transpose)
         assert_close(got[0::2], to64(a[0::2]) @ wt, BF16, "transpose %d" % transpose)
+
+
+@pytest.mark.parametrize("out_f, in_f, tokens, nnz, transpose", [
+    (3744, 3360, 7261, 1230, True),
+    (2016, 3936, 15003, 706, True),     # an odd number of k-blocks, 118 MB: lines asked for ahead
+    (3072, 1952, 13826, 677, False),
+])
+def test_operands_that_the_stream_kernel_reads_again(cuda, out_f, in_f, tokens, nnz, transpose):
+    """Large dense operands with few blocks to a column go to the column kernel by its estimate; a forward product without a workspace does not."""
+    n, k = (out_f, in_f) if transpose else (in_f, out_f)
+    assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16, True) == "ddsc_kernel"
+    if transpose:
+        assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16, False) != "ddsc_kernel"
+    np.random.seed(nnz)
+    torch.manual_seed(nnz)
+    m = BlockSparseMatrix.randn((out_f, in_f), nnz, device="cpu", dtype=BF16).to(cuda)
+    w = O.to_dense(to64(m.data), m.build_coo_block_index().cpu().numpy(), (out_f, in_f))
+    a = torch.randn(tokens, k).to(BF16)
+    print(n, k, tokens, nnz, transpose, flush=True)
+    got = m.reverse_matmul(a.to(cuda), transpose=transpose)
+    rows = np.r_[0:260, tokens - 260:tokens]
+    assert_close(got[rows], to64(a[rows]) @ (w.T if transpose else w), BF16, "rows at either end")
