@@ -554,9 +554,9 @@ static double split_us(long long M, int n, int k, int nnz) {
     const double units = (double)M / SP_BM * groups / 256, full = units < 1.0 ? units : 1.0;
     return 6.61 + 0.00319 * nnz + split_tiles(M, groups).rounds * (0.101 * (k / 32) + 1.07 * nnz / (n / 32) * (0.669 + 0.331 * full) + 2.48);
 }
-// Which problems: a density of 0.2 and more, six columns and more, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and not
+// Which problems: a density of 0.2 and more, groups of 8 columns that are filled to three quarters, 512 tokens, 4.3 GFLOP (2^21 tokens x blocks), and not
 // where the estimates see stream_kernel ahead by a tenth.  Below that density a panel is split for too few products (0.15: 0.8 to 1.1 times as fast, 0.05:
-// half as fast); with fewer columns waves have none; with fewer tokens or products the launch that splits and the first panels weigh too much.
+// half as fast); with emptier groups waves have no column; with fewer tokens or products the launch that splits and the first panels weigh too much.
 // The tenth is for a result's bits: those of a token are the same, to the last bit, in all calls of a pattern that are served alike, and a line
 // at level estimates would part the calls of a 4096 -> 4096 layer of density 0.25 seven times between 512 and 2177 tokens.  Of the 821 products 802 are taken, 1.28
 // times faster on average (706 and 1.31 where the estimate has to be 1.08 below), 24 of them more than 2 % slower, the worst 0.83 times as fast, where
@@ -566,12 +566,12 @@ static double split_us(long long M, int n, int k, int nnz) {
 // 59 -> 105 us).
 // (Between 1.5 and 2 2^20 tokens x blocks, what the estimate has an eighth faster is 1.10 times as fast with even columns, 1 of 13 slower, and 0.99 with Zipf rows, 6 of 13
 // slower, down to 0.79: which of these a pattern is is not known here.)
-// Groups that are less than three quarters full (9, 10, 11 and 17 columns) take what the estimate, 9 % long for them, leaves: of 56 products 22, 1.14 times as fast, one 3 % slower
-// (15776 tokens 1472 -> 288 density 0.73 97 -> 75 us, 12170 tokens 2368 -> 544 density 0.41 133 -> 110; 35 with an estimate 7 % shorter, four slower, down to 0.93).
+// (Of 56 products of 9, 10, 11 and 17 columns the estimate, 9 % long for them, would take 22, 1.14 times as fast.  They stay with the fp32 instructions: results of few
+// products, as one value to a token gives them, are up to 1.6e-7 off here and one rounding there.)
 constexpr double SPLIT_MARGIN = 0.91;
 static bool split_kernel_fits(long long M, int n, int k, int nnz) {
     const long long cols = n / 32, groups = split_groups(n);
-    if (5ll * nnz < cols * (k / 32) || (cols < SP_NC && 4 * cols < 3 * SP_NC) || M < 512 || M * nnz < (1 << 21)) return false;
+    if (5ll * nnz < cols * (k / 32) || 4 * cols < 3 * SP_NC * groups || M < 512 || M * nnz < (1 << 21)) return false;
     // units have 32-bit numbers; the waves that wait for one that multiplies a column again (a microsecond per block) must not give up
     if (k > (1 << 16) || (M + 31) / 32 * groups >= (1 << 28)) return false;
     return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] { return SPLIT_MARGIN * split_us(M, n, k, nnz) < choose_stream(4, M, n, k, nnz).us; });
