@@ -19,6 +19,22 @@ def test_make_builds_what_the_package_loads():
     assert "-packed-fp32-ops" in plan
 
 
+def test_make_knows_every_header():
+    """A change to any header that the library is made of makes the library old."""
+    rules = subprocess.run(["make", "-npq", "-C", CSRC], capture_output=True, text=True).stdout
+    included, seen = ["pbs_hip.hip"], set()
+    while included:
+        path = os.path.normpath(os.path.join(CSRC, included.pop()))
+        if path in seen:
+            continue
+        seen.add(path)
+        with open(path) as f:
+            included += [os.path.join(os.path.dirname(path), name) for name in re.findall(r'^#include "(.*)"', f.read(), re.M)]
+    for library in ("libpbs_hip.so", "libpbs_hip_check.so"):
+        needs = re.search(r"^%s: (.*)$" % re.escape(library), rules, re.M).group(1).split()
+        assert seen <= {os.path.normpath(os.path.join(CSRC, n)) for n in needs}, library
+
+
 def test_version_of_the_header():
     with open(HEADER) as f:
         assert int(re.search(r"#define PBS_ABI_VERSION (\d+)", f.read()).group(1)) == native.ABI_VERSION
