@@ -382,12 +382,15 @@ static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
     return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)at.grid), dim3(KS * 64), 0, stream, a);
 }
 
-// fp32 with enough token tiles: the number of tiles that a wave of walk_kernel takes, or 0 for stream_kernel.  The estimate: launch, the blocks of the fullest CU, a wave's own
-// chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75, runs of 1 to 3) within 8 % on average.  It has to be a fourteenth below
-// stream_kernel's, from 10 us on.  How uneven columns are is not known here, and a wave multiplies a column alone: so a full column may take as long as the launch
-// at most (half a microsecond per block).  Of 260 products that stream_kernel served 89 are taken, 1.105 times as fast on average, two of them, with Zipf rows, slower (0.91 and 0.95); without
-// the bound on full columns one of 9 Zipf products was at 0.57, without the 10 us three small ones between 0.83 and 0.91.
-constexpr double WALK_MARGIN = 0.93, WALK_LEAST = 10.0, WALK_BLOCK = 0.5;
+// fp32 with enough token tiles and short columns: the number of tiles that a wave of walk_kernel takes, or 0 for stream_kernel.  The estimate: launch, the blocks of the fullest
+// CU, a wave's own chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75, runs of 1 to 3) within 8 % on average.  It has to be a
+// ninth below stream_kernel's, from 10 us on, where that would take tiles of 64 tokens (against its tiles of 32 it is 0.92 to 1.08 times as fast).
+// How uneven columns are is not known here, and a wave multiplies a column alone: so a contraction has at most 32 blocks, and a full column of them takes at most 0.4 of the launch (a
+// wave's block takes half a microsecond).  Of 280 products drawn from those that are taken two are slower (Zipf rows, 0.95 and 0.97), the others 1.12 times as fast on average.  With a
+// full column of any length, as long as the launch, 21 of 174 products with Zipf rows were slower, down to 0.64 (922 tokens 672 -> 2656 density 0.14 12.4 -> 19.5 us, 5163 tokens 3488 -> 3200 density
+// 0.056 139 -> 182), and even ones longer than 1024 features gained 4 % on average.
+constexpr double WALK_MARGIN = 0.89, WALK_LEAST = 10.0, WALK_BLOCK = 0.5, WALK_FULL = 0.4;
+constexpr int WALK_MAX_K = 1024;
 constexpr int WALK_RUNS = 3;
 static long long walk_grid(int m_tiles, int xcd_t, int n, int run) {
     const long long tiles = (m_tiles + xcd_t - 1) / xcd_t, sets = NUM_XCD / xcd_t;
@@ -395,17 +398,16 @@ static long long walk_grid(int m_tiles, int xcd_t, int n, int run) {
 }
 static int choose_walk(long long M, int n, int k, int nnz) {
     return answer<int>(Sizes{M, n, k, nnz, 0}, [&] {
-        const double us = choose_stream(4, M, n, k, nnz).us;
-        // (a lane's offset into its token tile is a 32-bit number)
-        if (us < WALK_LEAST || 16ll * WALK_TT * k * 4 > 0xffffffffll) return 0;
+        const StreamChoice stream = choose_stream(4, M, n, k, nnz);
+        if (stream.us < WALK_LEAST || stream.shape.tt != 4 || k > WALK_MAX_K) return 0;
         const StreamGrid at = stream_grid(4, WALK_TT, M, n, k, nnz);
         const double blocks = (double)nnz / (n / 32);
         int best = 0;
-        double least = WALK_MARGIN * us;
+        double least = WALK_MARGIN * stream.us;
         for (int run = 1; run <= WALK_RUNS; ++run) {
             const double per_cu = std::ceil((double)((at.m_tiles + run - 1) / run) * (n / 32) / 256.0);
             const double t = 3.6 + per_cu * run * (0.122 * blocks + 0.136) + run * 0.493 * (std::ceil(blocks) + 1.0) + 0.0712e-6 * (double)M * ((double)n + k);
-            if (t >= least || WALK_BLOCK * run * (k / 32) > t || walk_grid(at.m_tiles, at.xcd_t, n, run) > (1ll << 30)) continue;
+            if (t >= least || WALK_BLOCK * run * (k / 32) > WALK_FULL * t || walk_grid(at.m_tiles, at.xcd_t, n, run) > (1ll << 30)) continue;
             least = t;
             best = run;
         }

@@ -7,7 +7,6 @@ from oracle import block_sparse_oracle as O
 from pytorch_block_sparse_amd import BlockSparseMatrix, native, workloads
 from tests.helpers import assert_close, to64
 
-pytestmark = pytest.mark.gpu
 F32 = torch.float32
 
 
@@ -20,16 +19,27 @@ def _blocks(out_f, in_f, nnz, zipf, seed):
     return [(int(p) // grid[1], int(p) % grid[1]) for p in where]
 
 
+@pytest.mark.parametrize("n, k, tokens, nnz", [
+    (2656, 672, 922, 247), (1856, 768, 2528, 132), (960, 672, 5473, 137),   # 0.64 to 0.85 times as fast where columns are uneven: a full one would take half of the launch
+    (3200, 3488, 5163, 610), (4064, 2240, 2323, 693), (2144, 2880, 10753, 374),   # 0.77 to 0.85: a long one, more than that of its work
+    (1984, 992, 4001, 480), (640, 448, 14976, 129),   # nothing to gain
+])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_columns_that_may_be_long(n, k, tokens, nnz, transpose):
+    """The host does not know how uneven columns are: what loses with uneven ones stays with stream_kernel."""
+    assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, F32, False) == "stream_kernel"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n, k, tokens, nnz, transpose, zipf", [
     (3808, 384, 13134, 72, True, False),        # columns without blocks
-    (640, 448, 14976, 129, True, False),
+    (640, 448, 14976, 60, True, False),
     (1792, 256, 13092 - 13092 % 32, 70, False, False),   # whole tiles only
     (1792, 256, 13092 - 13092 % 32 + 1, 70, True, False),  # one token in the last tile
     (1248, 608, 12843, 75, False, False),
     (1088, 480, 9000, 120, True, True),         # uneven columns
-    (1984, 992, 4001, 480, False, False),
-    (3072, 2400, 16001, 1350, False, False),    # sums of four
-    (3072, 2400, 16001, 1350, True, True),      # and lists of more than 64 entries
+    (3072, 1024, 14000, 450, True, False),      # the longest contraction
+    (3072, 1024, 14001, 450, False, True),
 ])
 @pytest.mark.parametrize("bias", [False, True])
 def test_same_bits_as_stream_kernel(cuda, n, k, tokens, nnz, transpose, zipf, bias):
@@ -47,9 +57,7 @@ def test_same_bits_as_stream_kernel(cuda, n, k, tokens, nnz, transpose, zipf, bi
     m = m.to(cuda)
     x = torch.randn(tokens, k, device=cuda)
     b = torch.randn(n, device=cuda) if bias else None
-    ends = (m.row_start_ends_a if transpose else m.col_start_ends_b).cpu()
-    print(n, k, tokens, nnz, transpose, zipf, bias, "longest", int(ends.diff().max()), flush=True)
-    assert k <= 2048 or not zipf or ends.diff().max() > 64
+    print(n, k, tokens, nnz, transpose, zipf, bias, flush=True)
     ptr, entries = (m.row_start_ends_a, m.cols_a) if transpose else (m.col_start_ends_b, m.rows_b)
     plan = native.blocksparse_matmul_plan(ptr, entries, n, k)
     run = lambda rows: native.blocksparse_matmul(rows, m.data.detach(), plan, n, k, nnz, transpose, bias=b)
