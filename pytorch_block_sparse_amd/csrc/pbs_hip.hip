@@ -362,83 +362,42 @@ static StreamGrid stream_grid(int esz, int tt, long long M, int n, int k, int nn
     });
 }
 
+static StreamArgs stream_args(const DdsArgs& g, const StreamGrid& at) { return {g.a, g.data, g.plan, g.bias, g.out, g.M, g.N, g.K, at.m_tiles, at.xcd_t, at.group}; }
+
 template <typename T, int TRANS, int TT, int KS>
 static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
     constexpr int WPE = TT == 8 ? 2 : (TT == 4 ? 3 : 4);   // waves per SIMD that the registers have to allow
-    StreamArgs a;
-    a.a = g.a;
-    a.data = g.data;
-    a.plan = g.plan;
-    a.bias = g.bias;
-    a.out = g.out;
-    a.M = g.M;
-    a.N = g.N;
-    a.K = g.K;
     const StreamGrid at = stream_grid(sizeof(T), TT, g.M, g.N, g.K, g.nnz);
-    a.m_tiles = at.m_tiles;
-    a.xcd_t = at.xcd_t;
-    a.group = at.group;
     if (at.grid > (1ll << 30)) return PBS_ERR_TOO_LARGE;
-    return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)at.grid), dim3(KS * 64), 0, stream, a);
+    return launch((stream_kernel<T, TRANS, TT, KS, WPE>), dim3((unsigned)at.grid), dim3(KS * 64), 0, stream, stream_args(g, at));
 }
 
-// fp32 with enough token tiles and short columns: the number of tiles that a wave of walk_kernel takes, or 0 for stream_kernel.  The estimate: launch, the blocks of the fullest
-// CU, a wave's own chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75, runs of 1 to 3) within 8 % on average.  It has to be a
+// fp32 with enough token tiles and short columns: whether walk_kernel takes it from stream_kernel.  The estimate: launch, the blocks of the fullest
+// CU, a wave's own chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75) within 8 % on average.  It has to be a
 // ninth below stream_kernel's, from 10 us on, where that would take tiles of 64 tokens (against its tiles of 32 it is 0.92 to 1.08 times as fast).
 // How uneven columns are is not known here, and a wave multiplies a column alone: so a contraction has at most 32 blocks, and a full column of them takes at most 0.4 of the launch (a
-// wave's block takes half a microsecond).  Of 280 products drawn from those that are taken two are slower (Zipf rows, 0.95 and 0.97), the others 1.12 times as fast on average.  With a
+// wave's block takes half a microsecond).  Of 280 products drawn from those that are taken, a quarter with uneven columns, one is slower (0.98), the others 1.12 times as fast on average.  With a
 // full column of any length, as long as the launch, 21 of 174 products with Zipf rows were slower, down to 0.64 (922 tokens 672 -> 2656 density 0.14 12.4 -> 19.5 us, 5163 tokens 3488 -> 3200 density
 // 0.056 139 -> 182), and even ones longer than 1024 features gained 4 % on average.
 constexpr double WALK_MARGIN = 0.89, WALK_LEAST = 10.0, WALK_BLOCK = 0.5, WALK_FULL = 0.4;
-constexpr int WALK_MAX_K = 1024;
-constexpr int WALK_RUNS = 3;
-static long long walk_grid(int m_tiles, int xcd_t, int n, int run) {
-    const long long tiles = (m_tiles + xcd_t - 1) / xcd_t, sets = NUM_XCD / xcd_t;
-    return NUM_XCD * ((tiles + run - 1) / run) * ((n / 32 + sets - 1) / sets);
-}
-static int choose_walk(long long M, int n, int k, int nnz) {
-    return answer<int>(Sizes{M, n, k, nnz, 0}, [&] {
+static bool choose_walk(long long M, int n, int k, int nnz) {
+    return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] {
         const StreamChoice stream = choose_stream(4, M, n, k, nnz);
-        if (stream.us < WALK_LEAST || stream.shape.tt != 4 || k > WALK_MAX_K) return 0;
+        if (stream.us < WALK_LEAST || stream.shape.tt != 4 || stream.shape.ks != 2 || k > WALK_MAX_K) return false;
         const StreamGrid at = stream_grid(4, WALK_TT, M, n, k, nnz);
-        const double blocks = (double)nnz / (n / 32);
-        int best = 0;
-        double least = WALK_MARGIN * stream.us;
-        for (int run = 1; run <= WALK_RUNS; ++run) {
-            const double per_cu = std::ceil((double)((at.m_tiles + run - 1) / run) * (n / 32) / 256.0);
-            const double t = 3.6 + per_cu * run * (0.122 * blocks + 0.136) + run * 0.493 * (std::ceil(blocks) + 1.0) + 0.0712e-6 * (double)M * ((double)n + k);
-            if (t >= least || WALK_BLOCK * run * (k / 32) > WALK_FULL * t || walk_grid(at.m_tiles, at.xcd_t, n, run) > (1ll << 30)) continue;
-            least = t;
-            best = run;
-        }
-        return best;
+        const double blocks = (double)nnz / (n / 32), per_cu = std::ceil((double)at.m_tiles * (n / 32) / 256.0);
+        const double t = 3.6 + per_cu * (0.122 * blocks + 0.136) + 0.493 * (std::ceil(blocks) + 1.0) + 0.0712e-6 * (double)M * ((double)n + k);
+        return t < WALK_MARGIN * stream.us && WALK_BLOCK * (k / 32) <= WALK_FULL * t && at.grid <= (1ll << 30);
     });
-}
-template <int TRANS>
-static int launch_walk(const DdsArgs& g, int run, hipStream_t stream) {
-    WalkArgs w;
-    StreamArgs& a = w.s;
-    a.a = g.a;
-    a.data = g.data;
-    a.plan = g.plan;
-    a.bias = g.bias;
-    a.out = g.out;
-    a.M = g.M;
-    a.N = g.N;
-    a.K = g.K;
-    const StreamGrid at = stream_grid(4, WALK_TT, g.M, g.N, g.K, g.nnz);
-    a.m_tiles = at.m_tiles;
-    a.xcd_t = at.xcd_t;
-    a.group = at.group / run < 1 ? 1 : at.group / run;   // (in runs)
-    w.run = run;
-    const dim3 grid((unsigned)walk_grid(at.m_tiles, at.xcd_t, g.N, run));
-    return stream_waves_f32(g.N, g.nnz) == 4 ? launch(walk_kernel<TRANS, 4>, grid, dim3(64), 0, stream, w) : launch(walk_kernel<TRANS, 2>, grid, dim3(64), 0, stream, w);
 }
 
 template <typename T, int TRANS>
 static int launch_stream(const DdsArgs& g, hipStream_t stream) {
     if constexpr (sizeof(T) == 4) {
-        if (const int run = choose_walk(g.M, g.N, g.K, g.nnz)) return launch_walk<TRANS>(g, run, stream);
+        if (choose_walk(g.M, g.N, g.K, g.nnz)) {
+            const StreamGrid at = stream_grid(4, WALK_TT, g.M, g.N, g.K, g.nnz);
+            return launch(walk_kernel<TRANS>, dim3((unsigned)at.grid), dim3(64), 0, stream, stream_args(g, at));
+        }
     }
     const StreamShape s = choose_stream(sizeof(T), g.M, g.N, g.K, g.nnz).shape;
 #define PBS_STREAM(TT, KS) \
