@@ -1,0 +1,27 @@
+"""Which bf16 products the column kernel takes by its estimate (the choice is made on the host)."""
+import pytest
+import torch
+
+from pytorch_block_sparse_amd import native
+
+BF16 = torch.bfloat16
+
+
+@pytest.mark.parametrize("n, k, tokens, density, transpose, kernel", [
+    # faster in the kernel that they have left: 0.87 and 0.91 of its speed in the column kernel
+    (1984, 3264, 15459, 0.156, True, "dds16_kernel"),
+    (1984, 3200, 16294, 0.166, True, "dds16_kernel"),
+    # 0.93 to 0.96: forward products of short contractions with half of the blocks and more
+    (2496, 1248, 5380, 0.712, True, "panel_chunk_kernel"),
+    (928, 1184, 14262, 0.737, True, "panel_chunk_kernel"),
+    # 0.92 to 0.95: input gradients at nearly level estimates
+    (3936, 2016, 4855, 0.297, False, "panel_chunk_kernel"),
+    (1408, 1056, 12675, 0.369, False, "panel_chunk_kernel"),
+    # 1.1 to 1.4 times as fast
+    (1728, 2720, 13394, 0.32, True, "ddsc_kernel"),
+    (2016, 3936, 15003, 0.0912, True, "ddsc_kernel"),
+    (1952, 3072, 13826, 0.1157, False, "ddsc_kernel"),
+])
+def test_faster_kernel(n, k, tokens, density, transpose, kernel):
+    nnz = int(density * (n // 32) * (k // 32))
+    assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16) == kernel
