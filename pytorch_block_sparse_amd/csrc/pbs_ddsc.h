@@ -278,7 +278,7 @@ struct DdscArgs {
     int M, N, K, nnz;
     int m_tiles, n_groups, group_ints;
     int wg_per_group;      // workgroups that share the token tiles of one column group
-    int touch;             // whether lines are asked for DC_AHEAD steps ahead
+    int touch;             // whether lines are asked for DC_AHEAD steps ahead (where columns are even)
     int stream_step;       // of their numbering (stream_and_group)
 };
 
@@ -351,16 +351,22 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     const int ni = has_col ? __builtin_amdgcn_readlane(v_hdr, 1 + wave) : 0;
     // items of the group -> LDS, column after column (the host launches this kernel only when they fit: K <= 4096)
     int ioff = 0;
+    bool touch = false;
     {
-        int off = 0;
+        int off = 0, most = 0, columns = 0;
 #pragma unroll
         for (int c = 0; c < NW; ++c) {
             const int n = __builtin_amdgcn_readlane(v_hdr, 1 + c);
             if (c == wave) ioff = off;
+            most = n > most ? n : most;
+            columns += n > 0 ? 1 : 0;
             if (off + n <= DC_ITEMS_LDS)
                 for (int i = tid; i < 2 * n; i += C::NT) s_items[2 * off + i] = gplan[DC_HDR + KP + c * 2 * KB + i];
             off += n;
         }
+        // (its longest column up to 2.2 times the average: patterns of 6 and more blocks to a column without any structure; with Zipf rows a full column
+        // is longer than that, and 134 such forward products were 0.5 to 1 % slower with touches)
+        touch = g.touch && 5 * most * columns <= 11 * off;
         for (int i = tid; i < ns; i += C::NT) s_steps[i] = gplan[DC_HDR + i];
         for (int i = tid; i < NW * 64 + 64; i += C::NT) s_done[i] = 0;   // done, landed, failure word
         // the bias of this wave's 32 result columns (zeros without one): the stores of a tile must not wait for a load
@@ -393,12 +399,15 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     bool gave_up = false;
     int md = 0;            // last minimum of done[] seen (it only grows)
 
-    // One word of each of the 128 lines of a step.  A dense operand that is not in the last-level cache (256 MB, for all operands and results) arrives a memory
+    // One word of each of the 128 rows of a step.  A dense operand that is not in the last-level cache (256 MB, for all operands and results) arrives a memory
     // access later than the ring is deep for: 4096 -> 4096 density 0.25, 16384 tokens take 168 us with the same operand in every call and 196 with three in turn.
-    // So who copies a step then asks for the lines of the step a ring further on, one workgroup of all that read them for the chip: 183 us.  What has to arrive early is
-    // the line in the last-level cache; a touch fills 16 KB of L1 like a copy, so one in each of the two L2s that a panel is read through took 186 us, and 171 for 169 where the
-    // operand is there (the training step 584 us and 553 with the same tensors every time, now 574 and 542; without touches 598 and 551).  With few groups to share it
-    // it costs up to 13 %, and dense patterns, which wait for their products, gain nothing: the host decides (touches).  5 to 16 steps
+    // So who copies a step then asks for the lines of the step a ring further on, one column group of all that read a panel, told by the panel: 183 us.  (By the number of the step,
+    // which stands for another panel in a group whose list leaves k-pairs out, some lines were asked for several times and some never: 250 even products 1.03 times as fast as without touches,
+    // 1.07 now.  Of a panel that the group does not read no line is asked for.  Of an odd number of k-blocks every other row begins in the middle of a line: the line's other half is the
+    // next step's, which asks for it a step later.)
+    // What has to arrive early is the line in the last-level cache; a touch fills 16 KB of L1 like a copy, so one in each of the two L2s that a panel is read through took 186 us, and 171 for 169 where the
+    // operand is there (the training step 584 us and 553 with the same tensors every time, with one for the chip 574 and 542; without touches 598 and 551).  Dense patterns and those with
+    // long columns wait for their products and gain nothing: the host decides by the sizes (touches), the group by its longest column.  5 to 16 steps
     // ahead are level, 24 and 40 1 to 2 % slower; the first steps touched before the loop, 2 us for every call.  Non-temporal touches are 10 % slower, past the L1 (sc0, sc1) level.
     const unsigned lds_dump = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(smem + C::DUMP_OFF));
     auto touch_step = [&](int t) __attribute__((always_inline)) {
@@ -410,6 +419,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
         const int a_last_row = g.M - 1 - m0;
         int pair = __builtin_amdgcn_readfirstlane(s_steps[step]);
         pair = pair < 0 ? 0 : (pair >= KP ? KP - 1 : pair);
+        if ((unsigned)(p + tile * g.wg_per_group + pair) % (unsigned)g.n_groups != (unsigned)ng) return;
         const unsigned char* src = uniform_ptr(A + (size_t)m0 * a_row_bytes + (size_t)pair * C::ROWB);
         int lc = lane;
         asm volatile("" : "+v"(lc));
@@ -469,7 +479,7 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
         dma4_lane0((unsigned)(uintptr_t)(s_landed + (t & (RS - 1))),
                    uniform_ptr(reinterpret_cast<const unsigned char*>(g.seq + ((t + 1) & (DC_SEQ_INTS - 1)))));
 #endif
-        if (g.touch && t + DC_AHEAD < nsteps && (unsigned)(t + DC_AHEAD) % (unsigned)g.n_groups == (unsigned)ng) touch_step(t + DC_AHEAD);
+        if (touch && t + DC_AHEAD < nsteps) touch_step(t + DC_AHEAD);
     };
 
     // ---------------- progress words ----------------

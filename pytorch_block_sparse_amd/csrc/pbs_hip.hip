@@ -235,12 +235,12 @@ static bool column_kernel_fits(long long M, int n, int k, int nnz) {
     return n >= DDSC_WIDE_RESULT && k >= 1024 && per_column >= 2.0;
 }
 
-// Whether its copies ask for lines ahead (pbs_ddsc.h): a dense operand of 100 MB and more is taken to be in memory.  Of 60 products with operands of 12 to 98 MB, three in
-// turn, it makes 6 to 9 one to seven hundredths faster and the others up to 9 slower (with one group in a set up to 13); of 16 with 98 to 134 MB and columns of up to 48 blocks
-// 14 faster, 1.01 to 1.10 times, two level.  With 62 to 64 blocks to a column training steps are 1 % faster (4096 -> 4096) or 2 % slower (3328 -> 3264), with 96 level.
+// Whether its copies ask for lines ahead (pbs_ddsc.h): a dense operand of 100 MB and more is taken to be in memory (of 60 products with operands of 12 to 98 MB, three in
+// turn, it makes 6 to 9 one to seven hundredths faster and the others up to 9 slower), with four groups of columns to share the asking (with three 1.00, two of nine slower) and columns of up to 32 blocks (with 33
+// to 48 1.01 times as fast, 8 of 35 slower, down to 0.95).  250 products drawn from those: even ones 1.05 times as fast, with an odd number of k-blocks 1.08, two slower (0.965, 0.975); with
+// Zipf rows 260 others 1.00 (0.91 to 1.09).
 static bool touches(long long M, int n, int k, int nnz) {
-    const int groups = column_groups(n);
-    return 2.0 * (double)M * k >= 100e6 && (groups & 1 ? groups : groups / 2) >= 2 && nnz <= 48ll * (n / 32);
+    return 2.0 * (double)M * k >= 100e6 && column_groups(n) >= 4 && nnz <= 32ll * (n / 32);
 }
 // FM: the blocks are given in fragment order (the forward product's copy) instead of [n][k] as stored
 template <bool FM>
