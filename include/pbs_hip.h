@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define PBS_ABI_VERSION 9
+#define PBS_ABI_VERSION 10
 #define PBS_BLOCK 32
 
 /* element type of dense operands, packed data and results (accumulation is fp32) */
@@ -338,7 +338,7 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
                                         int dtype, void* stream);
 
 /*
- * Diagnostics.  Neither has a counterpart in the reference.
+ * Diagnostics.  None has a counterpart in the reference.
  *
  * pbs_protocol_failures: the kernels for large problems (dds16_kernel, ddsc_kernel, split_kernel) synchronise their waves
  * through progress words in LDS with bounded waits instead of barriers.  A wait that runs into its bound means a
@@ -350,11 +350,20 @@ int pbs_blocksparse_matmul_back_noalloc(const void* dense_a, const void* dense_b
  * ("stream_kernel", "walk_kernel", "split_kernel", "panel_kernel", "panel_chunk_kernel", "dds16_kernel", "ddsc_kernel"; "sdd_row_kernel", "sdd_split_kernel",
  * "sdd_bf16_kernel", with " + sdd_reduce_kernel" when the token range is split), for benchmark labels.  "" for arguments the product
  * entry points reject.
+ *
+ * pbs_blocksparse_matmul_kernel_form: that name and, behind a comma, what a test of a form of the kernel has to know: "lines ahead" where copies of
+ * "ddsc_kernel" may ask for them.
+ * pbs_blocksparse_matmul_back_kernel_form: of "sdd_bf16_kernel" its partition, as "11 even bands of 8 rows x 2 rectangles x 11 slices" ("even": of equal numbers of
+ * rows, 8 at most).  The texts are the calling thread's until its next call.
  */
 int pbs_protocol_failures(unsigned* count);
 const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int nnz, int transpose, int dtype,
                                                int with_workspace);
+const char* pbs_blocksparse_matmul_kernel_form(int64_t tokens, int n, int k, int nnz, int transpose, int dtype,
+                                               int with_workspace);
 const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_features, int in_features, int nnz,
+                                                    int dtype);
+const char* pbs_blocksparse_matmul_back_kernel_form(int64_t tokens, int out_features, int in_features, int nnz,
                                                     int dtype);
 
 #ifdef __cplusplus

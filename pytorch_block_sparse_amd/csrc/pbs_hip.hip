@@ -5,8 +5,10 @@
 
 #include <atomic>
 #include <cmath>
+#include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <string>
 #include <tuple>
 
 #include "pbs_common.h"
@@ -1515,6 +1517,13 @@ const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int
     return c.part == PART_COLUMN ? "ddsc_kernel" : (c.part == PART_WIDE ? "dds16_kernel" : (!c.panel.splits ? "stream_kernel" : (c.panel.ways ? "panel_chunk_kernel" : "panel_kernel")));
 }
 
+const char* pbs_blocksparse_matmul_kernel_form(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace) {
+    static thread_local char text[96];
+    const std::string name = pbs_blocksparse_matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace);
+    std::snprintf(text, sizeof text, "%s%s", name.c_str(), name == "ddsc_kernel" && touches(tokens, n, k, nnz) ? ", lines ahead" : "");
+    return text;
+}
+
 const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
     if ((dtype != PBS_DTYPE_F32 && dtype != PBS_DTYPE_BF16) || tokens <= 0 || out_features <= 0 || in_features <= 0 ||
         nnz <= 0 || (out_features % 32) || (in_features % 32))
@@ -1523,6 +1532,15 @@ const char* pbs_blocksparse_matmul_back_kernel_name(int64_t tokens, int out_feat
     if (p.slices > 0 && p.split) return p.slices > 1 ? "sdd_split_kernel + sdd_reduce_kernel" : "sdd_split_kernel";
     if (p.slices > 0) return p.slices > 1 ? "sdd_row_kernel + sdd_reduce_kernel" : "sdd_row_kernel";
     return p.rect.nsplit > 1 ? "sdd_bf16_kernel + sdd_reduce_kernel" : "sdd_bf16_kernel";
+}
+
+const char* pbs_blocksparse_matmul_back_kernel_form(int64_t tokens, int out_features, int in_features, int nnz, int dtype) {
+    static thread_local char text[128];
+    const char* name = pbs_blocksparse_matmul_back_kernel_name(tokens, out_features, in_features, nnz, dtype);
+    if (!name[0] || plan_back(dtype, tokens, out_features, in_features, nnz, false, true).slices > 0) return name;
+    const SddPlan p = plan_back(dtype, tokens, out_features, in_features, nnz, false, true).rect;
+    std::snprintf(text, sizeof text, "%s, %d %sbands of %d rows x %d rectangles x %d slices", name, p.tiles_r, p.even ? "even " : "", p.rows, p.tiles_c, p.nsplit);
+    return text;
 }
 
 }  // extern "C"

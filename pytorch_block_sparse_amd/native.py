@@ -16,7 +16,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libpbs_hip.so")
 
-ABI_VERSION = 9   # PBS_ABI_VERSION of the header that the prototypes below restate
+ABI_VERSION = 10   # PBS_ABI_VERSION of the header that the prototypes below restate
 
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
 SUPPORTED_DTYPES = tuple(DTYPE_CODES)
@@ -77,7 +77,9 @@ _PROTOTYPES = {
     "pbs_blocksparse_matmul_back_noalloc_init": (_i32, []),
     "pbs_protocol_failures": (_i32, [ctypes.POINTER(ctypes.c_uint)]),
     "pbs_blocksparse_matmul_kernel_name": (ctypes.c_char_p, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_matmul_kernel_form": (ctypes.c_char_p, [_i64, _i32, _i32, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul_back_kernel_name": (ctypes.c_char_p, [_i64, _i32, _i32, _i32, _i32]),
+    "pbs_blocksparse_matmul_back_kernel_form": (ctypes.c_char_p, [_i64, _i32, _i32, _i32, _i32]),
     "pbs_blocksparse_matmul_back_noalloc": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
 }
 
@@ -151,8 +153,18 @@ def matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace=True)
         tokens, n, k, nnz, 1 if transpose else 0, DTYPE_CODES[dtype], 1 if with_workspace else 0).decode()
 
 
+def matmul_kernel_form(tokens, n, k, nnz, transpose, dtype, with_workspace=True):
+    """That name and in which of its forms the kernel runs (for tests of a form)."""
+    return load().pbs_blocksparse_matmul_kernel_form(
+        tokens, n, k, nnz, 1 if transpose else 0, DTYPE_CODES[dtype], 1 if with_workspace else 0).decode()
+
+
 def matmul_back_kernel_name(tokens, out_features, in_features, nnz, dtype):
     return load().pbs_blocksparse_matmul_back_kernel_name(tokens, out_features, in_features, nnz, DTYPE_CODES[dtype]).decode()
+
+
+def matmul_back_kernel_form(tokens, out_features, in_features, nnz, dtype):
+    return load().pbs_blocksparse_matmul_back_kernel_form(tokens, out_features, in_features, nnz, DTYPE_CODES[dtype]).decode()
 
 
 def _stream(index=None):

@@ -29,11 +29,15 @@ BF16 = torch.bfloat16
 ])
 def test_every_tile_of_every_group(cuda, monkeypatch, kernel, out_f, in_f, tokens):
     monkeypatch.setenv("PBS_COLUMN_KERNEL", "1" if kernel == "column" else "0")
-    nnz = out_f // 32
+    nnz = out_f // 32 * (8 if in_f == 4096 else 1)
     assert native.matmul_kernel_name(tokens, out_f, in_f, nnz, True, BF16, kernel == "column") == ("ddsc_kernel" if kernel == "column" else "dds16_kernel")
+    if in_f == 4096:
+        assert native.matmul_kernel_form(tokens, out_f, in_f, nnz, True, BF16).endswith(", lines ahead")
     np.random.seed(out_f)
     torch.manual_seed(out_f)
-    m = BlockSparseMatrix.randn((out_f, in_f), nnz, device="cpu", dtype=BF16).to(cuda)
+    # (a group whose columns are uneven does not ask ahead)
+    blocks = [(r, (16 * j + r) % 128) for r in range(out_f // 32) for j in range(8)] if in_f == 4096 else None
+    m = BlockSparseMatrix.randn((out_f, in_f), None if blocks else nnz, blocks=blocks, device="cpu", dtype=BF16).to(cuda)
     x = torch.randn(tokens, in_f).to(BF16)
     w = O.to_dense(to64(m.data), m.build_coo_block_index().cpu().numpy(), (out_f, in_f))
     print(kernel, out_f, in_f, tokens, flush=True)
@@ -71,6 +75,7 @@ def test_operands_that_the_stream_kernel_reads_again(cuda, out_f, in_f, tokens, 
     """Large dense operands with few blocks to a column go to the column kernel by its estimate; a forward product without a workspace does not."""
     n, k = (out_f, in_f) if transpose else (in_f, out_f)
     assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16, True) == "ddsc_kernel"
+    assert native.matmul_kernel_form(tokens, n, k, nnz, transpose, BF16).endswith(", lines ahead") == (out_f == 2016)
     if transpose:
         assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16, False) != "ddsc_kernel"
     np.random.seed(nnz)

@@ -10,18 +10,18 @@ from tests.test_gpu_row_gradient import _layer
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tokens,out_f,in_f,counts", [
-    (13007, 992, 1056, [24]),            # bands of 8 rows at most, a rectangle more in each; odd numbers of rows and of columns
-    (13007, 992, 1504, [47]),            # every block: twice the bands, the last of three rows
-    (13007, 1056, 1152, [27, 35, 19]),   # a band more, rows of different lengths
-    (13007, 2112, 992, [18]),            # two more bands of an even number of rows
-    (13007, 2112, 1504, [15]),           # bands of 16 rows at most
-    (13007, 1504, 1056, [33, 1, 0]),     # rows are dealt to the bands by their blocks
+@pytest.mark.parametrize("tokens,out_f,in_f,counts,partition", [
+    (13007, 992, 1056, [24], "4 even bands of 8 rows x 4 rectangles"),            # a rectangle more in each band; odd numbers of rows and of columns
+    (13007, 992, 1504, [47], "8 even bands of 8 rows x 3 rectangles"),            # every block: twice the bands, the last of three rows
+    (13007, 1056, 1152, [27, 35, 19], "6 even bands of 8 rows x 3 rectangles"),   # a band more, rows of different lengths
+    (13007, 2112, 992, [18], "11 even bands of 8 rows x 2 rectangles"),           # two more bands of an even number of rows
+    (13007, 2112, 1504, [15], "6 even bands of 16 rows x 3 rectangles"),          # bands of 16 rows at most
+    (13007, 1504, 1056, [33, 1, 0], "6 bands of 8 rows x 3 rectangles"),          # not even: rows are dealt to the bands by their blocks
 ])
-def test_even_partitions(cuda, tokens, out_f, in_f, counts):
+def test_even_partitions(cuda, tokens, out_f, in_f, counts, partition):
     dtype = torch.bfloat16
     m = _layer(out_f, in_f, counts, dtype, cuda, 5)
-    assert native.matmul_back_kernel_name(tokens, out_f, in_f, m.cols_a.shape[0], dtype).startswith("sdd_bf16_kernel")
+    assert native.matmul_back_kernel_form(tokens, out_f, in_f, m.cols_a.shape[0], dtype).startswith("sdd_bf16_kernel + sdd_reduce_kernel, " + partition)
     print(tokens, out_f, in_f, counts, flush=True)
     g = torch.Generator().manual_seed(tokens)
     x, dy = (torch.randn((tokens, f), generator=g).to(dtype) for f in (in_f, out_f))
