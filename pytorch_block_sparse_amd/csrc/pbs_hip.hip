@@ -799,8 +799,11 @@ static SddPlan plan_small(long long M, int N, int K, int nnz) {
 }
 // Operands beyond 52 MB: more rectangles than there have to be where the fullest would hold more blocks than the accumulators.  It takes two passes over its tokens then, and the
 // launch waits for it: 77 blocks take 1.4 times as long as 66.  The fullest one: the rows of the largest band, the columns (dealt in pairs by their blocks)
-// of the largest rectangle, and 1.6 times the deviation of a band's blocks.  Fitted to 34 problems of 90 MB and more in 16 partitions each, within 6 % on average.
-// Of 50 others 11 are partitioned in another way than by rectangle_us, 1.20 to 1.42 times as fast, one with Zipf rows 5 % slower.
+// of the largest rectangle, and 1.6 times the deviation of a band's blocks.  Fitted to 34 problems of 90 MB and more in 16 partitions each, within 6 % on average; the ratio of two
+// partitions of a problem, where the blocks of the fullest rectangle are known, within 5 % for 270 of 52 to 260 MB.
+// Of 600 problems of 52 MB and more that it partitions in another way than rectangle_us (one in six), the 300 without structure are 1.23 times as fast, 20 of them slower (down to
+// 0.85: what is fullest is up to chance), and the 300 with Zipf rows 1.24 times, 20 slower (0.81).  Taken only where the fullest rectangle is likelier to take two passes (1, 0 and -2
+// deviations instead of 1.6 for the partition that is left) 13, 5 and 0 of the 300 are slower, but the others gain 1.22, 1.21 and 1.15.
 // us: 15343 tokens 1760 -> 2784 density 0.71 249 -> 166, 13000 tokens 2304 -> 2752 density 0.3 140 -> 96, 12000 tokens 3072 -> 3072 density 0.3 153 -> 119,
 // 16384 tokens 2048 -> 2048 density 0.6 171 -> 127; 4096 -> 4096 at density 0.25 and 0.5 as before.
 static double partition_us(const SddPlan& p, int N, int K, int nnz) {
@@ -1022,6 +1025,10 @@ static int launch_rectangles(const BackArgs& b, const BackPlan& plan, void* work
     a.nnz = b.nnz;
     a.rows = p.rows;
     a.even = p.even;
+    // (a column unit more than the others in the largest rectangle, and a block for how they are dealt)
+    const double units = (b.K / 32 + 1) / 2, share = std::ceil(units / p.tiles_c) / units, mean = (double)b.nnz / ((double)p.tiles_r * p.tiles_c);
+    const double band_room = (std::ceil(mean / SddBf16Cfg<16>::QMAX) * SddBf16Cfg<16>::QMAX - 1.0) / share;
+    a.band_room = band_room < 2147483647.0 ? (int)band_room : 2147483647;
     a.tiles_r = p.tiles_r;
     a.tiles_c = p.tiles_c;
     a.nsplit = p.nsplit;

@@ -18,6 +18,7 @@ struct SddArgs {
     int M, N, K, nnz;
     int rows;                // block rows of a rectangle, 16 or 8
     int even;                // whether the rows are spread evenly over the bands
+    int band_room;           // then: blocks of a band that its rectangles hold in as many passes as the average one takes
     int tiles_r, tiles_c, nsplit;
     int tokens_per_split;    // multiple of TC
 };
@@ -25,15 +26,25 @@ struct SddArgs {
 // Which block rows of W form row band `band` of rectangles (SR places; -1 = no row).  Normally they are
 // rows SR*band .. SR*band + SR - 1, or (`even`) as many consecutive ones as in the other bands.  When the per-row block counts are very uneven (largest > 2x the
 // mean) the rows are ranked by count and dealt to the bands in serpentine order, so that all
-// rectangles hold about the same number of blocks.  Every workgroup derives its own band from the
+// rectangles hold about the same number of blocks.  So they are in an even partition, which is there for rectangles that take one pass less over their tokens, when
+// the fullest band has more than `band_room` blocks, with which its rectangles take a pass more than the average one: where long rows
+// are full the largest is below twice the mean and bands as uneven as they get.  (300 problems with Zipf rows in even partitions: without it 1.12 times as fast as in as few rectangles as
+// possible, 88 of them slower, down to 0.73; with it 1.24 times, 20 slower, down to 0.81.  2848 -> 2304 density 0.63, 8606 tokens 199 -> 124 us.  Without structure one in a hundred is dealt: level.)
+// Every workgroup derives its own band from the
 // row pointer array (a few microseconds at most; above SDD_BALANCE_MAX_ROWS rows the natural order
 // is kept).  Called by all threads of the workgroup; `scratch` is LDS for nblk_r ints.  Returns
 // whether the row pointers were scanned; then s_ptr_copy (nblk_r + 1 ints of LDS) holds them.
 constexpr int SDD_BALANCE_MAX_ROWS = 1024;
 static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__ ptr, int nnz, int nblk_r, int tiles_r, int band,
-                                                     int SR, bool even, int* s_rowid, int* scratch, int tid, int nthreads,
+                                                     int SR, bool even, int band_room, int* s_rowid, int* scratch, int tid, int nthreads,
                                                      int* s_ptr_copy) {
     bool skewed = false;
+    const int pairs = (nblk_r + 1) / 2;
+    const float per_band = __builtin_amdgcn_rcpf((float)tiles_r);
+    // (even bands in whole pairs of rows: 128 bytes of G.  Up to 512 pairs and as many bands the quotient is that of the integers)
+    auto first_row = [&](int b) {
+        return !even ? b * SR : 2 * (nblk_r <= SDD_BALANCE_MAX_ROWS ? (int)(((float)(pairs * b) + 0.5f) * per_band) : (int)((long long)pairs * b / tiles_r));
+    };
     const bool scanned = nblk_r <= SDD_BALANCE_MAX_ROWS && tiles_r >= 2;
     if (scanned) {
         for (int r = tid; r < nblk_r; r += nthreads) {
@@ -44,7 +55,13 @@ static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__
         }
         __syncthreads();
         // (every wave for itself: as atomics on two words the lanes of a wave take turns, 10500 cycles for 128 rows instead of 2300)
-        int most = 0, sum = 0;
+        int most = 0, sum = 0, fullest = 0;
+        if (even)
+            for (int b = tid & 63; b < tiles_r; b += 64) {
+                const int hi = first_row(b + 1);
+                const int n = s_ptr_copy[hi < nblk_r ? hi : nblk_r] - s_ptr_copy[first_row(b)];
+                fullest = n > fullest ? n : fullest;
+            }
         for (int r = tid & 63; r < nblk_r; r += 64) {
             const int n = scratch[r];
             most = n > most ? n : most;
@@ -52,16 +69,15 @@ static __device__ __forceinline__ bool sdd_band_rows(const int32_t* __restrict__
         }
 #pragma unroll
         for (int d = 32; d > 0; d >>= 1) {
-            const int m = __shfl_xor(most, d);
+            const int m = __shfl_xor(most, d), f = __shfl_xor(fullest, d);
             most = m > most ? m : most;
+            fullest = f > fullest ? f : fullest;
             sum += __shfl_xor(sum, d);
         }
-        skewed = (long long)most * nblk_r > 2ll * sum;
+        skewed = (long long)most * nblk_r > 2ll * sum || (even && fullest > band_room);
     }
     if (tid < SR) {
-        // (even bands in whole pairs of rows: 128 bytes of G)
-        const int pairs = (nblk_r + 1) / 2, lo = even ? 2 * (int)((long long)pairs * band / tiles_r) : band * SR;
-        const int hi = even ? 2 * (int)((long long)pairs * (band + 1) / tiles_r) : lo + SR, r = lo + tid;
+        const int lo = first_row(band), hi = even ? first_row(band + 1) : lo + SR, r = lo + tid;
         s_rowid[tid] = (!skewed && r < hi && r < nblk_r) ? r : -1;
     }
     __syncthreads();

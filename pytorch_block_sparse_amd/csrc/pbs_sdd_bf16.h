@@ -84,7 +84,7 @@ static __device__ __forceinline__ void sdd_bf16_prologue(const SddArgs& a, int t
     int* s_ug = s_cnt + UMAX;                   // [UMAX] rectangle * 8 + place of each column unit
     int* s_scan = s_ug + UMAX;                  // [SDD_BALANCE_MAX_ROWS + 2] scratch of the row scan
     int* s_ptr_copy = s_scan + SDD_BALANCE_MAX_ROWS + 2;   // [SDD_BALANCE_MAX_ROWS + 1] row pointers, if scanned
-    const bool have_ptr = sdd_band_rows(a.ptr, a.nnz, nblk_r, a.tiles_r, band, SR, a.even != 0, s_rowid, s_scan, tid, NT, s_ptr_copy);
+    const bool have_ptr = sdd_band_rows(a.ptr, a.nnz, nblk_r, a.tiles_r, band, SR, a.even != 0, a.band_room, s_rowid, s_scan, tid, NT, s_ptr_copy);
     __syncthreads();
     if (tid < SR) {
         const int r = s_rowid[tid];

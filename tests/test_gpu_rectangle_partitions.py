@@ -17,6 +17,10 @@ pytestmark = pytest.mark.gpu
     (13007, 2112, 992, [18], "11 even bands of 8 rows x 2 rectangles"),           # two more bands of an even number of rows
     (13007, 2112, 1504, [15], "6 even bands of 16 rows x 3 rectangles"),          # bands of 16 rows at most
     (13007, 1504, 1056, [33, 1, 0], "6 bands of 8 rows x 3 rectangles"),          # not even: rows are dealt to the bands by their blocks
+    (13007, 2112, 1056, [31] * 16 + [8] * 50, "6 even bands of 16 rows x 3 rectangles"),   # dealt: the longest rows have more than twice the mean
+    # dealt: none has, but consecutive rows would make bands of 176 to 264 and 40 blocks where three rectangles have room for 216 (of 47 columns 16 in the largest)
+    (13007, 1056, 1504, [44] * 16 + [8] * 17, "6 even bands of 8 rows x 3 rectangles"),
+    (13007, 2112, 1056, [22] * 33 + [5] * 33, "6 even bands of 16 rows x 3 rectangles"),
 ])
 def test_even_partitions(cuda, tokens, out_f, in_f, counts, partition):
     dtype = torch.bfloat16
