@@ -904,26 +904,28 @@ struct BackPlan {
     int per_unit; // blocks of a unit, at most
     bool split;   // fp32 in parts
     int passes, chunks_per_slice;
-    SddPlan rect;
+    SddPlan rect; // of rectangles only
     int partials;            // sums of this many slices in the workspace, or none
     size_t partial_bytes;
 };
 static BackPlan plan_back_anew(int dtype, long long M, int N, int K, int nnz, bool lists, size_t workspace_limit) {
-    BackPlan p;
+    BackPlan p{};
     const RowChoice row = choose_row(dtype, M, N, K, nnz, lists, workspace_limit);
     p.slices = row.slices;
     p.per_unit = row.per_unit;
     p.split = row.split;
-    p.rect = plan_sdd(M, N, K, nnz);
-    // (the workspace of sixteen rows also where eight need less: what an entry point without one refuses does not follow the estimates)
-    const int tall = plan_rectangles(M, N, K, 16).nsplit;
-    int n = tall > p.rect.nsplit ? tall : p.rect.nsplit;
+    int n = 0;
     if (p.slices > 0) {
         const long long chunks = (M + ROW_TC - 1) / ROW_TC, shares = (long long)row.slices * row.passes;
         p.chunks_per_slice = (int)((chunks + shares - 1) / shares);
         const long long filled = (chunks + p.chunks_per_slice - 1) / p.chunks_per_slice;   // slices with tokens
         p.slices = n = (int)(filled < row.slices ? filled : row.slices);
         p.passes = (int)((filled + n - 1) / n);   // (the last launch may have slices without tokens, which add nothing)
+    } else {
+        p.rect = plan_sdd(M, N, K, nnz);
+        // (the workspace of sixteen rows also where eight need less: what an entry point without one refuses does not follow the estimates)
+        const int tall = plan_rectangles(M, N, K, 16).nsplit;
+        n = tall > p.rect.nsplit ? tall : p.rect.nsplit;
     }
     p.partials = n > 1 ? n : 0;
     return p;
