@@ -114,8 +114,8 @@ static inline int column_groups(int n) { return (n / 32 + DC_NB - 1) / DC_NB; }
 static inline size_t column_table_bytes(int n) { return ((size_t)column_groups(n) * DC_NB * sizeof(int) + 63) / 64 * 64; }
 static inline size_t column_plan_bytes(int n, int k) {
     // k-pairs, and the lists of a group of 16 columns must fit the kernel's LDS area (16 * k / 32 items)
-    // (an odd number of them where no panel kernel holds the whole contraction, and not next to the largest k: the size of the plan of 4064 features stays as it was)
-    if (k % 64 && (k <= PANEL_MAX_K || DC_NB * (k / 32 + 1) >= DC_ITEMS_LDS)) return 0;
+    // (an odd number of k-blocks where no panel kernel holds the whole contraction)
+    if (k % 64 && k <= PANEL_MAX_K) return 0;
     if (DC_NB * (k / 32) > DC_ITEMS_LDS) return 0;
     return column_table_bytes(n) + ((size_t)column_groups(n) * ddsc_plan_group_ints(k / 32) + DC_SEQ_INTS) * sizeof(int);
 }

@@ -103,8 +103,7 @@ def test_plan_argument_checks(lib):
     # contraction sizes that are not a multiple of 64 have no k-pair plans
     assert lib.pbs_blocksparse_matmul_plan_bytes(64, 96) == 4 * (1 * (3 + 2) * 16 * 4 + 64)
     # nor does the column kernel serve contractions whose lists would not fit its LDS area
-    assert (lib.pbs_blocksparse_matmul_plan_bytes(512, 8192) - lib.pbs_blocksparse_matmul_plan_bytes(512, 8192 - 32)
-            < lib.pbs_blocksparse_matmul_plan_bytes(512, 4096) - lib.pbs_blocksparse_matmul_plan_bytes(512, 4096 - 32))
+    assert lib.pbs_blocksparse_matmul_plan_bytes(512, 4096 + 64) < lib.pbs_blocksparse_matmul_plan_bytes(512, 4096)
     assert lib.pbs_blocksparse_matmul_plan_bytes(100, 64) == 0
     f = lib.pbs_blocksparse_matmul_plan
     assert f(p, p, 64, 100, 1, p, 1 << 20, null) == ERR_SHAPE

@@ -49,6 +49,8 @@ def test_every_tile_of_every_group(cuda, monkeypatch, kernel, out_f, in_f, token
     (1056, 1120, 300, 35 * 33),      # every block
     (1120, 1056, 128 * 129 + 77, 60),
     (2080, 4000, 128 * 70, 2500),    # lists of more than 64 items
+    (1056, 4064, 128 * 70 + 1, 127 * 33),   # every block, in the longest lists: 2032 items of a group in the room for 2048
+    (4064, 2080, 300, 2500),
 ])
 def test_odd_numbers_of_k_blocks(cuda, monkeypatch, out_f, in_f, tokens, nnz):
     """The last pair of k-blocks is one k-block: its second half is never multiplied, whatever lies behind the row (here NaN: the next row's start)."""

@@ -8,13 +8,15 @@ import torch
 from pytorch_block_sparse_amd import BlockSparseMatrix, native
 
 
-@pytest.mark.parametrize("n, k", [(32, 32), (64, 96), (4096, 4096), (3072, 768), (512, 8192), (1504, 992)])
+@pytest.mark.parametrize("n, k", [(32, 32), (64, 96), (4096, 4096), (3072, 768), (512, 8192), (1504, 992), (992, 1024),
+                                  (1504, 1056), (2080, 4000), (512, 4064), (512, 4128)])
 def test_size_of_the_parts(n, k):
     lib = native.load()
     cols, kb = n // 32, k // 32
     lists = (cols + 7) // 8 * (8 * 16 + kb * 8 * 8)
     wide = 0 if kb % 2 else (cols + 15) // 16 * (kb // 2 + 2) * 256 + 1024
-    column = 0 if kb % 2 or kb > 128 else (cols + 15) // 16 * (64 + (64 + kb // 2 + 32 * kb) * 4) + 16384 * 4
+    # (an odd number of k-blocks from 1056 features on; the lists of 16 columns of up to 128 blocks)
+    column = 0 if kb > 128 or (kb % 2 and k <= 1024) else (cols + 15) // 16 * (64 + (64 + (kb + 1) // 2 + 32 * kb) * 4) + 16384 * 4
     assert lib.pbs_blocksparse_matmul_plan_part_bytes(n, k) == lists + wide + column <= lib.pbs_blocksparse_matmul_plan_bytes(n, k)
     assert lib.pbs_blocksparse_matmul_plan_part_bytes(n, k + 1) == 0
     p = ctypes.c_void_p(0x1000)
