@@ -238,11 +238,12 @@ static bool column_kernel_fits(long long M, int n, int k, int nnz) {
 }
 
 // Whether its copies ask for lines ahead (pbs_ddsc.h): a dense operand of 100 MB and more is taken to be in memory (of 60 products with operands of 12 to 98 MB, three in
-// turn, it makes 6 to 9 one to seven hundredths faster and the others up to 9 slower), with four groups of columns to share the asking (with three 1.00, two of nine slower) and columns of up to 32 blocks (with 33
-// to 48 1.01 times as fast, 8 of 35 slower, down to 0.95).  250 products drawn from those: even ones 1.05 times as fast, with an odd number of k-blocks 1.08, two slower (0.965, 0.975); with
-// Zipf rows 260 others 1.00 (0.91 to 1.09).
+// turn, it makes 6 to 9 one to seven hundredths faster and the others up to 9 slower), with four groups of columns to share the asking (with three 0.96 to 1.03, of 76 products
+// of up to 48 blocks a column 35 at least 2 % slower) and columns of up to 40 blocks, 48 where every other row begins in the middle of a line (even products of 33 to 40 blocks a column 1.034
+// times as fast, with an odd number of k-blocks 1.055, and of 41 to 48 1.05, where an even number is level; of 49 to 64 8 of 38 and 6 of 32 are slower).  250 products of up to 32 blocks a
+// column: even ones 1.05 times as fast, with an odd number of k-blocks 1.08, two slower (0.965, 0.975); with Zipf rows 260 others 1.00 (0.91 to 1.09).
 static bool touches(long long M, int n, int k, int nnz) {
-    return 2.0 * (double)M * k >= 100e6 && column_groups(n) >= 4 && nnz <= 32ll * (n / 32);
+    return 2.0 * (double)M * k >= 100e6 && column_groups(n) >= 4 && nnz <= (k % 64 ? 48ll : 40ll) * (n / 32);
 }
 // FM: the blocks are given in fragment order (the forward product's copy) instead of [n][k] as stored
 template <bool FM>

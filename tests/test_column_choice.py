@@ -25,3 +25,16 @@ BF16 = torch.bfloat16
 def test_faster_kernel(n, k, tokens, density, transpose, kernel):
     nnz = int(density * (n // 32) * (k // 32))
     assert native.matmul_kernel_name(tokens, n, k, nnz, transpose, BF16) == kernel
+
+
+@pytest.mark.parametrize("n, k, tokens, per_column, ahead", [
+    (4096, 3840, 15649, 35, True),     # 1.07 times as fast
+    (3808, 4000, 12795, 47, True),     # 1.05: an odd number of k-blocks
+    (3552, 3648, 15579, 44, False),    # level
+    (3808, 4000, 12795, 52, False),
+    (1376, 3072, 16158, 38, False),    # three groups of columns
+    (4096, 3840, 12800, 35, False),    # 98 MB
+])
+def test_lines_asked_for_ahead(n, k, tokens, per_column, ahead):
+    form = native.matmul_kernel_form(tokens, n, k, per_column * (n // 32), False, BF16)
+    assert form == ("ddsc_kernel, lines ahead" if ahead else "ddsc_kernel")
