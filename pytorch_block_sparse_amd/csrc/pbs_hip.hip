@@ -377,12 +377,12 @@ static int launch_stream_shape(const DdsArgs& g, hipStream_t stream) {
 
 // fp32 with enough token tiles and short columns: whether walk_kernel takes it from stream_kernel.  The estimate: launch, the blocks of the fullest
 // CU, a wave's own chain, memory; fitted to 222 products (256 to 4096 features, 600 to 16384 tokens, densities 0.05 to 0.75) within 8 % on average.  It has to be a
-// ninth below stream_kernel's, from 10 us on, where that would take tiles of 64 tokens (against its tiles of 32 it is 0.92 to 1.08 times as fast).
-// How uneven columns are is not known here, and a wave multiplies a column alone: so a contraction has at most 32 blocks, and a full column of them takes at most 0.4 of the launch (a
-// wave's block takes half a microsecond).  Of 280 products drawn from those that are taken, a quarter with uneven columns, one is slower (0.98), the others 1.12 times as fast on average.  With a
-// full column of any length, as long as the launch, 21 of 174 products with Zipf rows were slower, down to 0.64 (922 tokens 672 -> 2656 density 0.14 12.4 -> 19.5 us, 5163 tokens 3488 -> 3200 density
-// 0.056 139 -> 182), and even ones longer than 1024 features gained 4 % on average.
-constexpr double WALK_MARGIN = 0.89, WALK_LEAST = 10.0, WALK_BLOCK = 0.5, WALK_FULL = 0.4;
+// fourteenth below stream_kernel's, from 10 us on, where that would take tiles of 64 tokens (against its tiles of 32 it is 0.92 to 1.08 times as fast).
+// How uneven columns are is not known here, and a wave multiplies a column alone: so a contraction has at most 32 blocks, and a full column of them takes at most 0.65 of the launch (a
+// wave's block takes half a microsecond).  Of products drawn from those that are taken 300 with even columns are 1.14 times as fast on average, none slower, and 250 with Zipf rows 1.11 times, four
+// slower (0.93).  With full columns of 0.65 to 1 of the launch 8 of 15 with Zipf rows were slower, down to 0.73 (922 tokens 672 -> 2656 density 0.14 11.7 -> 18.0 us), and with contractions of 1056 to 2048 features
+// 11 of 49 (4893 tokens 1184 -> 3456 density 0.19 76 -> 104), where even ones would gain 1.08.
+constexpr double WALK_MARGIN = 0.93, WALK_LEAST = 10.0, WALK_BLOCK = 0.5, WALK_FULL = 0.65;
 static bool choose_walk(long long M, int n, int k, int nnz) {
     return answer<bool>(Sizes{M, n, k, nnz, 0}, [&] {
         const StreamChoice stream = choose_stream(4, M, n, k, nnz);

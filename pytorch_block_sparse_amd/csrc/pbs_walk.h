@@ -6,8 +6,8 @@
 //
 // What bounds it: the texture path (8 KB per block, 0.87 of the cycles of its matrix instructions) and memory.  Tiles of 64 tokens copy 12 KB for twice the
 // products, but 12 KB and 162 registers a wave leave three waves to a SIMD: 2 to 20 % slower; of 48 tokens between the two, of 16 5 to 15 % slower, of 128 spilled.
-// Measured, us, stream_kernel -> here: 672 -> 3200 density 0.21, 3133 tokens 41.1 -> 34.7; 352 -> 2080 density 0.15, 8586 tokens 36.2 -> 31.1; 704 -> 1856 density 0.09, 8054 tokens
-// 33.3 -> 29.6; 928 -> 3808 density 0.085, 9066 tokens 80.5 -> 74.1; input gradient of 2240 -> 704 density 0.11, 8819 tokens 47.8 -> 41.2.
+// Measured, us, stream_kernel -> here: 672 -> 3200 density 0.21, 3133 tokens 39.1 -> 31.1; 352 -> 2080 density 0.15, 8586 tokens 33.8 -> 29.3; 704 -> 1856 density 0.09, 8054 tokens
+// 32.1 -> 27.9; 992 -> 1984 density 0.25 with Zipf rows, 4001 tokens 48.8 -> 43.0; 448 -> 640 density 0.46, 14976 tokens 44.0 -> 39.7.
 #pragma once
 #include <type_traits>
 
