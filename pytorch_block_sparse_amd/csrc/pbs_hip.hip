@@ -637,12 +637,13 @@ static ProductChoice choose_product_anew(long long M, int n, int k, int nnz, int
     const double ts = choose_stream(esz, M, n, k, nnz).us;
     const double tw = wide ? wide_us(M, n, k, nnz) : 1e300;
     // Outside column_kernel_fits, and inside where panel_first has put a panel kernel before it, from 2048 tokens and 1024 features on, where its estimate is below those of
-    // the stream and the panel kernels: by a fourteenth, against panel_chunk_kernel by a seventh in the input gradient and by a fifth in forward products of up to 2048
-    // features half of whose blocks are there (that kernel's estimate, with its tenth, is up to 15 % long in these).  Not in place of the wide kernel, whose estimate is from before its workgroups were
+    // the stream and the panel kernels: by a fourteenth, against panel_chunk_kernel by a seventh in input gradients with contractions of up to 1500 features, and by a fifth in forward products of
+    // up to 1350 half of whose blocks are there (that kernel's estimate, with its tenth, is up to 15 % long in these).  Not in place of the wide kernel, whose estimate is from before its workgroups were
     // dealt within the XCDs' CUs: three such products were slower, 0.87 to 0.92.
-    // Of 680 products drawn from those that it takes so (half with Zipf rows, of which the host knows nothing) 12 are slower, ten of them with Zipf rows, down to 0.88, the others 1.24 times as fast
-    // (13394 tokens 2720 -> 1728 density 0.32 118 -> 69 us, 5332 tokens 3616 -> 1888 density 0.32 77 -> 49, 3983 tokens 3648 -> 1568 density 0.33 35 -> 29).  Of 170 products that a fourteenth against all kernels
-    // takes besides, 23 are slower, down to 0.88, 1.07 times as fast on average; of 120 that a seventh against all leaves out besides, 12, 1.14 times.
+    // Of 200 products drawn from those that a seventh, a fifth of up to 2048 features, and the wide kernel's estimate wherever it is the smallest had left to the others, 39 against
+    // stream_kernel are 1.23 times as fast, none slower, against panel_chunk_kernel 100 even ones 1.08 times (four slower, 0.95) and 61 with Zipf rows, of which the host knows nothing, 1.08 times (nine
+    // slower, down to 0.87); 200 that the seventh and the fifth leave out now would be 0.99 times as fast (13394 tokens 2720 -> 1728 density 0.32 114 -> 70 us, 4855 tokens 3936 -> 2016
+    // density 0.3 input gradient 52 -> 49, 3983 tokens 3648 -> 1568 density 0.33 35 -> 29).
     if (runs && M >= 2048 && k >= 1024) {
         // (an operand of more than 40 MB goes through memory again for the sets of columns that an XCD has of stream_kernel's, which its estimate does not count: 11386 tokens 3808 -> 2720
         // with 7 blocks a column 68 us where it has 48.  So up to 16 % are added to it here: of 90 drawn layers 13 products more are the column kernel's, 1.23 times as fast, none slower: 15003
@@ -650,9 +651,9 @@ static ProductChoice choose_product_anew(long long M, int n, int k, int nnz, int
         // 1.13 times as fast.)
         const double mb = 2e-6 * (double)M * k, far = ts + (mb > 40.0 ? std::fmin(2.5e-4 * (mb - 40.0) * n, 0.16 * ts) : 0.0);
         const double least = tp < far ? tp : far;
-        const bool dense = k <= 2048 && 2ll * nnz >= (long long)(n / 32) * (k / 32);
-        const double below = tp >= far ? 0.93 : (!transpose ? 0.86 : (dense ? 0.80 : 0.93));
-        if (least < tw && column_anywhere_us(M, n, k, nnz, transpose != 0) < below * least) return {PART_COLUMN, NO_PANEL};
+        const bool wide_first = tw < ts && tw < tp, dense = 2ll * nnz >= (long long)(n / 32) * (k / 32);
+        const double below = tp >= far ? 0.93 : (!transpose ? (k <= 1500 ? 0.86 : 0.93) : (dense && k <= 1350 ? 0.80 : 0.93));
+        if (!wide_first && column_anywhere_us(M, n, k, nnz, transpose != 0) < below * least) return {PART_COLUMN, NO_PANEL};
     }
     if (column && M >= 8192) return {PART_LIST, panel};
     if (tp < ts && tp < tw && tp < tc) return {PART_LIST, panel};

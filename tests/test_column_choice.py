@@ -14,9 +14,13 @@ BF16 = torch.bfloat16
     # 0.93 to 0.96: forward products of short contractions with half of the blocks and more
     (2496, 1248, 5380, 0.712, True, "panel_chunk_kernel"),
     (928, 1184, 14262, 0.737, True, "panel_chunk_kernel"),
-    # 0.92 to 0.95: input gradients at nearly level estimates
-    (3936, 2016, 4855, 0.297, False, "panel_chunk_kernel"),
+    # 0.94: input gradients of short contractions at nearly level estimates
     (1408, 1056, 12675, 0.369, False, "panel_chunk_kernel"),
+    # of longer ones 1.07 times as fast in the column kernel
+    (3936, 2016, 4855, 0.297, False, "ddsc_kernel"),
+    # 1.1 to 1.25: the wide kernel's estimate is below the column kernel's bound, but not below the stream kernel's
+    (1760, 3232, 10051, 0.19, False, "ddsc_kernel"),
+    (2144, 2720, 16379, 0.13, False, "ddsc_kernel"),
     # 1.1 to 1.4 times as fast
     (1728, 2720, 13394, 0.32, True, "ddsc_kernel"),
     (2016, 3936, 15003, 0.0912, True, "ddsc_kernel"),
