@@ -335,8 +335,8 @@ __global__ __launch_bounds__(DC_NB * 64) void ddsc_kernel(DdscArgs g) {
     // so a panel is fetched into two L2s and the blocks an XCD keeps re-reading (once per token tile) are 4 MB
     // at 4096 x 4096, which its L2 holds.  All groups per XCD (a panel in one L2, 8 MB of blocks) is 1.2 % slower
     // at both densities, a quarter of the groups per XCD 6 % slower at density 0.25.
-    // us, whole streams to an XCD -> here (16384 tokens if no other number): 3584 -> 3584 density 0.25 230 -> 175, 9000 tokens 158 -> 110; 3072 -> 1536 input gradient
-    // 165 -> 110; 2304 -> 2752, 13000 tokens 127 -> 81; 2560 -> 2560 124 -> 109; layers of 512, 1024, 2048 and 4096 features as before.
+    // us, whole streams to an XCD -> here: 9000 tokens 3584 -> 3584 density 0.25 135 -> 79; 13000 tokens 2304 -> 2752 density 0.3 104 -> 81; 16384 tokens 2560 -> 2560 density 0.25 106 -> 85, 3072 -> 1536
+    // input gradient at densities 0.25 and 0.5 100 -> 70 and 140 -> 99.  254 drawn products whose whole streams are more workgroups than an XCD has CUs are 1.16 times as fast, 200 others level.
     int ng, p;
     if (!stream_and_group(blockIdx.x, g.wg_per_group, g.stream_step, g.n_groups, g.n_groups & 1 ? 1 : 2, p, ng)) return;
     const int ntiles = (g.m_tiles - p + g.wg_per_group - 1) / g.wg_per_group;   // token tiles p, p + P, ...

@@ -898,6 +898,7 @@ static RowChoice choose_row(int dtype, long long M, int N, int K, int nnz, bool 
                 for (int p = one_list ? ROW_NB : 2; p <= ROW_NB; ++p) consider(ROW_SPLIT, p);
         }
     }
+    // (of a density below 0.1, and up to 52 MB, the partition is that of plan_small)
     if (rectangles && fits && (large ? 0.9 : 1.0) * rectangle_us(plan_small(M, N, K, nnz), nnz) < best_us) best.slices = 0;
     return best;
 }

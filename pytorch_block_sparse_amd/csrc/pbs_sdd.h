@@ -29,7 +29,7 @@ struct SddArgs {
 // rectangles hold about the same number of blocks.  So they are in an even partition, which is there for rectangles that take one pass less over their tokens, when
 // the fullest band has more than `band_room` blocks, with which its rectangles take a pass more than the average one: where long rows
 // are full the largest is below twice the mean and bands as uneven as they get.  (300 problems with Zipf rows in even partitions: without it 1.12 times as fast as in as few rectangles as
-// possible, 88 of them slower, down to 0.73; with it 1.24 times, 20 slower, down to 0.81.  2848 -> 2304 density 0.63, 8606 tokens 199 -> 124 us.  Without structure one in a hundred is dealt: level.)
+// possible, 88 of them slower, down to 0.73; with it 1.24 times, 20 slower, down to 0.81.  2304 -> 2848 density 0.63, 8606 tokens 199 -> 124 us.  Without structure one in a hundred is dealt: level.)
 // Every workgroup derives its own band from the
 // row pointer array (a few microseconds at most; above SDD_BALANCE_MAX_ROWS rows the natural order
 // is kept).  Called by all threads of the workgroup; `scratch` is LDS for nblk_r ints.  Returns
