@@ -7,8 +7,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
-#include <string>
 #include <tuple>
 
 #include "pbs_common.h"
@@ -1531,8 +1531,8 @@ const char* pbs_blocksparse_matmul_kernel_name(int64_t tokens, int n, int k, int
 
 const char* pbs_blocksparse_matmul_kernel_form(int64_t tokens, int n, int k, int nnz, int transpose, int dtype, int with_workspace) {
     static thread_local char text[96];
-    const std::string name = pbs_blocksparse_matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace);
-    std::snprintf(text, sizeof text, "%s%s", name.c_str(), name == "ddsc_kernel" && touches(tokens, n, k, nnz) ? ", lines ahead" : "");
+    const char* name = pbs_blocksparse_matmul_kernel_name(tokens, n, k, nnz, transpose, dtype, with_workspace);
+    std::snprintf(text, sizeof text, "%s%s", name, !std::strcmp(name, "ddsc_kernel") && touches(tokens, n, k, nnz) ? ", lines ahead" : "");
     return text;
 }
 
